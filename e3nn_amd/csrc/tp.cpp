@@ -50,6 +50,7 @@ struct SubKernel {
   std::unique_ptr<SubKernel> fused_dw;
   hipFunction_t fn_fused_dw[kMaxDevices] = {nullptr};
   hipFunction_t fn_fused_dw_x2[kMaxDevices] = {nullptr};  // ... and the gradient of the second input
+  hipFunction_t fn_rowgrad[kMaxDevices] = {nullptr}, fn_rowgrad_x2[kMaxDevices] = {nullptr}, fn_rowgrad_reduce[kMaxDevices] = {nullptr};
 };
 
 struct e3x_plan {
@@ -73,6 +74,8 @@ struct e3x_plan {
   // uvu with the spherical harmonics 0 .. lmax as second input: variants of the kernels of `subs` that form the
   // harmonics from the edge vectors themselves, per (normalize, normalization), built on first use
   std::map<int, std::vector<std::unique_ptr<SubKernel>>> sh_subs;
+  // uvu: the backward pass of a message step grouped by destination (see rowgrad_row_bytes), built on first use
+  std::unique_ptr<SubKernel> rowgrad;
   // uvu, bf16 storage: the message kernel (gather + product + scatter) with the contraction on the matrix cores,
   // when the instruction set fits it; the plain product keeps the kernels of `subs`
   std::unique_ptr<SubKernel> msg_mfma;
@@ -195,9 +198,10 @@ std::vector<std::vector<int>> split_uvu_paths(const e3x_plan& P, int acc_limit =
   return parts;
 }
 
-// extra_cfg: more constants for the generated namespace; tpl: the device template to specialise (default: uvu.inc)
+// extra_cfg: more constants for the generated namespace; tpl: the device template to specialise (default: uvu.inc);
+// fixed_upl: multiplicity indices per lane of a template that is written for one value
 int build_uvu_source(e3x_plan& P, SubKernel& K, std::string* src, bool bwd_only = false, const std::string* extra_cfg = nullptr,
-                     const char* tpl = nullptr) {
+                     const char* tpl = nullptr, int fixed_upl = 0) {
   int max_mul = 1;
   std::vector<char> used1(P.in1.size(), 0), usedo(P.out.size(), 0);
   long long unrolled = 0;
@@ -238,6 +242,7 @@ int build_uvu_source(e3x_plan& P, SubKernel& K, std::string* src, bool bwd_only 
     while (b < upl && (max_mul + b - 1) / b > 64) b *= 2;
     upl = env_int("E3X_UVU_BWD_UPL", b);
   }
+  if (fixed_upl) upl = fixed_upl;
   if (upl != 1 && upl != 2 && upl != 4) return fail(E3X_ERR_INVALID, "E3X_UVU_UPL must be 1, 2 or 4");
   for (size_t a = 0; a < P.in1.size(); ++a)
     if (used1[a] && P.in1[a].mul % upl) return fail(E3X_ERR_INVALID, "uvu kernel: multiplicity not divisible by UPL");
@@ -1021,6 +1026,57 @@ int load_uvu_fused_dw_function(e3x_plan* P, int dev) {
   return E3X_OK;
 }
 
+// The backward pass of a message step grouped by destination (templates/uvu_rowgrad.inc): fp32, per-edge weights, more
+// than 32 channels (a wavefront takes 64), the gradient row of a channel in registers beside two sets of edge operands
+// at two wavefronts per SIMD.  It moves three rows of the node features' width per edge (gather, scratch written, scratch
+// read) where the kernel on the transposed plan gathers one row of the messages' width: taken when the messages are
+// more than three times as wide.  Returns the scratch bytes per edge, 0 for plans it is not meant for.
+int64_t rowgrad_row_bytes(const e3x_plan* P) {
+  if (env_int("E3X_UVU_ROWGRAD", 1) == 0 || P->family != "uvu" || P->dtype != E3X_F32 || P->shared_weights || P->weight_numel == 0 ||
+      P->in2_dim < 1 || P->in2_dim > 32)
+    return 0;
+  int max_mul = 1, x1regs = 0, accregs = 0, wregs = 0;
+  std::vector<char> used1(P->in1.size(), 0), usedo(P->out.size(), 0);
+  for (const auto& p : P->paths) {
+    max_mul = std::max(max_mul, P->in1[p.in1].mul);
+    if (!used1[p.in1]) { used1[p.in1] = 1; x1regs += 2 * P->in1[p.in1].l + 1; }
+    if (!usedo[p.out]) { usedo[p.out] = 1; accregs += 2 * P->out[p.out].l + 1; }
+    if (p.has_w) wregs += P->in2[p.in2].mul;
+  }
+  const int chunks = (max_mul + 63) / 64;
+  if (max_mul <= 32 || chunks > 8 || accregs + 2 * (x1regs + wregs) + 2 * (int)P->in2_dim > 224) return 0;
+  const int64_t bytes = (int64_t)((x1regs + 3) / 4) * 4 * chunks * 64 * 4;
+  return P->out_dim * 4 > 3 * bytes ? bytes : 0;
+}
+
+int prepare_rowgrad(e3x_plan* P) {
+  std::lock_guard<std::mutex> lock(P->mu);
+  if (P->rowgrad) return E3X_OK;
+  std::unique_ptr<SubKernel> R(new SubKernel);
+  for (size_t i = 0; i < P->paths.size(); ++i) R->path_ids.push_back((int)i);
+  std::string src;
+  int rc;
+  if ((rc = build_uvu_source(*P, *R, &src, false, nullptr, e3x::kTplUvuRowgrad, 1))) return rc;
+  if ((rc = e3x::get_code_object("uvu_rowgrad", src, &R->key, &R->hsaco))) return rc;
+  P->rowgrad = std::move(R);
+  return E3X_OK;
+}
+
+int load_rowgrad_functions(e3x_plan* P, int dev) {
+  std::lock_guard<std::mutex> lock(P->mu);
+  SubKernel* R = P->rowgrad.get();
+  if (R->module[dev]) return E3X_OK;
+  hipModule_t mod = nullptr;
+  hipError_t err = hipModuleLoad(&mod, R->hsaco.c_str());
+  if (err != hipSuccess) return fail(E3X_ERR_HIP, "hipModuleLoad(" + R->hsaco + ") failed: " + hipGetErrorString(err));
+  if (hipModuleGetFunction(&R->fn_rowgrad[dev], mod, "e3x_uvu_rowgrad") != hipSuccess ||
+      hipModuleGetFunction(&R->fn_rowgrad_x2[dev], mod, "e3x_uvu_rowgrad_x2") != hipSuccess ||
+      hipModuleGetFunction(&R->fn_rowgrad_reduce[dev], mod, "e3x_uvu_rowgrad_reduce") != hipSuccess)
+    return fail(E3X_ERR_HIP, "kernels of e3x_uvu_rowgrad missing from " + R->hsaco);
+  R->module[dev] = mod;
+  return E3X_OK;
+}
+
 // ---- uvu message kernel with the spherical harmonics formed in the kernel -------------------------------------
 // lmax when irreps_in2 is 1x0e + 1x1o + ... + 1x(lmax)(parity (-1)^l) with 1 <= lmax <= 3, else -1
 int sh_lmax_of(const e3x_plan* P) {
@@ -1496,6 +1552,60 @@ extern "C" int e3x_tp_gather_scatter_grad_w(e3x_plan* P, const void* table, cons
       return fail(E3X_ERR_HIP, std::string("e3x_tp_gather_scatter_grad_w: launch failed: ") + hipGetErrorString(err));
     x2_accumulate = 1;
   }
+  return E3X_OK;
+}
+
+extern "C" int e3x_tp_plan_prepare_message_backward(e3x_plan* P) {
+  if (!P) return fail(E3X_ERR_INVALID, "e3x_tp_plan_prepare_message_backward: null plan");
+  if (!rowgrad_row_bytes(P)) return E3X_ERR_INVALID;  // (no message: callers ask to find out)
+  return prepare_rowgrad(P);
+}
+
+// scratch beyond this many bytes is not asked for: the caller then takes the kernels that need none
+constexpr int64_t kRowgradMaxScratch = 16LL << 30;
+
+extern "C" size_t e3x_tp_message_backward_workspace_bytes(const e3x_plan* P, int64_t E) {
+  const int64_t row = P && E > 0 ? rowgrad_row_bytes(P) : 0;
+  return row && E <= kRowgradMaxScratch / row ? (size_t)(E * row) : 0;
+}
+
+extern "C" int e3x_tp_message_backward(e3x_plan* P, const void* node_x, const void* edge_attr, const void* w, const void* grad_out,
+                                       const void* src, int idx_bits, const int32_t* rowptr, const int32_t* perm,
+                                       const int32_t* row_order, const int32_t* src_rows, const int32_t* rowptr_by_src,
+                                       const int32_t* perm_by_src, void* grad_x, void* grad_w, void* grad_x2, int64_t E,
+                                       int64_t num_src_nodes, int64_t num_out_nodes, void* workspace, size_t workspace_bytes,
+                                       void* stream) {
+  if (!P) return fail(E3X_ERR_INVALID, "e3x_tp_message_backward: null plan");
+  const int64_t scratch_row = rowgrad_row_bytes(P);
+  if (!scratch_row) return fail(E3X_ERR_INVALID, "e3x_tp_message_backward: the plan does not fit the kernel (see e3x_tp_plan_prepare_message_backward)");
+  if (idx_bits != 32 && idx_bits != 64) return fail(E3X_ERR_INVALID, "e3x_tp_message_backward: idx_bits must be 32 or 64");
+  if (E <= 0 || E >= (1LL << 31) || num_src_nodes <= 0 || num_out_nodes <= 0 || num_src_nodes >= (1LL << 31) || num_out_nodes >= (1LL << 31) - 8)
+    return fail(E3X_ERR_INVALID, "e3x_tp_message_backward: sizes must be in [1, 2^31)");
+  if (!node_x || !edge_attr || !w || !grad_out || !src || !rowptr || !rowptr_by_src || !grad_x || !grad_w || !workspace)
+    return fail(E3X_ERR_INVALID, "e3x_tp_message_backward: null pointer");
+  if (workspace_bytes < (size_t)(E * scratch_row) || ((uintptr_t)workspace & 15))
+    return fail(E3X_ERR_INVALID, "e3x_tp_message_backward: workspace smaller than e3x_tp_message_backward_workspace_bytes() or not 16-byte aligned");
+  hipStream_t st = (hipStream_t)stream;
+  int dev, rc;
+  if ((rc = current_device(&dev))) return rc;
+  if ((rc = prepare_rowgrad(P))) return rc;
+  if ((rc = load_rowgrad_functions(P, dev))) return rc;
+  SubKernel* R = P->rowgrad.get();
+  int idx64 = idx_bits == 64;
+  if (src_rows) {
+    src = src_rows;
+    idx64 = kSrcInRowOrderHost;
+  }
+  long long n_rows = num_out_nodes, n_src = num_src_nodes;
+  void* args[] = {(void*)&node_x, (void*)&edge_attr, (void*)&w,      (void*)&grad_out, (void*)&src,    (void*)&idx64,   (void*)&rowptr,
+                  (void*)&perm,   (void*)&row_order, (void*)&n_rows, (void*)&n_src,    (void*)&grad_w, (void*)&grad_x2, (void*)&workspace};
+  const long long blocks = (n_rows + 7) / 8 * 8;  // a workgroup per row, contiguous eighths of the rows per XCD
+  hipError_t err = hipModuleLaunchKernel(grad_x2 ? R->fn_rowgrad_x2[dev] : R->fn_rowgrad[dev], (unsigned)blocks, 1, 1, 64 * R->chunks, 1, 1,
+                                         0, st, args, nullptr);
+  if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_message_backward: launch failed: ") + hipGetErrorString(err));
+  void* rargs[] = {(void*)&workspace, (void*)&rowptr_by_src, (void*)&perm_by_src, (void*)&grad_x, (void*)&n_src};
+  err = hipModuleLaunchKernel(R->fn_rowgrad_reduce[dev], (unsigned)n_src, 1, 1, 256, 1, 1, 0, st, rargs, nullptr);
+  if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_message_backward: launch failed: ") + hipGetErrorString(err));
   return E3X_OK;
 }
 

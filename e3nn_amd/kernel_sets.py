@@ -164,6 +164,12 @@ def narrow_message():
     return message_tensor_product(f, SH2, irreps_out=f)
 
 
+def ragged_wide_message():
+    # 72 / 130 / 100 channels with one output block per path: the backward pass grouped by destination (messages ten times
+    # as wide as the features) with partly filled wavefronts
+    return message_tensor_product("72x0e+130x1o+100x2e", SH3, keep="0e+1o+2e+1e+2o+3o")
+
+
 def all_tensor_products():
     """(name, TensorProduct, dtypes) for everything that must be in the kernel cache."""
     out = [
@@ -195,6 +201,7 @@ def all_tensor_products():
         ("right_small", right_small(), (torch.float32,)),
         ("odd_mul", odd_mul(), (torch.float32,)),
         ("narrow_message", narrow_message(), (torch.float32, torch.bfloat16)),
+        ("ragged_wide_message", ragged_wide_message(), (torch.float32,)),
     ]
     return out
 
@@ -202,7 +209,7 @@ def all_tensor_products():
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
 BACKWARD_CASES = ["cfg1", "cfg3_merged", "cfg3_builder", "cfg4_A", "cfg5", "mfma_small", "mfma_full_tiles", "outer_split", "node_fctp", "node_block",
                   "node_wide_out", "node_narrow", "node_partial_tile", "radial_layer", "odd_mul", "unaligned_mfma", "unaligned_offsets",
-                  "mixed_modes", "scalar_exact", "narrow_message"]  # fmt: skip
+                  "mixed_modes", "scalar_exact", "narrow_message", "ragged_wide_message"]  # fmt: skip
 
 
 def linear_channels(norm="element"):

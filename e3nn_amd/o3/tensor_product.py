@@ -180,6 +180,29 @@ class _Plan:
             )
         return out, grad_w, grad_x2
 
+    def message_backward(self, node_x, edge_attr, w, grad_out, edges, want_x2=False):
+        """``(grad_node_x, grad_w, grad_edge_attr or None)`` of the message step from the kernel grouped by destination;
+        None when the plan or the size of its scratch is outside what that kernel is meant for."""
+        L = _lib.lib()
+        ws_bytes = L.e3x_tp_message_backward_workspace_bytes(self.handle, edges.num_edges)
+        if ws_bytes == 0:
+            return None
+        by_src = edges.transposed()
+        grad_x, grad_w = torch.empty_like(node_x), torch.empty_like(w)
+        grad_x2 = torch.empty_like(edge_attr) if want_x2 else None
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=node_x.device)
+        with torch.cuda.device(node_x.device):
+            _lib.check(
+                L.e3x_tp_message_backward(
+                    self.handle, _lib.ptr(node_x), _lib.ptr(edge_attr), _lib.ptr(w), _lib.ptr(grad_out), _lib.ptr(edges.edge_src),
+                    edges.edge_src.element_size() * 8, _lib.ptr(edges.rowptr), _lib.ptr(edges.walk_perm), _lib.ptr(edges.row_order),
+                    _lib.ptr(edges.src_rows), _lib.ptr(by_src.rowptr), _lib.ptr(by_src.walk_perm), _lib.ptr(grad_x), _lib.ptr(grad_w),
+                    _lib.ptr(grad_x2), edges.num_edges, node_x.shape[0], edges.num_nodes, _lib.ptr(ws), ws_bytes,
+                    _lib.stream_ptr(node_x.device),
+                )  # fmt: skip
+            )
+        return grad_x, grad_w, grad_x2
+
     def gather_scatter_radial(self, table, edge_attr, edge_scalars, w1, w2, act_kind, act_cst, variance_in, variance_out,
                               gather_idx, edges, num_table_rows):
         """``gather_scatter`` with the per-edge weights computed in the kernel by the two-layer network
@@ -370,7 +393,11 @@ def _message_gradients(tp, edges, node_x, edge_attr, w, g, need1, need2, needw):
     g1 = g2 = gw = None
     needw = needw and tp.weight_numel > 0
     if need1 and needw and dt == torch.float32:
-        # every gradient from one pass over the weights and one gather of g per edge
+        # every gradient from one pass over the weights: grouped by destination where the messages are much wider than
+        # the node features, else with one gather of g per edge
+        res = tp._plan(dt).message_backward(node_x, edge_attr, w, g, edges, need2 and edge_attr.shape[1] > 0)
+        if res is not None:
+            return res[0], (res[2] if need2 else None), res[1]
         res = tp._grad_plan("x1", dt).gather_scatter_grad_w(
             g, edge_attr, w, node_x, edges.edge_dst, edges.transposed(), need2 and edge_attr.shape[1] > 0
         )
@@ -749,6 +776,9 @@ class TensorProduct(torch.nn.Module):
         if self._live_mode() == "uvu":
             _lib.check(_lib.lib().e3x_tp_plan_prepare_backward_w(self._plan(dtype).handle))
             if dtype == torch.float32 and not self.shared_weights and self.weight_numel:
+                rc = _lib.lib().e3x_tp_plan_prepare_message_backward(self._plan(dtype).handle)
+                if rc != _lib.ERR_INVALID:
+                    _lib.check(rc)
                 # the message-step backward kernel on the transposed plan, where the instruction set fits it
                 rc = _lib.lib().e3x_tp_plan_prepare_gather_scatter_grad_w(self._grad_plan("x1", dtype).handle)
                 if rc != _lib.ERR_INVALID:

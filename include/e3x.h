@@ -308,6 +308,26 @@ int e3x_tp_gather_scatter_grad_w(e3x_plan* plan, const void* table, const void* 
                                  void* grad_w, void* grad_x2, int64_t E, int64_t num_table_rows, int64_t num_out_rows,
                                  void* stream);
 
+/* The backward pass of a message step grouped by DESTINATION, called on the forward plan: from grad_out[num_out_nodes,
+ * out_dim] the gradients grad_x[num_src_nodes, in1_dim], grad_w[E, weight_numel] and, unless NULL, grad_x2[E, in2_dim] of
+ *   out[n] = sum over the edges e -> n of plan(node_x[src[e]], edge_attr[e], w[e]).
+ * rowptr / perm (/ row_order / src_rows) group the edges by destination as for e3x_tp_gather_scatter_ws, rowptr_by_src /
+ * perm_by_src by source.  Each edge leaves its share of grad_x in the workspace
+ * (e3x_tp_message_backward_workspace_bytes(plan, E)), which a second kernel sums per source node in the order of the
+ * edges: no atomics, run-to-run identical.  For messages several times as wide as the node features it moves a
+ * fraction of the bytes of e3x_tp_gather_scatter_grad_w, which gathers a row of grad_out per edge.
+ * e3x_tp_plan_prepare_message_backward builds the code object (no GPU needed) and returns E3X_ERR_INVALID, without a
+ * message, for plans it is not meant for (fp32, per-edge weights, more than 32 channels, messages more than three times
+ * as wide as the scratch row); the workspace size reads 0 then, and where it would exceed 16 GiB. */
+int e3x_tp_plan_prepare_message_backward(e3x_plan* plan);
+size_t e3x_tp_message_backward_workspace_bytes(const e3x_plan* plan, int64_t E);
+int e3x_tp_message_backward(e3x_plan* plan, const void* node_x, const void* edge_attr, const void* w, const void* grad_out,
+                            const void* src, int idx_bits, const int32_t* rowptr, const int32_t* perm,
+                            const int32_t* row_order, const int32_t* src_rows, const int32_t* rowptr_by_src,
+                            const int32_t* perm_by_src, void* grad_x, void* grad_w, void* grad_x2, int64_t E,
+                            int64_t num_src_nodes, int64_t num_out_nodes, void* workspace, size_t workspace_bytes,
+                            void* stream);
+
 /* Weight gradient of the `uvw` product: grad_w[weight_numel] (shared weights, summed over the batch with
  * fp32 atomics, so the last bits depend on the order) or grad_w[Z, weight_numel] (per-sample weights), from
  * x1[Z, in1_dim], x2[Z, in2_dim], grad_out[Z, out_dim].  The reference obtains it by autograd through

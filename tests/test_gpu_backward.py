@@ -92,6 +92,40 @@ def test_fused_message_gradients(maker, N, E, idx):
     assert torch.equal(a5.grad, a4.grad) and torch.equal(c5.grad, c4.grad)
 
 
+@pytest.mark.parametrize("maker", [lambda: ks.cfg4("A"), ks.ragged_wide_message])
+@pytest.mark.parametrize("degrees,idx,grouped", [([0, 1, 63, 64, 65, 0, 130, 2], torch.int64, True), ([3, 0, 0, 129], torch.int32, False), ([1], torch.int64, True)])
+def test_message_gradients_grouped_by_destination(maker, degrees, idx, grouped):
+    # messages much wider than the node features: rows without edges, one edge, around the blocks of 64 edges, an odd
+    # and an even number of them; sources without edges get exact zeros
+    tp = maker()
+    spec = oracle_spec(tp)
+    N, E, n_src = len(degrees), sum(degrees), 9
+    dst = torch.repeat_interleave(torch.arange(N), torch.tensor(degrees))
+    src = torch.randint(1, n_src, (E,), generator=torch.Generator().manual_seed(3))
+    if not grouped:
+        dst = dst[torch.randperm(E, generator=torch.Generator().manual_seed(4))]
+    node_x, attr, w = seeded(n_src, tp.irreps_in1.dim, seed=1), seeded(E, tp.irreps_in2.dim, seed=2), seeded(E, tp.weight_numel, seed=3)
+    cot = seeded(N, tp.irreps_out.dim, seed=4)
+    _, (r1, r2, rw) = _oracle_grads(lambda a, b, c: tp_gather_scatter_torch(spec, a, b, c, src, dst, N), (node_x, attr, w), cot)
+    edges = DstSortedEdges(src.to(idx).to(DEV), dst.to(idx).to(DEV), N, n_src)
+    plan = tp._plan(torch.float32)
+    x, a, ww, g = (t.to(DEV) for t in (node_x, attr, w, cot))
+    for want_x2 in (True, False):
+        junk = torch.full((E, tp.weight_numel), float("nan"), device=DEV)  # see test_uvu_plain_gradients
+        del junk
+        gx, gw, gx2 = plan.message_backward(x, a, ww, g, edges, want_x2)
+        assert_close(gw, rw.numpy(), what="d/dweight")
+        # sums of at most E rows: 24-bit products, one rounding per addition
+        assert_close(gx, r1.numpy(), atol=1e-5 * max(1.0, float(r1.abs().max())), what="d/dnode_x")
+        assert not gx[0].any()
+        assert (gx2 is not None) == want_x2
+        if want_x2:
+            # 64 x 64-channel sums of products of four N(0, 1) factors per path
+            assert_close(gx2, r2.numpy(), atol=1e-5 * max(1.0, float(r2.abs().max())), what="d/dedge_attr")
+        again = plan.message_backward(x, a, ww, g, edges, want_x2)
+        assert torch.equal(again[0], gx) and torch.equal(again[1], gw)
+
+
 @pytest.mark.parametrize("maker,Z", [(lambda: ks.golden_tp("fctp_small_cfg5_like"), 6), (ks.cfg1, 50), (ks.mfma_small, 70),
                                      (lambda: ks.golden_tp("fctp_per_sample_weights"), 5), (ks.node_fctp, 90), (ks.radial_layer, 77), (ks.node_wide_out, 45), (ks.node_narrow, 40)])  # fmt: skip
 def test_uvw_input_gradients(maker, Z):
