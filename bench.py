@@ -324,14 +324,16 @@ def bench_uvw(args, dev, dtype=torch.float32):
 
 
 def split_operand_fractions(arithmetic, flops, ms):
-    """Both readings of an fp32 product that runs as six bf16 matrix products of three-way split operands:
+    """Both readings of an fp32 product that runs as six bf16 matrix products of three-way split operands, or three fp16
+    products of two-way split ones (the two instructions have one peak):
     ``frac`` prices the 2mnk flops of the fp32 product against the fp32 matrix peak (what the caller gets);
-    ``frac_of_bf16_peak_executed`` prices the six products the matrix cores execute against the peak of the instruction
+    ``frac_of_bf16_peak_executed`` prices the products the matrix cores execute against the peak of the instruction
     they execute.  On the fp32 instruction the two coincide and only ``frac`` is reported."""
     if "split" not in arithmetic:
         return {}
+    products = 3 if "three products" in arithmetic else 6
     return {"frac_fp32_equivalent": flops / (ms * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
-            "frac_of_bf16_peak_executed": 6 * flops / (ms * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS}  # fmt: skip
+            "frac_of_bf16_peak_executed": products * flops / (ms * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS}  # fmt: skip
 
 
 def with_env(name, value, fn):

@@ -44,6 +44,7 @@ struct SubKernel {
   bool bwd_lds = false;
   hipFunction_t fn_dw[kMaxDevices] = {nullptr};
   hipFunction_t fn_pack[kMaxDevices] = {nullptr};
+  hipFunction_t fn_max[kMaxDevices] = {nullptr};
   // uvu: the edge-parallel backward kernel is a code object of its own (other lane layout), built on first use
   std::unique_ptr<SubKernel> bwd;
   // uvu, transposed plan of a message step: the fused kernel that also writes the weight gradient, built on first use
@@ -80,6 +81,9 @@ struct e3x_plan {
   // when the instruction set fits it; the plain product keeps the kernels of `subs`
   std::unique_ptr<SubKernel> msg_mfma;
   int msg_groups = 0;  // wavefronts per output row
+  // uvw_mfma, fp32 storage: the kernel on pairs of fp16 operands, where the instruction set fits it (see half_fits)
+  std::unique_ptr<SubKernel> half;
+  int half_targets = 0;    // grid.y
   // uvw_mfma: the weight-gradient kernel is a code object of its own, built on first use
   std::unique_ptr<SubKernel> dw;
   long long dw_tiles = 0;  // grid.x: the largest tile count of a path
@@ -563,7 +567,25 @@ bool uvw_mfma_eligible(const e3x_plan& P, int dtype) {
 }
 bool uvw_mfma_eligible(const e3x_plan& P) { return uvw_mfma_eligible(P, P.dtype); }
 
-int build_uvw_mfma_source(e3x_plan& P, std::string* src) {
+// The kernel on pairs of fp16 operands (templates/uvw_mfma_half.inc): fp32 storage, multiplicities 64 or 128 on the inputs
+// (the K operand in registers, the row maximum among neighbouring lanes), multiples of 64 on the output, l <= 2 there (the
+// seven accumulator tiles of l = 3 do not fit beside the operands), rows in 16-byte pieces.  The weights are packed on
+// every call into a workspace; without one, or with misaligned rows, the kernel of uvw_mfma.inc runs.
+bool half_fits(const e3x_plan& P) {
+  if (P.family != "uvw_mfma" || P.dtype != E3X_F32 || env_int("E3X_UVW_SPLIT", 1) == 0 || env_int("E3X_UVW_HALF", 1) == 0) return false;
+  if ((P.in1_dim | P.in2_dim) & 3) return false;
+  for (const auto& p : P.paths) {
+    const int U = P.in1[p.in1].mul, V = P.in2[p.in2].mul;
+    if ((U != 64 && U != 128) || (V != 64 && V != 128) || P.out[p.out].mul % 64 || P.out[p.out].l > 2) return false;
+    if (((P.off1[p.in1] | P.off2[p.in2] | p.woff) & 3) || std::max(P.in1[p.in1].l, P.in2[p.in2].l) > 3) return false;
+  }
+  return true;
+}
+constexpr int kHalfMaxBlocks = 64;  // MAX_BLOCKS of the template
+// packed weights | inverse scales and block maxima of every path
+size_t half_workspace_bytes(const e3x_plan& P) { return (size_t)P.weight_numel * 4 + P.paths.size() * (kHalfMaxBlocks + 4) * 4 + 256; }
+
+int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   // Output channels per workgroup.  fp32: 128 (two accumulator tiles per wave, 64 KB of LDS, two workgroups per CU at
   // 256 registers) wherever every output multiplicity is a multiple of 128, else 64 (48 KB, three workgroups at 168
   // registers).  Measured on 128x0e+128x1o+128x2e squared, 65536 rows: 61.3 ms at 64 channels, 56.3 ms at 128 -- a
@@ -572,7 +594,7 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src) {
   int wt = env_int("E3X_UVW_WT", P.dtype == E3X_F32 ? 128 : 64), kmax = 32;
   for (const auto& p : P.paths)
     if (P.out[p.out].mul % 128) wt = 64;
-  if (P.dtype != E3X_F32) wt = 64;
+  if (P.dtype != E3X_F32 || half) wt = 64;
   std::ostringstream s, nzs, ps, ts;
   emit_header(s, P);
   // split-operand matrix steps (see the template) in fp32 storage; weight chunks of 16 K rows then keep the LDS at
@@ -583,9 +605,9 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src) {
   for (const auto& p : P.paths)
     if (P.in1[p.in1].mul % 64 || P.in2[p.in2].mul % 64 || P.out[p.out].mul % 64) full = false;
   const int split = P.dtype == E3X_F32 ? env_int("E3X_UVW_SPLIT", full ? 1 : 0) : 0;
-  if (split) s << "#define E3X_UVW_SPLIT 1\n";
-  P.arithmetic = P.dtype != E3X_F32 ? "bf16 matrix instruction" : split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
-  if (P.dtype == E3X_F32) s << "#define E3X_UVW_KC " << env_int("E3X_UVW_KC", split ? 16 : 32) << "\n";
+  if (split && !half) s << "#define E3X_UVW_SPLIT 1\n";
+  P.arithmetic = half ? "fp16 matrix instruction, three products of scaled two-way split operands" : P.dtype != E3X_F32 ? "bf16 matrix instruction" : split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
+  if (P.dtype == E3X_F32 && !half) s << "#define E3X_UVW_KC " << env_int("E3X_UVW_KC", split ? 16 : 32) << "\n";
   if (env_int("E3X_UVW_KS", 0)) s << "#define E3X_UVW_KS " << env_int("E3X_UVW_KS", 0) << "\n";
   // two waves per SIMD (256 registers) for 128-channel tiles and for l = 3 outputs, whose seven accumulator tiles do not
   // fit the 168 registers of three (64x1o+64x2e squared -> 32x3o: 3122 registers' worth of spills there, none here)
@@ -605,7 +627,8 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src) {
       // operand is synthesised; take the cheapest
       // (the bf16 kernel scales accumulators only: its matrix passes are cheap next to the fp32 epilogue)
       const bool okU = a.mul % 32 == 0 && a.mul <= k_cap(P.dtype), okV = b.mul % 32 == 0 && b.mul <= k_cap(P.dtype);
-      const bool synth = P.dtype == E3X_F32 && env_int("E3X_UVW_SYNTH", 1) && d3 < std::min(d1, d2) && okU;
+      // (so does the kernel on pairs of fp16 operands)
+      const bool synth = P.dtype == E3X_F32 && !half && env_int("E3X_UVW_SYNTH", 1) && d3 < std::min(d1, d2) && okU;
       const bool k_is_x2 = !synth && okV && (!okU || d2 < d1);
       kmax = std::max(kmax, k_is_x2 ? b.mul : a.mul);
       if (synth) dka = std::max(dka, d1);
@@ -652,8 +675,8 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src) {
   s << "struct Target { int out_off, d3, w0, wn, path_beg, path_end; };\n";  // wn: channels in the tile (64, or 32 at the end)
   s << "constexpr int N_TARGET = " << n_target << ";\nconstexpr Target targets[N_TARGET] = {\n" << ts.str() << "};\n";
   s << "}  // namespace cfg\n";
-  P.n_targets = n_target;
-  *src = s.str() + e3x::kTplCommon + (P.dtype == E3X_BF16 ? e3x::kTplUvwMfmaBf16 : e3x::kTplUvwMfma);
+  (half ? P.half_targets : P.n_targets) = n_target;
+  *src = s.str() + e3x::kTplCommon + (half ? e3x::kTplUvwMfmaHalf : P.dtype == E3X_BF16 ? e3x::kTplUvwMfmaBf16 : e3x::kTplUvwMfma);
   return E3X_OK;
 }
 
@@ -931,6 +954,18 @@ int load_functions(e3x_plan* P, int dev) {
       if (hipModuleGetFunction(&K->fn_dw[dev], mod, "e3x_uvw_small_dw") != hipSuccess)
         return fail(E3X_ERR_HIP, "kernel e3x_uvw_small_dw missing from " + K->hsaco);
     }
+    K->module[dev] = mod;
+  }
+  if (P->half && !P->half->module[dev]) {
+    SubKernel* K = P->half.get();
+    hipModule_t mod = nullptr;
+    hipError_t err = hipModuleLoad(&mod, K->hsaco.c_str());
+    if (err != hipSuccess)
+      return fail(E3X_ERR_HIP, "hipModuleLoad(" + K->hsaco + ") failed: " + hipGetErrorString(err));
+    if (hipModuleGetFunction(&K->fn_plain[dev], mod, "e3x_uvw_half_plain") != hipSuccess ||
+        hipModuleGetFunction(&K->fn_pack[dev], mod, "e3x_uvw_half_pack") != hipSuccess ||
+        hipModuleGetFunction(&K->fn_max[dev], mod, "e3x_uvw_half_max") != hipSuccess)
+      return fail(E3X_ERR_HIP, "kernels of e3x_uvw_half missing from " + K->hsaco);
     K->module[dev] = mod;
   }
   if (P->msg_mfma && !P->msg_mfma->module[dev]) {
@@ -1248,6 +1283,19 @@ extern "C" int e3x_tp_plan_create(const e3x_tp_desc* d, e3x_plan** out) {
     P->key += (P->key.empty() ? "" : "+") + K->key;
     P->subs.push_back(std::move(K));
   }
+  if (!P->paths.empty() && half_fits(*P)) {
+    std::unique_ptr<SubKernel> K(new SubKernel);
+    std::string src;
+    K->waves_per_block = 8;
+    if ((rc = build_uvw_mfma_source(*P, &src, true))) return rc;
+    rc = e3x::get_code_object("uvw_half", src, &K->key, &K->hsaco);
+    // LDS addresses as scalar operands of inline assembly: see above
+    if (rc == E3X_ERR_COMPILE && !env_int("E3X_NO_JIT", 0))
+      rc = e3x::get_code_object("uvw_half", "#define E3X_UVWH_SCALAR_ADDR 1\n" + src, &K->key, &K->hsaco);
+    if (rc) return rc;
+    P->key += "+" + K->key;
+    P->half = std::move(K);
+  }
   if (P->family == "uvu" && env_int("E3X_UVU_MFMA", 1)) {
     std::unique_ptr<SubKernel> K(new SubKernel);
     std::string src;
@@ -1294,6 +1342,7 @@ static int zero_output(e3x_plan* P, void* out, int64_t rows, hipStream_t st) {
 static bool needs_packed_weights(const e3x_plan* P) { return P->family == "uvw_mfma" && P->dtype == E3X_BF16; }
 
 extern "C" size_t e3x_tp_forward_workspace_bytes(const e3x_plan* P) {
+  if (P && P->half) return half_workspace_bytes(*P);  // (taken when given; e3x_tp_forward runs without)
   return (P && needs_packed_weights(P)) ? (size_t)P->weight_numel * 2 : 0;
 }
 
@@ -1318,6 +1367,27 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
   }
   if ((rc = load_functions(P, dev))) return rc;
   long long n_rows = Z;
+  if (P->half && workspace && workspace_bytes >= half_workspace_bytes(*P) &&
+      !(((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)w | (uintptr_t)workspace) & 15)) {
+    SubKernel* K = P->half.get();
+    const unsigned n_path = (unsigned)P->paths.size();
+    unsigned* w_max = (unsigned*)((char*)workspace + (size_t)P->weight_numel * 4);
+    float* w_inverse = (float*)(w_max + (size_t)n_path * kHalfMaxBlocks);
+    long long entries = 0;
+    for (const auto& p : P->paths) entries = std::max(entries, (long long)P->in1[p.in1].mul * P->in2[p.in2].mul * P->out[p.out].mul / 8);
+    const long long blocks = (Z + 127) / 128;
+    if (blocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_forward: batch too large for one launch");
+    void* margs[] = {(void*)&w, (void*)&w_max};
+    void* pargs[] = {(void*)&w, (void*)&w_max, (void*)&workspace, (void*)&w_inverse};
+    void* args[] = {(void*)&x1, (void*)&x2, (void*)&workspace, (void*)&w_inverse, (void*)&out, (void*)&n_rows};
+    hipError_t err = hipModuleLaunchKernel(K->fn_max[dev], kHalfMaxBlocks, n_path, 1, 256, 1, 1, 0, st, margs, nullptr);
+    if (err == hipSuccess)
+      err = hipModuleLaunchKernel(K->fn_pack[dev], (unsigned)((entries + 255) / 256), n_path, 1, 256, 1, 1, 0, st, pargs, nullptr);
+    if (err == hipSuccess)
+      err = hipModuleLaunchKernel(K->fn_plain[dev], (unsigned)blocks, (unsigned)P->half_targets, 1, 512, 1, 1, 0, st, args, nullptr);
+    if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
+    return E3X_OK;
+  }
   if (needs_packed_weights(P)) {
     // the matrix-core kernel reads the weights repacked into octets of consecutive K indices
     if (!workspace || workspace_bytes < (size_t)P->weight_numel * 2)

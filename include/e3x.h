@@ -120,8 +120,9 @@ int e3x_tp_plan_info(const e3x_plan* plan, int64_t* weight_numel, int64_t* in1_d
                      int64_t* out_dim, const char** family, const char** cache_key);
 
 /* Which instruction forms the products of the plan's kernels: "fp32 vector ALU", "fp32 matrix instruction",
- * "bf16 matrix instruction" (bf16 storage) or "bf16 matrix instruction, six products of three-way split operands"
- * (fp32 storage, fp32-accurate; see e3x_tp_forward).  which = 0: forward; which = 1: the "uvw" weight gradient on the
+ * "bf16 matrix instruction" (bf16 storage), "bf16 matrix instruction, six products of three-way split operands" or
+ * "fp16 matrix instruction, three products of scaled two-way split operands" (fp32 storage, fp32-accurate; see
+ * e3x_tp_forward and e3x_tp_forward_ws).  which = 0: forward; which = 1: the "uvw" weight gradient on the
  * matrix cores, "" until that kernel has been built (e3x_tp_plan_prepare_backward_w).  No counterpart in the
  * reference; benchmarks use it to state the peak a kernel is measured against.  The string lives as long as the plan. */
 const char* e3x_tp_plan_arithmetic(const e3x_plan* plan, int which);
@@ -140,7 +141,13 @@ int e3x_tp_forward(e3x_plan* plan, const void* x1, const void* x2, const void* w
                    void* stream);
 /* The same with caller-owned device scratch.  Plans of the "uvw_mfma" family in bf16 storage repack the
  * weights for the matrix cores on every call and need e3x_tp_forward_workspace_bytes(plan) bytes (16-byte
- * aligned, as x1 and x2 must be); every other plan needs none and e3x_tp_forward is enough. */
+ * aligned, as x1 and x2 must be).  fp32 plans of that family with input multiplicities of 64 or 128, output multiplicities
+ * that are multiples of 64 and output degrees up to 2 take the workspace when it is given and x1, x2, w and it are 16-byte
+ * aligned: the products are then three cross products of operands split into two fp16 pieces each, after scaling by
+ * powers of two (the first or second input's row per irrep component, the weights per path), which is faster than and at
+ * least as accurate as the six bf16 products of e3x_tp_forward.  An element below 2^-17 of the largest of its row and
+ * irrep (a weight: of its path) then carries an error of 2^-40 of that largest one instead of a relative one.  Every other
+ * plan needs no workspace and e3x_tp_forward is enough. */
 size_t e3x_tp_forward_workspace_bytes(const e3x_plan* plan);
 int e3x_tp_forward_ws(e3x_plan* plan, const void* x1, const void* x2, const void* w, void* out, int64_t Z,
                       void* workspace, size_t workspace_bytes, void* stream);

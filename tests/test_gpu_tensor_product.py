@@ -300,6 +300,47 @@ def _uvw_weight_gradient_fp64(tp, x1, x2, cot):
     return np.concatenate(blocks)
 
 
+@pytest.mark.parametrize("Z", [1, 127, 128, 129, 300])
+def test_uvw_on_pairs_of_fp16_operands(Z):
+    # edges of the 128-row tiles; rows of either input and the weights of a path scaled over the exponent range, also
+    # the input gradients (transposed plans: other K operands and component counts)
+    tp = ks.mfma_full_tiles()
+    assert "fp16" in tp._plan(torch.float32).arithmetic
+    sc = torch.tensor([1.0, 1e-12, 1e15, 1e-25, 1e20]).repeat(Z // 5 + 1)[:Z, None]
+    x1, x2 = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2)
+    w = torch.cat([seeded(t.path_shape[0] * t.path_shape[1] * t.path_shape[2], seed=10 + i) for i, t in enumerate(tp.instructions)])
+    spec = oracle_spec(tp)
+    ref = otp.tp_forward(spec, x1.numpy(), x2.numpy(), w.numpy())
+
+    def close(got, want, what):
+        # sums of some 1e4 products: fp32 accumulation leaves about 4e-7 of the 2-norm, the pairs 6e-8 of a term
+        err = got.double().cpu().numpy() - want
+        assert np.linalg.norm(err) < 1e-6 * np.linalg.norm(want), (what, np.linalg.norm(err) / np.linalg.norm(want))
+        assert np.abs(err).max() < 3e-5 * np.sqrt((want**2).mean()), what
+
+    out = tp(x1.to(DEV), x2.to(DEV), w.to(DEV))
+    close(out, ref, "rows of one scale")
+    y1, y2 = x1 * sc, x2 / sc
+    close(tp(y1.to(DEV), y2.to(DEV), w.to(DEV)), otp.tp_forward(spec, (y1.double() / sc).numpy(), (y2.double() * sc).numpy(), w.numpy()), "scaled rows")
+    close(tp(x1.to(DEV), x2.to(DEV), (w * 1e-20).to(DEV)).double() * 1e20, otp.tp_forward(spec, x1.numpy(), x2.numpy(), ((w * 1e-20).double() * 1e20).numpy()), "small weights")
+    # without a workspace (and so for rows that are not 16-byte aligned) the kernel on bf16 pieces runs
+    from e3nn_amd import _lib
+
+    a, b, c, plain = x1.to(DEV), x2.to(DEV), w.to(DEV), torch.empty_like(out)
+    _lib.check(_lib.lib().e3x_tp_forward(tp._plan(torch.float32).handle, _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), _lib.ptr(plain), Z, _lib.stream_ptr(a.device)))
+    close(plain, ref, "without a workspace")
+    # input gradients against 64-bit autograd of the einsums
+    a, b = a.requires_grad_(), b.requires_grad_()
+    cot = seeded(Z, tp.irreps_out.dim, seed=5)
+    g1, g2 = torch.autograd.grad(tp(a, b, c), (a, b), cot.to(DEV))
+    from oracle.torch_cpu import tp_forward_torch
+
+    d1, d2 = x1.double().requires_grad_(), x2.double().requires_grad_()
+    r1, r2 = torch.autograd.grad(tp_forward_torch(spec, d1, d2, w.double()), (d1, d2), cot.double())
+    close(g1, r1.numpy(), "d/dx1")
+    close(g2, r2.numpy(), "d/dx2")
+
+
 def test_uvw_weight_gradient_on_the_dense_configuration():
     # the weight gradient of config 5's own instruction set (11 paths of 128 x 128 x 128, 23 M weights) on the
     # split-operand matrix-core kernel; 300 rows end inside a batch chunk of the kernel.  The float64 reference is the
