@@ -7,6 +7,7 @@
 // permutation (and therefore the summation order) is unique for a given edge list.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -199,6 +200,221 @@ __global__ __launch_bounds__(kBlock) void fill_zero_bytes_kernel(unsigned char* 
   if (tid < n - tail0) p[tail0 + tid] = 0;
 }
 
+// ---- edge list in one pass: e3x_edges_build ---------------------------------------------------------------
+// Counting sort by destination.  What bounds the set-up of a neighbour list is launches and host round trips, not bytes:
+// 176 852 edges on 5 003 nodes took four library sorts (some 30 launches, 0.17 ms of kernels) and four stream
+// synchronisations.  Here: counts, two scan kernels, placement, one pass over the rows, one ranking kernel, one read-back.
+//   count    rank of an edge inside its row by an atomic on the row's counter; neighbouring lanes with the same
+//            destination take one atomic together, so a list that is already grouped costs one atomic per run.  The
+//            ranks depend on the order of the atomics;
+//   place    edge ids at rowptr[row] + rank;
+//   rows     a wavefront per row puts its ids in ascending order (the stable order, whatever the ranks were) and finds the
+//            row's two smallest sources.  A list that was grouped already skips the sorting (perm is the identity);
+//   order    rows ranked by their key by counting smaller keys.
+constexpr int kScanTile = 4096;
+constexpr int kRowMax = 1024;  // longest row that is put in order here
+enum { kBadSrc = 0, kBadDst, kUnsorted, kOverflow, kScore, kFlags };
+
+__global__ __launch_bounds__(kBlock) void edges_zero_kernel(int* __restrict__ p, long long n) {
+  for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock) p[i] = 0;
+}
+
+template <typename SrcT, typename DstT>
+__global__ __launch_bounds__(kBlock) void edges_count_kernel(const SrcT* __restrict__ src, const DstT* __restrict__ dst, long long E,
+                                                             long long N, long long n_src, int* __restrict__ counts,
+                                                             int* __restrict__ rank, int* __restrict__ flags) {
+  const int lane = threadIdx.x & 63;
+  bool bad_s = false, bad_d = false, unsorted = false;
+  const long long e_end = (E + 63) / 64 * 64;  // whole wavefronts: the shuffles run with every lane
+  for (long long e = (long long)blockIdx.x * kBlock + threadIdx.x; e < e_end; e += (long long)gridDim.x * kBlock) {
+    const bool live = e < E;
+    long long d = -1;
+    if (live) {
+      d = (long long)dst[e];
+      const long long s = (long long)src[e];
+      if (s < -n_src || s >= n_src) bad_s = true;
+      if (d < 0 || d >= N) {
+        bad_d = true;
+        d = -1;
+      }
+    }
+    const int key = (int)d;
+    int prev = __shfl_up(key, 1, 64);
+    if (lane == 0 && e > 0 && live) prev = (int)(long long)dst[e - 1];
+    if (live && e > 0 && prev > key) unsorted = true;
+    const unsigned long long heads = __ballot(lane == 0 || prev != key);
+    const unsigned long long upto = heads & (~0ull >> (63 - lane));
+    const int head = 63 - __clzll((long long)upto);
+    const unsigned long long after = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
+    const int end = after ? __ffsll((long long)after) - 1 : 64;
+    int base = 0;
+    if (lane == head && key >= 0) base = atomicAdd(&counts[key], end - head);
+    base = __shfl(base, head, 64);
+    if (live) rank[e] = base + lane - head;
+  }
+  if (bad_s) atomicOr(&flags[kBadSrc], 1);
+  if (bad_d) atomicOr(&flags[kBadDst], 1);
+  if (__ballot(unsorted) && lane == 0) atomicOr(&flags[kUnsorted], 1);
+}
+
+// sums[b] = sum of tile b of the counts
+__global__ __launch_bounds__(kBlock) void edges_scan_sums_kernel(const int* __restrict__ counts, long long N, int* __restrict__ sums) {
+  __shared__ int part[kBlock / 64];
+  const long long i0 = (long long)blockIdx.x * kScanTile;
+  int v = 0;
+  for (int i = threadIdx.x; i < kScanTile; i += kBlock) v += i0 + i < N ? counts[i0 + i] : 0;
+  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+  if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kBlock / 64; ++i) v += part[i];
+    sums[blockIdx.x] = v;
+  }
+}
+
+// rowptr[n] = sum of counts[0 .. n - 1], n = 0 .. N; every workgroup adds up the sums of the tiles before its own
+__global__ __launch_bounds__(kBlock) void edges_scan_kernel(const int* __restrict__ counts, long long N, const int* __restrict__ sums,
+                                                            int* __restrict__ rowptr) {
+  __shared__ int part[kBlock / 64], wsum[kBlock / 64];
+  constexpr int PER = kScanTile / kBlock;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+  int before = 0;
+  for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlock) before += sums[i];
+  for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off, 64);
+  if (lane == 0) part[wave] = before;
+  const long long i0 = (long long)blockIdx.x * kScanTile + threadIdx.x * PER;
+  int c[PER], mine = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    c[k] = i0 + k < N ? counts[i0 + k] : 0;
+    mine += c[k];
+  }
+  int incl = mine;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int t = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += t;
+  }
+  if (lane == 63) wsum[wave] = incl;
+  __syncthreads();
+  int run = incl - mine;
+  for (int i = 0; i < kBlock / 64; ++i) {
+    run += part[i];
+    if (i < wave) run += wsum[i];
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    if (i0 + k <= N) rowptr[i0 + k] = run;
+    run += c[k];
+  }
+}
+
+template <typename DstT>
+__global__ __launch_bounds__(kBlock) void edges_place_kernel(const DstT* __restrict__ dst, long long E, long long N,
+                                                             const int* __restrict__ rowptr, const int* __restrict__ rank,
+                                                             const int* __restrict__ flags, int* __restrict__ placed) {
+  if (!flags[kUnsorted]) return;
+  for (long long e = (long long)blockIdx.x * kBlock + threadIdx.x; e < E; e += (long long)gridDim.x * kBlock) {
+    const long long d = (long long)dst[e];
+    if (d >= 0 && d < N) placed[rowptr[d] + rank[e]] = (int)e;
+  }
+}
+
+// smallest and second smallest distinct value of the two pairs
+__device__ __forceinline__ void merge_two_smallest(unsigned& k1, unsigned& k2, unsigned a1, unsigned a2) {
+  const unsigned lo = k1 < a1 ? k1 : a1, hi = k1 < a1 ? a1 : k1;  // lo <= hi
+  const unsigned rest = k2 < a2 ? k2 : a2;
+  k1 = lo;
+  k2 = hi > lo && hi < rest ? hi : rest;  // (a pair's second is larger than its first, so rest > lo)
+}
+
+template <typename SrcT>
+__global__ __launch_bounds__(kBlock) void edges_rows_kernel(const SrcT* __restrict__ src, const int* __restrict__ rowptr,
+                                                            const int* __restrict__ placed, long long N, long long n_src,
+                                                            int* __restrict__ perm, unsigned* __restrict__ keys,
+                                                            unsigned* __restrict__ second, int* __restrict__ flags) {
+  __shared__ int ids[kBlock / 64][kRowMax];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+  const long long row = (long long)blockIdx.x * (kBlock / 64) + wave;
+  if (row >= N) return;
+  const bool sorted = !flags[kUnsorted];
+  const int beg = rowptr[row], n = rowptr[row + 1] - beg;
+  if (!sorted && n > kRowMax) {  // the host takes the general sort
+    if (lane == 0) atomicOr(&flags[kOverflow], 1);
+    return;
+  }
+  unsigned k1 = 0xffffffffu, k2 = 0xffffffffu;
+  for (int i = lane; i < n; i += 64) {
+    const int id = sorted ? beg + i : placed[beg + i];
+    if (!sorted) ids[wave][i] = id;
+    else perm[beg + i] = id;
+    long long s = (long long)src[id];
+    if (s < 0) s += n_src;
+    const unsigned v = (unsigned)s;
+    if (v < k1) {
+      k2 = k1;
+      k1 = v;
+    } else if (v > k1 && v < k2) {
+      k2 = v;
+    }
+  }
+  if (!sorted) {
+    // (one wavefront wrote these and reads them back: its LDS operations complete in order)
+    __builtin_amdgcn_wave_barrier();
+    for (int i = lane; i < n; i += 64) {
+      const int id = ids[wave][i];
+      int smaller = 0;
+      for (int j = 0; j < n; ++j) smaller += ids[wave][j] < id;
+      perm[beg + smaller] = id;
+    }
+  }
+  if (keys) {
+    for (int off = 32; off >= 1; off >>= 1) {
+      const unsigned a1 = (unsigned)__shfl_xor((int)k1, off, 64), a2 = (unsigned)__shfl_xor((int)k2, off, 64);
+      merge_two_smallest(k1, k2, a1, a2);
+    }
+    if (lane == 0) {
+      keys[row] = k1;
+      second[row] = k2;
+    }
+  }
+}
+
+// The position of a row in the order of (key of the key of its key, key of its key, key, number), the last three levels
+// only for one node set, found by counting the rows in front of it: N^2 comparisons spread over the chip.  A
+// workgroup takes 64 rows (a lane each), its 16 wavefronts a sixteenth of every tile of keys.
+constexpr long long kRankMax = 16384;
+constexpr int kRankTile = 2048;
+__global__ __launch_bounds__(1024) void edges_order_kernel(const unsigned* __restrict__ keys, int N, int levels, int* __restrict__ order) {
+  __shared__ unsigned long long tile[kRankTile];
+  __shared__ int part[16][64];
+  auto composite = [&](int n) {
+    const unsigned k = keys[n];
+    unsigned l1 = 0, l2 = 0;
+    if (levels) {
+      l1 = k < (unsigned)N ? keys[k] : 0xffffffffu;
+      l2 = l1 < (unsigned)N ? keys[l1] : 0xffffffffu;
+    }
+    return ((unsigned long long)(l2 & 0xffffu) << 48) | ((unsigned long long)(l1 & 0xffffu) << 32) | ((unsigned long long)(k & 0xffffu) << 16) | (unsigned)n;
+  };
+  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+  const int row = blockIdx.x * 64 + lane;
+  const unsigned long long mine = composite(row < N ? row : N - 1);
+  int smaller = 0;
+  for (int t0 = 0; t0 < N; t0 += kRankTile) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < kRankTile; i += 1024) tile[i] = t0 + i < N ? composite(t0 + i) : ~0ull;
+    __syncthreads();
+#pragma unroll 8
+    for (int i = 0; i < kRankTile / 16; ++i) smaller += tile[wave * (kRankTile / 16) + i] < mine;
+  }
+  part[wave][lane] = smaller;
+  __syncthreads();
+  if (wave == 0 && row < N) {
+    for (int i = 1; i < 16; ++i) smaller += part[i][lane];
+    order[smaller] = row;
+  }
+}
+
 unsigned grid_for(long long n, int per_block) {
   long long b = (n + per_block - 1) / per_block;
   if (b < 1) b = 1;
@@ -373,6 +589,120 @@ extern "C" int e3x_row_order_build(const void* src, int idx_bits, const int32_t*
         hipStreamSynchronize(st) != hipSuccess)
       return e3x::fail(E3X_ERR_HIP, "e3x_row_order_build: reading back the score failed");
   }
+  return E3X_OK;
+}
+
+// Where the counting sort pays and its kernels are safe: rows of moderate average length (a few long ones send the call to
+// the general sort after the fact), tile sums that one workgroup adds up.
+static bool counting_sort_fits(int64_t E, int64_t N) { return E > 0 && N > 0 && N <= (1 << 22) && E / N <= 256; }
+static bool rank_order_fits(int64_t N, int64_t n_src) { return N <= kRankMax && n_src < 65535; }
+
+static size_t edges_small_bytes(int64_t E, int64_t N) {
+  // flags | counts | tile sums | rank | placed | keys | second
+  const size_t n4 = align_up((size_t)N * 4, 256), e4 = align_up((size_t)E * 4, 256);
+  return 256 + n4 + align_up((size_t)((N + 1 + kScanTile - 1) / kScanTile) * 4, 256) + 2 * e4 + 2 * n4;
+}
+
+extern "C" size_t e3x_edges_workspace_bytes(int64_t E, int64_t num_nodes) {
+  if (E < 0 || num_nodes < 0) return 0;
+  const size_t general = std::max(e3x_csr_workspace_bytes(E, num_nodes), e3x_row_order_workspace_bytes(num_nodes));
+  return std::max(general, counting_sort_fits(E, num_nodes) ? edges_small_bytes(E, num_nodes) : (size_t)256);
+}
+
+namespace {
+template <typename SrcT, typename DstT>
+void launch_edges(const SrcT* src, const DstT* dst, long long E, long long N, long long n_src, int* rowptr, int* perm, int* flags,
+                  int* counts, int* sums, int* rank, int* placed, unsigned* keys, unsigned* second, hipStream_t st) {
+  const unsigned tiles = (unsigned)((N + 1 + kScanTile - 1) / kScanTile);
+  // flags and counters lie next to each other
+  hipLaunchKernelGGL(edges_zero_kernel, dim3(grid_for(64 + N, kBlock)), dim3(kBlock), 0, st, flags, 64 + N);
+  hipLaunchKernelGGL((edges_count_kernel<SrcT, DstT>), dim3(grid_for(E, kBlock)), dim3(kBlock), 0, st, src, dst, E, N, n_src, counts, rank, flags);
+  hipLaunchKernelGGL(edges_scan_sums_kernel, dim3(tiles), dim3(kBlock), 0, st, counts, N, sums);
+  hipLaunchKernelGGL(edges_scan_kernel, dim3(tiles), dim3(kBlock), 0, st, counts, N, sums, rowptr);
+  hipLaunchKernelGGL((edges_place_kernel<DstT>), dim3(grid_for(E, kBlock)), dim3(kBlock), 0, st, dst, E, N, rowptr, rank, flags, placed);
+  hipLaunchKernelGGL((edges_rows_kernel<SrcT>), dim3((unsigned)((N + kBlock / 64 - 1) / (kBlock / 64))), dim3(kBlock), 0, st, src, rowptr,
+                     placed, N, n_src, perm, keys, second, flags);
+}
+
+template <typename DstT>
+__global__ __launch_bounds__(kBlock) void unsorted_kernel(const DstT* __restrict__ dst, long long E, int* __restrict__ flag) {
+  bool unsorted = false;
+  for (long long e = (long long)blockIdx.x * kBlock + threadIdx.x + 1; e < E; e += (long long)gridDim.x * kBlock)
+    if (dst[e] < dst[e - 1]) unsorted = true;
+  if (unsorted) atomicOr(flag, 1);
+}
+}  // namespace
+
+extern "C" int e3x_edges_build(const void* src, int src_bits, const void* dst, int dst_bits, int64_t E, int64_t num_nodes,
+                               int64_t num_src_nodes, int32_t* rowptr, int32_t* perm, int32_t* row_order, int32_t* grouped,
+                               int32_t* shared_pairs, void* workspace, size_t workspace_bytes, void* stream) {
+  if (E < 0 || num_nodes < 0 || num_src_nodes < 0 || E >= (1LL << 31) || num_nodes >= (1LL << 31))
+    return e3x::fail(E3X_ERR_INVALID, "e3x_edges_build: E and num_nodes must fit in int32");
+  if ((src_bits != 32 && src_bits != 64) || (dst_bits != 32 && dst_bits != 64))
+    return e3x::fail(E3X_ERR_INVALID, "e3x_edges_build: index widths must be 32 or 64 bits");
+  if (!rowptr || (E > 0 && (!src || !dst || !perm)) || !grouped || !shared_pairs || (workspace_bytes && !workspace))
+    return e3x::fail(E3X_ERR_INVALID, "e3x_edges_build: null pointer");
+  if (workspace_bytes < e3x_edges_workspace_bytes(E, num_nodes))
+    return e3x::fail(E3X_ERR_INVALID, "e3x_edges_build: workspace smaller than e3x_edges_workspace_bytes()");
+  hipStream_t st = (hipStream_t)stream;
+  *grouped = 1;
+  *shared_pairs = 0;
+  bool order_done = false;
+  if (counting_sort_fits(E, num_nodes)) {
+    const size_t n4 = align_up((size_t)num_nodes * 4, 256), e4 = align_up((size_t)E * 4, 256);
+    char* p = (char*)workspace;
+    int* flags = (int*)p;
+    int* counts = (int*)(p += 256);
+    int* sums = (int*)(p += n4);
+    int* rank = (int*)(p += align_up((size_t)((num_nodes + 1 + kScanTile - 1) / kScanTile) * 4, 256));
+    int* placed = (int*)(p += e4);
+    unsigned* keys = (unsigned*)(p += e4);
+    unsigned* second = (unsigned*)(p += n4);
+    const bool ranks = row_order && rank_order_fits(num_nodes, num_src_nodes);
+    unsigned* k = ranks ? keys : nullptr;
+#define E3X_EDGES(S, D) launch_edges((const S*)src, (const D*)dst, E, num_nodes, num_src_nodes, rowptr, perm, flags, counts, sums, rank, placed, k, second, st)
+    if (src_bits == 64 && dst_bits == 64) E3X_EDGES(long long, long long);
+    else if (src_bits == 64) E3X_EDGES(long long, int);
+    else if (dst_bits == 64) E3X_EDGES(int, long long);
+    else E3X_EDGES(int, int);
+#undef E3X_EDGES
+    if (ranks) {
+      hipLaunchKernelGGL(edges_order_kernel, dim3((unsigned)((num_nodes + 63) / 64)), dim3(1024), 0, st, keys, (int)num_nodes,
+                         num_src_nodes == num_nodes && num_nodes > 1 ? 1 : 0, row_order);
+      hipLaunchKernelGGL(order_score_kernel, dim3(grid_for(num_nodes, kBlock)), dim3(kBlock), 0, st, row_order, keys, second,
+                         (long long)num_nodes, flags + kScore);
+    }
+    int h[kFlags] = {0};
+    if (hipGetLastError() != hipSuccess) return e3x::fail(E3X_ERR_HIP, "e3x_edges_build: launch failed");
+    if (hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
+      return e3x::fail(E3X_ERR_HIP, "e3x_edges_build: reading back the flags failed");
+    if (h[kBadSrc]) return e3x::fail(E3X_ERR_INDEX, "index out of range in gather source");
+    if (h[kBadDst]) return e3x::fail(E3X_ERR_INDEX, "index out of range in scatter destination");
+    *grouped = !h[kUnsorted];
+    if (!h[kOverflow]) {
+      *shared_pairs = ranks ? h[kScore] : 0;
+      order_done = ranks;
+    } else {  // a row too long to be put in order here
+      const int rc = e3x_csr_build(dst, dst_bits, E, num_nodes, rowptr, perm, workspace, workspace_bytes, stream);
+      if (rc != E3X_OK) return rc;
+    }
+  } else {
+    int rc = e3x_index_check(src, src_bits, E, num_src_nodes, stream);
+    if (rc != E3X_OK) return rc;
+    if ((rc = e3x_csr_build(dst, dst_bits, E, num_nodes, rowptr, perm, workspace, workspace_bytes, stream)) != E3X_OK) return rc;
+    if (E > 1) {
+      int* flag = (int*)workspace;
+      hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(kBlock), 0, st, flag, 1);
+      if (dst_bits == 64) hipLaunchKernelGGL((unsorted_kernel<long long>), dim3(grid_for(E, kBlock)), dim3(kBlock), 0, st, (const long long*)dst, (long long)E, flag);
+      else hipLaunchKernelGGL((unsorted_kernel<int>), dim3(grid_for(E, kBlock)), dim3(kBlock), 0, st, (const int*)dst, (long long)E, flag);
+      int h = 0;
+      if (hipMemcpyAsync(&h, flag, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
+        return e3x::fail(E3X_ERR_HIP, "e3x_edges_build: reading back the flags failed");
+      *grouped = !h;
+    }
+  }
+  if (row_order && !order_done)
+    return e3x_row_order_build(src, src_bits, rowptr, perm, E, num_nodes, num_src_nodes, row_order, shared_pairs, workspace, workspace_bytes, stream);
   return E3X_OK;
 }
 

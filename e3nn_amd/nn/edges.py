@@ -107,42 +107,31 @@ class DstSortedEdges:
         L = _lib.lib()
         with torch.cuda.device(dev):
             st = _lib.stream_ptr(dev)
-            _lib.check(L.e3x_index_check(_lib.ptr(self.edge_src), self.edge_src.element_size() * 8, E, self.num_src_nodes, st))
             self.rowptr = torch.empty(self.num_nodes + 1, dtype=torch.int32, device=dev)
             self.perm = torch.empty(E, dtype=torch.int32, device=dev)
-            ws_bytes = L.e3x_csr_workspace_bytes(E, self.num_nodes)
+            # rows that share their smallest source are processed next to each other (they share most of their
+            # sources, which then sit in L2): locality taken from the graph, not from the caller's node numbering
+            self.row_order = None
+            if locality_order and self.num_nodes > 0:
+                self.row_order = torch.empty(self.num_nodes, dtype=torch.int32, device=dev)
+            ws_bytes = L.e3x_edges_workspace_bytes(E, self.num_nodes)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            grouped, pairs = ctypes.c_int32(0), ctypes.c_int32(0)
             _lib.check(
-                L.e3x_csr_build(
-                    _lib.ptr(self.edge_dst), self.edge_dst.element_size() * 8, E, self.num_nodes, _lib.ptr(self.rowptr),
-                    _lib.ptr(self.perm), _lib.ptr(ws), ws_bytes, st,
+                L.e3x_edges_build(
+                    _lib.ptr(self.edge_src), self.edge_src.element_size() * 8, _lib.ptr(self.edge_dst), self.edge_dst.element_size() * 8,
+                    E, self.num_nodes, self.num_src_nodes, _lib.ptr(self.rowptr), _lib.ptr(self.perm), _lib.ptr(self.row_order),
+                    ctypes.byref(grouped), ctypes.byref(pairs), _lib.ptr(ws), ws_bytes, st,
                 )  # fmt: skip
             )
             # A list that is already grouped by destination (what neighbour searches emit: torch_cluster's
             # radius_graph, which the reference's models call, returns its pairs sorted by the query node) is walked
             # by position: the stable sort is then the identity and the kernels are handed no permutation, so that
             # per-edge rows are read as one contiguous run per destination.
-            self.walk_perm = self.perm
-            if E > 1 and bool((self.edge_dst[1:] >= self.edge_dst[:-1]).all()):
-                self.walk_perm = None
-            # rows that share their smallest source are processed next to each other (they share most of their
-            # sources, which then sit in L2): locality taken from the graph, not from the caller's node numbering
-            self.row_order = None
-            if locality_order and self.num_nodes > 0:
-                self.row_order = torch.empty(self.num_nodes, dtype=torch.int32, device=dev)
-                ws_bytes = L.e3x_row_order_workspace_bytes(self.num_nodes)
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-                pairs = ctypes.c_int32(0)
-                _lib.check(
-                    L.e3x_row_order_build(
-                        _lib.ptr(self.edge_src), self.edge_src.element_size() * 8, _lib.ptr(self.rowptr), _lib.ptr(self.perm),
-                        E, self.num_nodes, self.num_src_nodes, _lib.ptr(self.row_order), ctypes.byref(pairs), _lib.ptr(ws),
-                        ws_bytes, st,
-                    )  # fmt: skip
-                )
+            self.walk_perm = None if E > 1 and grouped.value else self.perm
+            if self.row_order is not None:
                 # rows that follow each other in the order and agree in their two smallest sources: next to nothing
                 # on a graph without neighbourhood structure, where the order would only scatter the rows
                 self.locality_score = pairs.value / self.num_nodes
                 if locality_order == "auto" and self.locality_score < 0.02:
                     self.row_order = None
-

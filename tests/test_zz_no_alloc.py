@@ -51,6 +51,61 @@ def test_static_scratch_matches_workspace_entry_point_twice_in_a_row():
             assert np.array_equal(rp_s, rp_r) and np.array_equal(pm_s, pm_r), (E, N)
 
 
+def _graph(kind, E, N, n_src, g):
+    src, dst = torch.randint(0, n_src, (E,), generator=g), torch.randint(0, N, (E,), generator=g)
+    if kind == "grouped":
+        dst = torch.sort(dst)[0]
+    if kind == "star":  # one row longer than a wavefront puts in order: the general sort
+        dst[: E // 2] = N // 2
+    if kind == "long":  # the longest that it does
+        dst = dst % (N - 1) + 1
+        dst[torch.randperm(E, generator=g)[:1024]] = 0
+    if kind == "band":  # rows that share sources
+        src = (dst + torch.randint(-3, 4, (E,), generator=g)) % n_src
+    if kind == "negative":
+        src = src - n_src * torch.randint(0, 2, (E,), generator=g)
+    return src, dst
+
+
+@pytest.mark.parametrize("kind,E,N,n_src", [
+    ("random", 1, 1, 1), ("random", 2, 5, 3), ("random", 5000, 63, 70), ("random", 4097, 4096, 4096), ("random", 9000, 4097, 4097),
+    ("grouped", 6001, 300, 300), ("band", 20000, 2500, 2500), ("star", 6000, 50, 50), ("long", 9000, 400, 400), ("negative", 3000, 200, 150),
+    ("random", 300, 1, 40), ("random", 30000, 16384, 16384), ("random", 30000, 16385, 16385), ("random", 3000, 100, 70000), ("band", 60, 8200, 8200),
+])  # fmt: skip
+@pytest.mark.parametrize("src_t,dst_t", [(torch.int64, torch.int64), (torch.int32, torch.int64)])
+def test_edge_list_in_one_call_matches_the_separate_entry_points(kind, E, N, n_src, src_t, dst_t):
+    import ctypes
+
+    L = _lib.lib()
+    src, dst = (t.to(DEV) for t in _graph(kind, E, N, n_src, torch.Generator().manual_seed(E + N)))
+    src, dst = src.to(src_t), dst.to(dst_t)
+    st, bits = _lib.stream_ptr(DEV), (src.element_size() * 8, dst.element_size() * 8)
+    want_ptr, want_perm = (torch.from_numpy(a).to(DEV) for a in _build(dst, N, static=False))
+    want_order, want_pairs = torch.empty(N, dtype=torch.int32, device=DEV), ctypes.c_int32(-1)
+    n = L.e3x_row_order_workspace_bytes(N)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    _lib.check(L.e3x_row_order_build(_lib.ptr(src), bits[0], _lib.ptr(want_ptr), _lib.ptr(want_perm), E, N, n_src, _lib.ptr(want_order),
+                                     ctypes.byref(want_pairs), _lib.ptr(ws), n, st))  # fmt: skip
+    for with_order in (True, False):
+        rowptr, perm, order = (torch.full((k,), -7, dtype=torch.int32, device=DEV) for k in (N + 1, E, N))
+        grouped, pairs = ctypes.c_int32(-1), ctypes.c_int32(-1)
+        n = L.e3x_edges_workspace_bytes(E, N)
+        ws = torch.full((n,), 255, dtype=torch.uint8, device=DEV)
+        _lib.check(L.e3x_edges_build(_lib.ptr(src), bits[0], _lib.ptr(dst), bits[1], E, N, n_src, _lib.ptr(rowptr), _lib.ptr(perm),
+                                     _lib.ptr(order) if with_order else None, ctypes.byref(grouped), ctypes.byref(pairs), _lib.ptr(ws), n, st))  # fmt: skip
+        assert torch.equal(rowptr, want_ptr) and torch.equal(perm, want_perm)
+        assert grouped.value == int(bool((dst[1:] >= dst[:-1]).all()))
+        if with_order:
+            assert torch.equal(order, want_order) and pairs.value == want_pairs.value
+    for bad_src, bad_dst in ((n_src, 0), (-n_src - 1, 0), (0, N), (0, -1)):
+        s, d = src.clone(), dst.clone()
+        s[E // 2], d[E // 2] = bad_src, bad_dst
+        rc = L.e3x_edges_build(_lib.ptr(s), bits[0], _lib.ptr(d), bits[1], E, N, n_src, _lib.ptr(rowptr), _lib.ptr(perm), _lib.ptr(order),
+                               ctypes.byref(grouped), ctypes.byref(pairs), _lib.ptr(ws), n, st)  # fmt: skip
+        with pytest.raises(IndexError, match="gather source" if bad_dst == 0 else "scatter destination"):
+            _lib.check(rc)
+
+
 def test_static_scratch_reports_bad_indices_and_clears_the_flag():
     with torch.cuda.device(DEV):
         bad = torch.tensor([0, 3, 9, 1], dtype=torch.int64, device=DEV)
