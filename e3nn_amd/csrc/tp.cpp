@@ -794,16 +794,18 @@ bool mfma_dw_fits(const e3x_plan& P) {
 // Tables of the matrix-core weight-gradient kernel: per path the M operand is the input with the smaller l.
 
 int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
+  bool split_operands = false;
+  int obmax = 1, nrmax = 1;
   std::ostringstream s, nzs, ps;
   emit_header(s, P);
   if (env_int("E3X_DW_ZC", 0)) s << "#define E3X_DW_ZC " << env_int("E3X_DW_ZC", 0) << "\n";
   if (std::getenv("E3X_DW_SYNTH")) s << "#define E3X_DW_SYNTH " << env_int("E3X_DW_SYNTH", 1) << "\n";
   if (std::getenv("E3X_DW_PAIR")) s << "#define E3X_DW_PAIR " << env_int("E3X_DW_PAIR", 1) << "\n";
   {
-    // Split operands (six bf16 products per fp32 one) pay where the 64 x 64 tiles are full: the vector ALU then
-    // prepares operands for 4 x 12 matrix instructions per pass; with 32-wide blocks half of them multiply padding and
-    // the fp32 instruction, which needs no splitting, is faster (measured: 128-wide blocks 73 -> 60 ms, the 32-wide
-    // node-wise layers of the convolution block 0.71 -> 0.78 ms).  A 32-channel path whose outer indices go two to a
+    // Split operands (three fp16 products per fp32 one) pay where the 64 x 64 tiles are full: the vector ALU then
+    // prepares operands for 4 x 6 matrix instructions per pass; with 32-wide blocks half of them multiply padding and
+    // the fp32 instruction, which needs no splitting, is faster (measured with six products: 128-wide blocks 73 -> 60
+    // ms, the 32-wide node-wise layers of the convolution block 0.71 -> 0.78 ms).  A 32-channel path whose outer indices go two to a
     // tile (E3X_DW_PAIR in the template) has no padded columns either: those layers 0.25 -> 0.19 and 0.11 -> 0.09 ms.
     bool full = true;
     const bool pairing = env_int("E3X_DW_PAIR", 1) != 0;
@@ -819,7 +821,8 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
     }
     const int split = env_int("E3X_DW_SPLIT", full ? 1 : 0);
     s << "#define E3X_DW_SPLIT " << split << "\n";
-    P.arithmetic_dw = split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
+    split_operands = split != 0;
+    P.arithmetic_dw = split ? "fp16 matrix instruction, three products of scaled two-way split operands" : "fp32 matrix instruction";
   }
   if (std::getenv("E3X_DW_OCC")) s << "#define E3X_DW_OCC " << env_int("E3X_DW_OCC", 3) << "\n";
   int n_nz = 0, n_path = 0, dkmax = 1, drmax = 1;
@@ -848,7 +851,10 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
     const int K = k_is_x2 ? b.mul : a.mul, O = k_is_x2 ? a.mul : b.mul;
     dkmax = std::max(dkmax, dK);
     drmax = std::max(drmax, dR);
-    const int ob = O % 4 == 0 ? 4 : (O % 2 == 0 ? 2 : 1);  // outer indices per workgroup
+    // Outer indices per workgroup.  On split operands 8: what a chunk of rows costs before its first matrix step (loads,
+    // largest magnitudes, scaling) is shared by twice the passes of 4 (128-wide blocks, 65 536 rows: 51.2 -> 43.8 ms).
+    const int ob = split_operands && O % 8 == 0 ? 8 : O % 4 == 0 ? 4 : (O % 2 == 0 ? 2 : 1);
+    obmax = std::max(obmax, ob), nrmax = std::max(nrmax, std::max(d3, dK));
     ps << "  {" << (k_is_x2 ? "true" : "false") << ", " << (k_is_x2 ? P.off2[p.in2] : P.off1[p.in1]) << ", " << dK << ", "
        << K << ", " << (k_is_x2 ? P.off1[p.in1] : P.off2[p.in2]) << ", " << dR << ", " << O << ", " << ob << ", " << P.offo[p.out]
        << ", " << d3 << ", " << W << ", " << p.woff << ", " << (k_is_x2 ? stride_v : stride_u) << ", "
@@ -856,7 +862,7 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
     tiles = std::max(tiles, (long long)((K + 63) / 64) * ((W + 63) / 64) * (O / ob));
     ++n_path;
   }
-  s << "constexpr int WT = 64, OBMAX = 4, DKMAX = " << dkmax << ", DRMAX = " << drmax << ";\n";
+  s << "constexpr int WT = 64, OBMAX = " << obmax << ", NRMAX = " << nrmax << ", DKMAX = " << dkmax << ", DRMAX = " << drmax << ";\n";
   s << "struct Nz { int s, r, k; float c; };\nconstexpr int N_NZ = " << n_nz << ";\nconstexpr Nz nz[N_NZ] = {\n"
     << nzs.str() << "};\n";
   s << "struct DPath { bool k_is_x2; int koff, dK, K, roff, dR, O, OB, goff, d3, W; long long wbase, wk_stride, wo_stride; "

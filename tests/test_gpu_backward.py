@@ -126,6 +126,31 @@ def test_message_gradients_grouped_by_destination(maker, degrees, idx, grouped):
         assert torch.equal(again[0], gx) and torch.equal(again[1], gw)
 
 
+@pytest.mark.parametrize("maker,Z", [(ks.mfma_full_tiles, 1), (ks.mfma_full_tiles, 31), (ks.mfma_full_tiles, 33), (ks.mfma_full_tiles, 400), (ks.node_block, 65)])
+@pytest.mark.parametrize("ramp", [0, 6, -6])
+def test_uvw_weight_gradient_on_pairs_of_fp16_operands(maker, Z, ramp):
+    # edges of the chunks of 32 rows; scales that grow (the accumulators are rescaled chunk by chunk) and that fall
+    tp = maker()
+    spec = oracle_spec(tp)
+    scale = torch.logspace(-ramp / 2, ramp / 2, Z)[:, None]
+    x1, x2, g = seeded(Z, tp.irreps_in1.dim, seed=1) * scale, seeded(Z, tp.irreps_in2.dim, seed=2), seeded(Z, tp.irreps_out.dim, seed=3) * 1e-20
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
+    plan = tp._plan(torch.float32)
+    got = plan.backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True)
+    assert "fp16" in plan.arithmetic_weight_gradient
+    # sums of at most 400 x 25 products: 4e-7 of the 2-norm from fp32 accumulation, 6e-8 of a term from the pairs
+    assert float((got.double().cpu() - ref).norm() / ref.norm()) < 1e-6
+    # an infinity spoils the gradients that it enters, and only these
+    if tp.irreps_in1.dim == tp.irreps_in1[0].dim + tp.irreps_in1[1].dim and Z > 1:
+        x1[0, 0] = float("inf")
+        bad = plan.backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True)
+        per_u = torch.isfinite(bad).cpu()
+        t = tp.instructions[0]
+        block = per_u[: t.path_shape[0] * t.path_shape[1] * t.path_shape[2]].view(t.path_shape)
+        assert t.i_in1 == 0 and not block[0].any() and block[1:].all()
+
+
 @pytest.mark.parametrize("maker,Z", [(lambda: ks.golden_tp("fctp_small_cfg5_like"), 6), (ks.cfg1, 50), (ks.mfma_small, 70),
                                      (lambda: ks.golden_tp("fctp_per_sample_weights"), 5), (ks.node_fctp, 90), (ks.radial_layer, 77), (ks.node_wide_out, 45), (ks.node_narrow, 40)])  # fmt: skip
 def test_uvw_input_gradients(maker, Z):
