@@ -140,7 +140,7 @@ class _BlockModule(torch.nn.Module):
         Z = x.shape[0]
         res = torch.empty(Z, in_dim if grad_out is not None else out_dim, dtype=x.dtype, device=x.device)
         L = _lib.lib()
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             if grad_out is None:
                 rc = L.e3x_gate_forward(self._acts, self._n[0], self._gates, self._n[1], _lib.ptr(x), _lib.ptr(res), Z, in_dim,
                                         out_dim, _storage(x), _lib.stream_ptr(x.device))  # fmt: skip
@@ -155,7 +155,7 @@ class _BlockModule(torch.nn.Module):
         in_dim, out_dim = self._dims
         Z = x.shape[0]
         gx, gg = torch.empty_like(x), torch.empty_like(grad_out)
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             rc = _lib.lib().e3x_gate_backward2(self._acts, self._n[0], self._gates, self._n[1], _lib.ptr(x), _lib.ptr(grad_out),
                                                _lib.ptr(cot), _lib.ptr(gg), _lib.ptr(gx), Z, in_dim, out_dim, _storage(x), _lib.stream_ptr(x.device))  # fmt: skip
         _lib.check(rc)

@@ -48,7 +48,7 @@ class DstSortedEdges:
         if self._src_rows is None and self.num_edges > 0 and os.environ.get("E3X_SRC_ROWS", "1") != "0":
             dev = self.edge_src.device
             rows = torch.empty(self.num_edges, dtype=torch.int32, device=dev)
-            with torch.cuda.device(dev):
+            with _lib.on_device(dev):
                 _lib.check(
                     _lib.lib().e3x_src_rows_build(
                         _lib.ptr(self.edge_src), self.edge_src.element_size() * 8, _lib.ptr(self.perm), self.num_edges,
@@ -105,7 +105,7 @@ class DstSortedEdges:
         self.num_edges = E = edge_src.numel()
         dev = edge_src.device
         L = _lib.lib()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             st = _lib.stream_ptr(dev)
             self.rowptr = torch.empty(self.num_nodes + 1, dtype=torch.int32, device=dev)
             self.perm = torch.empty(E, dtype=torch.int32, device=dev)

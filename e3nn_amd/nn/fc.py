@@ -236,7 +236,7 @@ class _FusedPlan:
     def backward_w(self, x, g):
         hs = self._args[0]
         gw = torch.empty(hs[0], hs[1], device=x.device, dtype=torch.float32)
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             _lib.check(
                 _lib.lib().e3x_fc_backward_w(self.handle, _lib.ptr(x), _lib.ptr(g), _lib.ptr(gw), x.shape[0], _lib.stream_ptr(x.device))
             )
@@ -249,7 +249,7 @@ class _FusedPlan:
         ws = torch.empty(self.workspace_bytes, device=x.device, dtype=torch.uint8)
         ptrs = (ctypes.c_void_p * len(weights))(*[w.data_ptr() for w in weights])
         assert z is None or (z.shape == out.shape and z.is_contiguous() and z.dtype == torch.float32)
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             _lib.check(
                 L.e3x_fc_forward_epilogue(self.handle, _lib.ptr(x), ptrs, _lib.ptr(z) if z is not None else None, _lib.ptr(out),
                                           Z, _lib.ptr(ws), self.workspace_bytes, _lib.stream_ptr(x.device))

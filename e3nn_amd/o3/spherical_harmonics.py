@@ -4,6 +4,7 @@ API of the reference's ``e3nn.o3.SphericalHarmonics`` / ``e3nn.o3.spherical_harm
 (e3nn/o3/_spherical_harmonics.py:14-112, :115-190).
 """
 import ctypes
+import functools
 from typing import Any, List, Union
 
 import torch
@@ -15,9 +16,40 @@ from .irreps import Irreps
 _NORMALIZATION = {"integral": _lib.NORM_INTEGRAL, "component": _lib.NORM_COMPONENT, "norm": _lib.NORM_NORM}
 
 
+@functools.lru_cache(maxsize=64)
+def _degrees(ls):
+    return (ctypes.c_int32 * len(ls))(*ls)
+
+
+def _rows(x):
+    """``x[..., 3]`` as contiguous rows."""
+    return x if x.ndim == 2 and x.shape[1] == 3 and x.is_contiguous() else x.reshape(-1, 3).contiguous()
+
+
+def _forward(x, ls, normalize, normalization):
+    if not x.is_cuda:
+        raise RuntimeError("e3nn_amd.o3.spherical_harmonics runs on the GPU only; got a CPU tensor")
+    if x.dtype != torch.float32:
+        raise TypeError(f"spherical_harmonics kernel supports float32 input, got {x.dtype}")
+    xyz = _rows(x)
+    n, n_out = xyz.shape[0], sum(2 * l + 1 for l in ls)
+    out = torch.empty(n, n_out, dtype=x.dtype, device=x.device)
+    _launch("e3x_sh_forward", ls, normalize, normalization, n, x.device, xyz, out)
+    return out if x.ndim == 2 and n == x.shape[0] else out.reshape(x.shape[:-1] + (n_out,))
+
+
+def _backward(x, g, ls, normalize, normalization):
+    """``(grad_x <g, Y(x)>, rows of x, rows of g)``."""
+    xyz = _rows(x)
+    g2 = g.reshape(xyz.shape[0], sum(2 * l + 1 for l in ls)).contiguous()  # the width spelled out: -1 is ambiguous for n = 0
+    gx = torch.empty_like(xyz)
+    _launch("e3x_sh_backward", ls, normalize, normalization, xyz.shape[0], x.device, xyz, g2, gx)
+    return gx if x.ndim == 2 and x.shape[1] == 3 else gx.reshape(x.shape[:-1] + (3,)), xyz, g2
+
+
 def _launch(entry, ls, normalize, normalization, n, device, *tensors):
-    arr = (ctypes.c_int32 * len(ls))(*ls)
-    with torch.cuda.device(device):
+    arr = _degrees(ls)
+    with _lib.on_device(device):
         _lib.check(
             getattr(_lib.lib(), entry)(
                 arr, len(ls), int(bool(normalize)), _NORMALIZATION[normalization], *[_lib.ptr(t) for t in tensors], n,
@@ -29,24 +61,15 @@ def _launch(entry, ls, normalize, normalization, n, device, *tensors):
 class _SphericalHarmonicsFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, ls, normalize, normalization):
-        if not x.is_cuda:
-            raise RuntimeError("e3nn_amd.o3.spherical_harmonics runs on the GPU only; got a CPU tensor")
-        if x.dtype != torch.float32:
-            raise TypeError(f"spherical_harmonics kernel supports float32 input, got {x.dtype}")
-        batch = x.shape[:-1]
-        xyz = x.reshape(-1, 3).contiguous()
-        n = xyz.shape[0]
-        n_out = sum(2 * l + 1 for l in ls)
-        out = torch.empty(n, n_out, dtype=x.dtype, device=x.device)
-        _launch("e3x_sh_forward", ls, normalize, normalization, n, x.device, xyz, out)
+        out = _forward(x, ls, normalize, normalization)
         ctx.save_for_backward(x)
         ctx.cfg = (ls, normalize, normalization)
-        return out.reshape(batch + (n_out,))
+        return out
 
     @staticmethod
     def backward(ctx, g):
         (x,) = ctx.saved_tensors
-        return _ShBackwardFn.apply(x, g, *ctx.cfg), None, None, None
+        return _sh_backward(x, g, *ctx.cfg), None, None, None
 
 
 class _ShBackwardFn(torch.autograd.Function):
@@ -55,15 +78,10 @@ class _ShBackwardFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, g, ls, normalize, normalization):
-        batch = x.shape[:-1]
-        xyz = x.reshape(-1, 3).contiguous()
-        n = xyz.shape[0]
-        g2 = g.reshape(n, sum(2 * l + 1 for l in ls)).contiguous()  # the width spelled out: -1 is ambiguous for n = 0
-        gx = torch.empty_like(xyz)
-        _launch("e3x_sh_backward", ls, normalize, normalization, n, x.device, xyz, g2, gx)
+        gx, xyz, g2 = _backward(x, g, ls, normalize, normalization)
         ctx.save_for_backward(xyz, g2)
-        ctx.cfg = (ls, normalize, normalization, batch, g.shape)
-        return gx.reshape(batch + (3,))
+        ctx.cfg = (ls, normalize, normalization, x.shape[:-1], g.shape)
+        return gx
 
     @staticmethod
     @once_differentiable
@@ -80,11 +98,17 @@ class _ShBackwardFn(torch.autograd.Function):
 
 
 def _sh_forward(x, ls, normalize, normalization):
-    return _SphericalHarmonicsFn.apply(x, tuple(ls), normalize, normalization)
+    ls = tuple(ls)
+    if _lib.unrecorded(x):
+        return _forward(x, ls, normalize, normalization)
+    return _SphericalHarmonicsFn.apply(x, ls, normalize, normalization)
 
 
 def _sh_backward(x, g, ls, normalize, normalization):
-    return _ShBackwardFn.apply(x, g, tuple(ls), normalize, normalization)
+    ls = tuple(ls)
+    if _lib.unrecorded(x, g):
+        return _backward(x, g, ls, normalize, normalization)[0]
+    return _ShBackwardFn.apply(x, g, ls, normalize, normalization)
 
 
 class SphericalHarmonics(torch.nn.Module):
@@ -141,7 +165,7 @@ class SphericalHarmonics(torch.nn.Module):
             raise NotImplementedError("spherical_harmonics maximum l implemented is 12, send us an email to ask for more")
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return _SphericalHarmonicsFn.apply(x, tuple(self._ls_list), self.normalize, self.normalization)
+        return _sh_forward(x, self._ls_list, self.normalize, self.normalization)
 
 
 def spherical_harmonics(

@@ -104,7 +104,7 @@ class _Plan:
         if self.family == "uvw_node":
             # rows and weights are read with 16-byte loads
             x1, w = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, w))
-        with torch.cuda.device(x1.device):
+        with _lib.on_device(x1.device):
             _lib.check(
                 _lib.lib().e3x_tp_forward_ws(
                     self.handle, _lib.ptr(x1), _lib.ptr(x2), _lib.ptr(w), _lib.ptr(out), Z,
@@ -117,7 +117,7 @@ class _Plan:
         """``out[n] = sum_{e: edges groups e under n} TP(table[gather_idx[e]], edge_attr[e], w[e])``."""
         out = torch.empty(edges.num_nodes, self.out_dim, dtype=table.dtype, device=table.device)
         L = _lib.lib()
-        with torch.cuda.device(table.device):
+        with _lib.on_device(table.device):
             # scratch of the matrix-core message kernel (the node table in operand order); 0 for every other plan
             ws_bytes = L.e3x_tp_gather_scatter_workspace_bytes(self.handle, num_table_rows)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=table.device) if ws_bytes else None
@@ -141,7 +141,7 @@ class _Plan:
             return None
         _lib.check(rc)
         out = torch.empty(edges.num_nodes, self.out_dim, dtype=table.dtype, device=table.device)
-        with torch.cuda.device(table.device):
+        with _lib.on_device(table.device):
             _lib.check(
                 L.e3x_tp_gather_scatter_sh(
                     self.handle, _lib.ptr(table), _lib.ptr(edge_vec), _lib.ptr(w), _lib.ptr(gather_idx),
@@ -168,7 +168,7 @@ class _Plan:
         out = torch.empty(edges.num_nodes, self.out_dim, dtype=table.dtype, device=table.device)
         grad_w = torch.empty(edges.num_edges, self.weight_numel, dtype=table.dtype, device=table.device)
         grad_x2 = torch.empty_like(edge_attr) if want_x2 else None
-        with torch.cuda.device(table.device):
+        with _lib.on_device(table.device):
             _lib.check(
                 L.e3x_tp_gather_scatter_grad_w(
                     self.handle, _lib.ptr(table), _lib.ptr(edge_attr), _lib.ptr(w), _lib.ptr(row_x), _lib.ptr(gather_idx),
@@ -191,7 +191,7 @@ class _Plan:
         grad_x, grad_w = torch.empty_like(node_x), torch.empty_like(w)
         grad_x2 = torch.empty_like(edge_attr) if want_x2 else None
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=node_x.device)
-        with torch.cuda.device(node_x.device):
+        with _lib.on_device(node_x.device):
             _lib.check(
                 L.e3x_tp_message_backward(
                     self.handle, _lib.ptr(node_x), _lib.ptr(edge_attr), _lib.ptr(w), _lib.ptr(grad_out), _lib.ptr(edges.edge_src),
@@ -208,7 +208,7 @@ class _Plan:
         """``gather_scatter`` with the per-edge weights computed in the kernel by the two-layer network
         ``(edge_scalars, w1, w2)``; returns None when the library does not take this instruction set or network."""
         out = torch.empty(edges.num_nodes, self.out_dim, dtype=table.dtype, device=table.device)
-        with torch.cuda.device(table.device):
+        with _lib.on_device(table.device):
             rc = _lib.lib().e3x_tp_gather_scatter_radial(
                 self.handle, _lib.ptr(table), _lib.ptr(edge_attr), _lib.ptr(edge_scalars), _lib.ptr(w1), _lib.ptr(w2),
                 w1.shape[0], w1.shape[1], act_kind, act_cst, float(variance_in), float(variance_out), _lib.ptr(gather_idx),
@@ -230,7 +230,7 @@ class _Plan:
         gw = torch.empty(shape, dtype=x1.dtype, device=x1.device)
         # the matrix-core kernel reads rows with 16-byte loads
         x1, x2, grad_out = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2, grad_out))
-        with torch.cuda.device(x1.device):
+        with _lib.on_device(x1.device):
             _lib.check(
                 _lib.lib().e3x_tp_backward_w_uvw(
                     self.handle, _lib.ptr(x1), _lib.ptr(x2), _lib.ptr(grad_out), _lib.ptr(gw), x1.shape[0],
@@ -248,7 +248,7 @@ class _Plan:
         if w is None and self.shared_weights and self.weight_numel:
             w = x1.new_zeros(self.weight_numel)
         bits = src.element_size() * 8 if src is not None else 64
-        with torch.cuda.device(x1.device):
+        with _lib.on_device(x1.device):
             _lib.check(
                 _lib.lib().e3x_tp_backward_w_x2(
                     self.handle, _lib.ptr(x1), _lib.ptr(x2), _lib.ptr(w), _lib.ptr(grad_out), _lib.ptr(src), _lib.ptr(dst),
@@ -381,6 +381,8 @@ class _TensorProductFn:
 
     @staticmethod
     def apply(x1, x2, w, tp):
+        if _lib.unrecorded(x1, x2, w):
+            return tp._plan(x1.dtype).forward(x1, x2, w)
         return _TpSlot.apply(_OUT, tp, x1, x2, w)
 
 
@@ -441,7 +443,20 @@ class _GatherScatterFn:
 
     @staticmethod
     def apply(node_x, edge_attr, w, tp, edges):
+        if _lib.unrecorded(node_x, edge_attr, w):
+            return tp._plan(node_x.dtype).gather_scatter(node_x, edge_attr, w, edges.edge_src, edges, node_x.shape[0])
         return _MessageSlot.apply(_OUT, tp, edges, node_x, edge_attr, w)
+
+
+def _gather_scatter_sh(node_x, edge_vec, w, tp, edges, normalize, normalization):
+    from .spherical_harmonics import _NORMALIZATION
+
+    out = tp._plan(node_x.dtype).gather_scatter_sh(
+        node_x, edge_vec, w, edges.edge_src, edges, node_x.shape[0], normalize, _NORMALIZATION[normalization]
+    )
+    if out is None:
+        raise NotImplementedError("forward_gather_scatter_sh needs irreps_in2 = 0e + 1o + ... up to l <= 3 (multiplicity 1)")
+    return out
 
 
 class _GatherScatterShFn(torch.autograd.Function):
@@ -452,13 +467,7 @@ class _GatherScatterShFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, node_x, edge_vec, w, tp, edges, normalize, normalization):
-        from .spherical_harmonics import _NORMALIZATION
-
-        out = tp._plan(node_x.dtype).gather_scatter_sh(
-            node_x, edge_vec, w, edges.edge_src, edges, node_x.shape[0], normalize, _NORMALIZATION[normalization]
-        )
-        if out is None:
-            raise NotImplementedError("forward_gather_scatter_sh needs irreps_in2 = 0e + 1o + ... up to l <= 3 (multiplicity 1)")
+        out = _gather_scatter_sh(node_x, edge_vec, w, tp, edges, normalize, normalization)
         ctx.tp, ctx.edges, ctx.sh = tp, edges, (normalize, normalization)
         ctx.save_for_backward(node_x, edge_vec, w)
         return out
@@ -658,10 +667,18 @@ class TensorProduct(torch.nn.Module):
 
     def _live_mode(self):
         """"uvu" / "uvw" for the two families with backward kernels, "general" for anything else, None if empty."""
-        live = {t.connection_mode for t in self.instructions if 0 not in t.path_shape}
-        if not live:
-            return None
-        return next(iter(live)) if len(live) == 1 and live <= {"uvu", "uvw"} else "general"
+        mode = self.__dict__.get("_mode", 0)  # of the instructions, which are fixed at construction
+        if mode == 0:
+            live = {t.connection_mode for t in self.instructions if 0 not in t.path_shape}
+            mode = None if not live else next(iter(live)) if len(live) == 1 and live <= {"uvu", "uvw"} else "general"
+            self.__dict__["_mode"] = mode
+        return mode
+
+    def _all_uvu(self):
+        value = self.__dict__.get("_uvu_only")
+        if value is None:
+            value = self.__dict__["_uvu_only"] = all(t.connection_mode == "uvu" for t in self.instructions)
+        return value
 
     def _plan(self, dtype: torch.dtype) -> _Plan:
         if dtype not in _DTYPES:
@@ -894,6 +911,8 @@ class TensorProduct(torch.nn.Module):
         if w.numel() and w.device != x.device:
             raise RuntimeError("weights and inputs must be on the same device")
         # broadcast all batch dimensions (everything but the last)
+        if x.ndim == 2 and y.ndim == 2 and x.shape[0] == y.shape[0] and self.shared_weights and self.weight_numel and self._live_mode() != "general":
+            return _TensorProductFn.apply(x.contiguous(), y.to(x.dtype).contiguous(), w.to(x.dtype).contiguous(), self)
         if self.shared_weights or self.weight_numel == 0:
             batch = torch.broadcast_shapes(x.shape[:-1], y.shape[:-1])
         else:
@@ -930,7 +949,7 @@ class TensorProduct(torch.nn.Module):
         Pass a prebuilt ``DstSortedEdges`` as ``edges`` to amortise the index preprocessing
         over several calls on the same graph.
         """
-        if any(t.connection_mode != "uvu" for t in self.instructions):
+        if not self._all_uvu():
             raise NotImplementedError("forward_gather_scatter needs an all-uvu TensorProduct")
         torch._assert(node_x.ndim == 2 and node_x.shape[-1] == self._in1_dim, "Incorrect shape for node_x")
         torch._assert(edge_attr.ndim == 2 and edge_attr.shape[-1] == self._in2_dim, "Incorrect shape for edge_attr")
@@ -956,7 +975,7 @@ class TensorProduct(torch.nn.Module):
         weight, edges=edges)`` with the harmonics formed inside the kernel: ``edge_vec[E, 3]`` (float32) is read in
         place of the stored ``[E, (lmax + 1)^2]`` attributes.  Needs ``irreps_in2 = 0e + 1o + ...`` up to ``lmax <= 3``
         with multiplicity 1 (what the reference's convolutions feed the product, e3nn/nn/models/gate_points_2101.py:329)."""
-        if any(t.connection_mode != "uvu" for t in self.instructions):
+        if not self._all_uvu():
             raise NotImplementedError("forward_gather_scatter_sh needs an all-uvu TensorProduct")
         assert normalization in ["integral", "component", "norm"]
         torch._assert(node_x.ndim == 2 and node_x.shape[-1] == self._in1_dim, "Incorrect shape for node_x")
@@ -972,7 +991,8 @@ class TensorProduct(torch.nn.Module):
             w = w.to(node_x.dtype).contiguous()
         else:
             w = node_x.new_empty(0)
-        return _GatherScatterShFn.apply(node_x.contiguous(), edge_vec.contiguous(), w, self, edges, bool(normalize), normalization)
+        args = (node_x.contiguous(), edge_vec.contiguous(), w, self, edges, bool(normalize), normalization)
+        return _gather_scatter_sh(*args) if _lib.unrecorded(*args[:3]) else _GatherScatterShFn.apply(*args)
 
     def _radial_description(self, net):
         """Arguments of the library's fused radial-network kernel for ``net``; None when ``net`` is not a two-layer

@@ -442,3 +442,21 @@ def test_code_object_cache_remembers_rejected_sources_and_honours_no_jit(tmp_pat
     monkeypatch.delenv("E3X_UVW16_NBUF")
     plan = tp._plan(torch.bfloat16)  # the defaults build, into the same directory
     assert (tmp_path / (plan.key + ".hsaco")).exists() and plan.family == "uvw_mfma"
+
+
+def test_calls_skip_their_autograd_function_only_where_nothing_records():
+    from torch.autograd import forward_ad
+
+    from e3nn_amd._lib import unrecorded
+
+    a, b = torch.ones(2, 3), torch.ones(2, 3, requires_grad=True)
+    assert unrecorded(a) and not unrecorded(a, b)
+    with torch.no_grad():
+        assert unrecorded(a, b)
+        with forward_ad.dual_level():
+            assert not unrecorded(a)
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(unrecorded(t)), t)[1])(a)
+    torch.func.grad(lambda t: (seen.append(unrecorded(t)), t.sum())[1])(a)
+    torch.jit.trace(lambda t: (seen.append(unrecorded(t)), t + 1)[1], a, check_trace=False)
+    assert seen == [False] * 3
