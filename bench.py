@@ -28,7 +28,7 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, published
 # scaled by the 1 GiB copy kernel (profiles/uvu_sh_fused_nequip.txt), keyed by the code object the counters were read
 # on: a kernel that has changed since reports no traffic instead of a stale figure.
 NEQUIP_TRAFFIC_BYTES = {
-    "uvu_3da245a80ccf1772fda9e383+sh": (2 * 1523940 + 56250) * 1024,  # FETCH_SIZE 1523940 x 2 KiB + WRITE_SIZE 56250 KiB
+    "uvu_fd0990045e07b448628d53e7+sh": (2 * 1523934 + 56250) * 1024,  # FETCH_SIZE 1523934 x 2 KiB + WRITE_SIZE 56250 KiB
 }
 FP32_MFMA_PEAK_TFLOPS = 157.3
 BF16_MFMA_PEAK_TFLOPS = 2500.0
