@@ -802,10 +802,10 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
   if (std::getenv("E3X_DW_SYNTH")) s << "#define E3X_DW_SYNTH " << env_int("E3X_DW_SYNTH", 1) << "\n";
   if (std::getenv("E3X_DW_PAIR")) s << "#define E3X_DW_PAIR " << env_int("E3X_DW_PAIR", 1) << "\n";
   {
-    // Split operands (three fp16 products per fp32 one) pay where the 64 x 64 tiles are full: the vector ALU then
-    // prepares operands for 4 x 6 matrix instructions per pass; with 32-wide blocks half of them multiply padding and
-    // the fp32 instruction, which needs no splitting, is faster (measured with six products: 128-wide blocks 73 -> 60
-    // ms, the 32-wide node-wise layers of the convolution block 0.71 -> 0.78 ms).  A 32-channel path whose outer indices go two to a
+    // Split operands (six bf16 products per fp32 one) pay where the 64 x 64 tiles are full: the vector ALU then
+    // prepares operands for 4 x 12 matrix instructions per pass; with 32-wide blocks half of them multiply padding and
+    // the fp32 instruction, which needs no splitting, is faster (measured: 128-wide blocks 73 -> 60 ms, the 32-wide
+    // node-wise layers of the convolution block 0.71 -> 0.78 ms).  A 32-channel path whose outer indices go two to a
     // tile (E3X_DW_PAIR in the template) has no padded columns either: those layers 0.25 -> 0.19 and 0.11 -> 0.09 ms.
     bool full = true;
     const bool pairing = env_int("E3X_DW_PAIR", 1) != 0;
@@ -822,7 +822,7 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
     const int split = env_int("E3X_DW_SPLIT", full ? 1 : 0);
     s << "#define E3X_DW_SPLIT " << split << "\n";
     split_operands = split != 0;
-    P.arithmetic_dw = split ? "fp16 matrix instruction, three products of scaled two-way split operands" : "fp32 matrix instruction";
+    P.arithmetic_dw = split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
   }
   if (std::getenv("E3X_DW_OCC")) s << "#define E3X_DW_OCC " << env_int("E3X_DW_OCC", 3) << "\n";
   int n_nz = 0, n_path = 0, dkmax = 1, drmax = 1;
@@ -851,8 +851,8 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
     const int K = k_is_x2 ? b.mul : a.mul, O = k_is_x2 ? a.mul : b.mul;
     dkmax = std::max(dkmax, dK);
     drmax = std::max(drmax, dR);
-    // Outer indices per workgroup.  On split operands 8: what a chunk of rows costs before its first matrix step (loads,
-    // largest magnitudes, scaling) is shared by twice the passes of 4 (128-wide blocks, 65 536 rows: 51.2 -> 43.8 ms).
+    // Outer indices per workgroup.  On split operands 8: what a chunk of rows costs before its first matrix step is shared
+    // by twice the passes of 4 (128-wide blocks, 65 536 rows: 54.4 -> 49.0 ms, with the factors R formed once per row).
     const int ob = split_operands && O % 8 == 0 ? 8 : O % 4 == 0 ? 4 : (O % 2 == 0 ? 2 : 1);
     obmax = std::max(obmax, ob), nrmax = std::max(nrmax, std::max(d3, dK));
     ps << "  {" << (k_is_x2 ? "true" : "false") << ", " << (k_is_x2 ? P.off2[p.in2] : P.off1[p.in1]) << ", " << dK << ", "

@@ -128,8 +128,8 @@ def test_message_gradients_grouped_by_destination(maker, degrees, idx, grouped):
 
 @pytest.mark.parametrize("maker,Z", [(ks.mfma_full_tiles, 1), (ks.mfma_full_tiles, 31), (ks.mfma_full_tiles, 33), (ks.mfma_full_tiles, 400), (ks.node_block, 65)])
 @pytest.mark.parametrize("ramp", [0, 6, -6])
-def test_uvw_weight_gradient_on_pairs_of_fp16_operands(maker, Z, ramp):
-    # edges of the chunks of 32 rows; scales that grow (the accumulators are rescaled chunk by chunk) and that fall
+def test_uvw_weight_gradient_on_split_operands(maker, Z, ramp):
+    # edges of the chunks of 32 rows; scales that grow along the batch and that fall
     tp = maker()
     spec = oracle_spec(tp)
     scale = torch.logspace(-ramp / 2, ramp / 2, Z)[:, None]
@@ -138,8 +138,8 @@ def test_uvw_weight_gradient_on_pairs_of_fp16_operands(maker, Z, ramp):
     (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
     plan = tp._plan(torch.float32)
     got = plan.backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True)
-    assert "fp16" in plan.arithmetic_weight_gradient
-    # sums of at most 400 x 25 products: 4e-7 of the 2-norm from fp32 accumulation, 6e-8 of a term from the pairs
+    assert "split operands" in plan.arithmetic_weight_gradient
+    # sums of at most 400 x 25 products: 6e-7 of the 2-norm from fp32 accumulation, 6e-9 of a term from the pieces
     assert float((got.double().cpu() - ref).norm() / ref.norm()) < 1e-6
     # an infinity spoils the gradients that it enters, and only these
     if tp.irreps_in1.dim == tp.irreps_in1[0].dim + tp.irreps_in1[1].dim and Z > 1:
@@ -149,6 +149,45 @@ def test_uvw_weight_gradient_on_pairs_of_fp16_operands(maker, Z, ramp):
         t = tp.instructions[0]
         block = per_u[: t.path_shape[0] * t.path_shape[1] * t.path_shape[2]].view(t.path_shape)
         assert t.i_in1 == 0 and not block[0].any() and block[1:].all()
+
+
+@pytest.mark.parametrize("maker", [ks.mfma_full_tiles, ks.node_block])
+@pytest.mark.parametrize("sizes", ["x1 against x2", "x1 against g", "x2 against g", "masked row", "largest number", "channels"])
+def test_uvw_weight_gradient_of_numbers_of_different_sizes(maker, sizes):
+    # the sum runs over the rows: factors of very different sizes whose products are of one size, rows that contribute
+    # nothing beside large entries, channels of different sizes.  Powers of two, so that the scales are exact.
+    tp = maker()
+    spec = oracle_spec(tp)
+    Z = 300
+    x1, x2, g = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(Z, tp.irreps_out.dim, seed=3)
+    scale = [torch.ones(t.path_shape) for t in tp.instructions]
+    if "against" in sizes:
+        s = 2.0 ** torch.randint(-40, 41, (Z, 1), generator=torch.Generator().manual_seed(4))
+        factors = {"x1": x1, "x2": x2, "g": g}
+        up, down = sizes.split(" against ")
+        factors[up].mul_(s), factors[down].div_(s)
+    if sizes == "masked row":
+        x1[7] *= 2.0**33
+        g[7] = 0
+        x2[150] *= 2.0**40
+        x1[150] = 0
+    if sizes == "largest number":
+        x1[5] *= 2.0**-100
+        x2[5, 0] = 2e38
+        g[5] *= 0.1
+    if sizes == "channels":
+        def spread(x, irreps):
+            per_mul = [2.0 ** -torch.linspace(0, 27, m.mul).round() for m in irreps]
+            x.mul_(torch.cat([v.repeat_interleave(m.ir.dim) for v, m in zip(per_mul, irreps)]))
+            return per_mul
+        of1, ofo = spread(x1, tp.irreps_in1), spread(g, tp.irreps_out)
+        scale = [of1[t.i_in1][:, None, None] * ofo[t.i_out] * torch.ones(t.path_shape) for t in tp.instructions]
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True)
+    scale = torch.cat([s.double().reshape(-1) for s in scale])
+    # as above: 1e-6 of the 2-norm, every channel measured in units of its own size
+    assert float(((got.double().cpu() - ref) / scale).norm() / (ref / scale).norm()) < 1e-6
 
 
 @pytest.mark.parametrize("maker,Z", [(lambda: ks.golden_tp("fctp_small_cfg5_like"), 6), (ks.cfg1, 50), (ks.mfma_small, 70),
