@@ -582,7 +582,7 @@ bool half_fits(const e3x_plan& P) {
   return true;
 }
 constexpr int kHalfMaxBlocks = 64;  // MAX_BLOCKS of the template
-// packed weights | inverse scales and block maxima of every path
+// packed weights | block maxima and scale exponents of every path
 size_t half_workspace_bytes(const e3x_plan& P) { return (size_t)P.weight_numel * 4 + P.paths.size() * (kHalfMaxBlocks + 4) * 4 + 256; }
 
 int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
@@ -1378,14 +1378,14 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
     SubKernel* K = P->half.get();
     const unsigned n_path = (unsigned)P->paths.size();
     unsigned* w_max = (unsigned*)((char*)workspace + (size_t)P->weight_numel * 4);
-    float* w_inverse = (float*)(w_max + (size_t)n_path * kHalfMaxBlocks);
+    int* w_exp = (int*)(w_max + (size_t)n_path * kHalfMaxBlocks);
     long long entries = 0;
     for (const auto& p : P->paths) entries = std::max(entries, (long long)P->in1[p.in1].mul * P->in2[p.in2].mul * P->out[p.out].mul / 8);
     const long long blocks = (Z + 127) / 128;
     if (blocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_forward: batch too large for one launch");
     void* margs[] = {(void*)&w, (void*)&w_max};
-    void* pargs[] = {(void*)&w, (void*)&w_max, (void*)&workspace, (void*)&w_inverse};
-    void* args[] = {(void*)&x1, (void*)&x2, (void*)&workspace, (void*)&w_inverse, (void*)&out, (void*)&n_rows};
+    void* pargs[] = {(void*)&w, (void*)&w_max, (void*)&workspace, (void*)&w_exp};
+    void* args[] = {(void*)&x1, (void*)&x2, (void*)&workspace, (void*)&w_exp, (void*)&out, (void*)&n_rows};
     hipError_t err = hipModuleLaunchKernel(K->fn_max[dev], kHalfMaxBlocks, n_path, 1, 256, 1, 1, 0, st, margs, nullptr);
     if (err == hipSuccess)
       err = hipModuleLaunchKernel(K->fn_pack[dev], (unsigned)((entries + 255) / 256), n_path, 1, 256, 1, 1, 0, st, pargs, nullptr);

@@ -341,6 +341,19 @@ def test_uvw_on_pairs_of_fp16_operands(Z):
     close(g2, r2.numpy(), "d/dx2")
 
 
+@pytest.mark.parametrize("exponents", [(66, 66, -83), (-76, -76, 33), (100, -100, 0), (-60, 100, -50)])
+def test_uvw_on_pairs_of_fp16_operands_over_the_exponent_range(exponents):
+    # x1, x2 and weights of one size each whose product of all three is an ordinary number although that of two of
+    # them need not be: (x W) x, the order of the kernel without pairs, stays representable in every case
+    tp = ks.mfma_full_tiles()
+    x1, x2, w = seeded(70, tp.irreps_in1.dim, seed=1), seeded(70, tp.irreps_in2.dim, seed=2), seeded(tp.weight_numel, seed=3)
+    want = otp.tp_forward(oracle_spec(tp), x1.numpy(), x2.numpy(), w.numpy())
+    e1, e2, ew = (2.0**e for e in exponents)
+    got = tp((x1 * e1).to(DEV), (x2 * e2).to(DEV), (w * ew).to(DEV)).double().cpu().numpy() / (e1 * e2 * ew)
+    # as above: fp32 accumulation of some 1e4 products
+    assert np.linalg.norm(got - want) < 1e-6 * np.linalg.norm(want)
+
+
 def test_uvw_weight_gradient_on_the_dense_configuration():
     # the weight gradient of config 5's own instruction set (11 paths of 128 x 128 x 128, 23 M weights) on the
     # split-operand matrix-core kernel; 300 rows end inside a batch chunk of the kernel.  The float64 reference is the
