@@ -582,8 +582,13 @@ bool half_fits(const e3x_plan& P) {
   return true;
 }
 constexpr int kHalfMaxBlocks = 64;  // MAX_BLOCKS of the template
-// packed weights | block maxima and scale exponents of every path
-size_t half_workspace_bytes(const e3x_plan& P) { return (size_t)P.weight_numel * 4 + P.paths.size() * (kHalfMaxBlocks + 4) * 4 + 256; }
+// Row flags in the workspace: bit z % (32 kRowFlagWords) for row z, 512 KB for 4 million rows (rows of a larger batch that
+// share a bit are formed by the general kernel together).
+constexpr int kRowFlagWords = 1 << 17;
+// packed weights | row flags | block maxima and PathWeights (three words) of every path
+size_t half_workspace_bytes(const e3x_plan& P) {
+  return (size_t)P.weight_numel * 4 + kRowFlagWords * 4 + P.paths.size() * (kHalfMaxBlocks + 3) * 4;
+}
 
 int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   // Output channels per workgroup.  fp32: 128 (two accumulator tiles per wave, 64 KB of LDS, two workgroups per CU at
@@ -664,6 +669,7 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
     }
   }
   s << "constexpr int WT = " << wt << ", KMAX = " << kmax << ";\n";  // KMAX: the largest GEMM K extent
+  if (P.dtype == E3X_F32) s << "constexpr int ROW_FLAG_WORDS = " << kRowFlagWords << ";\n";
   for (const char* knob : {"E3X_UVW16_OS", "E3X_UVW16_NBUF", "E3X_UVW16_LEAD", "E3X_UVW16_RT2", "E3X_UVW16_RT2_ROWS", "E3X_UVW16_SHIFT", "E3X_UVW16_SHIFT1"})
     if (P.dtype == E3X_BF16 && std::getenv(knob)) s << "#define " << knob << " " << env_int(knob, 0) << "\n";
   s << "struct Nz { int s, r, k; float c; };\nconstexpr int N_NZ = " << n_nz << ";\nconstexpr Nz nz[N_NZ] = {\n"
@@ -1373,26 +1379,32 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
   }
   if ((rc = load_functions(P, dev))) return rc;
   long long n_rows = Z;
+  unsigned* row_flags = nullptr;
   if (P->half && workspace && workspace_bytes >= half_workspace_bytes(*P) &&
       !(((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)w | (uintptr_t)workspace) & 15)) {
     SubKernel* K = P->half.get();
     const unsigned n_path = (unsigned)P->paths.size();
-    unsigned* w_max = (unsigned*)((char*)workspace + (size_t)P->weight_numel * 4);
-    int* w_exp = (int*)(w_max + (size_t)n_path * kHalfMaxBlocks);
-    long long entries = 0;
-    for (const auto& p : P->paths) entries = std::max(entries, (long long)P->in1[p.in1].mul * P->in2[p.in2].mul * P->out[p.out].mul / 8);
+    row_flags = (unsigned*)((char*)workspace + (size_t)P->weight_numel * 4);
+    unsigned* w_max = row_flags + kRowFlagWords;
+    int* path_w = (int*)(w_max + (size_t)n_path * kHalfMaxBlocks);
+    int n_words = (int)std::min<long long>((Z + 63) / 64 * 2, kRowFlagWords);
+    long long columns = 0;
+    for (const auto& p : P->paths) {
+      const long long U = P->in1[p.in1].mul, V = P->in2[p.in2].mul;
+      columns = std::max(columns, std::max(U, V) * P->out[p.out].mul);  // (either input may be the K operand)
+    }
     const long long blocks = (Z + 127) / 128;
     if (blocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_forward: batch too large for one launch");
-    void* margs[] = {(void*)&w, (void*)&w_max};
-    void* pargs[] = {(void*)&w, (void*)&w_max, (void*)&workspace, (void*)&w_exp};
-    void* args[] = {(void*)&x1, (void*)&x2, (void*)&workspace, (void*)&w_exp, (void*)&out, (void*)&n_rows};
+    void* margs[] = {(void*)&w, (void*)&w_max, (void*)&path_w, (void*)&row_flags, (void*)&n_words};
+    void* pargs[] = {(void*)&w, (void*)&w_max, (void*)&workspace, (void*)&path_w};
+    void* args[] = {(void*)&x1, (void*)&x2, (void*)&workspace, (void*)&path_w, (void*)&row_flags, (void*)&out, (void*)&n_rows};
     hipError_t err = hipModuleLaunchKernel(K->fn_max[dev], kHalfMaxBlocks, n_path, 1, 256, 1, 1, 0, st, margs, nullptr);
     if (err == hipSuccess)
-      err = hipModuleLaunchKernel(K->fn_pack[dev], (unsigned)((entries + 255) / 256), n_path, 1, 256, 1, 1, 0, st, pargs, nullptr);
+      err = hipModuleLaunchKernel(K->fn_pack[dev], (unsigned)((columns + 255) / 256), n_path, 1, 256, 1, 1, 0, st, pargs, nullptr);
     if (err == hipSuccess)
       err = hipModuleLaunchKernel(K->fn_plain[dev], (unsigned)blocks, (unsigned)P->half_targets, 1, 512, 1, 1, 0, st, args, nullptr);
     if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
-    return E3X_OK;
+    // ... and the general kernel below forms the rows that this one flagged
   }
   if (needs_packed_weights(P)) {
     // the matrix-core kernel reads the weights repacked into octets of consecutive K indices
@@ -1408,7 +1420,7 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
       return fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
     w = workspace;
   }
-  void* args[] = {(void*)&x1, (void*)&x2, (void*)&w, (void*)&out, (void*)&n_rows};
+  void* args[] = {(void*)&x1, (void*)&x2, (void*)&w, (void*)&out, (void*)&n_rows, (void*)&row_flags};  // (flags: uvw_mfma, fp32)
   for (auto& K : P->subs) {
     long long blocks;
     unsigned grid_y = 1;

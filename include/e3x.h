@@ -144,10 +144,10 @@ int e3x_tp_forward(e3x_plan* plan, const void* x1, const void* x2, const void* w
  * aligned, as x1 and x2 must be).  fp32 plans of that family with input multiplicities of 64 or 128, output multiplicities
  * that are multiples of 64 and output degrees up to 2 take the workspace when it is given and x1, x2, w and it are 16-byte
  * aligned: the products are then three cross products of operands split into two fp16 pieces each, after scaling by
- * powers of two (the first or second input's row per irrep component, the weights per path), which is faster than and at
- * least as accurate as the six bf16 products of e3x_tp_forward.  An element below 2^-17 of the largest of its row and
- * irrep (a weight: of its path) then carries an error of 2^-40 of that largest one instead of a relative one.  Every other
- * plan needs no workspace and e3x_tp_forward is enough. */
+ * powers of two (the first or second input's row per irrep component, the weights per path), which is faster than the six
+ * bf16 products of e3x_tp_forward and as accurate on numbers of similar size.  Rows whose numbers differ so much in size
+ * that the pieces may not hold what a sum depends on (beside the weights of the path; decided for every row by itself)
+ * are formed by the kernel of e3x_tp_forward.  Every other plan needs no workspace and e3x_tp_forward is enough. */
 size_t e3x_tp_forward_workspace_bytes(const e3x_plan* plan);
 int e3x_tp_forward_ws(e3x_plan* plan, const void* x1, const void* x2, const void* w, void* out, int64_t Z,
                       void* workspace, size_t workspace_bytes, void* stream);

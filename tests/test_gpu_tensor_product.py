@@ -354,6 +354,56 @@ def test_uvw_on_pairs_of_fp16_operands_over_the_exponent_range(exponents):
     assert np.linalg.norm(got - want) < 1e-6 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("sizes", ["first input", "second input", "both inputs", "output"])
+def test_uvw_on_pairs_of_fp16_operands_with_channels_of_different_sizes(sizes):
+    # channels that span eight decades, made up for by the weights; the weights of the output channels span them too
+    tp = ks.mfma_full_tiles()
+    Z = 140
+    x1, x2 = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2)
+    spans = [[2.0 ** -torch.linspace(0, 27, m.mul).round() for m in ir] for ir in (tp.irreps_in1, tp.irreps_in2, tp.irreps_out)]
+    whole = [torch.cat([v.repeat_interleave(m.ir.dim) for v, m in zip(s, ir)]) for s, ir in zip(spans, (tp.irreps_in1, tp.irreps_in2, tp.irreps_out))]
+    first, second = sizes in ("first input", "both inputs"), sizes in ("second input", "both inputs")
+    ws, scale = [], torch.ones(tp.irreps_out.dim)
+    for i, t in enumerate(tp.instructions):
+        w = seeded(*t.path_shape, seed=10 + i)
+        w = w / spans[0][t.i_in1][:, None, None] if first else w
+        w = w / spans[1][t.i_in2][None, :, None] if second else w
+        ws.append((w * spans[2][t.i_out] if sizes == "output" else w).reshape(-1))
+    x1, x2 = x1 * whole[0] if first else x1, x2 * whole[1] if second else x2
+    scale = whole[2] if sizes == "output" else scale
+    w = torch.cat(ws)
+    want = otp.tp_forward(oracle_spec(tp), x1.numpy(), x2.numpy(), w.numpy()) / scale.numpy()
+    got = tp(x1.to(DEV), x2.to(DEV), w.to(DEV)).double().cpu().numpy() / scale.numpy()
+    # as above, every channel in its own size
+    assert np.linalg.norm(got - want) < 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("Z,odd", [(1, [0]), (128, [127]), (129, [128]), (300, [0, 40, 63, 64, 191, 299]), (200, range(64, 200)), (256, range(256)), (300, [])])
+def test_uvw_on_pairs_of_fp16_operands_leaves_rows_to_the_general_kernel(Z, odd):
+    # a row with one large channel per irrep is formed by the kernel of e3x_tp_forward, its neighbours are not: each
+    # row's result is that of the row alone, bit for bit
+    from e3nn_amd import _lib
+
+    tp = ks.mfma_full_tiles()
+    odd = torch.tensor(list(odd), dtype=torch.long)
+    x1, x2, w = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(tp.weight_numel, seed=3).to(DEV)
+    ordinary = tp(x1.to(DEV), x2.to(DEV), w)
+    for x, ir in ((x1, tp.irreps_in1), (x2, tp.irreps_in2)):
+        x[odd] *= torch.cat([(torch.where(torch.arange(m.mul) == 5, 1.0, 2.0**-30)).repeat_interleave(m.ir.dim) for m in ir])
+    a, b = x1.to(DEV), x2.to(DEV)
+    plain = torch.empty_like(ordinary)
+    _lib.check(_lib.lib().e3x_tp_forward(tp._plan(torch.float32).handle, _lib.ptr(a), _lib.ptr(b), _lib.ptr(w), _lib.ptr(plain), Z, _lib.stream_ptr(a.device)))
+    got = tp(a, b, w)
+    rest = torch.ones(Z, dtype=torch.bool)
+    rest[odd] = False
+    assert torch.equal(got[odd.to(DEV)], plain[odd.to(DEV)])
+    assert torch.equal(got[rest.to(DEV)], ordinary[rest.to(DEV)])
+    assert not rest.any() or not torch.equal(got[rest.to(DEV)], plain[rest.to(DEV)])  # (the two kernels do differ in the last bits)
+    # zero rows need no general kernel: exact zeros either way
+    a[Z // 2] = 0
+    assert not tp(a, b, w)[Z // 2].any()
+
+
 def test_uvw_weight_gradient_on_the_dense_configuration():
     # the weight gradient of config 5's own instruction set (11 paths of 128 x 128 x 128, 23 M weights) on the
     # split-operand matrix-core kernel; 300 rows end inside a batch chunk of the kernel.  The float64 reference is the
