@@ -611,7 +611,8 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
     if (P.in1[p.in1].mul % 64 || P.in2[p.in2].mul % 64 || P.out[p.out].mul % 64) full = false;
   const int split = P.dtype == E3X_F32 ? env_int("E3X_UVW_SPLIT", full ? 1 : 0) : 0;
   if (split && !half) s << "#define E3X_UVW_SPLIT 1\n";
-  P.arithmetic = half ? "fp16 matrix instruction, three products of scaled two-way split operands" : P.dtype != E3X_F32 ? "bf16 matrix instruction" : split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
+  if (!half)
+    P.arithmetic = P.dtype != E3X_F32 ? "bf16 matrix instruction" : split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
   if (P.dtype == E3X_F32 && !half) s << "#define E3X_UVW_KC " << env_int("E3X_UVW_KC", split ? 16 : 32) << "\n";
   if (env_int("E3X_UVW_KS", 0)) s << "#define E3X_UVW_KS " << env_int("E3X_UVW_KS", 0) << "\n";
   // two waves per SIMD (256 registers) for 128-channel tiles and for l = 3 outputs, whose seven accumulator tiles do not
@@ -1304,9 +1305,13 @@ extern "C" int e3x_tp_plan_create(const e3x_tp_desc* d, e3x_plan** out) {
     // LDS addresses as scalar operands of inline assembly: see above
     if (rc == E3X_ERR_COMPILE && !env_int("E3X_NO_JIT", 0))
       rc = e3x::get_code_object("uvw_half", "#define E3X_UVWH_SCALAR_ADDR 1\n" + src, &K->key, &K->hsaco);
-    if (rc) return rc;
-    P->key += "+" + K->key;
-    P->half = std::move(K);
+    if (rc && rc != E3X_ERR_COMPILE) return rc;
+    // (not to be had, as with a cache made without it and E3X_NO_JIT: the kernel above does everything that this one does)
+    if (!rc) {
+      P->arithmetic = "fp16 matrix instruction, three products of scaled two-way split operands";
+      P->key += "+" + K->key;
+      P->half = std::move(K);
+    }
   }
   if (P->family == "uvu" && env_int("E3X_UVU_MFMA", 1)) {
     std::unique_ptr<SubKernel> K(new SubKernel);

@@ -122,7 +122,7 @@ int e3x_tp_plan_info(const e3x_plan* plan, int64_t* weight_numel, int64_t* in1_d
 /* Which instruction forms the products of the plan's kernels: "fp32 vector ALU", "fp32 matrix instruction",
  * "bf16 matrix instruction" (bf16 storage), "bf16 matrix instruction, six products of three-way split operands" or
  * "fp16 matrix instruction, three products of scaled two-way split operands" (fp32 storage, fp32-accurate; see
- * e3x_tp_forward and e3x_tp_forward_ws).  which = 0: forward; which = 1: the "uvw" weight gradient on the
+ * e3x_tp_forward_ws, whose call with an aligned workspace the string describes).  which = 0: forward; which = 1: the "uvw" weight gradient on the
  * matrix cores, "" until that kernel has been built (e3x_tp_plan_prepare_backward_w).  No counterpart in the
  * reference; benchmarks use it to state the peak a kernel is measured against.  The string lives as long as the plan. */
 const char* e3x_tp_plan_arithmetic(const e3x_plan* plan, int which);

@@ -444,6 +444,23 @@ def test_code_object_cache_remembers_rejected_sources_and_honours_no_jit(tmp_pat
     assert (tmp_path / (plan.key + ".hsaco")).exists() and plan.family == "uvw_mfma"
 
 
+def test_plan_without_its_second_kernel(tmp_path, monkeypatch):
+    # a cache made for the kernel that every dense fp32 plan has, and no compiler: the plan runs on that kernel and says so
+    monkeypatch.setenv("E3X_KERNEL_CACHE", str(tmp_path))
+    def plan_of():
+        return o3.FullyConnectedTensorProduct("64x0e", "64x0e", "64x0e")._plan(torch.float32)
+
+    monkeypatch.setenv("E3X_UVW_HALF", "0")
+    one = plan_of()
+    monkeypatch.delenv("E3X_UVW_HALF")
+    monkeypatch.setenv("E3X_NO_JIT", "1")
+    plan = plan_of()
+    assert plan.key == one.key and plan.arithmetic == one.arithmetic and "six products" in plan.arithmetic
+    monkeypatch.setenv("E3X_NO_JIT", "0")
+    both = plan_of()
+    assert both.key.startswith(one.key + "+uvw_half") and "fp16" in both.arithmetic
+
+
 def test_calls_skip_their_autograd_function_only_where_nothing_records():
     from torch.autograd import forward_ad
 
