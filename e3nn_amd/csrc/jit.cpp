@@ -8,6 +8,7 @@
 // code objects of the old one.
 #include <atomic>
 #include <dlfcn.h>
+#include <elf.h>
 #include <fcntl.h>
 #include <spawn.h>
 #include <sys/stat.h>
@@ -207,6 +208,53 @@ int get_code_object(const std::string& family, const std::string& source, std::s
   if (std::rename(tmp_path.c_str(), path_out->c_str()) != 0)
     return fail(E3X_ERR_COMPILE, "cannot move the code object into the cache");
   return E3X_OK;
+}
+
+// The kernel descriptor <name>.kd of an AMDGPU ELF file holds the private segment size in its second word.  What the
+// compiler writes is a bundle: magic, number of entries, then (offset, size, length of the target's name, the name) each.
+long long private_segment_bytes(const std::string& path, const std::string& kernel) {
+  std::ifstream f(path, std::ios::binary);
+  std::stringstream ss;
+  ss << f.rdbuf();
+  const std::string data = ss.str();
+  auto read = [&](uint64_t at, auto* v) {
+    if (at > data.size() || data.size() - at < sizeof(*v)) return false;
+    std::memcpy(v, data.data() + at, sizeof(*v));
+    return true;
+  };
+  uint64_t elf = 0;
+  static const char kMagic[] = "__CLANG_OFFLOAD_BUNDLE__";
+  if (data.compare(0, sizeof(kMagic) - 1, kMagic) == 0) {
+    uint64_t count = 0, at = sizeof(kMagic) - 1, entry[3];
+    if (!read(at, &count)) return -1;
+    at += 8;
+    for (uint64_t i = 0; i < count && !elf; ++i) {
+      if (!read(at, &entry) || entry[2] > data.size()) return -1;
+      at += sizeof(entry);
+      if (at > data.size()) return -1;
+      if (data.substr(at, entry[2]).find("gfx950") != std::string::npos) elf = entry[0];
+      at += entry[2];
+    }
+    if (!elf) return -1;
+  }
+  Elf64_Ehdr eh;
+  if (!read(elf, &eh) || std::memcmp(eh.e_ident, ELFMAG, SELFMAG) != 0) return -1;
+  auto section = [&](uint64_t i, Elf64_Shdr* sh) { return i < eh.e_shnum && read(elf + eh.e_shoff + i * sizeof(*sh), sh); };
+  const std::string symbol = kernel + ".kd";
+  for (uint64_t i = 0; i < eh.e_shnum; ++i) {
+    Elf64_Shdr table, names, home;
+    if (!section(i, &table) || table.sh_type != SHT_DYNSYM || !section(table.sh_link, &names)) continue;
+    for (uint64_t s = 0; s < table.sh_size / sizeof(Elf64_Sym); ++s) {
+      Elf64_Sym sym;
+      if (!read(elf + table.sh_offset + s * sizeof(sym), &sym)) return -1;
+      const uint64_t at = elf + names.sh_offset + sym.st_name;
+      if (at > data.size() || data.compare(at, symbol.size() + 1, symbol.c_str(), symbol.size() + 1) != 0) continue;
+      uint32_t bytes = 0;
+      if (!section(sym.st_shndx, &home) || !read(elf + home.sh_offset + (sym.st_value - home.sh_addr) + 4, &bytes)) return -1;
+      return bytes;
+    }
+  }
+  return -1;
 }
 
 }  // namespace e3x

@@ -25,4 +25,7 @@ std::string cache_dir();
 int get_code_object(const std::string& family, const std::string& source, std::string* key_out,
                     std::string* path_out);
 
+// Private memory per lane that `kernel` of a code object asks for (spilled registers), -1 when the file does not say.
+long long private_segment_bytes(const std::string& path, const std::string& kernel);
+
 }  // namespace e3x

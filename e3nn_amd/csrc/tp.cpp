@@ -582,6 +582,11 @@ bool half_fits(const e3x_plan& P) {
   return true;
 }
 constexpr int kHalfMaxBlocks = 64;  // MAX_BLOCKS of the template
+// What the compiler makes of a set decides as well.  Private bytes per lane against the kernel of uvw_mfma.inc, which spills
+// nothing on these sets, 64 / 32 768 rows: 0 to 248 bytes 0.42 / 1.21 against 1.12 / 2.04 ms and more; 1664 bytes
+// (128x2e+128x3o times 64x1o+64x3o onto 64x2e+64x1e+64x2o) 2.04 / 5.20 against 2.18 / 6.29; 4548 bytes (an earlier state
+// of the kernel on the same set) 23.4 / 85.2.
+int half_max_private_bytes() { return env_int("E3X_UVW_HALF_PRIVATE", 2048); }
 // Row flags in the workspace: bit z % (32 kRowFlagWords) for row z, 512 KB for 4 million rows (rows of a larger batch that
 // share a bit are formed by the general kernel together).
 constexpr int kRowFlagWords = 1 << 17;
@@ -1307,7 +1312,7 @@ extern "C" int e3x_tp_plan_create(const e3x_tp_desc* d, e3x_plan** out) {
       rc = e3x::get_code_object("uvw_half", "#define E3X_UVWH_SCALAR_ADDR 1\n" + src, &K->key, &K->hsaco);
     if (rc && rc != E3X_ERR_COMPILE) return rc;
     // (not to be had, as with a cache made without it and E3X_NO_JIT: the kernel above does everything that this one does)
-    if (!rc) {
+    if (!rc && e3x::private_segment_bytes(K->hsaco, "e3x_uvw_half_plain") <= half_max_private_bytes()) {
       P->arithmetic = "fp16 matrix instruction, three products of scaled two-way split operands";
       P->key += "+" + K->key;
       P->half = std::move(K);

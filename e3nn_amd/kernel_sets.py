@@ -50,6 +50,12 @@ def mfma_full_tiles():
     return o3.FullyConnectedTensorProduct("64x0e+64x1o", "64x0e+64x1o+64x2e", "64x0e+128x1o+64x1e+64x2e")
 
 
+def dense_l3_inputs():
+    # l = 3 inputs, 128 and 64 channels: seven components of the K and of the R operand, contractions over 64 and over 128
+    # indices into one output
+    return o3.FullyConnectedTensorProduct("128x2e+128x3o", "64x1o+64x3o", "64x2e")
+
+
 def mfma_half_tiles():
     # output multiplicities 32 and 96: the matrix-core kernels end an irrep with a tile of 32 channels (bf16 storage:
     # half of the 64-channel workgroup tile computes on copies and stores nothing)
@@ -181,6 +187,7 @@ def all_tensor_products():
         ("cfg5", cfg5(), (torch.float32, torch.bfloat16)),
         ("mfma_small", mfma_small(), (torch.float32,)),
         ("mfma_full_tiles", mfma_full_tiles(), (torch.float32,)),
+        ("dense_l3_inputs", dense_l3_inputs(), (torch.float32,)),
         ("mfma_half_tiles", mfma_half_tiles(), (torch.float32, torch.bfloat16)),
         ("wide_k_l3", wide_k_l3(), (torch.float32, torch.bfloat16)),
         ("mfma_l3_out", mfma_l3_out(), (torch.float32,)),

@@ -404,6 +404,18 @@ def test_uvw_on_pairs_of_fp16_operands_leaves_rows_to_the_general_kernel(Z, odd)
     assert not tp(a, b, w)[Z // 2].any()
 
 
+@pytest.mark.parametrize("Z", [1, 129, 200])
+def test_uvw_on_pairs_of_fp16_operands_with_l3_inputs(Z):
+    tp = ks.dense_l3_inputs()
+    assert "fp16" in tp._plan(torch.float32).arithmetic
+    x1, x2, w = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(tp.weight_numel, seed=3)
+    want = otp.tp_forward(oracle_spec(tp), x1.numpy(), x2.numpy(), w.numpy())
+    got = tp(x1.to(DEV), x2.to(DEV), w.to(DEV)).double().cpu().numpy()
+    # four paths, 5 to 7 slices of 64 outer indices each: some 1500 roundings of the accumulator in a row, a random walk of
+    # 6e-8 sqrt(1500) / sqrt(3) of the running sum
+    assert np.linalg.norm(got - want) < 2e-6 * np.linalg.norm(want)
+
+
 def test_uvw_weight_gradient_on_the_dense_configuration():
     # the weight gradient of config 5's own instruction set (11 paths of 128 x 128 x 128, 23 M weights) on the
     # split-operand matrix-core kernel; 300 rows end inside a batch chunk of the kernel.  The float64 reference is the

@@ -461,6 +461,15 @@ def test_plan_without_its_second_kernel(tmp_path, monkeypatch):
     assert both.key.startswith(one.key + "+uvw_half") and "fp16" in both.arithmetic
 
 
+def test_plan_keeps_its_second_kernel_unless_it_spills(monkeypatch):
+    # 128-channel blocks up to l = 2 spill some 200 bytes per lane in the kernel on pairs, 64-channel ones nothing
+    assert "fp16" in ks.cfg5()._plan(torch.float32).arithmetic
+    monkeypatch.setenv("E3X_UVW_HALF_PRIVATE", "16")
+    plan = ks.cfg5()._plan(torch.float32)
+    assert "uvw_half" not in plan.key and "six products" in plan.arithmetic
+    assert "fp16" in ks.mfma_full_tiles()._plan(torch.float32).arithmetic
+
+
 def test_calls_skip_their_autograd_function_only_where_nothing_records():
     from torch.autograd import forward_ad
 
