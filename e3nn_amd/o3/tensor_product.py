@@ -182,19 +182,19 @@ class _Plan:
 
     def message_backward(self, node_x, edge_attr, w, grad_out, edges, want_x2=False):
         """``(grad_node_x, grad_w, grad_edge_attr or None)`` of the message step from the kernel grouped by destination;
-        None when the plan or the size of its scratch is outside what that kernel is meant for, or the scratch does not
-        fit the memory that is left."""
+        None when the plan or the size of its scratch is outside what that kernel is meant for, or the scratch and the
+        gradients beside it do not fit the memory that is left."""
         L = _lib.lib()
         ws_bytes = L.e3x_tp_message_backward_workspace_bytes(self.handle, edges.num_edges)
         if ws_bytes == 0:
             return None
         by_src = edges.transposed()
         try:
+            grad_x, grad_w = torch.empty_like(node_x), torch.empty_like(w)
+            grad_x2 = torch.empty_like(edge_attr) if want_x2 else None
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=node_x.device)
-        except torch.OutOfMemoryError:  # the kernels on the transposed plan need no scratch
+        except torch.OutOfMemoryError:  # the kernels on the transposed plan need the gradients but no scratch
             return None
-        grad_x, grad_w = torch.empty_like(node_x), torch.empty_like(w)
-        grad_x2 = torch.empty_like(edge_attr) if want_x2 else None
         with _lib.on_device(node_x.device):
             _lib.check(
                 L.e3x_tp_message_backward(

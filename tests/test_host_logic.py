@@ -470,6 +470,43 @@ def test_plan_keeps_its_second_kernel_unless_it_spills(monkeypatch):
     assert "fp16" in ks.mfma_full_tiles()._plan(torch.float32).arithmetic
 
 
+class _NoMemory:
+    """Stands in for an allocator of torch: from the ``n``-th matching call on there is no memory left."""
+
+    def __init__(self, fn, n, dtype=None):
+        self.fn, self.left, self.dtype = fn, n, dtype
+
+    def __call__(self, *args, **kw):
+        if self.dtype is None or kw.get("dtype") == self.dtype:
+            self.left -= 1
+            if self.left < 0:
+                raise torch.OutOfMemoryError("no memory left")
+        return self.fn(*args, **kw)
+
+
+@pytest.mark.parametrize("like,plain", [(0, 9), (1, 9), (2, 9), (9, 0)])
+def test_message_backward_gives_way_when_scratch_or_gradients_do_not_fit(monkeypatch, like, plain):
+    # nothing is launched: whatever does not fit, the caller is sent to the kernels without scratch
+    class Library:
+        def e3x_tp_message_backward_workspace_bytes(self, handle, edges):
+            return 1 << 20
+
+    class Edges:
+        num_edges = 5
+
+        def transposed(self):
+            return None
+
+    from e3nn_amd.o3.tensor_product import _Plan
+
+    plan = object.__new__(_Plan)
+    plan.handle = None
+    monkeypatch.setattr(_lib, "lib", Library)
+    monkeypatch.setattr(torch, "empty_like", _NoMemory(torch.empty_like, like))
+    monkeypatch.setattr(torch, "empty", _NoMemory(torch.empty, plain, torch.uint8))
+    assert plan.message_backward(torch.zeros(3, 4), torch.zeros(5, 2), torch.zeros(5, 6), torch.zeros(3, 8), Edges(), True) is None
+
+
 def test_calls_skip_their_autograd_function_only_where_nothing_records():
     from torch.autograd import forward_ad
 
