@@ -99,7 +99,12 @@ class _Plan:
         ws = None
         if ws_bytes:
             # scratch for the weights repacked for the matrix cores; the kernel reads rows with 16-byte loads
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x1.device)
+            try:
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x1.device)
+            except torch.OutOfMemoryError:
+                if x1.dtype != torch.float32:
+                    raise
+                ws_bytes = 0  # fp32: the general kernel needs none
             x1, x2 = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2))
         if self.family == "uvw_node":
             # rows and weights are read with 16-byte loads

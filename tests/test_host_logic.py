@@ -507,6 +507,34 @@ def test_message_backward_gives_way_when_scratch_or_gradients_do_not_fit(monkeyp
     assert plan.message_backward(torch.zeros(3, 4), torch.zeros(5, 2), torch.zeros(5, 6), torch.zeros(3, 8), Edges(), True) is None
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_dense_product_without_memory_for_its_packed_weights(monkeypatch, dtype):
+    # fp32 runs on the kernel that needs no workspace, bf16 has no other kernel
+    calls = []
+
+    class Library:
+        def e3x_tp_forward_workspace_bytes(self, handle):
+            return 1 << 20
+
+        def e3x_tp_forward_ws(self, handle, x1, x2, w, out, rows, workspace, workspace_bytes, stream):
+            calls.append((workspace, workspace_bytes))
+            return 0
+
+    from e3nn_amd.o3.tensor_product import _Plan
+
+    plan = object.__new__(_Plan)
+    plan.handle, plan.family, plan.out_dim = None, "uvw_mfma", 4
+    monkeypatch.setattr(_lib, "lib", Library)
+    monkeypatch.setattr(_lib, "stream_ptr", lambda device: None)
+    monkeypatch.setattr(torch, "empty", _NoMemory(torch.empty, 0, torch.uint8))
+    args = [torch.zeros(3, 8, dtype=dtype), torch.zeros(3, 8, dtype=dtype), torch.zeros(16, dtype=dtype)]
+    if dtype == torch.float32:
+        assert plan.forward(*args).shape == (3, 4) and calls == [(None, 0)]
+    else:
+        with pytest.raises(torch.OutOfMemoryError):
+            plan.forward(*args)
+
+
 def test_calls_skip_their_autograd_function_only_where_nothing_records():
     from torch.autograd import forward_ad
 
