@@ -147,8 +147,15 @@ class Convolution(torch.nn.Module):
             # the radial network inside the message kernel: the [E, weight_numel] weights are never stored
             messages = self.tp.forward_gather_scatter_radial(node_features, edge_attr, edge_scalars, self.fc, edges)
         if messages is None:
-            weight = self.fc(edge_scalars)
-            messages = self.tp.forward_gather_scatter(node_features, edge_attr, weight, edges=edges)
+            try:
+                weight = self.fc(edge_scalars)
+            except torch.OutOfMemoryError:
+                # the weights of all edges do not fit the memory that is left: once more without storing them
+                messages = None if wants_grad else self.tp.forward_gather_scatter_radial(node_features, edge_attr, edge_scalars, self.fc, edges)
+                if messages is None:
+                    raise
+            else:
+                messages = self.tp.forward_gather_scatter(node_features, edge_attr, weight, edges=edges)
         node_features = messages
         # lin2 and alpha are linear in the features, so the division by sqrt(num_neighbors) that the reference applies
         # to the summed messages (points_convolution.py:108) is applied to their outputs instead, which are four to a

@@ -331,6 +331,26 @@ def test_convolution_without_gradients_on_either_side_of_its_rule(N, E):
     assert float((got - want).norm()) < 1e-6 * float(want.norm())
 
 
+def test_convolution_without_memory_for_its_stored_weights(monkeypatch):
+    conv = ks.conv_wide().to(DEV)
+    src, dst = (torch.randint(0, 50, (700,), generator=torch.Generator().manual_seed(i)).to(DEV) for i in (1, 2))
+    edge_attr = o3.spherical_harmonics([0, 1, 2], seeded(700, 3, seed=3).to(DEV), True, "component")
+    args = (seeded(50, 288, seed=1).to(DEV), seeded(50, 4, seed=2).to(DEV), src, dst, edge_attr, seeded(700, 8, seed=4).to(DEV))
+    with torch.no_grad():
+        want = conv(*args)
+
+    def no_memory(x):
+        raise torch.OutOfMemoryError("no memory left")
+
+    monkeypatch.setattr(conv.fc, "forward", no_memory)
+    with torch.no_grad():
+        got = conv(*args)
+    # both sum the same products in fp32: 6e-8 of the 2-norm seen
+    assert float((got - want).norm()) < 1e-6 * float(want.norm())
+    with pytest.raises(torch.OutOfMemoryError):  # (a recorded pass needs the weights)
+        conv(*args)
+
+
 def test_convolution_block_forward_and_backward():
     conv = ks.conv_wide().to(DEV)
     with torch.no_grad():
