@@ -1697,7 +1697,10 @@ extern "C" int e3x_tp_message_backward(e3x_plan* P, const void* node_x, const vo
   long long n_rows = num_out_nodes, n_src = num_src_nodes;
   void* args[] = {(void*)&node_x, (void*)&edge_attr, (void*)&w,      (void*)&grad_out, (void*)&src,    (void*)&idx64,   (void*)&rowptr,
                   (void*)&perm,   (void*)&row_order, (void*)&n_rows, (void*)&n_src,    (void*)&grad_w, (void*)&grad_x2, (void*)&workspace};
-  const long long blocks = (n_rows + 7) / 8 * 8;  // a workgroup per row, contiguous eighths of the rows per XCD
+  // a workgroup per row, contiguous eighths of the rows per XCD, and one per piece of a long row beyond the first (PIECE of
+  // the template: 128 edges)
+  const long long blocks = (n_rows + 7) / 8 * 8 + (E - 1) / 128;
+  if (blocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_message_backward: too many rows for one launch");
   hipError_t err = hipModuleLaunchKernel(grad_x2 ? R->fn_rowgrad_x2[dev] : R->fn_rowgrad[dev], (unsigned)blocks, 1, 1, 64 * R->chunks, 1, 1,
                                          0, st, args, nullptr);
   if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_message_backward: launch failed: ") + hipGetErrorString(err));

@@ -93,7 +93,9 @@ def test_fused_message_gradients(maker, N, E, idx):
 
 
 @pytest.mark.parametrize("maker", [lambda: ks.cfg4("A"), ks.ragged_wide_message])
-@pytest.mark.parametrize("degrees,idx,grouped", [([0, 1, 63, 64, 65, 0, 130, 2], torch.int64, True), ([3, 0, 0, 129], torch.int32, False), ([1], torch.int64, True)])
+@pytest.mark.parametrize("degrees,idx,grouped", [([0, 1, 63, 64, 65, 0, 130, 2], torch.int64, True), ([3, 0, 0, 129], torch.int32, False), ([1], torch.int64, True),
+                                                # rows around one, two and three pieces of 128 edges
+                                                ([129, 0, 127, 300, 128, 0], torch.int32, True), ([5, 257, 0, 400], torch.int64, False)])
 def test_message_gradients_grouped_by_destination(maker, degrees, idx, grouped):
     # messages much wider than the node features: rows without edges, one edge, around the blocks of 64 edges, an odd
     # and an even number of them; sources without edges get exact zeros
