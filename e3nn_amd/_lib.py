@@ -18,6 +18,7 @@ MODE_UVW, MODE_UVU = 0, 1
 NORM_INTEGRAL, NORM_COMPONENT, NORM_NORM = 0, 1, 2
 ERR_INDEX = -4
 ERR_INVALID = -1
+ERR_COMPILE = -2
 
 c_void_p, c_int, c_int32, c_int64, c_size_t = ctypes.c_void_p, ctypes.c_int, ctypes.c_int32, ctypes.c_int64, ctypes.c_size_t
 

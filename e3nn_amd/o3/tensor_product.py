@@ -83,6 +83,7 @@ class _Plan:
         self.out_dim, self.in2_dim = irreps_out.dim, irreps_in2.dim
         self.arithmetic = L.e3x_tp_plan_arithmetic(handle, 0).decode()  # which instruction forms the products
         self._fused_grad_w = None  # whether the plan has the message-step backward kernel; asked on first use
+        self._by_destination = None  # ... and, on the forward plan, the one grouped by destination
 
     def __del__(self):
         try:
@@ -185,13 +186,24 @@ class _Plan:
             )
         return out, grad_w, grad_x2
 
+    def has_message_backward(self):
+        """Whether the plan has the message-step backward kernel grouped by destination, built on first use: not where it
+        is not meant for the plan or its code object cannot be had (a cache made without it, E3X_NO_JIT); the kernels on
+        the transposed plan then do all that it does."""
+        if self._by_destination is None:
+            rc = _lib.lib().e3x_tp_plan_prepare_message_backward(self.handle)
+            if rc not in (_lib.ERR_INVALID, _lib.ERR_COMPILE):
+                _lib.check(rc)
+            self._by_destination = rc not in (_lib.ERR_INVALID, _lib.ERR_COMPILE)
+        return self._by_destination
+
     def message_backward(self, node_x, edge_attr, w, grad_out, edges, want_x2=False):
         """``(grad_node_x, grad_w, grad_edge_attr or None)`` of the message step from the kernel grouped by destination;
-        None when the plan or the size of its scratch is outside what that kernel is meant for, or the scratch and the
-        gradients beside it do not fit the memory that is left."""
+        None when the plan does not have it, the size of its scratch is outside what it is meant for, or the scratch and
+        the gradients beside it do not fit the memory that is left."""
         L = _lib.lib()
         ws_bytes = L.e3x_tp_message_backward_workspace_bytes(self.handle, edges.num_edges)
-        if ws_bytes == 0:
+        if ws_bytes == 0 or not self.has_message_backward():
             return None
         by_src = edges.transposed()
         try:
@@ -802,9 +814,7 @@ class TensorProduct(torch.nn.Module):
         if self._live_mode() == "uvu":
             _lib.check(_lib.lib().e3x_tp_plan_prepare_backward_w(self._plan(dtype).handle))
             if dtype == torch.float32 and not self.shared_weights and self.weight_numel:
-                rc = _lib.lib().e3x_tp_plan_prepare_message_backward(self._plan(dtype).handle)
-                if rc != _lib.ERR_INVALID:
-                    _lib.check(rc)
+                self._plan(dtype).has_message_backward()
                 # the message-step backward kernel on the transposed plan, where the instruction set fits it
                 rc = _lib.lib().e3x_tp_plan_prepare_gather_scatter_grad_w(self._grad_plan("x1", dtype).handle)
                 if rc != _lib.ERR_INVALID:

@@ -500,7 +500,7 @@ def test_message_backward_gives_way_when_scratch_or_gradients_do_not_fit(monkeyp
     from e3nn_amd.o3.tensor_product import _Plan
 
     plan = object.__new__(_Plan)
-    plan.handle = None
+    plan.handle, plan._by_destination = None, True
     monkeypatch.setattr(_lib, "lib", Library)
     monkeypatch.setattr(torch, "empty_like", _NoMemory(torch.empty_like, like))
     monkeypatch.setattr(torch, "empty", _NoMemory(torch.empty, plain, torch.uint8))
@@ -533,6 +533,27 @@ def test_dense_product_without_memory_for_its_packed_weights(monkeypatch, dtype)
     else:
         with pytest.raises(torch.OutOfMemoryError):
             plan.forward(*args)
+
+
+def test_message_backward_whose_kernel_cannot_be_had(tmp_path, monkeypatch):
+    # a cache made without the kernel grouped by destination, and no compiler: the caller is sent to the transposed plan
+    monkeypatch.setenv("E3X_KERNEL_CACHE", str(tmp_path))
+
+    def product():
+        return message_tensor_product("64x0e", "0e+1o+2e+3o", keep="0e+1o+2e+3o").compile_backward()
+
+    class Edges:
+        num_edges = 5
+
+    product()
+    built = [p for p in tmp_path.iterdir() if p.name.startswith("uvu_rowgrad")]
+    assert built
+    for p in built:
+        p.unlink()
+    monkeypatch.setenv("E3X_NO_JIT", "1")
+    tp = product()
+    x, attr, w, g = torch.zeros(3, 64), torch.zeros(5, 16), torch.zeros(5, tp.weight_numel), torch.zeros(3, tp.irreps_out.dim)
+    assert tp._plan(torch.float32).message_backward(x, attr, w, g, Edges(), True) is None
 
 
 def test_calls_skip_their_autograd_function_only_where_nothing_records():
