@@ -864,7 +864,7 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
     dkmax = std::max(dkmax, dK);
     drmax = std::max(drmax, dR);
     // Outer indices per workgroup.  On split operands 8: what a chunk of rows costs before its first matrix step is shared
-    // by twice the passes of 4 (128-wide blocks, 65 536 rows: 54.4 -> 49.0 ms, with the factors R formed once per row).
+    // by twice the passes of 4 (128-wide blocks, 65 536 rows: 54.1 -> 47.6 ms, with the factors R formed once per row).
     const int ob = split_operands && O % 8 == 0 ? 8 : O % 4 == 0 ? 4 : (O % 2 == 0 ? 2 : 1);
     obmax = std::max(obmax, ob), nrmax = std::max(nrmax, std::max(d3, dK));
     ps << "  {" << (k_is_x2 ? "true" : "false") << ", " << (k_is_x2 ? P.off2[p.in2] : P.off1[p.in1]) << ", " << dK << ", "
