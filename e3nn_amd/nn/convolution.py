@@ -18,7 +18,10 @@ from .message import message_instructions
 # The message kernel with the radial network inside deals whole rows to 8192 workers: below about one row each it waits
 # for the longest rows on a half-empty chip.  A block without gradients, 32x0e+32x1o+32x2e, 35 edges per row, network inside
 # / two kernels: 60 rows 177 / 124 us, 1000 rows 250 / 152, 5003 rows 340 / 252, 8000 rows 386 / 334, 12 000 rows 420 / 429,
-# 50 000 rows 1154 / 1533.  The two kernels store the weights of all edges: not beyond 1 GiB of them.
+# 50 000 rows 1154 / 1533.  Other degrees shift the gain, not the line: at 3, 12, 120 and 400 edges per row the network inside
+# takes 0.94 to 1.10, 1.07 to 1.10, 1.06 to 2.45 and 1.08 to 3.64 times as long below it, and between 0.91 and 1.10 times
+# at 20 000 rows; sets that the kernel does not take (64 channels, 16 channels) run the two kernels on either side.  The two
+# kernels store the weights of all edges: not beyond 1 GiB of them, and not where these do not fit the memory that is left.
 _ROWS_INSIDE = 10_000
 _MAX_STORED_WEIGHTS = 1 << 28
 
