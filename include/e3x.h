@@ -161,7 +161,8 @@ int e3x_tp_forward_ws(e3x_plan* plan, const void* x1, const void* x2, const void
 size_t e3x_csr_workspace_bytes(int64_t E, int64_t num_nodes);
 int e3x_csr_build(const void* dst, int idx_bits, int64_t E, int64_t num_nodes, int32_t* rowptr, int32_t* perm,
                   void* workspace, size_t workspace_bytes, void* stream);
-/* Everything a message step needs from an edge list in one call with one synchronisation: the range checks of both index
+/* Everything a message step needs from an edge list in one call with one synchronisation (a few for lists of more than two
+ * million edges and for rows of more than 256 edges on average or 1024 at most): the range checks of both index
  * arrays (E3X_ERR_INDEX as from e3x_index_check, then as from e3x_csr_build), rowptr and perm of e3x_csr_build, unless
  * row_order is NULL the order of e3x_row_order_build, *grouped (whether dst was non-decreasing already: perm is the
  * identity) and *shared_pairs, all identical to what these functions give. */

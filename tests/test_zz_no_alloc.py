@@ -71,6 +71,9 @@ def _graph(kind, E, N, n_src, g):
     ("random", 1, 1, 1), ("random", 2, 5, 3), ("random", 5000, 63, 70), ("random", 4097, 4096, 4096), ("random", 9000, 4097, 4097),
     ("grouped", 6001, 300, 300), ("band", 20000, 2500, 2500), ("star", 6000, 50, 50), ("long", 9000, 400, 400), ("negative", 3000, 200, 150),
     ("random", 300, 1, 40), ("random", 30000, 16384, 16384), ("random", 30000, 16385, 16385), ("random", 3000, 100, 70000), ("band", 60, 8200, 8200),
+    # lists that are looked at before they are sorted, and the largest that are not
+    ("random", 2_000_001, 20_000, 20_000), ("grouped", 2_000_001, 20_000, 20_000), ("random", 2_000_000, 20_000, 20_000),
+    ("random", 2_000_001, 16_000, 16_000), ("star", 2_000_001, 20_000, 20_000),
 ])  # fmt: skip
 @pytest.mark.parametrize("src_t,dst_t", [(torch.int64, torch.int64), (torch.int32, torch.int64)])
 def test_edge_list_in_one_call_matches_the_separate_entry_points(kind, E, N, n_src, src_t, dst_t):
