@@ -378,6 +378,27 @@ def test_uvw_on_pairs_of_fp16_operands_with_channels_of_different_sizes(sizes):
     assert np.linalg.norm(got - want) < 1e-6 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("sizes", ["first input", "output"])
+def test_uvw_on_pairs_of_fp16_operands_with_channels_beyond_the_range_of_a_scale(sizes):
+    # every other channel 2^170 smaller: beside the large ones its scaled numbers are zero in fp32 already
+    tp = ks.mfma_full_tiles()
+    x1, x2 = seeded(140, tp.irreps_in1.dim, seed=1), seeded(140, tp.irreps_in2.dim, seed=2)
+    irreps = tp.irreps_in1 if sizes == "first input" else tp.irreps_out
+    spans = [torch.where(torch.arange(m.mul) % 2 == 0, 2.0**100, 2.0**-70) for m in irreps]
+    whole = torch.cat([v.repeat_interleave(m.ir.dim) for v, m in zip(spans, irreps)])
+    ws = [seeded(*t.path_shape, seed=10 + i) for i, t in enumerate(tp.instructions)]
+    ws = [torch.sign(w) + w.clamp(-1, 1) for w in ws]  # (none of them small by itself)
+    want = otp.tp_forward(oracle_spec(tp), x1.numpy(), x2.numpy(), torch.cat([w.reshape(-1) for w in ws]).numpy())
+    if sizes == "first input":  # made up for by the weights
+        x1, ws = x1 * whole, [w / spans[t.i_in1][:, None, None] for t, w in zip(tp.instructions, ws)]
+    else:
+        ws = [w * spans[t.i_out] for t, w in zip(tp.instructions, ws)]
+    got = tp(x1.to(DEV), x2.to(DEV), torch.cat([w.reshape(-1) for w in ws]).to(DEV)).double().cpu()
+    got = got.numpy() / (whole.double().numpy() if sizes == "output" else 1.0)
+    # as above, every channel in its own size
+    assert np.linalg.norm(got - want) < 1e-6 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("Z,odd", [(1, [0]), (128, [127]), (129, [128]), (300, [0, 40, 63, 64, 191, 299]), (200, range(64, 200)), (256, range(256)), (300, [])])
 def test_uvw_on_pairs_of_fp16_operands_leaves_rows_to_the_general_kernel(Z, odd):
     # a row with one large channel per irrep is formed by the kernel of e3x_tp_forward, its neighbours are not: each
