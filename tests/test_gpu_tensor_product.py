@@ -425,6 +425,24 @@ def test_uvw_on_pairs_of_fp16_operands_leaves_rows_to_the_general_kernel(Z, odd)
     assert not tp(a, b, w)[Z // 2].any()
 
 
+@pytest.mark.parametrize("Z,path", [(1, 0), (128, -1), (129, 0), (300, -1)])
+def test_uvw_on_pairs_of_fp16_operands_leaves_every_row_to_the_general_kernel(Z, path):
+    # one column of one path's weights with a few large entries suits no row: the call is the general kernel's, bit for bit
+    from e3nn_amd import _lib
+
+    tp = ks.mfma_full_tiles()
+    w = seeded(tp.weight_numel, seed=3).to(DEV)
+    view = list(tp.weight_views(w))[path]
+    view[:, :, 5] *= 1e-4
+    view[0, :, 5] = view[:, 0, 5] = 1.0
+    a, b = seeded(Z, tp.irreps_in1.dim, seed=1).to(DEV), seeded(Z, tp.irreps_in2.dim, seed=2).to(DEV)
+    a[Z // 2] = 0
+    got = tp(a, b, w)
+    plain = torch.empty_like(got)
+    _lib.check(_lib.lib().e3x_tp_forward(tp._plan(torch.float32).handle, _lib.ptr(a), _lib.ptr(b), _lib.ptr(w), _lib.ptr(plain), Z, _lib.stream_ptr(a.device)))
+    assert torch.equal(got, plain)
+
+
 @pytest.mark.parametrize("Z", [1, 129, 200])
 def test_uvw_on_pairs_of_fp16_operands_with_l3_inputs(Z):
     tp = ks.dense_l3_inputs()
