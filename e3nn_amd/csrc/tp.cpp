@@ -88,6 +88,9 @@ struct e3x_plan {
   std::unique_ptr<SubKernel> dw;
   long long dw_tiles = 0;  // grid.x: the largest tile count of a path
   int dw_paths = 0;        // grid.y
+  // ... of products whose multiplicities are all multiples of 64: the kernel of uvw_dw_wide.inc (then `dw` is not built)
+  std::unique_ptr<SubKernel> dw_wide;
+  std::vector<std::pair<int, long long>> dw_wide_paths;  // per path: passes per outer index, tiles of a batch slice
 };
 
 namespace {
@@ -887,10 +890,78 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
   return E3X_OK;
 }
 
+// Weight gradient of wide blocks (templates/uvw_dw_wide.inc): a wave's tile is 32 indices of one input and all of 128 (or
+// 64) of another, so every multiplicity has to be a multiple of 64; the combined operand of an input with l > 2 would not
+// leave the accumulators their registers.
+bool dw_wide_fits(const e3x_plan& P) {
+  if (!P.shared_weights || P.dtype != E3X_F32 || P.paths.empty() || env_int("E3X_DW_WIDE", 1) == 0 || env_int("E3X_DW_SPLIT", 1) == 0) return false;
+  for (const auto& p : P.paths) {
+    const e3x_irrep &a = P.in1[p.in1], &b = P.in2[p.in2], &c = P.out[p.out];
+    if (p.mode != E3X_MODE_UVW || !p.has_w || a.mul % 64 || b.mul % 64 || c.mul % 64 || a.l > 2 || b.l > 2 || c.l > 2) return false;
+  }
+  return true;
+}
+
+int build_uvw_dw_wide_source(e3x_plan& P, std::string* src) {
+  std::ostringstream s, nzs, ps;
+  emit_header(s, P);
+  P.dw_wide_paths.clear();
+  int n_nz = 0;
+  for (const auto& p : P.paths) {
+    const e3x_irrep* ir[3] = {&P.in1[p.in1], &P.in2[p.in2], &P.out[p.out]};
+    const int off[3] = {P.off1[p.in1], P.off2[p.in2], P.offo[p.out]};
+    const int d[3] = {2 * ir[0]->l + 1, 2 * ir[1]->l + 1, 2 * ir[2]->l + 1};
+    const long long stride[3] = {(long long)ir[1]->mul * ir[2]->mul, ir[2]->mul, 1};  // W_p[u, v, w] at woff + (u * V + v) * W + w
+    // N: the factor with the smallest l; R: an input (the output's channels stay a column of the tile), the one with the
+    // larger l where both are left, so that M has the fewer components to keep
+    int n = 2;
+    for (int i = 1; i >= 0; --i) if (d[i] < d[n]) n = i;
+    const int r = n == 0 ? 1 : n == 1 ? 0 : d[0] >= d[1] ? 0 : 1, m = 3 - n - r;
+    const auto& C = e3x::wigner_3j(ir[0]->l, ir[1]->l, ir[2]->l);
+    const int nz_beg = n_nz;
+    for (int i = 0; i < d[0]; ++i)
+      for (int j = 0; j < d[1]; ++j)
+        for (int k = 0; k < d[2]; ++k) {
+          const double cv = C[(i * d[1] + j) * d[2] + k] * p.pw;
+          const int at[3] = {i, j, k};
+          if (cv != 0.0) {
+            nzs << "  {" << at[m] << ", " << at[r] << ", " << at[n] << ", " << fstr(cv) << "},\n";
+            ++n_nz;
+          }
+        }
+    const int mb = ir[m]->mul % 128 == 0 ? 128 : 64, nb = ir[n]->mul % 128 == 0 ? 128 : 64;
+    const int outer = 2 * (128 / mb);  // outer indices per workgroup
+    const long long tiles = (long long)(ir[m]->mul / mb) * (ir[n]->mul / nb) * (ir[r]->mul / outer);
+    ps << "  {" << m << ", " << off[m] << ", " << d[m] << ", " << ir[m]->mul << ", " << n << ", " << off[n] << ", " << d[n] << ", "
+       << ir[n]->mul << ", " << r << ", " << off[r] << ", " << d[r] << ", " << ir[r]->mul << ", " << (n == 2 ? "true" : "false") << ", "
+       << p.woff << ", " << stride[m] << ", " << stride[n] << ", " << stride[r] << ", " << tiles << ", " << nz_beg << ", " << n_nz << "},\n";
+    P.dw_wide_paths.push_back({d[n], tiles});
+  }
+  s << "constexpr int DIMS[3] = {IN1_DIM, IN2_DIM, OUT_DIM};\n";
+  s << "struct Nz { int s, r, k; float c; };\nconstexpr int N_NZ = " << n_nz << ";\nconstexpr Nz nz[N_NZ] = {\n" << nzs.str() << "};\n";
+  s << "struct WPath { int m_src, m_off, dM, M, n_src, n_off, dN, N, r_src, r_off, dR, O; bool n_is_w; "
+       "long long wbase, m_stride, n_stride, o_stride; int tiles, nz_beg, nz_end; };\n";
+  s << "constexpr int N_WPATH = " << P.paths.size() << ";\nconstexpr WPath wpaths[N_WPATH] = {\n" << ps.str() << "};\n}  // namespace cfg\n";
+  *src = s.str() + e3x::kTplCommon + e3x::kTplUvwDwWide;
+  return E3X_OK;
+}
+
 // builds (or finds in the cache) the weight-gradient code object of a uvw_mfma plan
 int prepare_mfma_dw(e3x_plan* P) {
   std::lock_guard<std::mutex> lock(P->mu);
-  if (P->dw) return E3X_OK;
+  if (P->dw || P->dw_wide) return E3X_OK;
+  if (dw_wide_fits(*P)) {
+    std::unique_ptr<SubKernel> K(new SubKernel);
+    std::string src;
+    int rc = build_uvw_dw_wide_source(*P, &src);
+    if (!rc) rc = e3x::get_code_object("uvw_dw_wide", src, &K->key, &K->hsaco);
+    if (!rc) {
+      P->arithmetic_dw = "bf16 matrix instruction, six products of three-way split operands";
+      P->dw_wide = std::move(K);
+      return E3X_OK;
+    }
+    // a code object that cannot be had leaves the general kernel
+  }
   std::unique_ptr<SubKernel> K(new SubKernel);
   std::string src;
   int rc;
@@ -902,13 +973,14 @@ int prepare_mfma_dw(e3x_plan* P) {
 
 int load_dw_function(e3x_plan* P, int dev) {
   std::lock_guard<std::mutex> lock(P->mu);
-  SubKernel* K = P->dw.get();
+  SubKernel* K = P->dw_wide ? P->dw_wide.get() : P->dw.get();
+  const std::string name = P->dw_wide ? "e3x_uvw_dw_wide" : "e3x_uvw_mfma_dw";
   if (K->module[dev]) return E3X_OK;
   hipModule_t mod = nullptr;
   hipError_t err = hipModuleLoad(&mod, K->hsaco.c_str());
   if (err != hipSuccess) return fail(E3X_ERR_HIP, "hipModuleLoad(" + K->hsaco + ") failed: " + hipGetErrorString(err));
-  if (hipModuleGetFunction(&K->fn_dw[dev], mod, "e3x_uvw_mfma_dw") != hipSuccess)
-    return fail(E3X_ERR_HIP, "kernel e3x_uvw_mfma_dw missing from " + K->hsaco);
+  if (hipModuleGetFunction(&K->fn_dw[dev], mod, name.c_str()) != hipSuccess)
+    return fail(E3X_ERR_HIP, "kernel " + name + " missing from " + K->hsaco);
   K->module[dev] = mod;
   return E3X_OK;
 }
@@ -1944,6 +2016,46 @@ extern "C" int e3x_tp_plan_prepare_backward_w(e3x_plan* P) {
   return E3X_OK;  // uvw_small carries its gradient kernel in the forward code object
 }
 
+// Batch slices of the wide weight gradient: a slice of a path with d passes has 1/d of the rows of one with a single pass,
+// so that all workgroups cost the same (unit_rows / d, whole stages of 16).  512 workgroups run at once, two per CU.  Taken is
+// the split, of 48 rows or more per workgroup, that ends first, counted in rounds of workgroups and rows (90 ns each): what
+// a workgroup does besides its rows costs it about as much as 32 of them, 96 where it adds to what others have stored, and
+// there the gradient is cleared first, at 50 000 numbers in the time of a row.
+static int launch_dw_wide(e3x_plan* P, int dev, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, hipStream_t st) {
+  auto rows_of = [](long long unit, int d) { return (unit / d + 15) / 16 * 16; };  // as in the kernel
+  int unit_rows = 0, accumulate = 0;
+  long long jobs = 0;
+  double best = 1e300;
+  for (int n = 0; n <= 24; ++n) {
+    // n = 0: every path whole (7 passes at most)
+    const long long unit = n == 0 ? (Z + 15) / 16 * 16 * 7 : ((Z + n - 1) / n + 239) / 240 * 240;
+    if (unit >= (1LL << 31)) continue;
+    long long n_jobs = 0, least = Z;
+    double most = 0, work = 0;
+    bool sums = false;
+    for (const auto& [d, tiles] : P->dw_wide_paths) {
+      const long long rows = rows_of(unit, d), slices = (Z + rows - 1) / rows;
+      n_jobs += slices * tiles;
+      sums = sums || slices > 1;
+      least = std::min(least, rows);
+      most = std::max(most, (double)std::min<long long>(rows, Z) * d);
+      work += (double)Z * d * tiles;
+    }
+    if (least < std::min<long long>(Z, 48)) break;  // (more slices have fewer rows)
+    const double cost = std::ceil(work / most / 512) * (most + (sums ? 96 : 32)) + (sums ? 2e-5 * (double)P->weight_numel : 0);
+    if (cost < best) best = cost, jobs = n_jobs, unit_rows = (int)unit, accumulate = sums;
+  }
+  jobs = (jobs + 7) / 8 * 8;
+  if (unit_rows == 0 || jobs >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: batch too large for one launch");
+  int rc;
+  if (accumulate && (rc = e3x::fill_zero_bytes(grad_w, (size_t)P->weight_numel * 4, st))) return rc;
+  long long n_rows = Z;
+  void* args[] = {(void*)&x1, (void*)&x2, (void*)&grad_out, (void*)&grad_w, (void*)&n_rows, (void*)&unit_rows, (void*)&accumulate};
+  hipError_t err = hipModuleLaunchKernel(P->dw_wide->fn_dw[dev], (unsigned)jobs, 1, 1, 256, 1, 1, 0, st, args, nullptr);
+  if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_backward_w_uvw: launch failed: ") + hipGetErrorString(err));
+  return E3X_OK;
+}
+
 extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2, const void* grad_out, void* grad_w,
                                      int64_t Z, void* stream) {
   if (!P) return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: null plan");
@@ -1969,6 +2081,7 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
       return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: x1, x2 and grad_out must be 16-byte aligned");
     if ((rc = prepare_mfma_dw(P))) return rc;
     if ((rc = load_dw_function(P, dev))) return rc;
+    if (P->dw_wide) return launch_dw_wide(P, dev, x1, x2, grad_out, grad_w, Z, st);
     // batch slices: enough workgroups for a few waves of the chip, at least 256 rows each
     const long long wgs = P->dw_tiles * P->dw_paths;
     long long slices = (2048 + wgs - 1) / wgs;

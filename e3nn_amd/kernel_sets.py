@@ -50,6 +50,12 @@ def mfma_full_tiles():
     return o3.FullyConnectedTensorProduct("64x0e+64x1o", "64x0e+64x1o+64x2e", "64x0e+128x1o+64x1e+64x2e")
 
 
+def mfma_wide_blocks():
+    # ... blocks of 64, 128 and 192 up to l = 2 on all sides: every order of the factors in the weight gradient of wide blocks,
+    # the output's channels as either index of its tiles, one and several tiles of each
+    return o3.FullyConnectedTensorProduct("128x0e+64x1o+64x2e", "64x0e+128x1o+64x2e", "64x0e+64x1o+192x2e")
+
+
 def dense_l3_inputs():
     # l = 3 inputs, 128 and 64 channels: seven components of the K and of the R operand, contractions over 64 and over 128
     # indices into one output
@@ -187,6 +193,7 @@ def all_tensor_products():
         ("cfg5", cfg5(), (torch.float32, torch.bfloat16)),
         ("mfma_small", mfma_small(), (torch.float32,)),
         ("mfma_full_tiles", mfma_full_tiles(), (torch.float32,)),
+        ("mfma_wide_blocks", mfma_wide_blocks(), (torch.float32,)),
         ("dense_l3_inputs", dense_l3_inputs(), (torch.float32,)),
         ("mfma_half_tiles", mfma_half_tiles(), (torch.float32, torch.bfloat16)),
         ("wide_k_l3", wide_k_l3(), (torch.float32, torch.bfloat16)),
@@ -214,7 +221,7 @@ def all_tensor_products():
 
 
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
-BACKWARD_CASES = ["cfg1", "cfg3_merged", "cfg3_builder", "cfg4_A", "cfg5", "mfma_small", "mfma_full_tiles", "outer_split", "node_fctp", "node_block",
+BACKWARD_CASES = ["cfg1", "cfg3_merged", "cfg3_builder", "cfg4_A", "cfg5", "mfma_small", "mfma_full_tiles", "mfma_wide_blocks", "outer_split", "node_fctp", "node_block",
                   "node_wide_out", "node_narrow", "node_partial_tile", "radial_layer", "odd_mul", "unaligned_mfma", "unaligned_offsets",
                   "mixed_modes", "scalar_exact", "narrow_message", "ragged_wide_message"]  # fmt: skip
 

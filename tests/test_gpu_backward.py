@@ -153,6 +153,24 @@ def test_uvw_weight_gradient_on_split_operands(maker, Z, ramp):
         assert t.i_in1 == 0 and not block[0].any() and block[1:].all()
 
 
+@pytest.mark.parametrize("Z", [1, 15, 16, 17, 49, 97, 800])
+def test_uvw_weight_gradient_of_wide_blocks(Z):
+    # stages of 16 rows and their remainders; one batch slice per path (stored) and several (added); every role of the factors
+    tp = ks.mfma_wide_blocks()
+    spec = oracle_spec(tp)
+    x1, x2, g = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(Z, tp.irreps_out.dim, seed=3)
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True).double().cpu()
+    # sums of at most 800 x 25 products in fp32, as above; block by block, so that no path is lost among the others
+    offset = 0
+    for t in tp.instructions:
+        n = t.path_shape[0] * t.path_shape[1] * t.path_shape[2]
+        a, b = got[offset : offset + n], ref[offset : offset + n]
+        assert float((a - b).norm() / b.norm()) < 1e-6, t
+        offset += n
+
+
 @pytest.mark.parametrize("maker", [ks.mfma_full_tiles, ks.node_block])
 @pytest.mark.parametrize("sizes", ["x1 against x2", "x1 against g", "x2 against g", "masked row", "largest number", "channels"])
 def test_uvw_weight_gradient_of_numbers_of_different_sizes(maker, sizes):
