@@ -45,6 +45,7 @@ struct SubKernel {
   hipFunction_t fn_dw[kMaxDevices] = {nullptr};
   hipFunction_t fn_pack[kMaxDevices] = {nullptr};
   hipFunction_t fn_max[kMaxDevices] = {nullptr};
+  hipFunction_t fn_sum[kMaxDevices] = {nullptr};
   // uvu: the edge-parallel backward kernel is a code object of its own (other lane layout), built on first use
   std::unique_ptr<SubKernel> bwd;
   // uvu, transposed plan of a message step: the fused kernel that also writes the weight gradient, built on first use
@@ -83,7 +84,10 @@ struct e3x_plan {
   int msg_groups = 0;  // wavefronts per output row
   // uvw_mfma, fp32 storage: the kernel on pairs of fp16 operands, where the instruction set fits it (see half_fits)
   std::unique_ptr<SubKernel> half;
-  int half_targets = 0;    // grid.y
+  int half_targets = 0;    // tiles of 64 channels
+  // scalar outputs formed from both inputs: how many, their parts, the channels of all parts, the channels of all sums; and
+  // the tiles of the other outputs
+  int half_scalars = 0, half_parts = 0, half_part_width = 0, half_sums = 0, half_general = 0;
   // uvw_mfma: the weight-gradient kernel is a code object of its own, built on first use
   std::unique_ptr<SubKernel> dw;
   long long dw_tiles = 0;  // grid.x: the largest tile count of a path
@@ -593,10 +597,17 @@ int half_max_private_bytes() { return env_int("E3X_UVW_HALF_PRIVATE", 2048); }
 // Row flags in the workspace: bit z % (32 kRowFlagWords) for row z, 512 KB for 4 million rows (rows of a larger batch that
 // share a bit are formed by the general kernel together).
 constexpr int kRowFlagWords = 1 << 17;
-// packed weights | row flags | block maxima and PathWeights (three words) of every path
-size_t half_workspace_bytes(const e3x_plan& P) {
-  return (size_t)P.weight_numel * 4 + kRowFlagWords * 4 + P.paths.size() * (kHalfMaxBlocks + 3) * 4;
+// Scalar outputs of l x l (run_scalar_target of the template): workgroups of 256 rows that walk all paths where the chip is
+// full, that is where the 128-row x 64-channel workgroups of the other targets are more than its 256 CUs; below that a
+// workgroup per path and 32 K indices, whose parts go through the workspace.  Row for row the two give the same bits.
+// 128x0e+128x1o+128x2e squared, 1000 / 8192 rows: 1.40 ms in parts / 2.97 whole, 1.89 whole / 3.07 with 2l + 1 passes per
+// outer index in the place of either.
+long long half_part_rows(const e3x_plan& P) { return P.half_parts ? 128LL * (256 / std::max(1, P.half_targets)) : 0; }
+// packed weights | row flags | block maxima and PathWeights (three words) of every path | parts
+size_t half_parts_offset(const e3x_plan& P) {
+  return ((size_t)P.weight_numel * 4 + kRowFlagWords * 4 + P.paths.size() * (kHalfMaxBlocks + 3) * 4 + 15) / 16 * 16;
 }
+size_t half_workspace_bytes(const e3x_plan& P) { return half_parts_offset(P) + (size_t)half_part_rows(P) * P.half_part_width * 4; }
 
 int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   // Output channels per workgroup.  fp32: 128 (two accumulator tiles per wave, 64 KB of LDS, two workgroups per CU at
@@ -608,7 +619,7 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   for (const auto& p : P.paths)
     if (P.out[p.out].mul % 128) wt = 64;
   if (P.dtype != E3X_F32 || half) wt = 64;
-  std::ostringstream s, nzs, ps, ts;
+  std::ostringstream s, nzs, ps, ts, scalar_width, parts;
   emit_header(s, P);
   // split-operand matrix steps (see the template) in fp32 storage; weight chunks of 16 K rows then keep the LDS at
   // 72 KB with 128 output channels (two workgroups per CU)
@@ -630,6 +641,8 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   const int wpe = env_int("E3X_UVW_WPE", wt == 128 || out_l3 ? 2 : 0);
   if (wpe) s << "#define E3X_UVW_WPE " << wpe << "\n";
   int n_nz = 0, n_path = 0, n_target = 0, dka = 1, drmax = 1;
+  int n_scalar = 0;
+  if (half) P.half_parts = P.half_part_width = P.half_sums = P.half_general = 0;
   for (size_t c = 0; c < P.out.size(); ++c) {
     std::ostringstream mine;
     const int beg = n_path;
@@ -671,7 +684,26 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
     }
     if (n_path == beg) continue;
     ps << mine.str();
+    // fp16 pairs: a scalar output of l x l, l = 1 or 2, can form its operand from both inputs (run_scalar_target)
+    bool scalar = half && P.out[c].l == 0, product = false;
+    for (const auto& p : P.paths)
+      if (p.out == (int)c) scalar = scalar && P.in1[p.in1].l <= 2, product = product || P.in1[p.in1].l > 0;
+    const int width = !scalar || !product ? 0 : P.out[c].mul % 128 == 0 ? 128 : 64;
     for (int w0 = 0; w0 < P.out[c].mul; w0 += wt) {
+      scalar_width << (n_target ? ", " : "") << width;
+      P.half_general += half && !width;
+      if (width && w0 % width == 0) {  // its parts: one per path and 32 K indices
+        P.half_sums += width, ++n_scalar;
+        int path = beg;
+        for (const auto& p : P.paths) {
+          if (p.out != (int)c) continue;
+          for (int k = 0; k < P.in1[p.in1].mul; k += 32) {  // (x1 is the K operand of l x l where it tiles, and it does)
+            parts << "  {" << n_target << ", " << path << ", " << k / 32 << ", " << P.half_part_width << ", " << n_scalar - 1 << "},\n";
+            P.half_part_width += width, ++P.half_parts;
+          }
+          ++path;
+        }
+      }
       ts << "  {" << P.offo[c] << ", " << 2 * P.out[c].l + 1 << ", " << w0 << ", " << std::min(wt, P.out[c].mul - w0) << ", "
          << beg << ", " << n_path << "},\n";
       ++n_target;
@@ -689,6 +721,12 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   s << "constexpr int N_MPATH = " << n_path << ";\nconstexpr MPath mpaths[N_MPATH] = {\n" << ps.str() << "};\n";
   s << "struct Target { int out_off, d3, w0, wn, path_beg, path_end; };\n";  // wn: channels in the tile (64, or 32 at the end)
   s << "constexpr int N_TARGET = " << n_target << ";\nconstexpr Target targets[N_TARGET] = {\n" << ts.str() << "};\n";
+  if (half) {
+    s << "constexpr int scalar_width[N_TARGET] = {" << scalar_width.str() << "};\n";
+    s << "struct Part { int target, path, chunk, offset, scalar; };\nconstexpr int N_PART = " << P.half_parts << ", PART_WIDTH = " << P.half_part_width
+      << ";\nconstexpr Part part_table[N_PART + 1] = {\n" << parts.str() << "  {0, 0, 0, 0, 0}};\n";
+    P.half_scalars = n_scalar;
+  }
   s << "}  // namespace cfg\n";
   (half ? P.half_targets : P.n_targets) = n_target;
   *src = s.str() + e3x::kTplCommon + (half ? e3x::kTplUvwMfmaHalf : P.dtype == E3X_BF16 ? e3x::kTplUvwMfmaBf16 : e3x::kTplUvwMfma);
@@ -1054,7 +1092,8 @@ int load_functions(e3x_plan* P, int dev) {
       return fail(E3X_ERR_HIP, "hipModuleLoad(" + K->hsaco + ") failed: " + hipGetErrorString(err));
     if (hipModuleGetFunction(&K->fn_plain[dev], mod, "e3x_uvw_half_plain") != hipSuccess ||
         hipModuleGetFunction(&K->fn_pack[dev], mod, "e3x_uvw_half_pack") != hipSuccess ||
-        hipModuleGetFunction(&K->fn_max[dev], mod, "e3x_uvw_half_max") != hipSuccess)
+        hipModuleGetFunction(&K->fn_max[dev], mod, "e3x_uvw_half_max") != hipSuccess ||
+        hipModuleGetFunction(&K->fn_sum[dev], mod, "e3x_uvw_half_sum") != hipSuccess)
       return fail(E3X_ERR_HIP, "kernels of e3x_uvw_half missing from " + K->hsaco);
     K->module[dev] = mod;
   }
@@ -1480,14 +1519,20 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
     }
     const long long blocks = (Z + 127) / 128;
     if (blocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_forward: batch too large for one launch");
+    float* parts = P->half_parts && Z <= half_part_rows(*P) ? (float*)((char*)workspace + half_parts_offset(*P)) : nullptr;
+    int n_scalar = parts ? P->half_parts : P->half_scalars;
     void* margs[] = {(void*)&w, (void*)&w_max, (void*)&path_w, (void*)&row_flags, (void*)&n_words};
     void* pargs[] = {(void*)&w, (void*)&w_max, (void*)&workspace, (void*)&path_w};
-    void* args[] = {(void*)&x1, (void*)&x2, (void*)&workspace, (void*)&path_w, (void*)&row_flags, (void*)&out, (void*)&n_rows};
+    void* args[] = {(void*)&x1, (void*)&x2, (void*)&workspace, (void*)&path_w, (void*)&row_flags, (void*)&out, (void*)&n_rows, (void*)&n_scalar, (void*)&parts};
     hipError_t err = hipModuleLaunchKernel(K->fn_max[dev], kHalfMaxBlocks, n_path, 1, 256, 1, 1, 0, st, margs, nullptr);
     if (err == hipSuccess)
       err = hipModuleLaunchKernel(K->fn_pack[dev], (unsigned)((columns + 255) / 256), n_path, 1, 256, 1, 1, 0, st, pargs, nullptr);
     if (err == hipSuccess)
-      err = hipModuleLaunchKernel(K->fn_plain[dev], (unsigned)blocks, (unsigned)P->half_targets, 1, 512, 1, 1, 0, st, args, nullptr);
+      err = hipModuleLaunchKernel(K->fn_plain[dev], (unsigned)blocks, (unsigned)(n_scalar + P->half_general), 1, 512, 1, 1, 0, st, args, nullptr);
+    if (err == hipSuccess && parts) {
+      void* sargs[] = {(void*)&parts, (void*)&out, (void*)&n_rows};
+      err = hipModuleLaunchKernel(K->fn_sum[dev], (unsigned)((Z * P->half_sums + 255) / 256), 1, 1, 256, 1, 1, 0, st, sargs, nullptr);
+    }
     if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
     // ... and the general kernel below forms the rows that this one flagged
   }

@@ -443,6 +443,44 @@ def test_uvw_on_pairs_of_fp16_operands_leaves_every_row_to_the_general_kernel(Z,
     assert torch.equal(got, plain)
 
 
+@pytest.mark.parametrize("Z", [1, 255, 257, 6528, 6529, 6900])
+def test_uvw_on_pairs_of_fp16_operands_scalar_outputs(Z):
+    # scalar outputs whose operand is formed from both inputs: edges of the 256-row tiles, in parts (up to 6528 rows of this
+    # product) and whole; rows whose slices, channels or components differ in size or are zero.  A row's result does not
+    # depend on the batch it is in.
+    tp = ks.mfma_wide_blocks()
+    assert "fp16" in tp._plan(torch.float32).arithmetic
+    x1, x2, w = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(tp.weight_numel, seed=3)
+    kinds = ["plain", "one direction", "half of the channels", "one small component", "small and large rows", "holes", "one channel", "tiny channel"]
+    which = torch.arange(Z) % len(kinds)
+    for x, irreps in ((x1, tp.irreps_in1), (x2, tp.irreps_in2)):
+        for sl, (mul, ir) in zip(irreps.slices(), irreps):
+            for i, kind in enumerate(kinds):
+                v = x[which == i, sl].unflatten(1, (mul, ir.dim))
+                if kind == "one direction":
+                    v[:, :, 1:] = 0
+                elif kind == "half of the channels":
+                    v[:, ::2] = 0
+                elif kind == "one small component":
+                    v[:, :, -1] *= 2.0**-30
+                elif kind == "small and large rows":
+                    v *= 2.0**-70 if x is x1 else 2.0**66
+                elif kind == "holes" and ir.l:
+                    v[:, ::3, 0] = 0
+                elif kind == "one channel":
+                    v[:, 1:] = 0
+                elif kind == "tiny channel":
+                    v[:, 3] *= 2.0**-40
+                x[which == i, sl] = v.flatten(1)
+    got = tp(x1.to(DEV), x2.to(DEV), w.to(DEV)).cpu()
+    rows = torch.cat([torch.arange(min(Z, 16)), torch.arange(max(0, Z - 16), Z)]).unique()
+    want = otp.tp_forward(oracle_spec(tp), x1[rows].numpy(), x2[rows].numpy(), w.numpy())
+    for sl in tp.irreps_out.slices():  # row by row: sums of some 1e4 products in fp32, as above
+        err = np.linalg.norm(got[rows][:, sl].double().numpy() - want[:, sl], axis=1)
+        assert (err <= 1.5e-6 * np.linalg.norm(want[:, sl], axis=1)).all(), [kinds[int(which[r])] for r in rows[err > 1.5e-6 * np.linalg.norm(want[:, sl], axis=1)]]
+    assert torch.equal(tp(x1[rows].to(DEV), x2[rows].to(DEV), w.to(DEV)).cpu(), got[rows])
+
+
 @pytest.mark.parametrize("Z", [1, 129, 200])
 def test_uvw_on_pairs_of_fp16_operands_with_l3_inputs(Z):
     tp = ks.dense_l3_inputs()
