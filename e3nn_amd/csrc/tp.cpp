@@ -684,15 +684,15 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
     }
     if (n_path == beg) continue;
     ps << mine.str();
-    // fp16 pairs: a scalar output of l x l, l = 1 or 2, can form its operand from both inputs (run_scalar_target)
-    bool scalar = half && P.out[c].l == 0, product = false;
+    // fp16 pairs and bf16: a scalar output of l x l, l = 1 or 2, can form its operand from both inputs (run_scalar_target)
+    bool scalar = (half || P.dtype == E3X_BF16) && P.out[c].l == 0 && P.out[c].mul % 64 == 0, product = false;
     for (const auto& p : P.paths)
       if (p.out == (int)c) scalar = scalar && P.in1[p.in1].l <= 2, product = product || P.in1[p.in1].l > 0;
     const int width = !scalar || !product ? 0 : P.out[c].mul % 128 == 0 ? 128 : 64;
     for (int w0 = 0; w0 < P.out[c].mul; w0 += wt) {
       scalar_width << (n_target ? ", " : "") << width;
       P.half_general += half && !width;
-      if (width && w0 % width == 0) {  // its parts: one per path and 32 K indices
+      if (half && width && w0 % width == 0) {  // its parts: one per path and 32 K indices
         P.half_sums += width, ++n_scalar;
         int path = beg;
         for (const auto& p : P.paths) {
@@ -721,6 +721,7 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   s << "constexpr int N_MPATH = " << n_path << ";\nconstexpr MPath mpaths[N_MPATH] = {\n" << ps.str() << "};\n";
   s << "struct Target { int out_off, d3, w0, wn, path_beg, path_end; };\n";  // wn: channels in the tile (64, or 32 at the end)
   s << "constexpr int N_TARGET = " << n_target << ";\nconstexpr Target targets[N_TARGET] = {\n" << ts.str() << "};\n";
+  if (P.dtype == E3X_BF16) s << "constexpr int scalar_width[N_TARGET] = {" << scalar_width.str() << "};\n";
   if (half) {
     s << "constexpr int scalar_width[N_TARGET] = {" << scalar_width.str() << "};\n";
     s << "struct Part { int target, path, chunk, offset, scalar; };\nconstexpr int N_PART = " << P.half_parts << ", PART_WIDTH = " << P.half_part_width

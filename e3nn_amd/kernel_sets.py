@@ -193,7 +193,7 @@ def all_tensor_products():
         ("cfg5", cfg5(), (torch.float32, torch.bfloat16)),
         ("mfma_small", mfma_small(), (torch.float32,)),
         ("mfma_full_tiles", mfma_full_tiles(), (torch.float32,)),
-        ("mfma_wide_blocks", mfma_wide_blocks(), (torch.float32,)),
+        ("mfma_wide_blocks", mfma_wide_blocks(), (torch.float32, torch.bfloat16)),
         ("dense_l3_inputs", dense_l3_inputs(), (torch.float32,)),
         ("mfma_half_tiles", mfma_half_tiles(), (torch.float32, torch.bfloat16)),
         ("wide_k_l3", wide_k_l3(), (torch.float32, torch.bfloat16)),

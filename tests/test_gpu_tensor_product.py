@@ -608,6 +608,32 @@ def test_uvw_bf16_storage_small_multiplicities_in_256_row_workgroups():
     assert (part - out[-300:].float()).abs().max().item() <= 2.0**-7 * scale
 
 
+@pytest.mark.parametrize("Z", [13056, 13056 + 1, 13056 + 255])
+def test_uvw_bf16_storage_scalar_outputs(Z):
+    # beyond 13 056 rows of this product (51 tiles of 256 rows, 5 channel tiles) the scalar output's operand is formed from
+    # both inputs, in two bf16 pieces; the last workgroup holds one row, or all but one.
+    tp, tpb, wq = _bf16_uvw(make=ks.mfma_wide_blocks)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    xb = torch.randn(Z, tp.irreps_in1.dim, device=DEV, generator=g).to(torch.bfloat16)
+    yb = torch.randn(Z, tp.irreps_in2.dim, device=DEV, generator=g).to(torch.bfloat16)
+    out = tpb(xb, yb)
+    rows = torch.cat([torch.arange(0, 13056, 1999), torch.arange(13056 - 2, Z)[:40], torch.tensor([Z - 1])])
+    ref = _oracle_chunks(oracle_spec(tp), xb[rows].float().cpu().numpy(), yb[rows].float().cpu().numpy(), wq)
+    # one rounding of the output, 2^-9 of it; the pieces' 2^-17 of a term and the sums in fp32 vanish beside it
+    for sl in tp.irreps_out.slices():
+        err = out[rows][:, sl].detach().double().cpu().numpy() - ref[:, sl]
+        assert np.linalg.norm(err) < 2e-3 * np.linalg.norm(ref[:, sl])
+        assert (np.abs(err) <= 2.0**-8 * np.abs(ref[:, sl]) + 1e-5 * np.abs(ref[:, sl]).max()).all()
+    # rows and weights of sizes whose product is an ordinary number although that of two of them need not be
+    e1, e2 = (torch.tensor(e).repeat(Z // 3 + 1)[:Z, None].to(DEV) for e in ([80, -70, 0], [70, 30, -60]))
+    with torch.no_grad():
+        tpb.weight.mul_(2.0**-40)
+    scaled = tpb(torch.ldexp(xb, e1), torch.ldexp(yb, e2)).float()
+    if Z > 13056:
+        assert torch.equal(torch.ldexp(torch.ldexp(scaled, -e1), 40 - e2)[rows], out[rows].float())
+
+
+
 @pytest.mark.parametrize("Z", [300, 16384 + 77])
 def test_uvw_bf16_storage_tiles_of_32_channels(Z):
     # irreps of 32 and 96 channels: their last workgroup tile holds 32 channels instead of 64 (both row tilings)
