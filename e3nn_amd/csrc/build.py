@@ -19,7 +19,7 @@ SOURCES = ["api.cpp", "wigner.cpp", "jit.cpp", "tp.cpp", "fc.cpp", "sh.hip", "gr
 TEMPLATES = [("kTplCommon", "common.inc"), ("kTplUvu", "uvu.inc"), ("kTplUvuFc", "uvu_fc.inc"), ("kTplUvuRowgrad", "uvu_rowgrad.inc"), ("kTplUvuMfma", "uvu_mfma.inc"), ("kTplUvwSmall", "uvw_small.inc"),
              ("kTplUvwMfma", "uvw_mfma.inc"), ("kTplUvwMfmaBf16", "uvw_mfma_bf16.inc"), ("kTplUvwMfmaHalf", "uvw_mfma_half.inc"),
              ("kTplUvwMfmaDw", "uvw_mfma_dw.inc"), ("kTplUvwDwWide", "uvw_dw_wide.inc"),
-             ("kTplUvwNode", "uvw_node.inc"),
+             ("kTplUvwNode", "uvw_node.inc"), ("kTplUvwNodeDw", "uvw_node_dw.inc"),
              ("kTplFcMfma", "fc_mfma.inc"), ("kTplFcDw", "fc_dw.inc")]
 DEVICE_FLAGS = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 COMMON_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wno-unused-function", "-Wno-unused-result"]

@@ -17,6 +17,7 @@ extern const char* const kTplUvwMfmaHalf;
 extern const char* const kTplUvwMfmaDw;
 extern const char* const kTplUvwDwWide;
 extern const char* const kTplUvwNode;
+extern const char* const kTplUvwNodeDw;
 extern const char* const kTplFcMfma;
 extern const char* const kTplFcDw;
 

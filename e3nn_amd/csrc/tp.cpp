@@ -95,6 +95,10 @@ struct e3x_plan {
   // ... of products whose multiplicities are all multiples of 64: the kernel of uvw_dw_wide.inc (then `dw` is not built)
   std::unique_ptr<SubKernel> dw_wide;
   std::vector<std::pair<int, long long>> dw_wide_paths;  // per path: passes per outer index, tiles of a batch slice
+  // ... of node-wise layers (uvw_node): the kernel of uvw_node_dw.inc
+  std::unique_ptr<SubKernel> dw_node;
+  std::vector<std::pair<int, long long>> dw_node_paths;  // per path: components, tiles of a batch slice
+  int dw_node_per_cu = 2;                                // workgroups that a CU holds
 };
 
 namespace {
@@ -985,6 +989,42 @@ int build_uvw_dw_wide_source(e3x_plan& P, std::string* src) {
   return E3X_OK;
 }
 
+// Tables of the weight gradient of node-wise layers (templates/uvw_node_dw.inc).
+int build_uvw_node_dw_source(e3x_plan& P, std::string* src) {
+  std::ostringstream s, ps;
+  emit_header(s, P);
+  P.dw_node_paths.clear();
+  for (const auto& p : P.paths) {
+    const e3x_irrep &a = P.in1[p.in1], &b = P.in2[p.in2], &c = P.out[p.out];
+    const int d = 2 * a.l + 1, ut = (a.mul + 31) / 32, ct = (b.mul * c.mul + 31) / 32;
+    // the four waves of a workgroup side by side along u where there are tiles enough, else along the columns; up to four
+    // column tiles per workgroup
+    const int mtw = ut >= 3 ? 4 : ut, cg = 4 / mtw, tw = std::max(1, std::min(4, ct) / cg);
+    const long long tiles = (long long)((ut + mtw - 1) / mtw) * ((ct + tw * cg - 1) / (tw * cg));
+    ps << "  {" << P.off1[p.in1] << ", " << a.mul << ", " << d << ", " << P.off2[p.in2] << ", " << b.mul << ", " << P.offo[p.out] << ", "
+       << c.mul << ", " << p.woff << ", " << fstr(e3x::wigner_3j(a.l, 0, a.l)[0] * p.pw) << ", " << mtw << ", " << tw << ", " << tiles << "},\n";
+    P.dw_node_paths.push_back({d, tiles});
+  }
+  s << "struct NdPath { int x_off, U, d, o_off, V, g_off, W; long long wbase; float c; int MTW, TW, tiles; };\n";
+  s << "constexpr int N_NDPATH = " << P.paths.size() << ";\nconstexpr NdPath ndpaths[N_NDPATH] = {\n" << ps.str() << "};\n";
+  s << "constexpr int MIN_WGS = 2;\n}  // namespace cfg\n";  // workgroups per CU the register budget is set for (three spill at l = 2)
+  *src = s.str() + e3x::kTplCommon + e3x::kTplUvwNodeDw;
+  return E3X_OK;
+}
+
+int prepare_node_dw(e3x_plan* P) {
+  std::lock_guard<std::mutex> lock(P->mu);
+  if (P->dw_node) return E3X_OK;
+  std::unique_ptr<SubKernel> K(new SubKernel);
+  std::string src;
+  int rc;
+  if ((rc = build_uvw_node_dw_source(*P, &src))) return rc;
+  if ((rc = e3x::get_code_object("uvw_node_dw", src, &K->key, &K->hsaco))) return rc;
+  P->arithmetic_dw = "bf16 matrix instruction, six products of three-way split operands";
+  P->dw_node = std::move(K);
+  return E3X_OK;
+}
+
 // builds (or finds in the cache) the weight-gradient code object of a uvw_mfma plan
 int prepare_mfma_dw(e3x_plan* P) {
   std::lock_guard<std::mutex> lock(P->mu);
@@ -1024,15 +1064,13 @@ int load_dw_function(e3x_plan* P, int dev) {
   return E3X_OK;
 }
 
-// A uvw_node or uvw_mfma plan that the matrix-core gradient kernel does not take (multiplicities that are not
-// multiples of 32, operands that are not 16-byte aligned within their rows) gets its weight gradient from the
-// vector-ALU family: that code object is built on first use.  Decided from the plan alone, so that
-// e3x_tp_plan_prepare_backward_w and e3x_tp_backward_w_uvw agree.
-bool node_dw_on_valu(const e3x_plan* P) {
-  if (P->family == "uvw_node") return !uvw_mfma_eligible(*P) || !mfma_dw_fits(*P);
-  if (P->family == "uvw_mfma") return !mfma_dw_fits(*P);
-  return false;
-}
+// A uvw_mfma plan that the matrix-core gradient kernel does not take (operands that are not 16-byte aligned within their
+// rows) gets its weight gradient from the vector-ALU family, and so does a uvw_node plan whose gradient kernel cannot be had:
+// that code object is built on first use.
+bool mfma_dw_on_valu(const e3x_plan* P) { return P->family == "uvw_mfma" && !mfma_dw_fits(*P); }
+// A gradient of a few hundred numbers (a layer onto one scalar) is a sum over rows and hardly a matrix product: 96x0e x 4x0e
+// -> 1x0e, 50 000 rows, 58 us in the matrix-core kernel against 84 and twice the rounding error, from the sums of its slices.
+bool node_dw_on_valu(const e3x_plan* P) { return P->family == "uvw_node" && P->weight_numel < 1024; }
 
 int prepare_valu_dw(e3x_plan* P) {
   std::lock_guard<std::mutex> lock(P->mu);
@@ -2053,10 +2091,12 @@ extern "C" int e3x_tp_plan_prepare_backward_w(e3x_plan* P) {
     for (const auto& q : P->paths)
       if (q.mode != E3X_MODE_UVW)
         return fail(E3X_ERR_INVALID, "e3x_tp_plan_prepare_backward_w: no weight-gradient kernel for connection modes other than uvu / uvw");
-  if (node_dw_on_valu(P)) return prepare_valu_dw(P);
+  if (mfma_dw_on_valu(P) || node_dw_on_valu(P)) return prepare_valu_dw(P);
   if (P->family == "uvw_mfma" || P->family == "uvw_node") {
     if (P->dtype != E3X_F32) return fail(E3X_ERR_INVALID, "e3x_tp_plan_prepare_backward_w: fp32 storage only");
-    return prepare_mfma_dw(P);
+    if (P->family == "uvw_mfma") return prepare_mfma_dw(P);
+    const int rc = prepare_node_dw(P);
+    return rc == E3X_ERR_COMPILE ? prepare_valu_dw(P) : rc;
   }
   if (P->family == "uvu") return P->paths.empty() ? E3X_OK : prepare_uvu_bwd(P);
   return E3X_OK;  // uvw_small carries its gradient kernel in the forward code object
@@ -2102,6 +2142,53 @@ static int launch_dw_wide(e3x_plan* P, int dev, const void* x1, const void* x2, 
   return E3X_OK;
 }
 
+// Batch slices of the weight gradient of node-wise layers: as above, a path with d components per row has d times the slices,
+// of 32 rows or more.  Their number grows with the root of the batch, with which sums inside a slice and sums of slices lose
+// about the same to rounding (96x0e+128x1o+128x2e x 4x0e -> 32x0e+32x1o+32x2e, 400 000 rows, 85 / 170 slices: 970 / 870 us,
+// error 1.1e-6 / 8.8e-7 of the 2-norm), in whole rounds of the workgroups that run at once (50 000 rows: one round of 504
+// 114 us, one and a half 128).
+static int launch_node_dw(e3x_plan* P, int dev, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, hipStream_t st) {
+  int rc;
+  {
+    std::lock_guard<std::mutex> lock(P->mu);
+    SubKernel* K = P->dw_node.get();
+    if (!K->module[dev]) {
+      hipModule_t mod = nullptr;
+      hipError_t err = hipModuleLoad(&mod, K->hsaco.c_str());
+      if (err != hipSuccess) return fail(E3X_ERR_HIP, "hipModuleLoad(" + K->hsaco + ") failed: " + hipGetErrorString(err));
+      if (hipModuleGetFunction(&K->fn_dw[dev], mod, "e3x_uvw_node_dw") != hipSuccess)
+        return fail(E3X_ERR_HIP, "kernel e3x_uvw_node_dw missing from " + K->hsaco);
+      int per_cu = 0;
+      if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, K->fn_dw[dev], 256, 0) != hipSuccess || per_cu < 1) per_cu = 2;
+      P->dw_node_per_cu = std::min(per_cu, 3);
+      K->module[dev] = mod;
+    }
+  }
+  long long jobs = 0, units = 0;
+  int dmax = 1;
+  for (const auto& [d, tiles] : P->dw_node_paths) units += d * tiles, dmax = std::max(dmax, d);
+  const double root = std::sqrt(0.15 * (double)Z);
+  const long long slots = 256LL * P->dw_node_per_cu, rounds = std::max(1LL, (long long)(root * (double)units / (double)slots));
+  const long long n = std::max(1LL, std::min<long long>({rounds * slots / units, (long long)(2 * root), Z / (32LL * dmax)}));
+  // n = 1: every path whole
+  const long long unit = n == 1 ? (Z + 15) / 16 * 16 * 7 : (Z + n - 1) / n;
+  bool accumulate_ = false;
+  for (const auto& [d, tiles] : P->dw_node_paths) {
+    const long long rows = (unit / d + 15) / 16 * 16, slices = (Z + rows - 1) / rows;
+    jobs += slices * tiles;
+    accumulate_ = accumulate_ || slices > 1;
+  }
+  jobs = (jobs + 7) / 8 * 8;
+  if (unit >= (1LL << 31) || jobs >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: batch too large for one launch");
+  int unit_rows = (int)unit, accumulate = accumulate_;
+  if (accumulate && (rc = e3x::fill_zero_bytes(grad_w, (size_t)P->weight_numel * 4, st))) return rc;
+  long long n_rows = Z;
+  void* args[] = {(void*)&x1, (void*)&x2, (void*)&grad_out, (void*)&grad_w, (void*)&n_rows, (void*)&unit_rows, (void*)&accumulate};
+  hipError_t err = hipModuleLaunchKernel(P->dw_node->fn_dw[dev], (unsigned)jobs, 1, 1, 256, 1, 1, 0, st, args, nullptr);
+  if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_backward_w_uvw: launch failed: ") + hipGetErrorString(err));
+  return E3X_OK;
+}
+
 extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2, const void* grad_out, void* grad_w,
                                      int64_t Z, void* stream) {
   if (!P) return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: null plan");
@@ -2117,11 +2204,16 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
   hipStream_t st = (hipStream_t)stream;
   int dev, rc;
   if ((rc = current_device(&dev))) return rc;
-  // the node-wise family has no gradient kernel of its own: the matrix-core one where its tiling fits, else the vector-ALU one
-  const bool mfma = (P->family == "uvw_mfma" || P->family == "uvw_node") && !node_dw_on_valu(P);
+  const bool mfma = P->family == "uvw_mfma" && !mfma_dw_on_valu(P);
   if (Z == 0) return P->shared_weights ? e3x::fill_zero_bytes(grad_w, (size_t)P->weight_numel * 4, st) : E3X_OK;
   if (!grad_out || (P->in1_dim && !x1) || (P->in2_dim && !x2)) return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: null pointer");
   long long n_rows = Z;
+  bool valu = mfma_dw_on_valu(P) || node_dw_on_valu(P);
+  if (P->family == "uvw_node" && !valu) {
+    if ((rc = prepare_node_dw(P)) && rc != E3X_ERR_COMPILE) return rc;
+    valu = rc == E3X_ERR_COMPILE;  // (not to be had, as with a cache made without it and E3X_NO_JIT)
+    if (!valu) return launch_node_dw(P, dev, x1, x2, grad_out, grad_w, Z, st);
+  }
   if (mfma) {
     if (((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)grad_out) & 15)
       return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: x1, x2 and grad_out must be 16-byte aligned");
@@ -2148,7 +2240,7 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
   }
   if (P->shared_weights && (rc = e3x::fill_zero_bytes(grad_w, (size_t)P->weight_numel * 4, st))) return rc;
   hipFunction_t fn_dw = nullptr;
-  if (node_dw_on_valu(P)) {
+  if (valu) {
     if ((rc = prepare_valu_dw(P))) return rc;
     if ((rc = load_valu_dw_function(P, dev))) return rc;
     fn_dw = P->dw->fn_dw[dev];

@@ -222,7 +222,7 @@ def all_tensor_products():
 
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
 BACKWARD_CASES = ["cfg1", "cfg3_merged", "cfg3_builder", "cfg4_A", "cfg5", "mfma_small", "mfma_full_tiles", "mfma_wide_blocks", "outer_split", "node_fctp", "node_block",
-                  "node_wide_out", "node_narrow", "node_partial_tile", "radial_layer", "odd_mul", "unaligned_mfma", "unaligned_offsets",
+                  "node_wide_out", "node_narrow", "node_many_species", "node_partial_tile", "radial_layer", "odd_mul", "unaligned_mfma", "unaligned_offsets",
                   "mixed_modes", "scalar_exact", "narrow_message", "ragged_wide_message"]  # fmt: skip
 
 

@@ -171,6 +171,20 @@ def test_uvw_weight_gradient_of_wide_blocks(Z):
         offset += n
 
 
+@pytest.mark.parametrize("maker", [ks.node_block, ks.node_narrow, ks.node_wide_out, ks.node_many_species, ks.radial_layer])
+@pytest.mark.parametrize("Z", [1, 16, 17, 2500])
+def test_uvw_weight_gradient_of_node_wise_layers(maker, Z):
+    # stages of 16 rows and their remainders, one slice and several; tiles of both indices that are not full
+    tp = maker()
+    spec = oracle_spec(tp)
+    x1, x2, g = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(Z, tp.irreps_out.dim, seed=3)
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True).double().cpu()
+    # sums of at most 2500 x 7 products in fp32: a random walk of some hundred roundings of 6e-8 / sqrt(3)
+    assert float((got - ref).norm() / ref.norm()) < 1e-6
+
+
 @pytest.mark.parametrize("maker", [ks.mfma_full_tiles, ks.node_block])
 @pytest.mark.parametrize("sizes", ["x1 against x2", "x1 against g", "x2 against g", "masked row", "largest number", "channels"])
 def test_uvw_weight_gradient_of_numbers_of_different_sizes(maker, sizes):
