@@ -18,7 +18,8 @@ _NORMALIZATION = {"integral": _lib.NORM_INTEGRAL, "component": _lib.NORM_COMPONE
 
 @functools.lru_cache(maxsize=64)
 def _degrees(ls):
-    return (ctypes.c_int32 * len(ls))(*ls)
+    """The degrees as the library takes them, and the width of a row of the output."""
+    return (ctypes.c_int32 * len(ls))(*ls), sum(2 * l + 1 for l in ls)
 
 
 def _rows(x):
@@ -32,7 +33,7 @@ def _forward(x, ls, normalize, normalization):
     if x.dtype != torch.float32:
         raise TypeError(f"spherical_harmonics kernel supports float32 input, got {x.dtype}")
     xyz = _rows(x)
-    n, n_out = xyz.shape[0], sum(2 * l + 1 for l in ls)
+    n, n_out = xyz.shape[0], _degrees(ls)[1]
     out = torch.empty(n, n_out, dtype=x.dtype, device=x.device)
     _launch("e3x_sh_forward", ls, normalize, normalization, n, x.device, xyz, out)
     return out if x.ndim == 2 and n == x.shape[0] else out.reshape(x.shape[:-1] + (n_out,))
@@ -41,14 +42,15 @@ def _forward(x, ls, normalize, normalization):
 def _backward(x, g, ls, normalize, normalization):
     """``(grad_x <g, Y(x)>, rows of x, rows of g)``."""
     xyz = _rows(x)
-    g2 = g.reshape(xyz.shape[0], sum(2 * l + 1 for l in ls)).contiguous()  # the width spelled out: -1 is ambiguous for n = 0
+    n, n_out = xyz.shape[0], _degrees(ls)[1]
+    g2 = g if g.shape == (n, n_out) and g.is_contiguous() else g.reshape(n, n_out).contiguous()  # the width spelled out: -1 is ambiguous for n = 0
     gx = torch.empty_like(xyz)
-    _launch("e3x_sh_backward", ls, normalize, normalization, xyz.shape[0], x.device, xyz, g2, gx)
+    _launch("e3x_sh_backward", ls, normalize, normalization, n, x.device, xyz, g2, gx)
     return gx if x.ndim == 2 and x.shape[1] == 3 else gx.reshape(x.shape[:-1] + (3,)), xyz, g2
 
 
 def _launch(entry, ls, normalize, normalization, n, device, *tensors):
-    arr = _degrees(ls)
+    arr = _degrees(ls)[0]
     with _lib.on_device(device):
         _lib.check(
             getattr(_lib.lib(), entry)(
@@ -177,4 +179,13 @@ def spherical_harmonics(
     l = 0 constant and zeros elsewhere); ``normalization`` is ``'integral'``,
     ``'component'`` (:math:`\|Y^l\|^2 = 2l+1` on the sphere) or ``'norm'``.
     """
+    # the module's checks and irreps once per set of degrees: a call spent more time on them than on all the rest (a
+    # molecular-dynamics step of a block on 5003 nodes waits for it behind the read-back of its neighbour list)
+    if type(l) in (int, str) or (type(l) is list and all(type(i) is int for i in l)):
+        return _module(tuple(l) if type(l) is list else l, bool(normalize), normalization)(x)
     return SphericalHarmonics(l, normalize, normalization)(x)
+
+
+@functools.lru_cache(maxsize=64)
+def _module(l, normalize, normalization):
+    return SphericalHarmonics(list(l) if isinstance(l, tuple) else l, normalize, normalization)
