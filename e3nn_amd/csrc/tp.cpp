@@ -46,6 +46,7 @@ struct SubKernel {
   hipFunction_t fn_pack[kMaxDevices] = {nullptr};
   hipFunction_t fn_max[kMaxDevices] = {nullptr};
   hipFunction_t fn_sum[kMaxDevices] = {nullptr};
+  hipFunction_t fn_share[kMaxDevices] = {nullptr};
   // uvu: the edge-parallel backward kernel is a code object of its own (other lane layout), built on first use
   std::unique_ptr<SubKernel> bwd;
   // uvu, transposed plan of a message step: the fused kernel that also writes the weight gradient, built on first use
@@ -67,6 +68,7 @@ struct e3x_plan {
   bool zero_fill = false;  // some output irrep is reached by no instruction
   int n_targets = 0;       // uvw_mfma: grid.y
   std::vector<int> node_tile_rows;  // uvw_node: rows per workgroup of each target, in grid order
+  bool node_share = false;          // ... and the variant for small batches, a quarter of these rows, is in the code object
   // uvu: the message kernel with the radial network inside, one per network description, built on first use
   std::vector<std::unique_ptr<SubKernel>> radial;
   std::vector<std::unique_ptr<SubKernel>> radial_retired;  // kernels of earlier network descriptions: a launch may still hold them
@@ -827,6 +829,10 @@ int build_uvw_node_source(e3x_plan& P, std::string* src) {
     if (split) s << "#define E3X_NODE_SPLIT 1\n";
     P.arithmetic = split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
   }
+  // a wave per outer index (run_target's SHARE): two to four of them in every path
+  P.node_share = true;
+  for (const auto& p : P.paths) P.node_share = P.node_share && P.in2[p.in2].mul >= 2 && P.in2[p.in2].mul <= 4;
+  if (P.node_share) s << "#define E3X_NODE_SHARE 1\nconstexpr int MAX_D = " << max_d << ";\n";
   // workgroups per CU the register budget is set for: three when their weights fit (160 KB of LDS per CU)
   s << "constexpr int MIN_WGS = " << env_int("E3X_NODE_WGS", max_blocks <= 48 && max_d <= 5 ? 3 : 2) << ";\n";
   s << "}  // namespace cfg\n";
@@ -1116,6 +1122,10 @@ int load_functions(e3x_plan* P, int dev) {
     if (P->family == "uvw_mfma" && P->dtype == E3X_BF16) {
       if (hipModuleGetFunction(&K->fn_pack[dev], mod, "e3x_uvw_mfma_pack") != hipSuccess)
         return fail(E3X_ERR_HIP, "kernel e3x_uvw_mfma_pack missing from " + K->hsaco);
+    }
+    if (P->family == "uvw_node" && P->node_share) {
+      if (hipModuleGetFunction(&K->fn_share[dev], mod, "e3x_uvw_node_share") != hipSuccess)
+        return fail(E3X_ERR_HIP, "kernel e3x_uvw_node_share missing from " + K->hsaco);
     }
     if (P->family == "uvw_small") {
       if (hipModuleGetFunction(&K->fn_dw[dev], mod, "e3x_uvw_small_dw") != hipSuccess)
@@ -1593,6 +1603,7 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
   for (auto& K : P->subs) {
     long long blocks;
     unsigned grid_y = 1;
+    hipFunction_t fn = K->fn_plain[dev];
     if (P->family == "uvw_mfma") {
       const int rows = 16 * K->waves_per_block;  // fp32: 4 waves, 64 rows; bf16: 8 waves, 128 rows
       blocks = (Z + rows - 1) / rows;
@@ -1608,6 +1619,15 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
         return fail(E3X_ERR_INVALID, "e3x_tp_forward: x1 and the weights must be 16-byte aligned");
       blocks = 0;
       for (int rows : P->node_tile_rows) blocks += (Z + rows - 1) / rows;
+      // Few rows: a quarter of them per workgroup, a wave per outer index, as long as these are one round of two per CU.
+      // x 4x0e, 5003 rows, us: 96x0e+128x1o+128x2e -> 32x0e+32x1o+32x2e 39.7 -> 28.3, 32x0e+32x1o+32x2e -> the same
+      // 14.1 -> 10.9, 96x0e -> 1x0e 16.8 -> 10.3 (20 rows 32.8 -> 16.9, 10.7 -> 8.5, 15.5 -> 9.0); beyond it the second
+      // 14.9 -> 17.0 at 8000 rows, the first 44.0 -> 46.1 at 12 000.
+      if (P->node_share && blocks <= 128) {
+        fn = K->fn_share[dev];
+        blocks = 0;
+        for (int rows : P->node_tile_rows) blocks += (Z + rows / 4 - 1) / (rows / 4);
+      }
     } else {
       const int groups = 64 / K->lanes;
       const long long items = (Z + groups - 1) / groups * K->chunks;
@@ -1616,7 +1636,7 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
     }
     if (blocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_forward: batch too large for one launch");
     hipError_t err =
-        hipModuleLaunchKernel(K->fn_plain[dev], (unsigned)blocks, grid_y, 1, 64 * K->waves_per_block, 1, 1, 0, st, args, nullptr);
+        hipModuleLaunchKernel(fn, (unsigned)blocks, grid_y, 1, 64 * K->waves_per_block, 1, 1, 0, st, args, nullptr);
     if (err != hipSuccess)
       return fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
   }

@@ -202,6 +202,19 @@ def test_uvw_matrix_core_kernel_against_oracle(maker, Z, family):
     assert_close(out, ref, what=str(tp))
 
 
+@pytest.mark.parametrize("maker", [ks.node_block, ks.node_narrow, ks.node_wide_out, ks.node_partial_tile])
+@pytest.mark.parametrize("Z", [1, 31, 33, 20000])
+def test_node_wise_kernel_small_and_large_batches(maker, Z):
+    # the four waves of a workgroup share 32 rows (64 of a scalar output) where the batch is small, 2 to 4 outer indices
+    tp = maker().to(DEV)
+    assert tp._plan(torch.float32).family == "uvw_node"
+    w = _fan_in_weights(tp)
+    x1, x2 = seeded(Z, tp.irreps_in1.dim, seed=21), seeded(Z, tp.irreps_in2.dim, seed=22)
+    out = tp(x1.to(DEV), x2.to(DEV), w.to(DEV))
+    rows = torch.cat([torch.arange(min(Z, 70)), torch.arange(max(0, Z - 70), Z)]).unique()
+    assert_close(out[rows], otp.tp_forward(oracle_spec(tp), x1[rows].numpy(), x2[rows].numpy(), w.numpy()), what=str(tp))
+
+
 @pytest.mark.parametrize("maker,Z", [(ks.node_fctp, 333), (ks.node_fctp, 1), (ks.node_wide_out, 130), (ks.node_narrow, 301), (ks.node_partial_tile, 257),
                                      (ks.node_many_species, 140)])  # fmt: skip
 def test_node_wise_kernel_in_bf16_storage_against_oracle(maker, Z):
