@@ -28,7 +28,7 @@ constexpr int kMaxLiveRegs = 192;
 
 struct e3x_fc_plan {
   std::vector<int> hs, hp;
-  int n_layers = 0, rows_per_wg = 0, waves = 8;
+  int n_layers = 0, rows_per_wave = 0, waves = 8;
   bool epilogue = false;  // outputs are multiplied by an activation derivative of a caller-supplied tensor
   int input_act = 0;      // the rows given are pre-activations: the network starts from input_cst * act(x)
   double input_cst = 1.0;
@@ -172,7 +172,7 @@ extern "C" int e3x_fc_plan_create_fused(const int32_t* hs, int32_t n_hs, int32_t
   if (const char* v = std::getenv("E3X_FC_WAVES")) waves = std::atoi(v);
   if ((rs != 1 && rs != 2) || waves < 1 || waves > 16) return fail(E3X_ERR_INVALID, "E3X_FC_RS must be 1 or 2, E3X_FC_WAVES 1..16");
   P->waves = waves;
-  P->rows_per_wg = waves * 32 * rs;
+  P->rows_per_wave = 32 * rs;
   std::ostringstream s;
   s << "// generated: one fully-connected network\n#include <stdint.h>\nnamespace cfg {\n";
   s << "constexpr int NL = " << NL << ";\nconstexpr int H[NL + 1] = {";
@@ -304,8 +304,8 @@ extern "C" int e3x_fc_forward_epilogue(e3x_fc_plan* P, const void* x, const void
     if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_fc_forward: pack launch failed: ") + hipGetErrorString(err));
   }
   long long n_rows = Z;
-  long long tiles = (Z + P->rows_per_wg - 1) / P->rows_per_wg;
-  long long blocks = tiles < P->n_cu[dev] ? tiles : P->n_cu[dev];  // one persistent workgroup per compute unit
+  const long long tiles = (Z + P->rows_per_wave - 1) / P->rows_per_wave;
+  long long blocks = tiles < P->n_cu[dev] ? tiles : P->n_cu[dev];  // one persistent workgroup per compute unit, fewer only if some would have no tile
   void* args[] = {&x, &workspace, &out, &n_rows, &z};
   hipError_t err = hipModuleLaunchKernel(P->fn_fwd[dev], (unsigned)blocks, 1, 1, 64 * P->waves, 1, 1, 0, st, args, nullptr);
   if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_fc_forward: launch failed: ") + hipGetErrorString(err));
