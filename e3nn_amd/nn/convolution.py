@@ -9,6 +9,7 @@
 """
 import torch
 
+from .. import _lib
 from ..o3.irreps import Irrep, Irreps
 from ..o3.tensor_product import _OUT, FullyConnectedTensorProduct, TensorProduct, _permuted_weights, _slot_backward, _TpSlot
 from .edges import DstSortedEdges
@@ -28,25 +29,42 @@ _MAX_STORED_WEIGHTS = 1 << 28
 
 class _Mix(torch.autograd.Function):
     """``sc + (c0 + alpha * c1) * conv`` with ``c0 = (1 - m) / sqrt(n)``, ``c1 = m / n`` (reference
-    points_convolution.py:110-113 with the division by sqrt(num_neighbors) moved behind lin2 and alpha): two elementwise
-    kernels forward and three backward, where autograd through the separate operations launches a dozen over the
-    [N, channels] arrays.  The backward pass is written in differentiable elementwise operations, so it can itself be
-    differentiated (``create_graph``)."""
+    points_convolution.py:110-113 with the division by sqrt(num_neighbors) moved behind lin2 and alpha): one kernel
+    forward and one backward in fp32, elementwise operations elsewhere.  Under ``create_graph`` the backward pass is
+    written in differentiable elementwise operations, so it can itself be differentiated."""
 
     @staticmethod
     def forward(ctx, sc, alpha, conv, c0, c1):
-        coeff = torch.addcmul(c0, alpha, c1)  # [N, channels]
-        ctx.save_for_backward(coeff, conv, c1, alpha, c0)
-        return torch.addcmul(sc, coeff, conv)
+        ctx.save_for_backward(alpha, conv, c0, c1)
+        if not _mix_in_one_kernel(sc, alpha, conv, c0, c1):
+            return torch.addcmul(sc, torch.addcmul(c0, alpha, c1), conv)
+        out = torch.empty_like(sc)
+        with _lib.on_device(sc.device):
+            _lib.check(_lib.lib().e3x_mix_forward(*(_lib.ptr(t) for t in (sc, alpha, conv, c0, c1, out)), *sc.shape, _lib.stream_ptr(sc.device)))
+        return out
 
     @staticmethod
     def backward(ctx, g):
-        coeff, conv, c1, alpha, c0 = ctx.saved_tensors
-        if torch.is_grad_enabled():
-            coeff = torch.addcmul(c0, alpha, c1)  # as a function of alpha
+        alpha, conv, c0, c1 = ctx.saved_tensors
         need_sc, need_alpha, need_conv = ctx.needs_input_grad[:3]
-        g_alpha = (g * conv * c1).sum(-1, keepdim=True) if need_alpha else None
-        return (g if need_sc else None), g_alpha, (g * coeff if need_conv else None), None, None
+        g_rows = g.contiguous()
+        if not torch.is_grad_enabled() and _mix_in_one_kernel(g_rows, alpha, conv, c0, c1):
+            g_alpha = torch.empty_like(alpha) if need_alpha else None
+            g_conv = torch.empty_like(conv) if need_conv else None
+            with _lib.on_device(g.device):
+                _lib.check(_lib.lib().e3x_mix_backward(*(_lib.ptr(t) for t in (g_rows, alpha, conv, c0, c1, g_alpha, g_conv)), *conv.shape, _lib.stream_ptr(g.device)))
+        else:
+            g_alpha = (g * conv * c1).sum(-1, keepdim=True) if need_alpha else None
+            g_conv = g * torch.addcmul(c0, alpha, c1) if need_conv else None
+        return (g if need_sc else None), g_alpha, g_conv, None, None
+
+
+def _mix_in_one_kernel(rows, alpha, conv, c0, c1):
+    return (
+        rows.is_cuda and rows.dim() == 2 and rows.shape == conv.shape and alpha.shape == (rows.shape[0], 1)
+        and c0.shape == c1.shape == rows.shape[1:]
+        and all(t.dtype == torch.float32 and t.is_contiguous() and t.device == rows.device for t in (rows, alpha, conv, c0, c1))
+    )  # fmt: skip
 
 
 class _Lin2Alpha(torch.autograd.Function):
@@ -56,38 +74,37 @@ class _Lin2Alpha(torch.autograd.Function):
     that autograd then adds to the first: three passes over an array as wide as the messages saved."""
 
     @staticmethod
-    def forward(ctx, features, attr, w_lin2, w_alpha, lin2, head):
-        ctx.lin2, ctx.head = lin2, head
-        scalars = features[:, : head.irreps_in1.dim].contiguous()
-        ctx.save_for_backward(features, attr, w_lin2, w_alpha, scalars)
+    def forward(ctx, features, attr, w_lin2, w_alpha, lin2, alpha, head):
+        ctx.lin2, ctx.alpha, ctx.head = lin2, alpha, head
+        ctx.save_for_backward(features, attr, w_lin2, w_alpha)
         dt = features.dtype
-        return lin2._plan(dt).forward(features, attr, w_lin2), head._plan(dt).forward(scalars, attr, w_alpha)
+        return lin2._plan(dt).forward(features, attr, w_lin2), alpha._plan(dt).forward(features, attr, w_alpha)
 
     @staticmethod
     def backward(ctx, g_conv, g_alpha):
-        lin2, head = ctx.lin2, ctx.head
-        features, attr, w_lin2, w_alpha, scalars = ctx.saved_tensors
+        lin2, alpha, head = ctx.lin2, ctx.alpha, ctx.head
+        features, attr, w_lin2, w_alpha = ctx.saved_tensors
+        k = head.irreps_in1.dim
         g_conv, g_alpha = g_conv.contiguous(), g_alpha.contiguous()
         if torch.is_grad_enabled():
             # under create_graph: the two products' own differentiable gradients
             need = ctx.needs_input_grad
-            k = head.irreps_in1.dim
             gf, _, gw_lin2 = _slot_backward(_TpSlot, _OUT, (features, attr, w_lin2), g_conv, (need[0], False, need[2]), lin2)
             gs, _, gw_alpha = _slot_backward(_TpSlot, _OUT, (features[:, :k].contiguous(), attr, w_alpha), g_alpha, (need[0], False, need[3]), head)
             if need[0]:
                 gf = gf + torch.nn.functional.pad(gs, (0, features.shape[1] - k))
-            return gf, None, gw_lin2, gw_alpha, None, None
+            return gf, None, gw_lin2, gw_alpha, None, None, None
         dt = features.dtype
         g_features = gw_lin2 = gw_alpha = None
         if ctx.needs_input_grad[2]:
             gw_lin2 = lin2._plan(dt).backward_w_uvw(features, attr, g_conv, True)
         if ctx.needs_input_grad[3]:
-            gw_alpha = head._plan(dt).backward_w_uvw(scalars, attr, g_alpha, True)
+            gw_alpha = alpha._plan(dt).backward_w_uvw(features, attr, g_alpha, True)
         if ctx.needs_input_grad[0]:
             g_features = lin2._grad_plan("x1", dt).forward(g_conv, attr, _permuted_weights(lin2, w_lin2, (2, 1, 0)))
             g_scalars = head._grad_plan("x1", dt).forward(g_alpha, attr, _permuted_weights(head, w_alpha, (2, 1, 0)))
-            g_features[:, : scalars.shape[1]] += g_scalars
-        return g_features, None, gw_lin2, gw_alpha, None, None
+            g_features[:, :k] += g_scalars
+        return g_features, None, gw_lin2, gw_alpha, None, None, None
 
 
 class Convolution(torch.nn.Module):
@@ -175,7 +192,7 @@ class Convolution(torch.nn.Module):
         ):
             node_conv_out, alpha = _Lin2Alpha.apply(
                 node_features.contiguous(), node_attr.to(node_features.dtype).contiguous(), self.lin2.weight, self.alpha.weight,
-                self.lin2, self._alpha_head,
+                self.lin2, self.alpha, self._alpha_head,
             )  # fmt: skip
         else:
             node_conv_out = self.lin2(node_features, node_attr)

@@ -391,6 +391,12 @@ int e3x_gate_forward(const e3x_act_block* acts, int32_t n_acts, const e3x_gate_b
 int e3x_gate_backward(const e3x_act_block* acts, int32_t n_acts, const e3x_gate_block* gates, int32_t n_gates, const void* x,
                       const void* grad_out, void* grad_x, int64_t Z, int64_t in_dim, int64_t out_dim, int32_t dtype,
                       void* stream);
+/* Mixing of a convolution block, rows of C columns in fp32: out = sc + (c0[c] + alpha[n] c1[c]) conv (reference
+ * points_convolution.py:110-113), and the gradients with respect to alpha[N] and conv[N, C] (either may be NULL). */
+int e3x_mix_forward(const float* sc, const float* alpha, const float* conv, const float* c0, const float* c1, float* out, int64_t N,
+                    int64_t C, void* stream);
+int e3x_mix_backward(const float* grad_out, const float* alpha, const float* conv, const float* c0, const float* c1, float* grad_alpha,
+                     float* grad_conv, int64_t N, int64_t C, void* stream);
 /* The derivative of e3x_gate_backward: for a cotangent cot_x[Z, in_dim] on its result,
  * grad_grad_out[Z, out_dim] = d<cot_x, grad_x>/d grad_out and grad_x[Z, in_dim] = d<cot_x, grad_x>/dx (second
  * derivatives of the activations; 0 for abs and relu away from 0).  The reference differentiates

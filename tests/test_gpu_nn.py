@@ -496,3 +496,22 @@ def test_node_wise_blocks_in_bf16_storage():
             continue
         assert pb.grad.dtype == torch.bfloat16, name
         assert_close(pb.grad, pf.grad.cpu().numpy(), **_bf16_tol(pf.grad, 10), what=f"convolution block d/d{name}, bf16 storage")
+
+
+@pytest.mark.parametrize("N,C", [(1, 3), (5, 288), (70, 290), (16390, 4), (3, 1028)])
+@pytest.mark.parametrize("wanted", ["all", "alpha", "conv"])
+def test_mixing_of_a_convolution_block(N, C, wanted):
+    # rows shorter and longer than a wavefront's 256 floats, columns that are no multiple of four, more rows than wavefronts
+    from e3nn_amd.nn.convolution import _Mix
+
+    sc, alpha, conv, g = seeded(N, C, seed=1), seeded(N, 1, seed=2), seeded(N, C, seed=3), seeded(N, C, seed=4)
+    c0, c1 = seeded(C, seed=5), seeded(C, seed=6)
+    leaves = [t.to(DEV).requires_grad_(wanted == "all" or name == wanted) for name, t in (("sc", sc), ("alpha", alpha), ("conv", conv))]
+    out = _Mix.apply(*leaves, c0.to(DEV), c1.to(DEV))
+    grads = dict(zip([n for n, t in zip(("sc", "alpha", "conv"), leaves) if t.requires_grad], torch.autograd.grad(out, [t for t in leaves if t.requires_grad], g.to(DEV))))
+    s, a, v, k0, k1, gd = (t.double() for t in (sc, alpha, conv, c0, c1, g))
+    want = {"sc": gd, "alpha": (gd * v * k1).sum(-1, keepdim=True), "conv": gd * (k0 + a * k1)}
+    # a few roundings of 6e-8 per element; the sum over C columns: a random walk of C / 64 of them per lane
+    assert_close(out, (s + (k0 + a * k1) * v).numpy(), atol=1e-5, rtol=1e-6)
+    for name, got in grads.items():
+        assert_close(got, want[name].numpy(), atol=1e-5 if name != "alpha" else 1e-6 * C**0.5 + 1e-5, rtol=1e-6, what=name)
