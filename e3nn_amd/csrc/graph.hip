@@ -126,6 +126,11 @@ __global__ __launch_bounds__(kBlock) void rowkey_kernel(const IdxT* __restrict__
   }
 }
 
+// whether rows a and b, b next to a in an order, have the same two smallest sources
+__device__ __forceinline__ bool counts_as_shared(const unsigned* __restrict__ keys, const unsigned* __restrict__ second, int a, int b) {
+  return keys[a] != 0xffffffffu && keys[a] == keys[b] && second[a] != 0xffffffffu && second[a] == second[b];
+}
+
 // counts the neighbours in the order that agree in BOTH smallest sources: chance alone makes rows share one
 // (a small id is the minimum of many rows), two in common mean overlapping source sets
 __global__ __launch_bounds__(kBlock) void order_score_kernel(const int* __restrict__ order, const unsigned* __restrict__ keys,
@@ -133,8 +138,7 @@ __global__ __launch_bounds__(kBlock) void order_score_kernel(const int* __restri
                                                              int* __restrict__ score) {
   int hits = 0;
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i + 1 < N; i += (long long)gridDim.x * kBlock) {
-    const int a = order[i], b = order[i + 1];
-    if (keys[a] != 0xffffffffu && keys[a] == keys[b] && second[a] != 0xffffffffu && second[a] == second[b]) ++hits;
+    if (counts_as_shared(keys, second, order[i], order[i + 1])) ++hits;
   }
   if (hits) atomicAdd(score, hits);
 }
@@ -203,7 +207,8 @@ __global__ __launch_bounds__(kBlock) void fill_zero_bytes_kernel(unsigned char* 
 // ---- edge list in one pass: e3x_edges_build ---------------------------------------------------------------
 // Counting sort by destination.  What bounds the set-up of a neighbour list is launches and host round trips, not bytes:
 // 176 852 edges on 5 003 nodes took four library sorts (some 30 launches, 0.17 ms of kernels) and four stream
-// synchronisations.  Here: counts, two scan kernels, placement, one pass over the rows, one ranking kernel, one read-back.
+// synchronisations.  Here: counts, one or two scan kernels, placement, one pass over the rows, one ranking kernel, one
+// read-back.
 //   count    rank of an edge inside its row by an atomic on the row's counter; neighbouring lanes with the same
 //            destination take one atomic together, so a list that is already grouped costs one atomic per run.  The
 //            ranks depend on the order of the atomics;
@@ -212,6 +217,9 @@ __global__ __launch_bounds__(kBlock) void fill_zero_bytes_kernel(unsigned char* 
 //            row's two smallest sources.  A list that was grouped already skips the sorting (perm is the identity);
 //   order    rows ranked by their key by counting smaller keys.
 constexpr int kScanTile = 4096;
+// Up to here the second of the two scan kernels does without the first: adding up three tiles before one's own is less than a
+// launch.  With the one ranking kernel below, set-up and step of a block on 5003 nodes 355 -> 339 us.
+constexpr unsigned kScanTilesDirect = 4;
 constexpr int kRowMax = 1024;  // longest row that is put in order here
 enum { kBadSrc = 0, kBadDst, kUnsorted, kOverflow, kScore, kFlags };
 
@@ -279,14 +287,20 @@ __global__ __launch_bounds__(kBlock) void edges_scan_sums_kernel(const int* __re
   }
 }
 
-// rowptr[n] = sum of counts[0 .. n - 1], n = 0 .. N; every workgroup adds up the sums of the tiles before its own
+// rowptr[n] = sum of counts[0 .. n - 1], n = 0 .. N; every workgroup adds up the sums of the tiles before its own, or, where
+// these are not given, the counts themselves
 __global__ __launch_bounds__(kBlock) void edges_scan_kernel(const int* __restrict__ counts, long long N, const int* __restrict__ sums,
                                                             int* __restrict__ rowptr) {
   __shared__ int part[kBlock / 64], wsum[kBlock / 64];
   constexpr int PER = kScanTile / kBlock;
   const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
   int before = 0;
-  for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlock) before += sums[i];
+  if (sums) {
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlock) before += sums[i];
+  } else {
+#pragma unroll 16
+    for (int i = threadIdx.x; i < (int)blockIdx.x * kScanTile; i += kBlock) before += counts[i];
+  }
   for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off, 64);
   if (lane == 0) part[wave] = before;
   const long long i0 = (long long)blockIdx.x * kScanTile + threadIdx.x * PER;
@@ -387,38 +401,83 @@ __global__ __launch_bounds__(kBlock) void edges_rows_kernel(const SrcT* __restri
 }
 
 // The position of a row in the order of (key of the key of its key, key of its key, key, number), the last three levels
-// only for one node set, found by counting the rows in front of it: N^2 comparisons spread over the chip.  A
-// workgroup takes 64 rows (a lane each), its 16 wavefronts a sixteenth of every tile of keys.
-constexpr long long kRankMax = 16384;
+// only for one node set, found by counting the rows in front of it: N^2 comparisons spread over the chip.  The row that
+// follows comes out of the same comparisons, and with it the pairs that order_score_kernel counts.  A workgroup takes ROWS
+// rows, its 16 wavefronts a sixteenth of every tile of keys, and the 64 / ROWS groups of lanes of a wavefront every
+// (64 / ROWS)th of these.
+// A step of few rows has few workgroups, and waits for the vector ALU (and to look up levels in memory, when it did) of the CUs
+// that have one.  Together with the count of the pairs as a kernel of its own, 64 rows a workgroup and 64-bit integers took
+// 7.5 / 8.5 / 17.4 / 23.1 / 32.1 / 46.5 us for 200 / 1000 / 5003 / 8192 / 12 000 / 16 384 rows; 16 rows 4.5 / 4.9 / 12.0 /
+// 17.2 / 31.3 / 50.6, 32 rows 5.3 / 5.5 / 12.5 / 16.8 / 32.0 / 42.7, 8 rows more from 1000 on (each workgroup reads all keys).
+constexpr long long kRankMax = 16384, kRankNarrow = 8192;  // (up to which: 16 rows)
 constexpr int kRankTile = 2048;
-__global__ __launch_bounds__(1024) void edges_order_kernel(const unsigned* __restrict__ keys, int N, int levels, int* __restrict__ order) {
-  __shared__ unsigned long long tile[kRankTile];
-  __shared__ int part[16][64];
+template <int ROWS>
+__global__ __launch_bounds__(1024) void edges_order_kernel(const unsigned* __restrict__ keys, const unsigned* __restrict__ second,
+                                                           int N, int levels, int* __restrict__ order, int* __restrict__ score) {
+  constexpr int GROUPS = 64 / ROWS, PER_WAVE = kRankTile / 16;
+  constexpr unsigned kNone = 0x7fe00000u;  // upper word of a number above every row's
+  __shared__ unsigned short key_of[kRankMax];
+  __shared__ double2 tile[kRankTile / 2];
+  __shared__ double part_next[16][ROWS];
+  __shared__ int part[16][ROWS];
+  // the keys as 16 bits (sources are numbered below 65535; a row without edges 65535), so that the levels are looked up in LDS
+  for (int i = threadIdx.x; i < N; i += 1024) key_of[i] = (unsigned short)keys[i];
+  __syncthreads();
+  // A row's levels and number as the bits of a positive normal double, whose order is that of the bits: one compare and one
+  // minimum a key where 64-bit integers take twice the instructions
   auto composite = [&](int n) {
-    const unsigned k = keys[n];
-    unsigned l1 = 0, l2 = 0;
+    const int k = key_of[n];
+    int l1 = 0, l2 = 0;
     if (levels) {
-      l1 = k < (unsigned)N ? keys[k] : 0xffffffffu;
-      l2 = l1 < (unsigned)N ? keys[l1] : 0xffffffffu;
+      l1 = k < N ? key_of[k] : 0xffff;
+      l2 = l1 < N ? min((int)key_of[l1], (int)kRankMax) : (int)kRankMax;  // (at least N where there is none)
     }
-    return ((unsigned long long)(l2 & 0xffffu) << 48) | ((unsigned long long)(l1 & 0xffffu) << 32) | ((unsigned long long)(k & 0xffffu) << 16) | (unsigned)n;
+    return __hiloint2double((l2 + 0x10) << 16 | l1, k << 16 | n);
   };
   const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
-  const int row = blockIdx.x * 64 + lane;
-  const unsigned long long mine = composite(row < N ? row : N - 1);
-  int smaller = 0;
+  const int row = blockIdx.x * ROWS + lane % ROWS, group = lane / ROWS;
+  const double mine = composite(row < N ? row : N - 1);
+  double next = __hiloint2double((int)kNone, 0);
+  int upto = 0;  // rows in front of this one, and itself
+  auto take = [&](double k) {
+    const bool le = k <= mine;
+    upto += le;
+    const double above = __hiloint2double(le ? (int)kNone : __double2hiint(k), __double2loint(k));
+    asm("v_min_f64 %0, %1, %2" : "=v"(next) : "v"(next), "v"(above));
+  };
   for (int t0 = 0; t0 < N; t0 += kRankTile) {
     __syncthreads();
-    for (int i = threadIdx.x; i < kRankTile; i += 1024) tile[i] = t0 + i < N ? composite(t0 + i) : ~0ull;
+    for (int i = threadIdx.x; i < kRankTile; i += 1024)
+      reinterpret_cast<double*>(tile)[i] = t0 + i < N ? composite(t0 + i) : __hiloint2double((int)kNone, 0);
     __syncthreads();
 #pragma unroll 8
-    for (int i = 0; i < kRankTile / 16; ++i) smaller += tile[wave * (kRankTile / 16) + i] < mine;
+    for (int i = 0; i < PER_WAVE / 2 / GROUPS; ++i) {
+      const double2 k = tile[wave * (PER_WAVE / 2) + i * GROUPS + group];
+      take(k.x);
+      take(k.y);
+    }
   }
-  part[wave][lane] = smaller;
+  for (int off = 32; off >= ROWS; off >>= 1) {
+    upto += __shfl_xor(upto, off, 64);
+    next = fmin(next, __shfl_xor(next, off, 64));
+  }
+  if (group == 0) {
+    part[wave][lane] = upto;
+    part_next[wave][lane] = next;
+  }
   __syncthreads();
-  if (wave == 0 && row < N) {
-    for (int i = 1; i < 16; ++i) smaller += part[i][lane];
-    order[smaller] = row;
+  if (wave == 0) {
+    bool hit = false;
+    if (group == 0 && row < N) {
+      for (int i = 1; i < 16; ++i) {
+        upto += part[i][lane];
+        next = fmin(next, part_next[i][lane]);
+      }
+      order[upto - 1] = row;
+      if ((unsigned)__double2hiint(next) < kNone) hit = counts_as_shared(keys, second, row, __double2loint(next) & 0xffff);
+    }
+    const int hits = __popcll(__ballot(hit));
+    if (lane == 0 && hits) atomicAdd(score, hits);
   }
 }
 
@@ -629,7 +688,8 @@ void launch_edges(const SrcT* src, const DstT* dst, long long E, long long N, lo
   // flags and counters lie next to each other
   hipLaunchKernelGGL(edges_zero_kernel, dim3(grid_for(64 + N, kBlock)), dim3(kBlock), 0, st, flags, 64 + N);
   hipLaunchKernelGGL((edges_count_kernel<SrcT, DstT>), dim3(grid_for(E, kBlock)), dim3(kBlock), 0, st, src, dst, E, N, n_src, counts, rank, flags);
-  hipLaunchKernelGGL(edges_scan_sums_kernel, dim3(tiles), dim3(kBlock), 0, st, counts, N, sums);
+  if (tiles > kScanTilesDirect) hipLaunchKernelGGL(edges_scan_sums_kernel, dim3(tiles), dim3(kBlock), 0, st, counts, N, sums);
+  else sums = nullptr;
   hipLaunchKernelGGL(edges_scan_kernel, dim3(tiles), dim3(kBlock), 0, st, counts, N, sums, rowptr);
   hipLaunchKernelGGL((edges_place_kernel<DstT>), dim3(grid_for(E, kBlock)), dim3(kBlock), 0, st, dst, E, N, rowptr, rank, flags, placed);
   hipLaunchKernelGGL((edges_rows_kernel<SrcT>), dim3((unsigned)((N + kBlock / 64 - 1) / (kBlock / 64))), dim3(kBlock), 0, st, src, rowptr,
@@ -695,10 +755,13 @@ extern "C" int e3x_edges_build(const void* src, int src_bits, const void* dst, i
     else E3X_EDGES(int, int);
 #undef E3X_EDGES
     if (ranks) {
-      hipLaunchKernelGGL(edges_order_kernel, dim3((unsigned)((num_nodes + 63) / 64)), dim3(1024), 0, st, keys, (int)num_nodes,
-                         num_src_nodes == num_nodes && num_nodes > 1 ? 1 : 0, row_order);
-      hipLaunchKernelGGL(order_score_kernel, dim3(grid_for(num_nodes, kBlock)), dim3(kBlock), 0, st, row_order, keys, second,
-                         (long long)num_nodes, flags + kScore);
+      const int levels = num_src_nodes == num_nodes && num_nodes > 1 ? 1 : 0;
+      const auto launch = [&](auto kernel, int rows) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((num_nodes + rows - 1) / rows)), dim3(1024), 0, st, keys, second, (int)num_nodes, levels,
+                           row_order, flags + kScore);
+      };
+      if (num_nodes <= kRankNarrow) launch(edges_order_kernel<16>, 16);
+      else launch(edges_order_kernel<32>, 32);
     }
     int h[kFlags] = {0};
     if (hipGetLastError() != hipSuccess) return e3x::fail(E3X_ERR_HIP, "e3x_edges_build: launch failed");

@@ -184,6 +184,33 @@ def test_row_processing_order(idx):
     assert geo.row_order is not None and geo.locality_score > 0.1, geo.locality_score
 
 
+@pytest.mark.parametrize("N", [1, 15, 17, 2049, 4096, 8192, 8193, 16383, 16384])
+def test_row_order_of_a_small_node_set(N):
+    """Row pointers, order and share of the counting set-up at the edges of its tiles, against sorting on the host: with and
+    without a node set of its own for the sources, rows without edges among them."""
+    rng = np.random.default_rng(N)
+    for n_src in (N, 65_534):
+        E = 3 * N
+        dst = rng.integers(0, N, E) // 3 * 2 % N  # every third row keeps no edge, and sources come in runs of neighbours
+        src = np.minimum((dst.astype(np.int64) // 8 * 8 + rng.integers(0, 9, E)) * n_src // N, n_src - 1)
+        edges = DstSortedEdges(torch.from_numpy(src).to(DEV), torch.from_numpy(dst).to(DEV), N, n_src, locality_order=True)
+        assert np.array_equal(edges.rowptr.cpu().numpy(), np.concatenate([[0], np.cumsum(np.bincount(dst, minlength=N))]))
+        none = 2**32 - 1
+        key, second = np.full(N, none), np.full(N, none)
+        np.minimum.at(key, dst, src)
+        above = src > key[dst]
+        np.minimum.at(second, dst[above], src[above])
+        k2 = k3 = np.zeros(N, dtype=np.int64)
+        if n_src == N and N > 1:
+            k2 = np.where(key < N, key[np.minimum(key, N - 1)], none)
+            k3 = np.where(k2 < N, key[np.minimum(k2, N - 1)], none)
+        order = np.lexsort((np.arange(N), key, k2, k3))
+        assert np.array_equal(edges.row_order.cpu().numpy(), order)
+        a, b = order[:-1], order[1:]
+        shared = ((key[a] == key[b]) & (key[a] != none) & (second[a] == second[b]) & (second[a] != none)).sum()
+        assert edges.locality_score == shared / N
+
+
 @pytest.mark.parametrize("maker,N,E,idx", [
     (lambda: ks.cfg3(True), 700, 26_000, torch.int64),
     (lambda: ks.cfg3(False), 300, 9_000, torch.int64),
