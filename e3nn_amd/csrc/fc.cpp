@@ -214,6 +214,10 @@ extern "C" int e3x_fc_plan_prepare_backward_w(e3x_fc_plan* P) {
   const int mt = (P->hs[0] + 31) / 32, nt = (P->hs[1] + 31) / 32;
   if (mt > 8) return fail(E3X_ERR_INVALID, "e3x_fc_backward_w: input width above 256");
   int ntw = std::min((nt + 3) / 4, std::max(1, 10 / mt));  // <= 160 accumulator registers per lane
+  // few tiles: every wave takes all of them for rows of its own (a split layer; the fp32 instruction keeps its form)
+  const char* split = std::getenv("E3X_FCDW_SPLIT");
+  const bool by_rows = nt <= 2 && mt * nt <= 4 && !(split && !std::atoi(split));
+  if (by_rows) ntw = nt;
   P->dw_col_groups = (nt + 4 * ntw - 1) / (4 * ntw);
   std::ostringstream s;
   s << "// generated: weight gradient of one dense layer\n#include <stdint.h>\n";
@@ -222,7 +226,7 @@ extern "C" int e3x_fc_plan_prepare_backward_w(e3x_fc_plan* P) {
   if (const char* v = std::getenv("E3X_FCDW_SPLIT")) s << "#define E3X_FCDW_SPLIT " << std::atoi(v) << "\n";
   if (const char* v = std::getenv("E3X_FCDW_SHARE")) s << "#define E3X_FCDW_SHARE " << std::atoi(v) << "\n";
   s << "namespace cfg {\n";
-  s << "constexpr int H_IN = " << P->hs[0] << ", H_OUT = " << P->hs[1] << ", NTW = " << ntw << ";\n";
+  s << "constexpr int H_IN = " << P->hs[0] << ", H_OUT = " << P->hs[1] << ", NTW = " << ntw << ";\nconstexpr bool BY_ROWS = " << (by_rows ? "true" : "false") << ";\n";
   s << "constexpr float SCALE = " << fstr(P->scale0) << ";\n";
   s << "constexpr int IN_ACT = " << P->input_act << ";\nconstexpr float IN_CST = " << fstr(P->input_cst) << ";\n}  // namespace cfg\n";
   const std::string src = s.str() + e3x::kTplCommon + e3x::kTplFcDw;

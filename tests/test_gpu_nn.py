@@ -239,6 +239,26 @@ def test_dense_layer_gradients_on_batches_around_one_trip(Z):
     assert_close(xd.grad, gz @ w0.T / np.sqrt(8.0), what=f"dense input gradient, Z = {Z}")
 
 
+@pytest.mark.parametrize("shape", [(8, 64), (3, 33), (33, 64), (100, 20), (128, 32), (65, 33)])
+@pytest.mark.parametrize("act", [None, "silu"])
+def test_dense_weight_gradient_of_few_tiles(shape, act):
+    """Layers of at most two column tiles and four tiles in all, where every wave takes trips of its own (65 -> 33 is past
+    that): batches around one trip, one workgroup and one round of trips.  A number is a sum over the rows on some 60 trips a
+    wave, four waves and at most 512 workgroups, so 1024 roundings of the sum of the magnitudes bound its error."""
+    net = nn.FullyConnectedNet([4, *shape], torch.nn.functional.silu) if act else nn.FullyConnectedNet(list(shape))
+    net = net.to(DEV)
+    layer = net.layer1 if act else net.layer0
+    for Z in (1, 16, 17, 63, 65, 257, 32_768 + 5, 250_003):
+        x, cot = seeded(Z, net.hs[0], seed=3 + Z).to(DEV), seeded(Z, shape[1], seed=5 + Z).to(DEV)
+        grad, = torch.autograd.grad(net(x), layer.weight, cot)
+        h = x.double()
+        if act:
+            h = onn.normalize2mom_const("silu") * torch.nn.functional.silu(h @ net.layer0.weight.detach().double() / 2.0)
+        scale = shape[0] ** -0.5
+        want, size = h.T @ cot.double() * scale, h.abs().T @ cot.abs().double() * scale
+        assert ((grad - want).abs() <= 1024 * 2.0**-24 * size).all(), (Z, ((grad - want).abs() / size).max().item())
+
+
 def test_fully_connected_net_wide_hidden_layer():
     """Outside the limits of the fused kernel every layer runs on the tensor-product kernels, forward and backward."""
     fc = dict(ks.nn_modules())["fc_wide_hidden"].to(DEV)
