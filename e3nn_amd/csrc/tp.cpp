@@ -487,7 +487,7 @@ bool build_uvu_msg_mfma_source(e3x_plan& P, SubKernel& K, std::string* src) {
 }
 
 // ---- uvw (lane <-> output multiplicity, VALU) ----------------------------------------
-int build_uvw_small_source(e3x_plan& P, SubKernel& K, std::string* src) {
+int build_uvw_small_source(e3x_plan& P, SubKernel& K, std::string* src, bool gradient_only = false) {
   int max_mul = 1;
   std::vector<char> usedo(P.out.size(), 0);
   bool all_uvw = true;
@@ -501,9 +501,10 @@ int build_uvw_small_source(e3x_plan& P, SubKernel& K, std::string* src) {
   // multiplicity idle)
   while (K.lanes < 64 && (P.in1_dim + P.in2_dim) * 16 * (64 / K.lanes) > 65536) K.lanes *= 2;
   K.chunks = (max_mul + K.lanes - 1) / K.lanes;
-  if ((P.in1_dim + P.in2_dim) * 16 * (64 / K.lanes) > 65536)
+  if (!gradient_only && (P.in1_dim + P.in2_dim) * 16 * (64 / K.lanes) > 65536)
     return fail(E3X_ERR_INVALID, "uvw kernel: input rows too long for the LDS staging buffer");
   std::ostringstream s;
+  if (gradient_only) s << "#define E3X_UVW_SMALL_DW_ONLY\n";
   emit_header(s, P, K.lanes, K.chunks);
   int reg = 0;
   s << "struct Out { int off, d, mul, reg; bool used; };\n";
@@ -1085,7 +1086,7 @@ int prepare_valu_dw(e3x_plan* P) {
   for (size_t i = 0; i < P->paths.size(); ++i) K->path_ids.push_back((int)i);
   std::string src;
   int rc;
-  if ((rc = build_uvw_small_source(*P, *K, &src))) return rc;
+  if ((rc = build_uvw_small_source(*P, *K, &src, true))) return rc;
   if ((rc = e3x::get_code_object("uvw_small", src, &K->key, &K->hsaco))) return rc;
   P->dw = std::move(K);
   return E3X_OK;

@@ -75,15 +75,18 @@ class _Lin2Alpha(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, features, attr, w_lin2, w_alpha, lin2, alpha, head):
-        ctx.lin2, ctx.alpha, ctx.head = lin2, alpha, head
-        ctx.save_for_backward(features, attr, w_lin2, w_alpha)
         dt = features.dtype
-        return lin2._plan(dt).forward(features, attr, w_lin2), alpha._plan(dt).forward(features, attr, w_alpha)
+        # the node-wise kernels read the scalars where they lie; the vector-ALU kernel stages whole rows, and takes a copy
+        in_place = head._plan(dt).family == "uvw_node" and features.shape[1] % 4 == 0
+        scalars, ctx.reads_scalars = (features, alpha) if in_place else (features[:, : head.irreps_in1.dim].contiguous(), head)
+        ctx.lin2, ctx.head = lin2, head
+        ctx.save_for_backward(features, attr, w_lin2, w_alpha, scalars)
+        return lin2._plan(dt).forward(features, attr, w_lin2), ctx.reads_scalars._plan(dt).forward(scalars, attr, w_alpha)
 
     @staticmethod
     def backward(ctx, g_conv, g_alpha):
-        lin2, alpha, head = ctx.lin2, ctx.alpha, ctx.head
-        features, attr, w_lin2, w_alpha = ctx.saved_tensors
+        lin2, head = ctx.lin2, ctx.head
+        features, attr, w_lin2, w_alpha, scalars = ctx.saved_tensors
         k = head.irreps_in1.dim
         g_conv, g_alpha = g_conv.contiguous(), g_alpha.contiguous()
         if torch.is_grad_enabled():
@@ -99,7 +102,7 @@ class _Lin2Alpha(torch.autograd.Function):
         if ctx.needs_input_grad[2]:
             gw_lin2 = lin2._plan(dt).backward_w_uvw(features, attr, g_conv, True)
         if ctx.needs_input_grad[3]:
-            gw_alpha = alpha._plan(dt).backward_w_uvw(features, attr, g_alpha, True)
+            gw_alpha = ctx.reads_scalars._plan(dt).backward_w_uvw(scalars, attr, g_alpha, True)
         if ctx.needs_input_grad[0]:
             g_features = lin2._grad_plan("x1", dt).forward(g_conv, attr, _permuted_weights(lin2, w_lin2, (2, 1, 0)))
             g_scalars = head._grad_plan("x1", dt).forward(g_alpha, attr, _permuted_weights(head, w_alpha, (2, 1, 0)))

@@ -57,6 +57,27 @@ def nn_golden():
     return np.load(os.path.join(GOLDEN, "nn_cases.npz")), meta
 
 
+# (features, node attributes) of blocks whose mixing coefficient is read from messages of 4224 numbers, too long for the
+# vector-ALU kernel to stage; of an ordinary width; with a handful of weights; and that are not whole 16-byte pieces
+ALPHA_CASES = [("384x0e+384x1o", "1x0e"), ("16x0e+16x1o", "4x0e"), ("8x0e+8x1o", "1x0e"), ("8x0e+7x1o", "9x0e")]
+
+
+def alpha_block(features, attr):
+    torch.manual_seed(1)
+    return nn.Convolution(features, attr, SH2, features, [8, 16], 4.0)
+
+
+def alpha_modules():
+    out = []
+    for i, case in enumerate(ALPHA_CASES):
+        conv = alpha_block(*case)
+        # (lin2 and alpha on the long messages have no kernel for the gradient of the node attributes, which a block does not
+        # ask for; those of a training step are built as they are used)
+        parts = [conv.sc, conv.lin1, conv.tp, conv.fc, conv.__dict__["_alpha_head"]] if i == 0 else [conv]
+        out.append((f"alpha_block{i}", torch.nn.ModuleList(p for p in parts if p is not None)))
+    return out
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
@@ -76,5 +97,5 @@ def golden_modules():
 
 def prebuild(verbose=True):
     """Every kernel the tests and the benchmark use: the package's list plus the fixtures' instruction sets."""
-    _ks.prebuild(verbose=verbose, extra_tensor_products=golden_tensor_products(), extra_modules=golden_modules(),
+    _ks.prebuild(verbose=verbose, extra_tensor_products=golden_tensor_products(), extra_modules=golden_modules() + alpha_modules(),
                  backward_cases=BACKWARD_CASES, backward_bf16_cases=BACKWARD_BF16_CASES)  # fmt: skip

@@ -535,3 +535,23 @@ def test_mixing_of_a_convolution_block(N, C, wanted):
     assert_close(out, (s + (k0 + a * k1) * v).numpy(), atol=1e-5, rtol=1e-6)
     for name, got in grads.items():
         assert_close(got, want[name].numpy(), atol=1e-5 if name != "alpha" else 1e-6 * C**0.5 + 1e-5, rtol=1e-6, what=name)
+
+
+@pytest.mark.parametrize("features,attr", ks.ALPHA_CASES)
+def test_alpha_of_a_convolution_block_on_wide_and_ragged_messages(features, attr):
+    """The mixing coefficient reads the leading scalars of the messages in place where a kernel can, else from a copy: its
+    weight gradient against the product restricted to the scalars, which is what a graph of the backward pass takes."""
+    conv = ks.alpha_block(features, attr).to(DEV)
+    N, E = 40, 150
+    src, dst = (torch.randint(0, N, (E,), generator=torch.Generator().manual_seed(i)).to(DEV) for i in (1, 2))
+    edge_attr = o3.spherical_harmonics([0, 1, 2], seeded(E, 3, seed=3).to(DEV), True, "component")
+    x = seeded(N, conv.irreps_node_input.dim, seed=1).to(DEV).requires_grad_()
+    node_attr = seeded(N, conv.irreps_node_attr.dim, seed=2).to(DEV)
+    out = conv(x, node_attr, src, dst, edge_attr, seeded(E, 8, seed=4).to(DEV))
+    cot = seeded(*out.shape, seed=5).to(DEV)
+    wanted = (conv.alpha.weight, conv.lin2.weight, x)
+    got = torch.autograd.grad(out, wanted, cot, retain_graph=True)
+    ref = torch.autograd.grad(out, wanted, cot, create_graph=True)
+    for a, b in zip(got, ref):
+        # both are sums of the same fp32 products, of 40 rows and at most a few thousand terms, in other orders
+        assert float((a - b).norm()) <= 1e-5 * float(b.norm())
