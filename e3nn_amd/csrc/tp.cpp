@@ -1076,8 +1076,21 @@ int load_dw_function(e3x_plan* P, int dev) {
 // that code object is built on first use.
 bool mfma_dw_on_valu(const e3x_plan* P) { return P->family == "uvw_mfma" && !mfma_dw_fits(*P); }
 // A gradient of a few hundred numbers (a layer onto one scalar) is a sum over rows and hardly a matrix product: 96x0e x 4x0e
-// -> 1x0e, 50 000 rows, 58 us in the matrix-core kernel against 84 and twice the rounding error, from the sums of its slices.
+// -> 1x0e, 50 000 rows, 58 us in the matrix-core kernel, with twice the rounding error from the sums of its slices, against 84
+// in e3x_uvw_small_dw and 20 in e3x_uvw_scalar_dw.
 bool node_dw_on_valu(const e3x_plan* P) { return P->family == "uvw_node" && P->weight_numel < 1024; }
+
+// ... where it couples scalars only, with few weights for an index of the first input: accumulators of the kernel that reads rows
+// as they lie (64 of them: 64 KB of LDS for the sums of the waves)
+bool scalar_dw_fits(const e3x_plan& P) {
+  if (P.family != "uvw_node") return false;
+  long long sums = 0;
+  for (const auto& p : P.paths) {
+    if (P.in1[p.in1].l || P.in2[p.in2].l || P.out[p.out].l) return false;
+    sums += (long long)(P.in1[p.in1].mul + 31) / 32 * P.in2[p.in2].mul * P.out[p.out].mul;
+  }
+  return sums <= 64;
+}
 
 int prepare_valu_dw(e3x_plan* P) {
   std::lock_guard<std::mutex> lock(P->mu);
@@ -1087,6 +1100,7 @@ int prepare_valu_dw(e3x_plan* P) {
   std::string src;
   int rc;
   if ((rc = build_uvw_small_source(*P, *K, &src, true))) return rc;
+  if (scalar_dw_fits(*P)) src = "#define E3X_UVW_SCALAR_DW\n" + src;
   if ((rc = e3x::get_code_object("uvw_small", src, &K->key, &K->hsaco))) return rc;
   P->dw = std::move(K);
   return E3X_OK;
@@ -1099,8 +1113,9 @@ int load_valu_dw_function(e3x_plan* P, int dev) {
   hipModule_t mod = nullptr;
   hipError_t err = hipModuleLoad(&mod, K->hsaco.c_str());
   if (err != hipSuccess) return fail(E3X_ERR_HIP, "hipModuleLoad(" + K->hsaco + ") failed: " + hipGetErrorString(err));
-  if (hipModuleGetFunction(&K->fn_dw[dev], mod, "e3x_uvw_small_dw") != hipSuccess)
-    return fail(E3X_ERR_HIP, "kernel e3x_uvw_small_dw missing from " + K->hsaco);
+  const std::string name = scalar_dw_fits(*P) ? "e3x_uvw_scalar_dw" : "e3x_uvw_small_dw";
+  if (hipModuleGetFunction(&K->fn_dw[dev], mod, name.c_str()) != hipSuccess)
+    return fail(E3X_ERR_HIP, "kernel " + name + " missing from " + K->hsaco);
   K->module[dev] = mod;
   return E3X_OK;
 }
@@ -2265,6 +2280,12 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
     if ((rc = prepare_valu_dw(P))) return rc;
     if ((rc = load_valu_dw_function(P, dev))) return rc;
     fn_dw = P->dw->fn_dw[dev];
+    if (scalar_dw_fits(*P)) {
+      long long rows_per_slice = std::max(128LL, ((long long)Z + 127) / 128);  // at most 128 workgroups (see the kernel), and a round of rows
+      void* args[] = {(void*)&x1, (void*)&x2, (void*)&grad_out, (void*)&grad_w, (void*)&n_rows, (void*)&rows_per_slice};
+      hipError_t err = hipModuleLaunchKernel(fn_dw, (unsigned)((Z + rows_per_slice - 1) / rows_per_slice), 1, 1, 1024, 1, 1, 0, st, args, nullptr);
+      return err == hipSuccess ? E3X_OK : fail(E3X_ERR_HIP, std::string("e3x_tp_backward_w_uvw: launch failed: ") + hipGetErrorString(err));
+    }
   } else {
     if ((rc = load_functions(P, dev))) return rc;
     fn_dw = P->subs[0]->fn_dw[dev];

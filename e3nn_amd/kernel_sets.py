@@ -86,6 +86,11 @@ def node_fctp():
     return o3.FullyConnectedTensorProduct("128x0e+64x1o+32x2e", "4x0e", "128x0e+64x1o+96x2e")
 
 
+def node_onto_scalars():
+    # scalars of several irreps, ragged against 32, onto a few scalars; the rest of the rows is not read
+    return o3.FullyConnectedTensorProduct("32x0e+16x1o+40x0e+8x0e", "4x0e", "2x0e")
+
+
 def node_many_species():
     # six species at 128 channels: 96 weight blocks per target, more than half of the LDS (one workgroup per CU)
     return o3.FullyConnectedTensorProduct("128x0e+64x1o", "6x0e", "64x0e+32x1o")
@@ -205,6 +210,7 @@ def all_tensor_products():
         ("outer_split", outer_split(), (torch.float32,)),
         ("node_block", node_block(), (torch.float32,)),
         ("node_many_species", node_many_species(), (torch.float32, torch.bfloat16)),
+        ("node_onto_scalars", node_onto_scalars(), (torch.float32,)),
         ("node_wide_out", node_wide_out(), (torch.float32, torch.bfloat16)),
         ("node_narrow", node_narrow(), (torch.float32, torch.bfloat16)),
         ("node_partial_tile", node_partial_tile(), (torch.float32, torch.bfloat16)),
@@ -222,7 +228,7 @@ def all_tensor_products():
 
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
 BACKWARD_CASES = ["cfg1", "cfg3_merged", "cfg3_builder", "cfg4_A", "cfg5", "mfma_small", "mfma_full_tiles", "mfma_wide_blocks", "outer_split", "node_fctp", "node_block",
-                  "node_wide_out", "node_narrow", "node_many_species", "node_partial_tile", "radial_layer", "odd_mul", "unaligned_mfma", "unaligned_offsets",
+                  "node_wide_out", "node_narrow", "node_many_species", "node_onto_scalars", "node_partial_tile", "radial_layer", "odd_mul", "unaligned_mfma", "unaligned_offsets",
                   "mixed_modes", "scalar_exact", "narrow_message", "ragged_wide_message"]  # fmt: skip
 
 

@@ -171,8 +171,8 @@ def test_uvw_weight_gradient_of_wide_blocks(Z):
         offset += n
 
 
-@pytest.mark.parametrize("maker", [ks.node_block, ks.node_narrow, ks.node_wide_out, ks.node_many_species, ks.radial_layer])
-@pytest.mark.parametrize("Z", [1, 16, 17, 2500])
+@pytest.mark.parametrize("maker", [ks.node_block, ks.node_narrow, ks.node_wide_out, ks.node_many_species, ks.radial_layer, ks.node_onto_scalars])
+@pytest.mark.parametrize("Z", [1, 16, 17, 63, 65, 2500])
 def test_uvw_weight_gradient_of_node_wise_layers(maker, Z):
     # stages of 16 rows and their remainders, one slice and several; tiles of both indices that are not full
     tp = maker()
