@@ -21,7 +21,7 @@ GOLDEN_GPU_CASES = [
 
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
 BACKWARD_CASES = _ks.BACKWARD_CASES + ["uvu_merged_cfg3_like_mul4", "uvu_builderA_cfg4_like_mul2", "uvu_shared_v2", "fctp_small_cfg5_like",
-                                       "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular"]  # fmt: skip
+                                       "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular", "zero_path_first", "zero_path_last"]  # fmt: skip
 BACKWARD_BF16_CASES = _ks.BACKWARD_BF16_CASES + ["uvu_shared_v2"]
 
 
@@ -78,9 +78,18 @@ def alpha_modules():
     return out
 
 
+def zero_path(first):
+    # scalars onto scalars, few weights, one of the two paths with a path weight of zero
+    return o3.TensorProduct("32x0e+32x0e", "4x0e", "2x0e", [(0, 0, 0, "uvw", True, 0.0 if first else 1.0), (1, 0, 0, "uvw", True, 1.0 if first else 0.0)])
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
+
+
+def edge_case_tensor_products():
+    return [("zero_path_first", zero_path(True), (torch.float32,)), ("zero_path_last", zero_path(False), (torch.float32,))]
 
 
 def golden_modules():
@@ -97,5 +106,5 @@ def golden_modules():
 
 def prebuild(verbose=True):
     """Every kernel the tests and the benchmark use: the package's list plus the fixtures' instruction sets."""
-    _ks.prebuild(verbose=verbose, extra_tensor_products=golden_tensor_products(), extra_modules=golden_modules() + alpha_modules(),
+    _ks.prebuild(verbose=verbose, extra_tensor_products=golden_tensor_products() + edge_case_tensor_products(), extra_modules=golden_modules() + alpha_modules(),
                  backward_cases=BACKWARD_CASES, backward_bf16_cases=BACKWARD_BF16_CASES)  # fmt: skip

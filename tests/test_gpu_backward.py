@@ -185,6 +185,22 @@ def test_uvw_weight_gradient_of_node_wise_layers(maker, Z):
     assert float((got - ref).norm() / ref.norm()) < 1e-6
 
 
+@pytest.mark.parametrize("first", [True, False])
+def test_uvw_weight_gradient_of_a_path_with_weight_zero(first):
+    # its weights have no part in the output, whatever the path beside it does: zeros exactly, also where rows are not finite
+    tp = ks.zero_path(first)
+    spec = oracle_spec(tp, [0.0, 1.0] if first else [1.0, 0.0])
+    Z = 300
+    x1, x2, g = seeded(Z, 64, seed=1), seeded(Z, 4, seed=2), seeded(Z, 2, seed=3)
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
+    dead, alive = (slice(0, 256), slice(256, 512)) if first else (slice(256, 512), slice(0, 256))
+    x1[7, 3 if first else 40] = float("inf")
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True).double().cpu()
+    assert not got[dead].any() and ref[alive].all()
+    assert float((got - ref)[alive].norm() / ref[alive].norm()) < 1e-6
+
+
 @pytest.mark.parametrize("maker", [ks.mfma_full_tiles, ks.node_block])
 @pytest.mark.parametrize("sizes", ["x1 against x2", "x1 against g", "x2 against g", "masked row", "largest number", "channels"])
 def test_uvw_weight_gradient_of_numbers_of_different_sizes(maker, sizes):
