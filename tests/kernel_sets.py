@@ -83,13 +83,23 @@ def zero_path(first):
     return o3.TensorProduct("32x0e+32x0e", "4x0e", "2x0e", [(0, 0, 0, "uvw", True, 0.0 if first else 1.0), (1, 0, 0, "uvw", True, 1.0 if first else 0.0)])
 
 
+def scalar_outputs():
+    # scalar outputs of l x l, l = 0, 1, 2, whose path coefficients are about 1, larger, and a hundred
+    weights = (1.0, 2.0, 1e4)
+    return o3.TensorProduct("64x0e+64x1o+64x2e", "64x0e+64x1o+64x2e", "64x0e+64x0e+64x0e",
+                            [(l, l, o, "uvw", True, pw) for o, pw in enumerate(weights) for l in range(3)], path_normalization="none")  # fmt: skip
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
 
 
 def edge_case_tensor_products():
-    return [("zero_path_first", zero_path(True), (torch.float32,)), ("zero_path_last", zero_path(False), (torch.float32,))]
+    return [
+        ("zero_path_first", zero_path(True), (torch.float32,)), ("zero_path_last", zero_path(False), (torch.float32,)),
+        ("scalar_outputs", scalar_outputs(), (torch.bfloat16,)),
+    ]  # fmt: skip
 
 
 def golden_modules():

@@ -646,6 +646,49 @@ def test_uvw_bf16_storage_scalar_outputs(Z):
         assert torch.equal(torch.ldexp(torch.ldexp(scaled, -e1), 40 - e2)[rows], out[rows].float())
 
 
+_SPECIAL_ROWS = 9
+
+
+def _special_rows(tp, x1, x2):
+    """The first rows of a batch for products of l x l: zero in either input, or in one irrep of it, and so small in one that
+    it takes a large other one to make an ordinary number."""
+    blocks1, blocks2 = tp.irreps_in1.slices(), tp.irreps_in2.slices()
+    x1[0] = 0
+    x2[1] = 0
+    x1[2] = x2[2] = 0
+    x1[3, blocks1[0]] = 0
+    x1[4, blocks1[1]] = x1[4, blocks1[2]] = 0
+    x1[5] *= 2.0**-120
+    x2[5] *= 2.0**110
+    x1[6] *= 2.0**110
+    x2[6] *= 2.0**-120
+    x1[7] *= 2.0**-60  # nothing of l = 0 in the first input, much of it in the second
+    x2[7] *= 2.0**-40
+    x1[7, blocks1[0]] = 0
+    x2[7, blocks2[0]] = 2.0**100
+    x1[8, 1:] = 0  # one number that is not zero
+    x1[8, 0] = 3.0
+
+
+@pytest.mark.parametrize("Z", [300, 21760, 21761])
+def test_uvw_bf16_storage_scalar_outputs_of_zero_rows_and_large_coefficients(Z):
+    # up to 21 760 rows (85 tiles of 256 rows, three channel tiles) in 2l + 1 passes per outer index, beyond with the operand
+    # formed from both inputs
+    tp = ks.scalar_outputs().to(DEV).to(torch.bfloat16)
+    with torch.no_grad():
+        tp.weight.copy_(seeded(tp.weight_numel, seed=5, scale=2.0**-6))
+    x1, x2 = seeded(Z, tp.irreps_in1.dim, seed=1).to(torch.bfloat16), seeded(Z, tp.irreps_in2.dim, seed=2).to(torch.bfloat16)
+    _special_rows(tp, x1, x2)
+    rows = torch.cat([torch.arange(_SPECIAL_ROWS + 3), torch.arange(Z - 3, Z)])
+    got = tp(x1.to(DEV), x2.to(DEV)).detach()[rows].double().cpu().numpy()
+    spec = oracle_spec(tp, [1.0] * 3 + [2.0] * 3 + [1e4] * 3, path_normalization="none")
+    want = _oracle_chunks(spec, x1[rows].float().numpy(), x2[rows].float().numpy(), tp.weight.detach().float().cpu().numpy())
+    assert not got[:3].any()
+    # a rounding of the output, 2^-9 of it; sums of 3 x 4096 terms in fp32 vanish beside the largest of the irrep
+    for sl in tp.irreps_out.slices():
+        size = np.abs(want[:, sl]).max(axis=1, keepdims=True)
+        assert (np.abs(got[:, sl] - want[:, sl]) <= 2.0**-8 * np.abs(want[:, sl]) + 1e-5 * size).all()
+
 
 @pytest.mark.parametrize("Z", [300, 16384 + 77])
 def test_uvw_bf16_storage_tiles_of_32_channels(Z):
