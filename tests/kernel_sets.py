@@ -90,6 +90,10 @@ def scalar_outputs():
                             [(l, l, o, "uvw", True, pw) for o, pw in enumerate(weights) for l in range(3)], path_normalization="none")  # fmt: skip
 
 
+def wide_scalar_output():
+    return o3.FullyConnectedTensorProduct("64x0e+64x1o+64x2e", "64x0e+64x1o+64x2e", "128x0e")
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
@@ -98,7 +102,7 @@ def golden_tensor_products():
 def edge_case_tensor_products():
     return [
         ("zero_path_first", zero_path(True), (torch.float32,)), ("zero_path_last", zero_path(False), (torch.float32,)),
-        ("scalar_outputs", scalar_outputs(), (torch.bfloat16,)),
+        ("scalar_outputs", scalar_outputs(), (torch.bfloat16,)), ("wide_scalar_output", wide_scalar_output(), (torch.float32, torch.bfloat16)),
     ]  # fmt: skip
 
 

@@ -690,6 +690,36 @@ def test_uvw_bf16_storage_scalar_outputs_of_zero_rows_and_large_coefficients(Z):
         assert (np.abs(got[:, sl] - want[:, sl]) <= 2.0**-8 * np.abs(want[:, sl]) + 1e-5 * size).all()
 
 
+def _infinite_rows(tp, x1, x2, w):
+    """``(rows, columns of the second input, signs)``: one infinity a row, in an irrep with l > 0 of the second input, and the
+    sign that it gives every scalar output: the sum over the first input's channels is taken before the infinity meets it."""
+    rows, signs = [], []
+    view = dict(zip(((t.i_in1, t.i_out) for t in tp.instructions), tp.weight_views(w)))
+    for row, (l, channel, component, sign) in enumerate([(1, 0, 0, 1), (1, 17, 2, -1), (2, 3, 4, 1), (2, 63, 0, -1)]):
+        column = tp.irreps_in2.slices()[l].start + channel * (2 * l + 1) + component
+        x2[row, column] = sign * float("inf")
+        mul = tp.irreps_in1[l].mul
+        x = x1[row, tp.irreps_in1.slices()[l]].reshape(mul, -1)[:, component].double()
+        cg = o3.wigner_3j(l, l, 0)[component, component, 0].double()
+        rows.append(row)
+        signs.append(torch.sign(sign * cg * (x @ view[l, 0][:, channel].double())))
+    return rows, torch.stack(signs)
+
+
+@pytest.mark.parametrize("Z", [300, 32_768, 32_769])
+def test_uvw_bf16_storage_scalar_outputs_of_infinite_rows(Z):
+    # an infinity stays one, whichever way the scalar output is formed (beyond 32 768 rows from both inputs), and keeps to its row
+    tp = ks.wide_scalar_output().to(DEV).to(torch.bfloat16)
+    x1, x2 = seeded(Z, tp.irreps_in1.dim, seed=1).to(torch.bfloat16), seeded(Z, tp.irreps_in2.dim, seed=2).to(torch.bfloat16)
+    ordinary = tp(x1.to(DEV), x2.to(DEV)).detach().float().cpu()
+    rows, signs = _infinite_rows(tp, x1, x2, tp.weight.detach().cpu())
+    got = tp(x1.to(DEV), x2.to(DEV)).detach().float().cpu()
+    assert torch.equal(got[rows], signs.float() * float("inf"))
+    rest = slice(len(rows), None)
+    # two roundings to bf16 of sums that agree to fp32
+    assert ((got[rest] - ordinary[rest]).abs() <= 2.0**-7 * ordinary[rest].abs() + 1e-5 * ordinary.abs().max()).all()
+
+
 @pytest.mark.parametrize("Z", [300, 16384 + 77])
 def test_uvw_bf16_storage_tiles_of_32_channels(Z):
     # irreps of 32 and 96 channels: their last workgroup tile holds 32 channels instead of 64 (both row tilings)
