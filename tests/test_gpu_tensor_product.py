@@ -720,6 +720,26 @@ def test_uvw_bf16_storage_scalar_outputs_of_infinite_rows(Z):
     assert ((got[rest] - ordinary[rest]).abs() <= 2.0**-7 * ordinary[rest].abs() + 1e-5 * ordinary.abs().max()).all()
 
 
+@pytest.mark.parametrize("Z", [4, 300, 16_384, 16_385])
+def test_uvw_on_pairs_of_fp16_operands_scalar_outputs_of_infinite_rows(Z):
+    # in fp32 an infinity meets channels of both signs, in parts (up to 16 384 rows of this product), whole and in the general
+    # kernel alike; the rows beside it keep every bit
+    from e3nn_amd import _lib
+
+    tp = ks.wide_scalar_output()
+    assert "fp16" in tp._plan(torch.float32).arithmetic
+    x1, x2, w = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(tp.weight_numel, seed=3)
+    ordinary = tp(x1.to(DEV), x2.to(DEV), w.to(DEV)).cpu()
+    rows, _ = _infinite_rows(tp, x1, x2, w)
+    a, b, w = x1.to(DEV), x2.to(DEV), w.to(DEV)
+    got = tp(a, b, w)
+    assert got[rows].isnan().all()
+    assert torch.equal(got[len(rows) :].cpu(), ordinary[len(rows) :])
+    general = torch.empty_like(got)
+    _lib.check(_lib.lib().e3x_tp_forward(tp._plan(torch.float32).handle, _lib.ptr(a), _lib.ptr(b), _lib.ptr(w), _lib.ptr(general), Z, _lib.stream_ptr(a.device)))
+    assert general[rows].isnan().all()
+
+
 @pytest.mark.parametrize("Z", [300, 16384 + 77])
 def test_uvw_bf16_storage_tiles_of_32_channels(Z):
     # irreps of 32 and 96 channels: their last workgroup tile holds 32 channels instead of 64 (both row tilings)
