@@ -624,7 +624,7 @@ def test_uvw_bf16_storage_small_multiplicities_in_256_row_workgroups():
 @pytest.mark.parametrize("Z", [13056, 13056 + 1, 13056 + 255])
 def test_uvw_bf16_storage_scalar_outputs(Z):
     # beyond 13 056 rows of this product (51 tiles of 256 rows, 5 channel tiles) the scalar output's operand is formed from
-    # both inputs, in two bf16 pieces; the last workgroup holds one row, or all but one.
+    # both inputs, in three bf16 pieces; the last workgroup holds one row, or all but one.
     tp, tpb, wq = _bf16_uvw(make=ks.mfma_wide_blocks)
     g = torch.Generator(device=DEV).manual_seed(5)
     xb = torch.randn(Z, tp.irreps_in1.dim, device=DEV, generator=g).to(torch.bfloat16)
@@ -632,7 +632,7 @@ def test_uvw_bf16_storage_scalar_outputs(Z):
     out = tpb(xb, yb)
     rows = torch.cat([torch.arange(0, 13056, 1999), torch.arange(13056 - 2, Z)[:40], torch.tensor([Z - 1])])
     ref = _oracle_chunks(oracle_spec(tp), xb[rows].float().cpu().numpy(), yb[rows].float().cpu().numpy(), wq)
-    # one rounding of the output, 2^-9 of it; the pieces' 2^-17 of a term and the sums in fp32 vanish beside it
+    # one rounding of the output, 2^-9 of it; the pieces hold 24 bits of a term, and the sums in fp32 vanish beside it
     for sl in tp.irreps_out.slices():
         err = out[rows][:, sl].detach().double().cpu().numpy() - ref[:, sl]
         assert np.linalg.norm(err) < 2e-3 * np.linalg.norm(ref[:, sl])
@@ -738,6 +738,41 @@ def test_uvw_on_pairs_of_fp16_operands_scalar_outputs_of_infinite_rows(Z):
     general = torch.empty_like(got)
     _lib.check(_lib.lib().e3x_tp_forward(tp._plan(torch.float32).handle, _lib.ptr(a), _lib.ptr(b), _lib.ptr(w), _lib.ptr(general), Z, _lib.stream_ptr(a.device)))
     assert general[rows].isnan().all()
+
+
+def test_uvw_bf16_storage_scalar_outputs_that_cancel():
+    # a row whose scalars, through large weights, take away all but 3e-6 of what vectors and l = 2 tensors add up to: what is
+    # left shows the sums before they are rounded to bf16
+    tp = ks.wide_scalar_output()
+    g = torch.Generator().manual_seed(1)
+    x1, x2, w = (torch.randn(n, generator=g).to(torch.bfloat16).double() for n in (tp.irreps_in1.dim, tp.irreps_in2.dim, tp.weight_numel))
+    x1[:64] = x2[:64] = 0
+    x1[0], x1[1], x2[0] = 1.0, 2.0**-8, 1.0
+    blocks = list(tp.weight_views(w))
+    blocks[0].zero_()
+
+    def product():
+        out = 0
+        for t, block in zip(tp.instructions, blocks):
+            a, b = (x[irreps.slices()[i]].reshape(64, -1) for x, irreps, i in ((x1, tp.irreps_in1, t.i_in1), (x2, tp.irreps_in2, t.i_in2)))
+            cg = t.path_weight * o3.wigner_3j(t.i_in1, t.i_in2, 0)[:, :, 0].double()
+            out = out + torch.einsum("ui,ij,vj,uvw->w", a, cg, b, block)
+        return out
+
+    size = product().norm()
+    c = tp.instructions[0].path_weight
+    blocks[0][0, 0] = (-product() / c).to(torch.bfloat16).double()
+    blocks[0][1, 0] = (-product() / c * 2.0**8).to(torch.bfloat16).double()
+    want = product()
+    assert 1e-6 * size < want.norm() < 1e-5 * size
+    tp = tp.to(DEV).to(torch.bfloat16)
+    with torch.no_grad():
+        tp.weight.copy_(w)
+    for Z in (300, 33_000):  # (beyond 32 768 rows the operand is formed from both inputs)
+        got = tp(*(x.to(torch.bfloat16).to(DEV).expand(Z, -1).contiguous() for x in (x1, x2))).detach()[[0, Z - 1]].double().cpu()
+        # 2 paths x 64 outer indices x 4 steps of 16 K indices x 3 pieces = 1536 sums in fp32, each cut to 2^-24 of a number no
+        # larger than the whole: a random walk of half of that
+        assert ((got - want).norm(dim=1) <= 1536**0.5 * 2.0**-25 * size).all()
 
 
 @pytest.mark.parametrize("Z", [300, 16384 + 77])
