@@ -2139,31 +2139,36 @@ extern "C" int e3x_tp_plan_prepare_backward_w(e3x_plan* P) {
 }
 
 // Batch slices of the wide weight gradient: a slice of a path with d passes has 1/d of the rows of one with a single pass,
-// so that all workgroups cost the same (unit_rows / d, whole stages of 16).  512 workgroups run at once, two per CU.  Taken is
-// the split, of 48 rows or more per workgroup, that ends first, counted in rounds of workgroups and rows (90 ns each): what
-// a workgroup does besides its rows costs it about as much as 32 of them, 96 where it adds to what others have stored, and
-// there the gradient is cleared first, at 50 000 numbers in the time of a row.
+// so that all workgroups cost the same (unit_rows / d, whole stages of 16; 48 rows or more).  512 workgroups run at once, two
+// per CU.  Taken is the split that ends first, counted in rounds of workgroups and rows (90 ns each): what a workgroup does
+// besides its rows costs it about as much as 32 of them, 96 where it adds to what others have stored, and there the gradient
+// is cleared first, at 50 000 numbers in the time of a row.
+// Where that leaves a sum many rows (few tiles, large batches), its rounding is most of the error: four workgroups for
+// every one that runs, of units of 240 rows at least.  64x0e x 64x0e -> 64x0e, 12 000 / 50 000 / 400 000 rows:
+// 89 / 201 / 1387 us, error against 64 bits 2.7e-7 / 3.8e-7 / 7.6e-7 of the 2-norm; 24 slices at most 69 / 239 / 1826 us and
+// 3.5e-7 / 9.0e-7 / 4.2e-6; uvw_mfma_dw.inc 94 / 270 / 1523 us and 3.1e-7 / 4.2e-7 / 1.5e-6.
 static int launch_dw_wide(e3x_plan* P, int dev, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, hipStream_t st) {
   auto rows_of = [](long long unit, int d) { return (unit / d + 15) / 16 * 16; };  // as in the kernel
   int unit_rows = 0, accumulate = 0;
-  long long jobs = 0;
+  long long jobs = 0, one_each = 0;  // (workgroups of one unit)
+  for (const auto& [d, tiles] : P->dw_wide_paths) one_each += d * tiles;
+  const long long n_min = std::min<long long>(Z / 128, 2048 / one_each);
+  const long long n_max = std::max(n_min, std::min<long long>(std::max(24LL, 2 * n_min), Z / 240 + 1));
   double best = 1e300;
-  for (int n = 0; n <= 24; ++n) {
+  for (long long n = n_min > 1 ? n_min : 0; n <= n_max; ++n) {
     // n = 0: every path whole (7 passes at most)
     const long long unit = n == 0 ? (Z + 15) / 16 * 16 * 7 : ((Z + n - 1) / n + 239) / 240 * 240;
     if (unit >= (1LL << 31)) continue;
-    long long n_jobs = 0, least = Z;
+    long long n_jobs = 0;
     double most = 0, work = 0;
     bool sums = false;
     for (const auto& [d, tiles] : P->dw_wide_paths) {
       const long long rows = rows_of(unit, d), slices = (Z + rows - 1) / rows;
       n_jobs += slices * tiles;
       sums = sums || slices > 1;
-      least = std::min(least, rows);
       most = std::max(most, (double)std::min<long long>(rows, Z) * d);
       work += (double)Z * d * tiles;
     }
-    if (least < std::min<long long>(Z, 48)) break;  // (more slices have fewer rows)
     const double cost = std::ceil(work / most / 512) * (most + (sums ? 96 : 32)) + (sums ? 2e-5 * (double)P->weight_numel : 0);
     if (cost < best) best = cost, jobs = n_jobs, unit_rows = (int)unit, accumulate = sums;
   }

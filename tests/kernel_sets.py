@@ -21,7 +21,8 @@ GOLDEN_GPU_CASES = [
 
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
 BACKWARD_CASES = _ks.BACKWARD_CASES + ["uvu_merged_cfg3_like_mul4", "uvu_builderA_cfg4_like_mul2", "uvu_shared_v2", "fctp_small_cfg5_like",
-                                       "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular", "zero_path_first", "zero_path_last"]  # fmt: skip
+                                       "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular", "zero_path_first", "zero_path_last",
+                                       "dense_one_path"]  # fmt: skip
 BACKWARD_BF16_CASES = _ks.BACKWARD_BF16_CASES + ["uvu_shared_v2"]
 
 
@@ -94,6 +95,10 @@ def wide_scalar_output():
     return o3.FullyConnectedTensorProduct("64x0e+64x1o+64x2e", "64x0e+64x1o+64x2e", "128x0e")
 
 
+def dense_one_path():
+    return o3.FullyConnectedTensorProduct("64x0e", "64x0e", "64x0e")
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
@@ -103,6 +108,7 @@ def edge_case_tensor_products():
     return [
         ("zero_path_first", zero_path(True), (torch.float32,)), ("zero_path_last", zero_path(False), (torch.float32,)),
         ("scalar_outputs", scalar_outputs(), (torch.bfloat16,)), ("wide_scalar_output", wide_scalar_output(), (torch.float32, torch.bfloat16)),
+        ("dense_one_path", dense_one_path(), (torch.float32,)),
     ]  # fmt: skip
 
 

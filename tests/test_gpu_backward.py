@@ -171,6 +171,22 @@ def test_uvw_weight_gradient_of_wide_blocks(Z):
         offset += n
 
 
+@pytest.mark.parametrize("Z", [129, 50_003, 400_003])
+def test_uvw_weight_gradient_of_few_wide_tiles(Z):
+    # 16 tiles for 512 workgroups: how many rows go into one sum decides the error
+    tp = ks.dense_one_path().to(DEV)
+    x1, x2, g = (seeded(Z, 64, seed=i).to(DEV) for i in (1, 2, 3))
+    got = tp._plan(torch.float32).backward_w_uvw(x1, x2, g, True).double()
+    ref = torch.zeros(64 * 64, 64, dtype=torch.float64, device=DEV)
+    for z in range(0, Z, 8192):
+        a, b, c = (x[z : z + 8192].double() for x in (x1, x2, g))
+        ref += (a[:, :, None] * b[:, None, :]).flatten(1).T @ c
+    ref = tp.instructions[0].path_weight * ref.flatten()
+    # at most 3200 rows a sum, six products for every 16 of them: a random walk of 1200 roundings of 2^-24 / sqrt(3), the same
+    # share of every slice
+    assert float((got - ref).norm() / ref.norm()) < 1200**0.5 * 2.0**-24 / 3**0.5
+
+
 @pytest.mark.parametrize("maker", [ks.node_block, ks.node_narrow, ks.node_wide_out, ks.node_many_species, ks.radial_layer, ks.node_onto_scalars])
 @pytest.mark.parametrize("Z", [1, 16, 17, 63, 65, 2500])
 def test_uvw_weight_gradient_of_node_wise_layers(maker, Z):
