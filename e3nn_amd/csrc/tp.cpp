@@ -1014,7 +1014,10 @@ int build_uvw_node_dw_source(e3x_plan& P, std::string* src) {
   }
   s << "struct NdPath { int x_off, U, d, o_off, V, g_off, W; long long wbase; float c; int MTW, TW, tiles; };\n";
   s << "constexpr int N_NDPATH = " << P.paths.size() << ";\nconstexpr NdPath ndpaths[N_NDPATH] = {\n" << ps.str() << "};\n";
-  s << "constexpr int MIN_WGS = 2;\n}  // namespace cfg\n";  // workgroups per CU the register budget is set for (three spill at l = 2)
+  s << "constexpr int MIN_WGS = 2;\n";  // workgroups per CU the register budget is set for (three spill at l = 2)
+  // sums as exact as the vector ALU's where the matrix-core kernel for whole tiles would not do (see the template)
+  const bool whole_tiles = uvw_mfma_eligible(P) && mfma_dw_fits(P);
+  s << "constexpr bool TWO_SUMS = " << (whole_tiles ? "false" : "true") << ";\n}  // namespace cfg\n";
   *src = s.str() + e3x::kTplCommon + e3x::kTplUvwNodeDw;
   return E3X_OK;
 }

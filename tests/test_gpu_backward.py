@@ -217,6 +217,22 @@ def test_uvw_weight_gradient_of_a_path_with_weight_zero(first):
     assert float((got - ref)[alive].norm() / ref[alive].norm()) < 1e-6
 
 
+@pytest.mark.parametrize("maker", [ks.node_ragged, ks.node_narrow, ks.node_partial_tile])
+def test_uvw_weight_gradient_of_ragged_node_wise_layers_is_as_exact_as_fp32(maker):
+    # multiplicities that are no multiples of 32, which the fp32 vector ALU sums with an error of 1.6e-7 at 1000 rows.  A slice
+    # of some 170 rows and components is 11 matrix steps, each cut by 2^-24 / sqrt(3) of a partial sum (two thirds of the
+    # whole on average), 0.8e-7; up to 30 slices are added with roundings of 2^-24 / sqrt(12), 0.6e-7; the product of the
+    # second input and g is rounded, 0.2e-7, and the operands' pieces end at 2^-25 of them, 0.4e-7: 1.1e-7 in all
+    tp = maker()
+    spec = oracle_spec(tp)
+    Z = 1000
+    x1, x2, g = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(Z, tp.irreps_out.dim, seed=3)
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True).double().cpu()
+    assert float((got - ref).norm() / ref.norm()) < 1.6e-7
+
+
 @pytest.mark.parametrize("maker", [ks.mfma_full_tiles, ks.node_block])
 @pytest.mark.parametrize("sizes", ["x1 against x2", "x1 against g", "x2 against g", "masked row", "largest number", "channels"])
 def test_uvw_weight_gradient_of_numbers_of_different_sizes(maker, sizes):
