@@ -49,6 +49,7 @@ _SIGNATURES = {
     "e3x_tp_plan_arithmetic": (ctypes.c_char_p, [c_void_p, c_int]),
     "e3x_tp_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "e3x_tp_forward_workspace_bytes": (c_size_t, [c_void_p]),
+    "e3x_tp_forward_workspace_bytes_for": (c_size_t, [c_void_p, c_int64]),
     "e3x_tp_forward_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_size_t, c_void_p]),
     "e3x_csr_workspace_bytes": (c_size_t, [c_int64, c_int64]),
     "e3x_csr_build": (c_int, [c_void_p, c_int, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -614,7 +614,8 @@ long long half_part_rows(const e3x_plan& P) { return P.half_parts ? 128LL * (256
 size_t half_parts_offset(const e3x_plan& P) {
   return ((size_t)P.weight_numel * 4 + kRowFlagWords * 4 + P.paths.size() * (kHalfMaxBlocks + 3) * 4 + 15) / 16 * 16;
 }
-size_t half_workspace_bytes(const e3x_plan& P) { return half_parts_offset(P) + (size_t)half_part_rows(P) * P.half_part_width * 4; }
+// ... the parts of a batch of Z rows: none where its workgroups walk all paths
+size_t half_parts_bytes(const e3x_plan& P, long long Z) { return Z < 0 || Z > half_part_rows(P) ? 0 : (size_t)Z * P.half_part_width * 4; }
 
 int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   // Output channels per workgroup.  fp32: 128 (two accumulator tiles per wave, 64 KB of LDS, two workgroups per CU at
@@ -1545,9 +1546,13 @@ static int zero_output(e3x_plan* P, void* out, int64_t rows, hipStream_t st) {
 
 static bool needs_packed_weights(const e3x_plan* P) { return P->family == "uvw_mfma" && P->dtype == E3X_BF16; }
 
-extern "C" size_t e3x_tp_forward_workspace_bytes(const e3x_plan* P) {
-  if (P && P->half) return half_workspace_bytes(*P);  // (taken when given; e3x_tp_forward runs without)
+extern "C" size_t e3x_tp_forward_workspace_bytes_for(const e3x_plan* P, int64_t Z) {
+  if (P && P->half) return half_parts_offset(*P) + half_parts_bytes(*P, Z);  // (taken when given; e3x_tp_forward runs without)
   return (P && needs_packed_weights(P)) ? (size_t)P->weight_numel * 2 : 0;
+}
+
+extern "C" size_t e3x_tp_forward_workspace_bytes(const e3x_plan* P) {
+  return e3x_tp_forward_workspace_bytes_for(P, P && P->half ? half_part_rows(*P) : 0);
 }
 
 extern "C" int e3x_tp_forward(e3x_plan* P, const void* x1, const void* x2, const void* w, void* out, int64_t Z,
@@ -1572,7 +1577,7 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
   if ((rc = load_functions(P, dev))) return rc;
   long long n_rows = Z;
   unsigned* row_flags = nullptr;
-  if (P->half && workspace && workspace_bytes >= half_workspace_bytes(*P) &&
+  if (P->half && workspace && workspace_bytes >= half_parts_offset(*P) &&
       !(((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)w | (uintptr_t)workspace) & 15)) {
     SubKernel* K = P->half.get();
     const unsigned n_path = (unsigned)P->paths.size();
@@ -1587,7 +1592,8 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
     }
     const long long blocks = (Z + 127) / 128;
     if (blocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_forward: batch too large for one launch");
-    float* parts = P->half_parts && Z <= half_part_rows(*P) ? (float*)((char*)workspace + half_parts_offset(*P)) : nullptr;
+    const size_t part_bytes = half_parts_bytes(*P, Z);  // (a workspace without room for them: whole)
+    float* parts = part_bytes && workspace_bytes >= half_parts_offset(*P) + part_bytes ? (float*)((char*)workspace + half_parts_offset(*P)) : nullptr;
     int n_scalar = parts ? P->half_parts : P->half_scalars;
     void* margs[] = {(void*)&w, (void*)&w_max, (void*)&path_w, (void*)&row_flags, (void*)&n_words};
     void* pargs[] = {(void*)&w, (void*)&w_max, (void*)&workspace, (void*)&path_w};

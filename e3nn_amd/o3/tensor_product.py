@@ -61,6 +61,8 @@ def _num_elements(mode, m1, m2):
 class _Plan:
     """Owner of one ``e3x_plan`` handle: a fused kernel specialised to one instruction set."""
 
+    _in_parts = False  # whether the scratch of a forward call depends on the batch
+
     def __init__(self, irreps_in1, irreps_in2, irreps_out, instructions, shared_weights: bool, dtype: torch.dtype):
         """``instructions``: tuples ``(i_in1, i_in2, i_out, mode, has_weight, path_weight)``, path weights final."""
         L = _lib.lib()
@@ -82,6 +84,7 @@ class _Plan:
         self.weight_numel, self.family, self.key = wn.value, fam.value.decode(), key.value.decode()
         self.out_dim, self.in2_dim = irreps_out.dim, irreps_in2.dim
         self.arithmetic = L.e3x_tp_plan_arithmetic(handle, 0).decode()  # which instruction forms the products
+        self._in_parts = L.e3x_tp_forward_workspace_bytes(handle) > L.e3x_tp_forward_workspace_bytes_for(handle, -1)
         self._fused_grad_w = None  # whether the plan has the message-step backward kernel; asked on first use
         self._by_destination = None  # ... and, on the forward plan, the one grouped by destination
 
@@ -96,23 +99,29 @@ class _Plan:
     def forward(self, x1, x2, w):
         Z = x1.shape[0]
         out = torch.empty(Z, self.out_dim, dtype=x1.dtype, device=x1.device)
-        ws_bytes = _lib.lib().e3x_tp_forward_workspace_bytes(self.handle)
-        ws = None
-        if ws_bytes:
+        L = _lib.lib()
+        if self._in_parts:
+            # with room for the parts of a small batch, or, where memory does not have it, for the weights alone
+            sizes = [L.e3x_tp_forward_workspace_bytes_for(self.handle, rows) for rows in (Z, -1)]
+        else:
+            sizes = [L.e3x_tp_forward_workspace_bytes(self.handle)]
+        ws, ws_bytes = None, 0
+        if sizes[0]:
             # scratch for the weights repacked for the matrix cores; the kernel reads rows with 16-byte loads
-            try:
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x1.device)
-            except torch.OutOfMemoryError:
-                if x1.dtype != torch.float32:
-                    raise
-                ws_bytes = 0  # fp32: the general kernel needs none
+            for n in sizes:
+                try:
+                    ws, ws_bytes = torch.empty(n, dtype=torch.uint8, device=x1.device), n
+                    break
+                except torch.OutOfMemoryError:
+                    if x1.dtype != torch.float32:
+                        raise  # (fp32: the general kernel needs none)
             x1, x2 = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2))
         if self.family == "uvw_node":
             # rows and weights are read with 16-byte loads
             x1, w = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, w))
         with _lib.on_device(x1.device):
             _lib.check(
-                _lib.lib().e3x_tp_forward_ws(
+                L.e3x_tp_forward_ws(
                     self.handle, _lib.ptr(x1), _lib.ptr(x2), _lib.ptr(w), _lib.ptr(out), Z,
                     _lib.ptr(ws) if ws is not None else None, ws_bytes, _lib.stream_ptr(x1.device),
                 )

@@ -147,8 +147,13 @@ int e3x_tp_forward(e3x_plan* plan, const void* x1, const void* x2, const void* w
  * powers of two (the first or second input's row per irrep component, the weights per path), which is faster than the six
  * bf16 products of e3x_tp_forward and as accurate on numbers of similar size.  Rows whose numbers differ so much in size
  * that the pieces may not hold what a sum depends on (beside the weights of the path; decided for every row by itself)
- * are formed by the kernel of e3x_tp_forward.  Every other plan needs no workspace and e3x_tp_forward is enough. */
+ * are formed by the kernel of e3x_tp_forward.  Every other plan needs no workspace and e3x_tp_forward is enough.
+ * e3x_tp_forward_workspace_bytes is enough for every batch, e3x_tp_forward_workspace_bytes_for for batches of Z rows: fp32
+ * plans with scalar outputs of l x l form these in parts where the chip would not be full, and only such a batch needs room
+ * for its parts.  Z < 0: the least that the call takes, without room for parts; a small batch runs the longer for it and has
+ * the same results to the last bit. */
 size_t e3x_tp_forward_workspace_bytes(const e3x_plan* plan);
+size_t e3x_tp_forward_workspace_bytes_for(const e3x_plan* plan, int64_t Z);
 int e3x_tp_forward_ws(e3x_plan* plan, const void* x1, const void* x2, const void* w, void* out, int64_t Z,
                       void* workspace, size_t workspace_bytes, void* stream);
 

@@ -492,6 +492,14 @@ def test_uvw_on_pairs_of_fp16_operands_scalar_outputs(Z):
         err = np.linalg.norm(got[rows][:, sl].double().numpy() - want[:, sl], axis=1)
         assert (err <= 1.5e-6 * np.linalg.norm(want[:, sl], axis=1)).all(), [kinds[int(which[r])] for r in rows[err > 1.5e-6 * np.linalg.norm(want[:, sl], axis=1)]]
     assert torch.equal(tp(x1[rows].to(DEV), x2[rows].to(DEV), w.to(DEV)).cpu(), got[rows])
+    # scratch without room for the parts: whole, to the same bits
+    from e3nn_amd import _lib
+
+    L, handle = _lib.lib(), tp._plan(torch.float32).handle
+    a, b, c = x1.to(DEV), x2.to(DEV), w.to(DEV)
+    out, ws = torch.empty(Z, tp.irreps_out.dim, device=DEV), torch.empty(L.e3x_tp_forward_workspace_bytes_for(handle, -1), dtype=torch.uint8, device=DEV)
+    _lib.check(L.e3x_tp_forward_ws(handle, _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), _lib.ptr(out), Z, _lib.ptr(ws), ws.numel(), _lib.stream_ptr(a.device)))
+    assert torch.equal(out.cpu(), got)
 
 
 @pytest.mark.parametrize("Z", [1, 129, 200])

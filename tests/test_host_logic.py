@@ -535,6 +535,51 @@ def test_dense_product_without_memory_for_its_packed_weights(monkeypatch, dtype)
             plan.forward(*args)
 
 
+@pytest.mark.parametrize("free,taken", [(1 << 30, 1100), (1099, 800), (799, 0)])
+def test_dense_product_in_parts_takes_the_scratch_that_memory_has(monkeypatch, free, taken):
+    # room for the parts of its three rows, else for the packed weights alone, else the kernel that needs none
+    calls = []
+
+    class Library:
+        def e3x_tp_forward_workspace_bytes_for(self, handle, rows):
+            return 800 + 100 * max(rows, 0)
+
+        def e3x_tp_forward_ws(self, handle, x1, x2, w, out, rows, workspace, workspace_bytes, stream):
+            calls.append((workspace is not None, workspace_bytes))
+            return 0
+
+    from e3nn_amd.o3.tensor_product import _Plan
+
+    plan = object.__new__(_Plan)
+    plan.handle, plan.family, plan.out_dim, plan._in_parts = None, "uvw_mfma", 4, True
+    empty = torch.empty
+
+    def limited(*size, **kw):
+        if kw.get("dtype") == torch.uint8 and size[0] > free:
+            raise torch.OutOfMemoryError("no memory left")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(_lib, "lib", Library)
+    monkeypatch.setattr(_lib, "stream_ptr", lambda device: None)
+    monkeypatch.setattr(torch, "empty", limited)
+    plan.forward(torch.zeros(3, 8), torch.zeros(3, 8), torch.zeros(16))
+    assert calls == [(taken > 0, taken)]
+
+
+def test_dense_product_asks_for_the_scratch_of_its_batch():
+    # 768 numbers of parts a row: K = 128 and 64 in chunks of 32, six of the 128 channels of the only output
+    plan = o3.FullyConnectedTensorProduct("128x0e+64x1o", "128x0e+64x1o", "128x0e")._plan(torch.float32)
+    L = _lib.lib()
+    least, most = (L.e3x_tp_forward_workspace_bytes_for(plan.handle, -1), L.e3x_tp_forward_workspace_bytes(plan.handle))
+    assert "fp16" in plan.arithmetic and plan._in_parts and least >= plan.weight_numel * 4
+    assert [L.e3x_tp_forward_workspace_bytes_for(plan.handle, rows) - least for rows in (0, 1, 100, 1 << 20)] == [0, 3072, 307200, 0]
+    rows = (most - least) // 3072
+    assert L.e3x_tp_forward_workspace_bytes_for(plan.handle, rows) == most and L.e3x_tp_forward_workspace_bytes_for(plan.handle, rows + 1) == least
+    # no scalar output of l x l, l > 0: nothing beside the packed weights, whatever the batch
+    plan = o3.FullyConnectedTensorProduct("64x0e+64x1o", "64x0e", "64x0e+64x1o")._plan(torch.float32)
+    assert "fp16" in plan.arithmetic and not plan._in_parts
+
+
 def test_message_backward_whose_kernel_cannot_be_had(tmp_path, monkeypatch):
     # a cache made without the kernel grouped by destination, and no compiler: the caller is sent to the transposed plan
     monkeypatch.setenv("E3X_KERNEL_CACHE", str(tmp_path))
