@@ -59,8 +59,9 @@ def nn_golden():
 
 
 # (features, node attributes) of blocks whose mixing coefficient is read from messages of 4224 numbers, too long for the
-# vector-ALU kernel to stage; of an ordinary width; with a handful of weights; and that are not whole 16-byte pieces
-ALPHA_CASES = [("384x0e+384x1o", "1x0e"), ("16x0e+16x1o", "4x0e"), ("8x0e+8x1o", "1x0e"), ("8x0e+7x1o", "9x0e")]
+# vector-ALU kernel to stage; of an ordinary width; with a handful of weights; and that are not whole 16-byte pieces, with
+# scalars that are and scalars that are not
+ALPHA_CASES = [("384x0e+384x1o", "1x0e"), ("16x0e+16x1o", "4x0e"), ("8x0e+8x1o", "1x0e"), ("16x0e+16x1o+1x1e", "4x0e"), ("8x0e+7x1o", "9x0e")]
 
 
 def alpha_block(features, attr):

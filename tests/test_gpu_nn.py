@@ -537,11 +537,36 @@ def test_mixing_of_a_convolution_block(N, C, wanted):
         assert_close(got, want[name].numpy(), atol=1e-5 if name != "alpha" else 1e-6 * C**0.5 + 1e-5, rtol=1e-6, what=name)
 
 
+@pytest.mark.parametrize("features,attr", ks.ALPHA_CASES[:-1])  # (the last has no scalars to read apart)
+def test_lin2_and_alpha_against_64_bits(features, attr):
+    # both products of the messages and all of their gradients: rows of 4224 numbers, a single attribute, ragged multiplicities
+    # and the copy of the scalars where rows are no whole pieces of 16 bytes
+    from e3nn_amd.nn.convolution import _Lin2Alpha
+    from oracle.torch_cpu import tp_forward_torch
+    from tests.helpers import oracle_spec
+
+    conv = ks.alpha_block(features, attr).to(DEV)
+    head, N = conv._alpha_head, 40
+    x, a, wa = seeded(N, conv.lin2.irreps_in1.dim, seed=1), seeded(N, conv.irreps_node_attr.dim, seed=2), seeded(conv.alpha.weight_numel, seed=3)
+    w2, g2, ga = seeded(conv.lin2.weight_numel, seed=4), seeded(N, conv.irreps_node_output.dim, seed=5), seeded(N, 1, seed=6)
+    leaves = [t.to(DEV).requires_grad_() for t in (x, w2, wa)]
+    out = _Lin2Alpha.apply(leaves[0], a.to(DEV), leaves[1], leaves[2], conv.lin2, conv.alpha, head)
+    got = [*out, *torch.autograd.grad(out, leaves, (g2.to(DEV), ga.to(DEV)))]
+    leaves = [t.double().requires_grad_() for t in (x, w2, wa)]
+    ref = tuple(tp_forward_torch(oracle_spec(tp), leaves[0], a.double(), w) for tp, w in ((conv.lin2, leaves[1]), (conv.alpha, leaves[2])))
+    ref = [*ref, *torch.autograd.grad(ref, leaves, (g2.double(), ga.double()))]
+    for what, p, q in zip(("lin2", "alpha", "d/dx", "d/dw lin2", "d/dw alpha"), got, ref):
+        # sums of at most 384 x 4 x 5 products in fp32: a random walk of some hundred roundings of 6e-8 / sqrt(3)
+        assert float((p.detach().double().cpu() - q.detach()).norm() / q.detach().norm()) < 1e-6, what
+
+
 @pytest.mark.parametrize("features,attr", ks.ALPHA_CASES)
 def test_alpha_of_a_convolution_block_on_wide_and_ragged_messages(features, attr):
-    """The mixing coefficient reads the leading scalars of the messages in place where a kernel can, else from a copy: its
-    weight gradient against the product restricted to the scalars, which is what a graph of the backward pass takes."""
+    """The mixing coefficient reads the leading scalars of the messages in place where a kernel can, else from a copy: the
+    gradients against those of the product restricted to the scalars, which is what a graph of the backward pass takes."""
     conv = ks.alpha_block(features, attr).to(DEV)
+    with torch.no_grad():
+        conv.alpha.weight.normal_()  # (zeros at first: alpha and its share of d/dx would be zero whatever is read)
     N, E = 40, 150
     src, dst = (torch.randint(0, N, (E,), generator=torch.Generator().manual_seed(i)).to(DEV) for i in (1, 2))
     edge_attr = o3.spherical_harmonics([0, 1, 2], seeded(E, 3, seed=3).to(DEV), True, "component")
