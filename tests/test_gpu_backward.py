@@ -201,6 +201,19 @@ def test_uvw_weight_gradient_of_node_wise_layers(maker, Z):
     assert float((got - ref).norm() / ref.norm()) < 1e-6
 
 
+@pytest.mark.parametrize("Z", [16_384, 16_385, 50_003])
+def test_uvw_weight_gradient_onto_scalars_of_many_rows(Z):
+    # beyond 128 rows a workgroup: several trips of 128 rows in each, the last one ragged (50 003 rows: 391 a workgroup)
+    tp = ks.node_onto_scalars()
+    x1, x2, g = seeded(Z, tp.irreps_in1.dim, seed=1), seeded(Z, tp.irreps_in2.dim, seed=2), seeded(Z, tp.irreps_out.dim, seed=3)
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(oracle_spec(tp), x1.double(), x2.double(), w), (w,), g.double())
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True).double().cpu()
+    # a lane adds up at most 16 rows, 32 lanes and 128 workgroups one after the other: a random walk of 176 roundings of
+    # 2^-24 / sqrt(3) of sums that are two thirds of the whole on average
+    assert float((got - ref).norm() / ref.norm()) < 176**0.5 * 2.0**-24 / 3**0.5
+
+
 @pytest.mark.parametrize("first", [True, False])
 def test_uvw_weight_gradient_of_a_path_with_weight_zero(first):
     # its weights have no part in the output, whatever the path beside it does: zeros exactly, also where rows are not finite
