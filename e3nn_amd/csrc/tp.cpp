@@ -953,6 +953,15 @@ bool dw_wide_fits(const e3x_plan& P) {
   return true;
 }
 
+// workgroups of one unit of rows (see launch_dw_wide)
+long long dw_wide_unit_jobs(const e3x_plan& P) {
+  long long n = 0;
+  for (const auto& [d, tiles] : P.dw_wide_paths) n += d * tiles;
+  return n;
+}
+// ... so few that the batch is cut beyond what fills the chip: its slices alternate in sign
+bool dw_wide_few_tiles(const e3x_plan& P) { return 2048 / dw_wide_unit_jobs(P) > 1; }
+
 int build_uvw_dw_wide_source(e3x_plan& P, std::string* src) {
   std::ostringstream s, nzs, ps;
   emit_header(s, P);
@@ -988,7 +997,7 @@ int build_uvw_dw_wide_source(e3x_plan& P, std::string* src) {
        << p.woff << ", " << stride[m] << ", " << stride[n] << ", " << stride[r] << ", " << tiles << ", " << nz_beg << ", " << n_nz << "},\n";
     P.dw_wide_paths.push_back({d[n], tiles});
   }
-  s << "constexpr int DIMS[3] = {IN1_DIM, IN2_DIM, OUT_DIM};\n";
+  s << "constexpr int DIMS[3] = {IN1_DIM, IN2_DIM, OUT_DIM};\nconstexpr bool ALTERNATE = " << (dw_wide_few_tiles(P) ? "true" : "false") << ";\n";
   s << "struct Nz { int s, r, k; float c; };\nconstexpr int N_NZ = " << n_nz << ";\nconstexpr Nz nz[N_NZ] = {\n" << nzs.str() << "};\n";
   s << "struct WPath { int m_src, m_off, dM, M, n_src, n_off, dN, N, r_src, r_off, dR, O; bool n_is_w; "
        "long long wbase, m_stride, n_stride, o_stride; int tiles, nz_beg, nz_end; };\n";
@@ -2153,15 +2162,15 @@ extern "C" int e3x_tp_plan_prepare_backward_w(e3x_plan* P) {
 // besides its rows costs it about as much as 32 of them, 96 where it adds to what others have stored, and there the gradient
 // is cleared first, at 50 000 numbers in the time of a row.
 // Where that leaves a sum many rows (few tiles, large batches), its rounding is most of the error: four workgroups for
-// every one that runs, of units of 240 rows at least.  64x0e x 64x0e -> 64x0e, 12 000 / 50 000 / 400 000 rows:
-// 89 / 201 / 1387 us, error against 64 bits 2.7e-7 / 3.8e-7 / 7.6e-7 of the 2-norm; 24 slices at most 69 / 239 / 1826 us and
-// 3.5e-7 / 9.0e-7 / 4.2e-6; uvw_mfma_dw.inc 94 / 270 / 1523 us and 3.1e-7 / 4.2e-7 / 1.5e-6.
+// every one that runs, of units of 240 rows at least, and every other slice works on the negative of its operand.
+// 64x0e x 64x0e -> 64x0e, 12 000 / 50 000 / 400 000 rows: 89 / 201 / 1387 us, error against 64 bits 2.7e-7 / 3.8e-7 / 7.6e-7 of the
+// 2-norm; 24 slices at most 69 / 239 / 1826 us and 3.5e-7 / 9.0e-7 / 4.2e-6; uvw_mfma_dw.inc 94 / 270 / 1523 us and 3.1e-7 /
+// 4.2e-7 / 1.5e-6.
 static int launch_dw_wide(e3x_plan* P, int dev, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, hipStream_t st) {
   auto rows_of = [](long long unit, int d) { return (unit / d + 15) / 16 * 16; };  // as in the kernel
   int unit_rows = 0, accumulate = 0;
-  long long jobs = 0, one_each = 0;  // (workgroups of one unit)
-  for (const auto& [d, tiles] : P->dw_wide_paths) one_each += d * tiles;
-  const long long n_min = std::min<long long>(Z / 128, 2048 / one_each);
+  long long jobs = 0;
+  const long long n_min = std::min<long long>(Z / 128, 2048 / dw_wide_unit_jobs(*P));
   const long long n_max = std::max(n_min, std::min<long long>(std::max(24LL, 2 * n_min), Z / 240 + 1));
   double best = 1e300;
   for (long long n = n_min > 1 ? n_min : 0; n <= n_max; ++n) {
