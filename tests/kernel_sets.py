@@ -22,7 +22,7 @@ GOLDEN_GPU_CASES = [
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
 BACKWARD_CASES = _ks.BACKWARD_CASES + ["uvu_merged_cfg3_like_mul4", "uvu_builderA_cfg4_like_mul2", "uvu_shared_v2", "fctp_small_cfg5_like",
                                        "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular", "zero_path_first", "zero_path_last",
-                                       "dense_one_path", "node_ragged"]  # fmt: skip
+                                       "dense_one_path", "node_ragged", "node_long_row"]  # fmt: skip
 BACKWARD_BF16_CASES = _ks.BACKWARD_BF16_CASES + ["uvu_shared_v2"]
 
 
@@ -104,6 +104,11 @@ def node_ragged():
     return o3.FullyConnectedTensorProduct("16x0e+16x1o+16x2e", "4x0e", "16x0e+16x1o+16x2e")
 
 
+def node_long_row():
+    # scalars onto one scalar, the longest row whose gradient the kernel for few scalars takes
+    return o3.FullyConnectedTensorProduct("960x0e", "1x0e", "1x0e")
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
@@ -114,6 +119,7 @@ def edge_case_tensor_products():
         ("zero_path_first", zero_path(True), (torch.float32,)), ("zero_path_last", zero_path(False), (torch.float32,)),
         ("scalar_outputs", scalar_outputs(), (torch.bfloat16,)), ("wide_scalar_output", wide_scalar_output(), (torch.float32, torch.bfloat16)),
         ("dense_one_path", dense_one_path(), (torch.float32,)), ("node_ragged", node_ragged(), (torch.float32,)),
+        ("node_long_row", node_long_row(), (torch.float32,)),
     ]  # fmt: skip
 
 

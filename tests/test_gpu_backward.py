@@ -214,6 +214,17 @@ def test_uvw_weight_gradient_onto_scalars_of_many_rows(Z):
     assert float((got - ref).norm() / ref.norm()) < 176**0.5 * 2.0**-24 / 3**0.5
 
 
+@pytest.mark.parametrize("Z", [1, 31, 65, 129, 16_385])
+def test_uvw_weight_gradient_of_long_rows_onto_a_scalar(Z):
+    # two rows of 960 numbers in flight a half-wave, trips of 64 rows a workgroup
+    tp = ks.node_long_row()
+    x1, x2, g = (seeded(Z, n, seed=i) for i, n in ((1, 960), (2, 1), (3, 1)))
+    ref = tp.instructions[0].path_weight * ((x2 * g).double().T @ x1.double()).flatten()
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True).double().cpu()
+    # the bound of the sets above (fewer rows a lane here), and two roundings of every product
+    assert float((got - ref).norm() / ref.norm()) < (176**0.5 + 2) * 2.0**-24 / 3**0.5
+
+
 @pytest.mark.parametrize("first", [True, False])
 def test_uvw_weight_gradient_of_a_path_with_weight_zero(first):
     # its weights have no part in the output, whatever the path beside it does: zeros exactly, also where rows are not finite
