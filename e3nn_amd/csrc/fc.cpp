@@ -194,7 +194,7 @@ extern "C" int e3x_fc_plan_create_fused(const int32_t* hs, int32_t n_hs, int32_t
   s << "constexpr int RS = " << rs << ", WAVES = " << waves << ";\n}  // namespace cfg\n";
   if (const char* v = std::getenv("E3X_FC_STREAM")) s << "#define E3X_FC_STREAM " << std::atoi(v) << "\n";
   if (const char* v = std::getenv("E3X_FC_STREAM_DIST")) s << "#define E3X_FC_STREAM_DIST " << std::max(1, std::atoi(v)) << "\n";
-  const std::string src = s.str() + e3x::kTplCommon + e3x::kTplFcMfma;
+  const std::string src = s.str() + e3x::kTplCommon + e3x::kTplPieces + e3x::kTplFcMfma;
   int rc = e3x::get_code_object("fc_mfma", src, &P->key, &P->hsaco);
   if (rc) return rc;
   *out = P.release();
@@ -229,7 +229,7 @@ extern "C" int e3x_fc_plan_prepare_backward_w(e3x_fc_plan* P) {
   s << "constexpr int H_IN = " << P->hs[0] << ", H_OUT = " << P->hs[1] << ", NTW = " << ntw << ";\nconstexpr bool BY_ROWS = " << (by_rows ? "true" : "false") << ";\n";
   s << "constexpr float SCALE = " << fstr(P->scale0) << ";\n";
   s << "constexpr int IN_ACT = " << P->input_act << ";\nconstexpr float IN_CST = " << fstr(P->input_cst) << ";\n}  // namespace cfg\n";
-  const std::string src = s.str() + e3x::kTplCommon + e3x::kTplFcDw;
+  const std::string src = s.str() + e3x::kTplCommon + e3x::kTplPieces + e3x::kTplFcDw;
   return e3x::get_code_object("fc_dw", src, &P->dw_key, &P->dw_hsaco);
 }
 

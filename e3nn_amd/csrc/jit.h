@@ -6,6 +6,7 @@ namespace e3x {
 
 // Device template sources, embedded at library build time from templates/*.inc.
 extern const char* const kTplCommon;
+extern const char* const kTplPieces;
 extern const char* const kTplUvu;
 extern const char* const kTplUvuFc;
 extern const char* const kTplUvuRowgrad;

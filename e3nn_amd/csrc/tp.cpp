@@ -738,7 +738,10 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   }
   s << "}  // namespace cfg\n";
   (half ? P.half_targets : P.n_targets) = n_target;
-  *src = s.str() + e3x::kTplCommon + (half ? e3x::kTplUvwMfmaHalf : P.dtype == E3X_BF16 ? e3x::kTplUvwMfmaBf16 : e3x::kTplUvwMfma);
+  *src = s.str() + e3x::kTplCommon;
+  if (half) *src += e3x::kTplUvwMfmaHalf;
+  else if (P.dtype == E3X_BF16) *src += e3x::kTplUvwMfmaBf16;
+  else *src += std::string(e3x::kTplPieces) + e3x::kTplUvwMfma;
   return E3X_OK;
 }
 
@@ -838,7 +841,7 @@ int build_uvw_node_source(e3x_plan& P, std::string* src) {
   // workgroups per CU the register budget is set for: three when their weights fit (160 KB of LDS per CU)
   s << "constexpr int MIN_WGS = " << env_int("E3X_NODE_WGS", max_blocks <= 48 && max_d <= 5 ? 3 : 2) << ";\n";
   s << "}  // namespace cfg\n";
-  *src = s.str() + e3x::kTplCommon + e3x::kTplUvwNode;
+  *src = s.str() + e3x::kTplCommon + e3x::kTplPieces + e3x::kTplUvwNode;
   return E3X_OK;
 }
 
@@ -937,7 +940,7 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
   s << "}  // namespace cfg\n";
   P.dw_tiles = tiles;
   P.dw_paths = n_path;
-  *src = s.str() + e3x::kTplCommon + e3x::kTplUvwMfmaDw;
+  *src = s.str() + e3x::kTplCommon + e3x::kTplPieces + e3x::kTplUvwMfmaDw;
   return E3X_OK;
 }
 
@@ -1002,7 +1005,7 @@ int build_uvw_dw_wide_source(e3x_plan& P, std::string* src) {
   s << "struct WPath { int m_src, m_off, dM, M, n_src, n_off, dN, N, r_src, r_off, dR, O; bool n_is_w; "
        "long long wbase, m_stride, n_stride, o_stride; int tiles, nz_beg, nz_end; };\n";
   s << "constexpr int N_WPATH = " << P.paths.size() << ";\nconstexpr WPath wpaths[N_WPATH] = {\n" << ps.str() << "};\n}  // namespace cfg\n";
-  *src = s.str() + e3x::kTplCommon + e3x::kTplUvwDwWide;
+  *src = s.str() + e3x::kTplCommon + e3x::kTplPieces + e3x::kTplUvwDwWide;
   return E3X_OK;
 }
 
@@ -1028,7 +1031,7 @@ int build_uvw_node_dw_source(e3x_plan& P, std::string* src) {
   // sums as exact as the vector ALU's where the matrix-core kernel for whole tiles would not do (see the template)
   const bool whole_tiles = uvw_mfma_eligible(P) && mfma_dw_fits(P);
   s << "constexpr bool TWO_SUMS = " << (whole_tiles ? "false" : "true") << ";\n}  // namespace cfg\n";
-  *src = s.str() + e3x::kTplCommon + e3x::kTplUvwNodeDw;
+  *src = s.str() + e3x::kTplCommon + e3x::kTplPieces + e3x::kTplUvwNodeDw;
   return E3X_OK;
 }
 
