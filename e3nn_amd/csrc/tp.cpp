@@ -496,15 +496,21 @@ int build_uvw_small_source(e3x_plan& P, SubKernel& K, std::string* src, bool gra
     max_mul = std::max(max_mul, P.out[p.out].mul);
     all_uvw = all_uvw && p.mode == E3X_MODE_UVW;
   }
+  // few outputs per row and many indices of the second input (a gradient of edge attributes): lanes <-> these (E3X_UVW_REDUCE)
+  int max_v = 1, min_v = 1 << 30;
+  for (const auto& p : P.paths) max_v = std::max(max_v, P.in2[p.in2].mul), min_v = std::min(min_v, P.in2[p.in2].mul);
+  const bool reduce = !gradient_only && all_uvw && !P.paths.empty() && P.out_dim <= 32 && min_v >= 8 * max_mul;
+  if (reduce) max_mul = max_v;
   K.lanes = max_mul > 32 ? 64 : pow2_at_least(max_mul, 16);
   // long input rows: fewer rows per wavefront so that the staged rows fit in LDS (lanes beyond the output
   // multiplicity idle)
   while (K.lanes < 64 && (P.in1_dim + P.in2_dim) * 16 * (64 / K.lanes) > 65536) K.lanes *= 2;
-  K.chunks = (max_mul + K.lanes - 1) / K.lanes;
+  K.chunks = reduce ? 1 : (max_mul + K.lanes - 1) / K.lanes;
   if (!gradient_only && (P.in1_dim + P.in2_dim) * 16 * (64 / K.lanes) > 65536)
     return fail(E3X_ERR_INVALID, "uvw kernel: input rows too long for the LDS staging buffer");
   std::ostringstream s;
   if (gradient_only) s << "#define E3X_UVW_SMALL_DW_ONLY\n";
+  if (reduce) s << "#define E3X_UVW_REDUCE\n";
   emit_header(s, P, K.lanes, K.chunks);
   int reg = 0;
   s << "struct Out { int off, d, mul, reg; bool used; };\n";
@@ -521,7 +527,7 @@ int build_uvw_small_source(e3x_plan& P, SubKernel& K, std::string* src, bool gra
   // shared weights of few (u, v) pairs live in registers, one per pair and lane (one chunk of output channels only)
   long long pairs = 0;
   for (const auto& p : P.paths) pairs += (long long)P.in1[p.in1].mul * P.in2[p.in2].mul;
-  const bool cached = all_uvw && P.shared_weights && K.chunks == 1 && pairs > 0 && pairs <= 64;
+  const bool cached = !reduce && all_uvw && P.shared_weights && K.chunks == 1 && pairs > 0 && pairs <= 64;
   K.cached_weights = cached;
   s << "constexpr int W_CACHE_REGS = " << (cached ? pairs : 0) << ";\n";
   s << "struct Path { int x1off, d1, U, x2off, d2, V, out, woff, wreg, mode; bool has_w; int nz_beg, nz_end; };\n";
@@ -2316,19 +2322,21 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
     if ((rc = load_functions(P, dev))) return rc;
     fn_dw = P->subs[0]->fn_dw[dev];
   }
-  // one thread per (path, v, w) column of the weight blocks
-  long long cols = 0;
-  for (const auto& q : P->paths) cols += (long long)P->in2[q.in2].mul * P->out[q.out].mul;
-  // with fewer than 256 columns a workgroup is (power of two >= columns) x (interleaved rows of its slice)
-  long long cpb = 1;
-  while (cpb < cols && cpb < 256) cpb *= 2;
-  const long long row_lanes = 256 / cpb;
-  const long long wblocks = (cols + cpb - 1) / cpb;
-  // enough batch slices to fill the chip a few times over, at least 16 rows per row lane
-  long long slices = (2048 + wblocks - 1) / wblocks;
-  if (slices > (Z + 16 * row_lanes - 1) / (16 * row_lanes)) slices = (Z + 16 * row_lanes - 1) / (16 * row_lanes);
-  if (slices < 1) slices = 1;
-  if (slices > 65535) slices = 65535;
+  // a workgroup per path, up to 256 of its (v, w) columns and 8 of its u (dw_jobs of the template)
+  long long wblocks = 0, row_lanes = 1;
+  for (const auto& q : P->paths) {
+    const long long cols = (long long)P->in2[q.in2].mul * P->out[q.out].mul;
+    long long cpb = 1;
+    while (cpb < cols && cpb < 256) cpb *= 2;
+    wblocks += (cols + cpb - 1) / cpb * ((P->in1[q.in1].mul + 7) / 8);
+    row_lanes = std::max(row_lanes, 256 / cpb);
+  }
+  if (wblocks == 0) return E3X_OK;
+  if (wblocks >= (1LL << 31)) return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: too many weights for one launch");
+  // enough batch slices to fill the chip a few times over, at least 4 rows per row lane (the slices of summed weights meet in
+  // atomics, one rounding each: at most 256 of them)
+  long long slices = std::min<long long>((2048 + wblocks - 1) / wblocks, (Z + 4 * row_lanes - 1) / (4 * row_lanes));
+  slices = std::max(1LL, std::min(slices, P->shared_weights ? 256LL : 65535LL));
   long long rows_per_slice = (Z + slices - 1) / slices;
   slices = (Z + rows_per_slice - 1) / rows_per_slice;
   void* args[] = {(void*)&x1, (void*)&x2, (void*)&grad_out, (void*)&grad_w, (void*)&n_rows, (void*)&rows_per_slice};

@@ -22,7 +22,8 @@ GOLDEN_GPU_CASES = [
 # instruction sets whose backward pass the GPU tests run (transposed plans are separate kernels)
 BACKWARD_CASES = _ks.BACKWARD_CASES + ["uvu_merged_cfg3_like_mul4", "uvu_builderA_cfg4_like_mul2", "uvu_shared_v2", "fctp_small_cfg5_like",
                                        "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular", "zero_path_first", "zero_path_last",
-                                       "dense_one_path", "node_ragged", "node_long_row"]  # fmt: skip
+                                       "dense_one_path", "node_ragged", "node_long_row", "few_channels", "few_channels_ragged",
+                                       "few_outputs", "few_outputs_per_sample"]  # fmt: skip
 BACKWARD_BF16_CASES = _ks.BACKWARD_BF16_CASES + ["uvu_shared_v2"]
 
 
@@ -109,6 +110,21 @@ def node_long_row():
     return o3.FullyConnectedTensorProduct("960x0e", "1x0e", "1x0e")
 
 
+def few_channels():
+    return o3.FullyConnectedTensorProduct("16x0e+16x1o", "0e+1o+2e", "16x0e+16x1o+16x2e")
+
+
+def few_channels_ragged():
+    # either input the one of more indices; more columns (v, w) than a workgroup has threads, and 9 u to blocks of 8
+    return o3.FullyConnectedTensorProduct("9x0e+5x1o", "3x0e+30x1o", "6x0e+11x1o")
+
+
+def few_outputs(per_sample=False):
+    # outputs summed over the lanes, with indices that are no multiple of them and more of them than lanes
+    kw = dict(internal_weights=False, shared_weights=False) if per_sample else {}
+    return o3.FullyConnectedTensorProduct("12x0e+7x1o", "20x0e+70x1o", "1x0e+2x1o+1x2e", **kw)
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
@@ -119,7 +135,9 @@ def edge_case_tensor_products():
         ("zero_path_first", zero_path(True), (torch.float32,)), ("zero_path_last", zero_path(False), (torch.float32,)),
         ("scalar_outputs", scalar_outputs(), (torch.bfloat16,)), ("wide_scalar_output", wide_scalar_output(), (torch.float32, torch.bfloat16)),
         ("dense_one_path", dense_one_path(), (torch.float32,)), ("node_ragged", node_ragged(), (torch.float32,)),
-        ("node_long_row", node_long_row(), (torch.float32,)),
+        ("node_long_row", node_long_row(), (torch.float32,)), ("few_channels", few_channels(), (torch.float32,)),
+        ("few_channels_ragged", few_channels_ragged(), (torch.float32,)), ("few_outputs", few_outputs(), (torch.float32, torch.bfloat16)),
+        ("few_outputs_per_sample", few_outputs(True), (torch.float32,)),
     ]  # fmt: skip
 
 
