@@ -113,7 +113,7 @@ class _Plan:
                     ws, ws_bytes = torch.empty(n, dtype=torch.uint8, device=x1.device), n
                     break
                 except torch.OutOfMemoryError:
-                    if x1.dtype != torch.float32:
+                    if x1.dtype != torch.float32 and n == sizes[-1]:
                         raise  # (fp32: the general kernel needs none)
             x1, x2 = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2))
         if self.family == "uvw_node":

@@ -593,6 +593,31 @@ def test_uvw_bf16_storage_full_size():
     assert abs(out.float().var().item() * 16384 - 1.0) < 0.1
 
 
+@pytest.mark.parametrize("make,Z", [(ks.mfma_small, 1), (ks.mfma_small, 128), (ks.mfma_small, 129), (ks.mfma_small, 4096), (ks.mfma_small, 4097),
+                                    (ks.mfma_wide_blocks, 70), (ks.mfma_wide_blocks, 1537)])  # fmt: skip
+def test_uvw_bf16_storage_few_rows_in_parts(make, Z):
+    # up to 128 workgroups of 128 rows and 64 channels: in parts, summed by another kernel (4097 rows of four outputs are 132)
+    from e3nn_amd import _lib
+
+    tp, tpb, wq = _bf16_uvw(make=make)
+    x1, x2 = (seeded(Z, d, seed=i).to(DEV).to(torch.bfloat16) for i, d in enumerate((tp.irreps_in1.dim, tp.irreps_in2.dim)))
+    x1[Z // 2, 5], x2[0, 70] = float("inf"), float("-inf")
+    L, handle = _lib.lib(), tpb._plan(torch.bfloat16).handle
+    room = [L.e3x_tp_forward_workspace_bytes_for(handle, n) for n in (Z, -1)]
+    assert (room[0] > room[1]) == ((Z + 127) // 128 * (4 if make is ks.mfma_small else 5) <= 128)
+    got, whole = tpb(x1, x2), torch.empty(Z, tp.irreps_out.dim, device=DEV, dtype=torch.bfloat16)
+    ws, w = torch.empty(room[1], dtype=torch.uint8, device=DEV), tpb.weight.detach()
+    _lib.check(L.e3x_tp_forward_ws(handle, _lib.ptr(x1), _lib.ptr(x2), _lib.ptr(w), _lib.ptr(whole), Z, _lib.ptr(ws), ws.numel(), _lib.stream_ptr(x1.device)))
+    # an infinity reaches the same outputs, as what it is or as NaN
+    assert torch.equal(got.isfinite(), whole.isfinite()) and not whole.isfinite().all()
+    rows = torch.cat([torch.arange(min(Z, 130)), torch.arange(max(0, Z - 20), Z)]).unique()
+    rows = rows[got[rows].isfinite().all(1).cpu()]
+    if len(rows):
+        ref = _oracle_chunks(oracle_spec(tp), x1[rows].float().cpu().numpy(), x2[rows].float().cpu().numpy(), wq)
+        # bf16 rounds to nearest with 8 significant bits; the fp32 sums vanish beside it
+        assert (np.abs(got[rows].detach().double().cpu().numpy() - ref) <= 2.0**-8 * np.abs(ref) + 1e-5 * np.abs(ref).max()).all()
+
+
 @pytest.mark.parametrize("Z", [8192 + 1, 16384 + 130, 16384 + 256 + 127])
 def test_uvw_bf16_storage_ragged_batches_in_256_row_workgroups(Z):
     # from 8192 rows on the 0e and 1o outputs are computed by workgroups of 256 rows (two row tiles per wavefront);
