@@ -17,7 +17,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libe3x.so")
 
 SOURCES = ["api.cpp", "wigner.cpp", "jit.cpp", "tp.cpp", "fc.cpp", "sh.hip", "graph.hip", "gate.hip"]
 TEMPLATES = [("kTplCommon", "common.inc"), ("kTplPieces", "pieces.inc"), ("kTplUvu", "uvu.inc"), ("kTplUvuFc", "uvu_fc.inc"), ("kTplUvuRowgrad", "uvu_rowgrad.inc"), ("kTplUvuMfma", "uvu_mfma.inc"), ("kTplUvwSmall", "uvw_small.inc"),
-             ("kTplUvwMfma", "uvw_mfma.inc"), ("kTplUvwMfmaBf16", "uvw_mfma_bf16.inc"), ("kTplUvwFew", "uvw_few.inc"), ("kTplUvwMfmaHalf", "uvw_mfma_half.inc"),
+             ("kTplUvwMfma", "uvw_mfma.inc"), ("kTplUvwMfmaBf16", "uvw_mfma_bf16.inc"), ("kTplUvwFew", "uvw_few.inc"), ("kTplUvwUnits", "uvw_units.inc"), ("kTplUvwMfmaHalf", "uvw_mfma_half.inc"),
              ("kTplUvwMfmaDw", "uvw_mfma_dw.inc"), ("kTplUvwDwWide", "uvw_dw_wide.inc"),
              ("kTplUvwNode", "uvw_node.inc"), ("kTplUvwNodeDw", "uvw_node_dw.inc"),
              ("kTplFcMfma", "fc_mfma.inc"), ("kTplFcDw", "fc_dw.inc")]

@@ -15,6 +15,7 @@ extern const char* const kTplUvwSmall;
 extern const char* const kTplUvwMfma;
 extern const char* const kTplUvwMfmaBf16;
 extern const char* const kTplUvwFew;
+extern const char* const kTplUvwUnits;
 extern const char* const kTplUvwMfmaHalf;
 extern const char* const kTplUvwMfmaDw;
 extern const char* const kTplUvwDwWide;

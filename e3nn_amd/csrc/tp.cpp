@@ -7,9 +7,11 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
+#include <numeric>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -91,7 +93,7 @@ struct e3x_plan {
   // scalar outputs formed from both inputs: how many, their parts, the channels of all parts, the channels of all sums; and
   // the tiles of the other outputs
   // uvw_mfma: what a batch of few rows takes in parts (see few_ranges): units, their fp32 sums per row, ranges of outer indices at most
-  int few_units = 0, few_width = 0, few_max_ranges = 0;
+  int few_units = 0, few_width = 0, few_max_ranges = 0, few_channels = 64;  // (channels of a tile)
   int half_scalars = 0, half_parts = 0, half_part_width = 0, half_sums = 0, half_general = 0;
   // uvw_mfma: the weight-gradient kernel is a code object of its own, built on first use
   std::unique_ptr<SubKernel> dw;
@@ -659,11 +661,13 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   if (wpe) s << "#define E3X_UVW_WPE " << wpe << "\n";
   int n_nz = 0, n_path = 0, n_target = 0, dka = 1, drmax = 1;
   int n_scalar = 0, units = 0, width_units = 0, min_blocks = 1 << 20;
+  long long longest = 0;
   if (half) P.half_parts = P.half_part_width = P.half_sums = P.half_general = 0;
   for (size_t c = 0; c < P.out.size(); ++c) {
     std::ostringstream mine;
     const int beg = n_path;
     int out_units = 0, out_width = 0;  // of a tile of this output
+    long long steps = 0;               // ... and outer indices times K that its workgroup walks
     for (const auto& p : P.paths) {
       if (p.out != (int)c) continue;
       const e3x_irrep &a = P.in1[p.in1], &b = P.in2[p.in2];
@@ -691,9 +695,10 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
               reached[k_is_x2 ? j : i] |= 1u << k;
             }
           }
+      if (synth) reached = {std::accumulate(reached.begin(), reached.end(), 0u, std::bit_or<unsigned>())};
       for (unsigned m : reached)
-        if (m) out_units += 1, out_width += 64 * __builtin_popcount(m);
-      min_blocks = std::min(min_blocks, (k_is_x2 ? a.mul : b.mul) / 8);
+        if (m) out_units += 1, out_width += wt * __builtin_popcount(m), steps += (long long)a.mul * b.mul;
+      min_blocks = std::min(min_blocks, std::max(1, (k_is_x2 ? a.mul : b.mul) / 8));
       const long long W = P.out[c].mul;
       // W_p[u, v, w] at woff + (u * V + v) * W + w
       const long long stride_u = (long long)b.mul * W, stride_v = W;
@@ -706,6 +711,7 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
       ++n_path;
     }
     if (n_path == beg) continue;
+    longest = std::max(longest, steps);
     ps << mine.str();
     // fp16 pairs and bf16: a scalar output of l x l, l = 1 or 2, can form its operand from both inputs (run_scalar_target)
     bool scalar = (half || P.dtype == E3X_BF16) && P.out[c].l == 0 && P.out[c].mul % 64 == 0, product = false;
@@ -733,8 +739,10 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
       units += out_units, width_units += out_width;
     }
   }
-  if (P.dtype == E3X_BF16) {
-    P.few_units = units, P.few_width = width_units, P.few_max_ranges = min_blocks;
+  if (P.dtype == E3X_BF16 || (longest >= 3072 && !half && !half_fits(P))) {
+    s << "#define E3X_UVW_FEW 1\n";
+    // (a walk of 3072 takes some 12 us in bf16 storage and 35 in fp32; a shorter one is not worth a second launch)
+    P.few_units = longest >= 3072 ? units : 0, P.few_width = width_units, P.few_max_ranges = min_blocks, P.few_channels = wt;
     s << "constexpr int FEW_UNITS = " << units << ", FEW_WIDTH = " << width_units << ";\n";
   }
   s << "constexpr int WT = " << wt << ", KMAX = " << kmax << ";\n";  // KMAX: the largest GEMM K extent
@@ -760,8 +768,8 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   (half ? P.half_targets : P.n_targets) = n_target;
   *src = s.str() + e3x::kTplCommon;
   if (half) *src += e3x::kTplUvwMfmaHalf;
-  else if (P.dtype == E3X_BF16) *src += std::string(e3x::kTplUvwMfmaBf16) + e3x::kTplUvwFew;
-  else *src += std::string(e3x::kTplPieces) + e3x::kTplUvwMfma;
+  else if (P.dtype == E3X_BF16) *src += std::string(e3x::kTplUvwMfmaBf16) + e3x::kTplUvwUnits + e3x::kTplUvwFew;
+  else *src += std::string(e3x::kTplPieces) + (P.few_units ? e3x::kTplUvwUnits : "") + e3x::kTplUvwMfma;
   return E3X_OK;
 }
 
@@ -1174,6 +1182,8 @@ int load_functions(e3x_plan* P, int dev) {
     if (P->family == "uvw_mfma" && P->dtype == E3X_BF16) {
       if (hipModuleGetFunction(&K->fn_pack[dev], mod, "e3x_uvw_mfma_pack") != hipSuccess)
         return fail(E3X_ERR_HIP, "kernel e3x_uvw_mfma_pack missing from " + K->hsaco);
+    }
+    if (P->few_units) {
       if (hipModuleGetFunction(&K->fn_parts[dev], mod, "e3x_uvw_few_parts") != hipSuccess ||
           hipModuleGetFunction(&K->fn_sum[dev], mod, "e3x_uvw_few_sum") != hipSuccess)
         return fail(E3X_ERR_HIP, "kernels for few rows missing from " + K->hsaco);
@@ -1581,30 +1591,35 @@ static int zero_output(e3x_plan* P, void* out, int64_t rows, hipStream_t st) {
 
 static bool needs_packed_weights(const e3x_plan* P) { return P->family == "uvw_mfma" && P->dtype == E3X_BF16; }
 
-static size_t packed_bytes(const e3x_plan* P) { return ((size_t)P->weight_numel * 2 + 15) / 16 * 16; }
+static size_t packed_bytes(const e3x_plan* P) { return needs_packed_weights(P) ? ((size_t)P->weight_numel * 2 + 15) / 16 * 16 : 0; }
 
-// Few rows in bf16 storage (templates/uvw_few.inc): a workgroup per unit (one slice of one path and output tile) and range of
-// its outer indices, as many ranges as keep the workgroups to one round of the 256 CUs.  Up to 128 workgroups of the ordinary
-// form, whole / in parts: 64x0e+32x1o times 32x0e+32x1o+32x2e onto 64x0e+64x1o+64x1e+64x2e 64 / 1480 / 4096 / 5000 rows (1 / 12 /
+// Few rows (templates/uvw_few.inc for bf16 storage, e3x_uvw_few_parts of uvw_mfma.inc for fp32): a workgroup per unit (one slice
+// of one path and output tile) and range of its outer indices, as many ranges as keep the workgroups to one round of the
+// chip, one workgroup per CU in bf16 storage and three in fp32.  In bf16 storage up to 128 workgroups of the ordinary form, whole
+// / in parts: 64x0e+32x1o times 32x0e+32x1o+32x2e onto 64x0e+64x1o+64x1e+64x2e 64 / 1480 / 4096 / 5000 rows (1 / 12 /
 // 32 / 40 tiles of 4 outputs) 58 / 69 / 70 / 71 and 28 / 46 / 65 / 75 us; 128x0e+128x1o+128x2e squared 64 / 1480 / 3000 / 5000
 // rows (6 outputs) 616 / 652 / 655 / 765 and 64 / 273 / 518 / 786.  Half and twice as many ranges at 64 rows: 28 and 29, 79 and
-// 80 us.  0: whole.
+// 80 us.  In fp32, where the kernel on pairs of fp16 operands does not fit, up to 384 (of 64 rows, so 6144 rows of four outputs):
+// the first of these products at 64 / 1480 / 4096 / 6000 rows 175 / 178 / 178 / 252 and 31 / 78 / 138 / 197 us, beyond it 253 and
+// 237 at 8192, 311 and 326 at 12 000, for scratch of 24 KB a row.  0: whole.
+static int few_tile_rows(const e3x_plan* P) { return P->dtype == E3X_BF16 ? 128 : 64; }
 static int few_ranges(const e3x_plan* P, long long Z) {
-  const long long tiles = (Z + 127) / 128;
-  if (!P->few_units || Z <= 0 || tiles * P->n_targets > 128) return 0;
-  return (int)std::max(1LL, std::min<long long>(P->few_max_ranges, 256 / (tiles * P->few_units)));
+  const long long tiles = (Z + few_tile_rows(P) - 1) / few_tile_rows(P);
+  const bool half_storage = P->dtype == E3X_BF16;
+  if (!P->few_units || Z <= 0 || tiles * P->n_targets > (half_storage ? 128 : 384)) return 0;
+  return (int)std::max(1LL, std::min<long long>(P->few_max_ranges, (half_storage ? 256 : 768) / (tiles * P->few_units)));
 }
 static size_t few_bytes(const e3x_plan* P, long long Z) { return (size_t)few_ranges(P, Z) * (size_t)std::max(Z, 0LL) * P->few_width * 4; }
 
 extern "C" size_t e3x_tp_forward_workspace_bytes_for(const e3x_plan* P, int64_t Z) {
   if (P && P->half) return half_parts_offset(*P) + half_parts_bytes(*P, Z);  // (taken when given; e3x_tp_forward runs without)
-  return (P && needs_packed_weights(P)) ? packed_bytes(P) + few_bytes(P, Z) : 0;
+  return P ? packed_bytes(P) + few_bytes(P, Z) : 0;
 }
 
 extern "C" size_t e3x_tp_forward_workspace_bytes(const e3x_plan* P) {
   if (P && P->few_units) {  // the most that a batch asks for
     size_t most = 0;
-    for (long long Z = 128; few_ranges(P, Z); Z += 128) most = std::max(most, few_bytes(P, Z));
+    for (long long Z = few_tile_rows(P); few_ranges(P, Z); Z += few_tile_rows(P)) most = std::max(most, few_bytes(P, Z));
     return packed_bytes(P) + most;
   }
   return e3x_tp_forward_workspace_bytes_for(P, P && P->half ? half_part_rows(*P) : 0);
@@ -1678,18 +1693,19 @@ extern "C" int e3x_tp_forward_ws(e3x_plan* P, const void* x1, const void* x2, co
     if (err != hipSuccess)
       return fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
     w = workspace;
-    const size_t part_bytes = few_bytes(P, Z);  // (a workspace without room for them: whole)
-    if (part_bytes && workspace_bytes >= packed_bytes(P) + part_bytes) {
-      SubKernel* K = P->subs[0].get();
-      float* parts = (float*)((char*)workspace + packed_bytes(P));
-      int n_ranges = few_ranges(P, Z);
-      void* fargs[] = {(void*)&x1, (void*)&x2, (void*)&w, (void*)&parts, (void*)&n_rows, (void*)&n_ranges};
-      err = hipModuleLaunchKernel(K->fn_parts[dev], (unsigned)((Z + 127) / 128), (unsigned)(P->few_units * n_ranges), 1, 512, 1, 1, 0, st, fargs, nullptr);
-      void* sargs[] = {(void*)&parts, (void*)&out, (void*)&n_rows, (void*)&n_ranges};
-      if (err == hipSuccess)
-        err = hipModuleLaunchKernel(K->fn_sum[dev], (unsigned)((Z * 16 + 255) / 256), (unsigned)P->n_targets, 1, 256, 1, 1, 0, st, sargs, nullptr);
-      return err == hipSuccess ? E3X_OK : fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
-    }
+  }
+  const size_t few = few_bytes(P, Z);
+  if (few && workspace && workspace_bytes >= packed_bytes(P) + few && !((uintptr_t)workspace & 15)) {  // (without room for the parts: whole)
+    SubKernel* K = P->subs[0].get();
+    float* parts = (float*)((char*)workspace + packed_bytes(P));
+    int n_ranges = few_ranges(P, Z);
+    const int tile = few_tile_rows(P), quads = P->few_channels / 4;
+    void* fargs[] = {(void*)&x1, (void*)&x2, (void*)&w, (void*)&parts, (void*)&n_rows, (void*)&n_ranges};
+    hipError_t err = hipModuleLaunchKernel(K->fn_parts[dev], (unsigned)((Z + tile - 1) / tile), (unsigned)(P->few_units * n_ranges), 1, 4 * tile, 1, 1, 0, st, fargs, nullptr);
+    void* sargs[] = {(void*)&parts, (void*)&out, (void*)&n_rows, (void*)&n_ranges};
+    if (err == hipSuccess)
+      err = hipModuleLaunchKernel(K->fn_sum[dev], (unsigned)((Z * quads + 255) / 256), (unsigned)P->n_targets, 1, 256, 1, 1, 0, st, sargs, nullptr);
+    return err == hipSuccess ? E3X_OK : fail(E3X_ERR_HIP, std::string("e3x_tp_forward: launch failed: ") + hipGetErrorString(err));
   }
   void* args[] = {(void*)&x1, (void*)&x2, (void*)&w, (void*)&out, (void*)&n_rows, (void*)&row_flags};  // (flags: uvw_mfma, fp32)
   for (auto& K : P->subs) {

@@ -85,6 +85,7 @@ class _Plan:
         self.out_dim, self.in2_dim = irreps_out.dim, irreps_in2.dim
         self.arithmetic = L.e3x_tp_plan_arithmetic(handle, 0).decode()  # which instruction forms the products
         self._in_parts = L.e3x_tp_forward_workspace_bytes(handle) > L.e3x_tp_forward_workspace_bytes_for(handle, -1)
+        self._packs = L.e3x_tp_forward_workspace_bytes_for(handle, -1) > 0
         self._fused_grad_w = None  # whether the plan has the message-step backward kernel; asked on first use
         self._by_destination = None  # ... and, on the forward plan, the one grouped by destination
 
@@ -107,7 +108,7 @@ class _Plan:
             sizes = [L.e3x_tp_forward_workspace_bytes(self.handle)]
         ws, ws_bytes = None, 0
         if sizes[0]:
-            # scratch for the weights repacked for the matrix cores; the kernel reads rows with 16-byte loads
+            # scratch for the weights repacked for the matrix cores and for the parts of a batch of few rows
             for n in sizes:
                 try:
                     ws, ws_bytes = torch.empty(n, dtype=torch.uint8, device=x1.device), n
@@ -115,7 +116,8 @@ class _Plan:
                 except torch.OutOfMemoryError:
                     if x1.dtype != torch.float32 and n == sizes[-1]:
                         raise  # (fp32: the general kernel needs none)
-            x1, x2 = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2))
+            if self._packs:  # rows are read with 16-byte loads
+                x1, x2 = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2))
         if self.family == "uvw_node":
             # rows and weights are read with 16-byte loads
             x1, w = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, w))

@@ -150,8 +150,9 @@ int e3x_tp_forward(e3x_plan* plan, const void* x1, const void* x2, const void* w
  * are formed by the kernel of e3x_tp_forward.  Every other plan needs no workspace and e3x_tp_forward is enough.
  * e3x_tp_forward_workspace_bytes is enough for every batch, e3x_tp_forward_workspace_bytes_for for batches of Z rows: fp32
  * plans with scalar outputs of l x l form these in parts where the chip would not be full, and only such a batch needs room
- * for its parts; so do bf16 plans with all outputs.  Z < 0: the least that the call takes, without room for parts; a small batch
- * runs the longer for it and has the same results, to the last bit in fp32, up to the order of its fp32 sums in bf16 storage. */
+ * for its parts; so do plans in bf16 storage, and fp32 plans that do not take pairs of fp16 operands, with all outputs.
+ * Z < 0: the least that the call takes, without room for parts; a small batch runs the longer for it and has the same results,
+ * to the last bit on pairs of fp16 operands, up to the order of its fp32 sums elsewhere. */
 size_t e3x_tp_forward_workspace_bytes(const e3x_plan* plan);
 size_t e3x_tp_forward_workspace_bytes_for(const e3x_plan* plan, int64_t Z);
 int e3x_tp_forward_ws(e3x_plan* plan, const void* x1, const void* x2, const void* w, void* out, int64_t Z,

@@ -119,6 +119,11 @@ def few_channels_ragged():
     return o3.FullyConnectedTensorProduct("9x0e+5x1o", "3x0e+30x1o", "6x0e+11x1o")
 
 
+def few_outer_indices():
+    # tiles of 32 channels, whose second wave column takes every other outer index, an odd number of which is left
+    return o3.FullyConnectedTensorProduct("128x0e+64x1o", "33x0e+3x1o", "32x1o+32x1e+32x2e")
+
+
 def few_outputs(per_sample=False):
     # outputs summed over the lanes, with indices that are no multiple of them and more of them than lanes
     kw = dict(internal_weights=False, shared_weights=False) if per_sample else {}
@@ -137,7 +142,7 @@ def edge_case_tensor_products():
         ("dense_one_path", dense_one_path(), (torch.float32,)), ("node_ragged", node_ragged(), (torch.float32,)),
         ("node_long_row", node_long_row(), (torch.float32,)), ("few_channels", few_channels(), (torch.float32,)),
         ("few_channels_ragged", few_channels_ragged(), (torch.float32,)), ("few_outputs", few_outputs(), (torch.float32, torch.bfloat16)),
-        ("few_outputs_per_sample", few_outputs(True), (torch.float32,)),
+        ("few_outer_indices", few_outer_indices(), (torch.float32,)), ("few_outputs_per_sample", few_outputs(True), (torch.float32,)),
     ]  # fmt: skip
 
 

@@ -618,6 +618,34 @@ def test_uvw_bf16_storage_few_rows_in_parts(make, Z):
         assert (np.abs(got[rows].detach().double().cpu().numpy() - ref) <= 2.0**-8 * np.abs(ref) + 1e-5 * np.abs(ref).max()).all()
 
 
+@pytest.mark.parametrize("make,Z", [(ks.mfma_small, 1), (ks.mfma_small, 64), (ks.mfma_small, 65), (ks.mfma_small, 6144), (ks.mfma_small, 6145),
+                                    (ks.mfma_half_tiles, 193), (ks.few_outer_indices, 70)])  # fmt: skip
+def test_uvw_fp32_few_rows_in_parts(make, Z):
+    # fp32 instruction, blocks of 32: up to 384 workgroups of 64 rows and one output tile (6145 rows of four outputs are 388)
+    from e3nn_amd import _lib
+
+    tp = make().to(DEV)
+    x1, x2, w = (seeded(*n, seed=i).to(DEV) for i, n in enumerate([(Z, tp.irreps_in1.dim), (Z, tp.irreps_in2.dim), (tp.weight_numel,)]))
+    ref = otp.tp_forward(oracle_spec(tp), x1[:200].cpu().numpy(), x2[:200].cpu().numpy(), w.cpu().numpy())
+    L, handle = _lib.lib(), tp._plan(torch.float32).handle
+    assert L.e3x_tp_forward_workspace_bytes_for(ks.unaligned_mfma()._plan(torch.float32).handle, Z) == 0  # too short a walk
+    assert L.e3x_tp_forward_workspace_bytes_for(handle, -1) == 0 and (L.e3x_tp_forward_workspace_bytes_for(handle, Z) > 0) == (Z != 6145)
+    whole = torch.empty(Z, tp.irreps_out.dim, device=DEV)
+
+    def both():
+        _lib.check(L.e3x_tp_forward(handle, _lib.ptr(x1), _lib.ptr(x2), _lib.ptr(w), _lib.ptr(whole), Z, _lib.stream_ptr(x1.device)))
+        return tp(x1, x2, w)
+
+    got = both()
+    # sums of some 1e4 products in fp32 lose about 4e-7 of the 2-norm
+    assert float((got - whole).norm()) < 1e-6 * float(whole.norm())
+    assert np.linalg.norm(got[:200].double().cpu().numpy() - ref) < 1e-6 * np.linalg.norm(ref)
+    # an infinity reaches the same outputs, as what it is or as NaN
+    x1[Z // 2, 5], x2[0, x2.shape[1] // 2] = float("inf"), float("-inf")
+    got = both()
+    assert torch.equal(got.isfinite(), whole.isfinite()) and not whole.isfinite().all()
+
+
 @pytest.mark.parametrize("Z", [8192 + 1, 16384 + 130, 16384 + 256 + 127])
 def test_uvw_bf16_storage_ragged_batches_in_256_row_workgroups(Z):
     # from 8192 rows on the 0e and 1o outputs are computed by workgroups of 256 rows (two row tiles per wavefront);
