@@ -596,8 +596,7 @@ bool uvw_mfma_eligible(const e3x_plan& P) { return uvw_mfma_eligible(P, P.dtype)
 // (the K operand in registers, the row maximum among neighbouring lanes), multiples of 64 on the output, l <= 2 there (the
 // seven accumulator tiles of l = 3 do not fit beside the operands), rows in 16-byte pieces.  The weights are packed on
 // every call into a workspace; without one, or with misaligned rows, the kernel of uvw_mfma.inc runs.
-bool half_fits(const e3x_plan& P) {
-  if (P.family != "uvw_mfma" || P.dtype != E3X_F32 || env_int("E3X_UVW_SPLIT", 1) == 0 || env_int("E3X_UVW_HALF", 1) == 0) return false;
+bool half_blocks(const e3x_plan& P) {
   if ((P.in1_dim | P.in2_dim) & 3) return false;
   for (const auto& p : P.paths) {
     const int U = P.in1[p.in1].mul, V = P.in2[p.in2].mul;
@@ -605,6 +604,9 @@ bool half_fits(const e3x_plan& P) {
     if (((P.off1[p.in1] | P.off2[p.in2] | p.woff) & 3) || std::max(P.in1[p.in1].l, P.in2[p.in2].l) > 3) return false;
   }
   return true;
+}
+bool half_fits(const e3x_plan& P) {
+  return P.family == "uvw_mfma" && P.dtype == E3X_F32 && env_int("E3X_UVW_SPLIT", 1) && env_int("E3X_UVW_HALF", 1) && half_blocks(P);
 }
 constexpr int kHalfMaxBlocks = 64;  // MAX_BLOCKS of the template
 // What the compiler makes of a set decides as well.  Private bytes per lane against the kernel of uvw_mfma.inc, which spills
@@ -739,7 +741,7 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
       units += out_units, width_units += out_width;
     }
   }
-  if (P.dtype == E3X_BF16 || (longest >= 3072 && !half && !half_fits(P))) {
+  if (P.dtype == E3X_BF16 || (longest >= 3072 && !half && !half_blocks(P))) {
     s << "#define E3X_UVW_FEW 1\n";
     // (a walk of 3072 takes some 12 us in bf16 storage and 35 in fp32; a shorter one is not worth a second launch)
     P.few_units = longest >= 3072 ? units : 0, P.few_width = width_units, P.few_max_ranges = min_blocks, P.few_channels = wt;

@@ -62,6 +62,7 @@ class _Plan:
     """Owner of one ``e3x_plan`` handle: a fused kernel specialised to one instruction set."""
 
     _in_parts = False  # whether the scratch of a forward call depends on the batch
+    _packs = True  # whether it holds repacked weights, whose kernels read rows with 16-byte loads
 
     def __init__(self, irreps_in1, irreps_in2, irreps_out, instructions, shared_weights: bool, dtype: torch.dtype):
         """``instructions``: tuples ``(i_in1, i_in2, i_out, mode, has_weight, path_weight)``, path weights final."""
@@ -116,7 +117,7 @@ class _Plan:
                 except torch.OutOfMemoryError:
                     if x1.dtype != torch.float32 and n == sizes[-1]:
                         raise  # (fp32: the general kernel needs none)
-            if self._packs:  # rows are read with 16-byte loads
+            if self._packs:
                 x1, x2 = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2))
         if self.family == "uvw_node":
             # rows and weights are read with 16-byte loads
