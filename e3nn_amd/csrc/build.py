@@ -14,6 +14,8 @@ PKG = os.path.dirname(HERE)
 LIB_DIR = os.path.join(PKG, "lib")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(LIB_DIR, "libe3x.so")
+HOST_PATH = os.path.join(LIB_DIR, "_e3x_host.so")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 SOURCES = ["api.cpp", "wigner.cpp", "jit.cpp", "tp.cpp", "fc.cpp", "sh.hip", "graph.hip", "gate.hip"]
 TEMPLATES = [("kTplCommon", "common.inc"), ("kTplPieces", "pieces.inc"), ("kTplUvu", "uvu.inc"), ("kTplUvuFc", "uvu_fc.inc"), ("kTplUvuRowgrad", "uvu_rowgrad.inc"), ("kTplUvuMfma", "uvu_mfma.inc"), ("kTplUvwSmall", "uvw_small.inc"),
@@ -81,14 +83,34 @@ def build_library(verbose=True, force=True):
     with open(vs, "w") as f:
         f.write("{ global: e3x_*; local: *; };\n")
     _run([hipcc(), "-shared", "-o", LIB_PATH] + objs + ["-ldl", "-Wl,--version-script=" + vs], verbose)
+    build_host(verbose, force)
     return LIB_PATH
+
+
+def build_host(verbose=True, force=True):
+    """The extension module of the host path, against libe3x.so and this interpreter's torch."""
+    import sysconfig
+
+    import torch
+
+    src = os.path.join(HERE, "host.cpp")
+    header = os.path.join(PKG, "..", "include", "e3x.h")
+    if not force and os.path.exists(HOST_PATH) and os.path.getmtime(HOST_PATH) > max(os.path.getmtime(src), os.path.getmtime(header)):
+        return
+    torch_dir = os.path.dirname(torch.__file__)
+    include = [os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"), ROCM + "/include",
+               sysconfig.get_paths()["include"]]  # fmt: skip
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-DTORCH_EXTENSION_NAME=_e3x_host", "-DUSE_ROCM",
+           "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]  # fmt: skip
+    cmd += [a for d in include for a in ("-isystem", d)] + [src, "-o", HOST_PATH, "-L" + LIB_DIR, "-l:libe3x.so", "-L" + os.path.join(torch_dir, "lib")]
+    _run(cmd + ["-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"], verbose)
 
 
 def ensure_built():
     """For test sessions, the smoke test and the benchmark: builds the library when it is not there (the package itself
     never does: it raises)."""
     lib = os.path.join(LIB_DIR, "libe3x.so")
-    if not os.path.exists(lib):
+    if not (os.path.exists(lib) and os.path.exists(HOST_PATH)):
         build_library(verbose=False, force=False)
     return lib
 

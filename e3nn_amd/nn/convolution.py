@@ -53,10 +53,21 @@ class _Mix(torch.autograd.Function):
             g_conv = torch.empty_like(conv) if need_conv else None
             with _lib.on_device(g.device):
                 _lib.check(_lib.lib().e3x_mix_backward(*(_lib.ptr(t) for t in (g_rows, alpha, conv, c0, c1, g_alpha, g_conv)), *conv.shape, _lib.stream_ptr(g.device)))
-        else:
-            g_alpha = (g * conv * c1).sum(-1, keepdim=True) if need_alpha else None
-            g_conv = g * torch.addcmul(c0, alpha, c1) if need_conv else None
-        return (g if need_sc else None), g_alpha, g_conv, None, None
+            return (g if need_sc else None), g_alpha, g_conv, None, None
+        return _mix_gradients(ctx.saved_tensors, g, ctx.needs_input_grad)
+
+
+def _mix_gradients(saved, g, needs):
+    """Differentiable gradients of the mixing."""
+    alpha, conv, c0, c1 = saved
+    g_alpha = (g * conv * c1).sum(-1, keepdim=True) if needs[1] else None
+    g_conv = g * torch.addcmul(c0, alpha, c1) if needs[2] else None
+    return (g if needs[0] else None), g_alpha, g_conv, None, None
+
+
+def _mix(sc, alpha, conv, c0, c1):
+    out = _lib.native().mix(sc, alpha, conv, c0, c1)
+    return _Mix.apply(sc, alpha, conv, c0, c1) if out is None else out
 
 
 def _mix_in_one_kernel(rows, alpha, conv, c0, c1):
@@ -65,6 +76,31 @@ def _mix_in_one_kernel(rows, alpha, conv, c0, c1):
         and c0.shape == c1.shape == rows.shape[1:]
         and all(t.dtype == torch.float32 and t.is_contiguous() and t.device == rows.device for t in (rows, alpha, conv, c0, c1))
     )  # fmt: skip
+
+
+def _lin2_alpha_gradients(lin2, head, saved, g_conv, g_alpha, need):
+    """Differentiable gradients of ``lin2`` and ``alpha``: the two products' own."""
+    features, attr, w_lin2, w_alpha = saved[:4]
+    k = head.irreps_in1.dim
+    gf, _, gw_lin2 = _slot_backward(_TpSlot, _OUT, (features, attr, w_lin2), g_conv.contiguous(), (need[0], False, need[2]), lin2)
+    gs, _, gw_alpha = _slot_backward(_TpSlot, _OUT, (features[:, :k].contiguous(), attr, w_alpha), g_alpha.contiguous(), (need[0], False, need[3]), head)
+    if need[0]:
+        gf = gf + torch.nn.functional.pad(gs, (0, features.shape[1] - k))
+    return gf, None, gw_lin2, gw_alpha
+
+
+_lib.connect({"mix_gradients": _mix_gradients, "lin2_alpha_gradients": _lin2_alpha_gradients})
+
+
+def _lin2_alpha(features, attr, w_lin2, w_alpha, lin2, alpha, head):
+    in_place = head._plan(features.dtype).family == "uvw_node" and features.shape[1] % 4 == 0
+    reads = alpha if in_place else head
+    packs = [(tp._plans.get("native") or tp._native_plans())[0] for tp in (lin2, reads, head)]
+    if None not in packs:
+        out = _lib.native().lin2_alpha(*packs, lin2, reads, head, alpha, head.irreps_in1.dim, in_place, features, attr, w_lin2, w_alpha)
+        if out is not None:
+            return out
+    return _Lin2Alpha.apply(features, attr, w_lin2, w_alpha, lin2, alpha, head)
 
 
 class _Lin2Alpha(torch.autograd.Function):
@@ -90,13 +126,7 @@ class _Lin2Alpha(torch.autograd.Function):
         k = head.irreps_in1.dim
         g_conv, g_alpha = g_conv.contiguous(), g_alpha.contiguous()
         if torch.is_grad_enabled():
-            # under create_graph: the two products' own differentiable gradients
-            need = ctx.needs_input_grad
-            gf, _, gw_lin2 = _slot_backward(_TpSlot, _OUT, (features, attr, w_lin2), g_conv, (need[0], False, need[2]), lin2)
-            gs, _, gw_alpha = _slot_backward(_TpSlot, _OUT, (features[:, :k].contiguous(), attr, w_alpha), g_alpha, (need[0], False, need[3]), head)
-            if need[0]:
-                gf = gf + torch.nn.functional.pad(gs, (0, features.shape[1] - k))
-            return gf, None, gw_lin2, gw_alpha, None, None, None
+            return (*_lin2_alpha_gradients(lin2, head, ctx.saved_tensors, g_conv, g_alpha, ctx.needs_input_grad), None, None, None)
         dt = features.dtype
         g_features = gw_lin2 = gw_alpha = None
         if ctx.needs_input_grad[2]:
@@ -193,7 +223,7 @@ class Convolution(torch.nn.Module):
             and node_attr.shape[:-1] == node_features.shape[:-1]
             and node_features.dtype == torch.float32
         ):
-            node_conv_out, alpha = _Lin2Alpha.apply(
+            node_conv_out, alpha = _lin2_alpha(
                 node_features.contiguous(), node_attr.to(node_features.dtype).contiguous(), self.lin2.weight, self.alpha.weight,
                 self.lin2, self.alpha, self._alpha_head,
             )  # fmt: skip
@@ -205,4 +235,4 @@ class Convolution(torch.nn.Module):
         if self.__dict__.get("_mix_key") != key:  # the two constant rows of the mixing, once per device
             self.__dict__["_mix_key"], self.__dict__["_mix_rows"] = key, ((1 - m) * inv, m * (inv * inv))
         c0, c1 = self.__dict__["_mix_rows"]
-        return _Mix.apply(node_self_connection, alpha, node_conv_out, c0, c1)
+        return _mix(node_self_connection, alpha, node_conv_out, c0, c1)

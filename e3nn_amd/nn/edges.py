@@ -6,7 +6,6 @@ The message-passing step of the reference is
 edges of each destination to be contiguous: ``DstSortedEdges`` validates both index
 arrays once and builds the row pointers and the stable permutation on the GPU.
 """
-import ctypes
 import os
 
 import torch
@@ -58,6 +57,15 @@ class DstSortedEdges:
             self._src_rows = rows
         return self._src_rows
 
+    def native(self):
+        """The tensors of the list as the host path takes them."""
+        if self._native is None:
+            self._native = _lib.native().Edges(
+                self.edge_src, self.edge_dst, self.rowptr, self.perm, self.walk_perm, self.row_order, self.src_rows, self.num_edges, self.num_nodes,
+                self.num_src_nodes,
+            )  # fmt: skip
+        return self._native
+
     def in_sorted_order(self, *edge_tensors):
         """Per-edge tensors ``[E, ...]`` rewritten in the order of the destination-sorted list (row ``k`` of a result is
         row ``perm[k]`` of the argument; differentiable).  Together with :meth:`sorted` this moves the permutation out
@@ -82,7 +90,7 @@ class DstSortedEdges:
             other.edge_src, other.edge_dst = src, self.edge_dst.index_select(0, self.perm)
             other._src_rows, other.walk_perm = src, None
             other.perm = torch.arange(self.num_edges, dtype=torch.int32, device=src.device)
-            other._transposed, other._sorted = None, other
+            other._transposed, other._sorted, other._native = None, other, None
             self._sorted = other
         return self._sorted
 
@@ -91,6 +99,7 @@ class DstSortedEdges:
         self._transposed = None
         self._sorted = None
         self._src_rows = None
+        self._native = None
         self._locality_order = locality_order
         if not (edge_src.is_cuda and edge_dst.is_cuda):
             raise RuntimeError("DstSortedEdges needs index tensors on the GPU")
@@ -103,35 +112,19 @@ class DstSortedEdges:
         self.edge_src = edge_src.contiguous()
         self.edge_dst = edge_dst.contiguous()
         self.num_edges = E = edge_src.numel()
-        dev = edge_src.device
-        L = _lib.lib()
-        with _lib.on_device(dev):
-            st = _lib.stream_ptr(dev)
-            self.rowptr = torch.empty(self.num_nodes + 1, dtype=torch.int32, device=dev)
-            self.perm = torch.empty(E, dtype=torch.int32, device=dev)
-            # rows that share their smallest source are processed next to each other (they share most of their
-            # sources, which then sit in L2): locality taken from the graph, not from the caller's node numbering
-            self.row_order = None
-            if locality_order and self.num_nodes > 0:
-                self.row_order = torch.empty(self.num_nodes, dtype=torch.int32, device=dev)
-            ws_bytes = L.e3x_edges_workspace_bytes(E, self.num_nodes)
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            grouped, pairs = ctypes.c_int32(0), ctypes.c_int32(0)
-            _lib.check(
-                L.e3x_edges_build(
-                    _lib.ptr(self.edge_src), self.edge_src.element_size() * 8, _lib.ptr(self.edge_dst), self.edge_dst.element_size() * 8,
-                    E, self.num_nodes, self.num_src_nodes, _lib.ptr(self.rowptr), _lib.ptr(self.perm), _lib.ptr(self.row_order),
-                    ctypes.byref(grouped), ctypes.byref(pairs), _lib.ptr(ws), ws_bytes, st,
-                )  # fmt: skip
-            )
-            # A list that is already grouped by destination (what neighbour searches emit: torch_cluster's
-            # radius_graph, which the reference's models call, returns its pairs sorted by the query node) is walked
-            # by position: the stable sort is then the identity and the kernels are handed no permutation, so that
-            # per-edge rows are read as one contiguous run per destination.
-            self.walk_perm = None if E > 1 and grouped.value else self.perm
-            if self.row_order is not None:
-                # rows that follow each other in the order and agree in their two smallest sources: next to nothing
-                # on a graph without neighbourhood structure, where the order would only scatter the rows
-                self.locality_score = pairs.value / self.num_nodes
-                if locality_order == "auto" and self.locality_score < 0.02:
-                    self.row_order = None
+        # rows that share their smallest source are processed next to each other (they share most of their
+        # sources, which then sit in L2): locality taken from the graph, not from the caller's node numbering
+        self.rowptr, self.perm, self.row_order, grouped, pairs = _lib.native().edges_build(
+            self.edge_src, self.edge_dst, self.num_nodes, self.num_src_nodes, bool(locality_order and self.num_nodes > 0)
+        )
+        # A list that is already grouped by destination (what neighbour searches emit: torch_cluster's
+        # radius_graph, which the reference's models call, returns its pairs sorted by the query node) is walked
+        # by position: the stable sort is then the identity and the kernels are handed no permutation, so that
+        # per-edge rows are read as one contiguous run per destination.
+        self.walk_perm = None if E > 1 and grouped else self.perm
+        if self.row_order is not None:
+            # rows that follow each other in the order and agree in their two smallest sources: next to nothing
+            # on a graph without neighbourhood structure, where the order would only scatter the rows
+            self.locality_score = pairs / self.num_nodes
+            if locality_order == "auto" and self.locality_score < 0.02:
+                self.row_order = None

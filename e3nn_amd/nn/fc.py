@@ -67,7 +67,39 @@ class _DenseFn:
 
     @staticmethod
     def apply(x, w, layer):
+        if layer._fwd.has_backward_w:
+            out = _lib.native().fc_layer(layer._fwd.native, layer._bwd.native, layer._scale * layer.h_out**0.5, layer, None, x, w)
+            if out is not None:
+                return out
         return _DenseSlot.apply(_G, layer, x, w)
+
+
+def _act_dense(z, w, layer, prev):
+    """``dense(act(z))`` of two consecutive layers, see ``_ActDenseFn``."""
+    fwd, bwd = layer.act_dense_plans(prev)
+    out = _lib.native().fc_layer(fwd.native, bwd.native, layer._scale * layer.h_out**0.5, layer, prev, z, w)
+    return _ActDenseFn.apply(z, w, layer, prev) if out is None else out
+
+
+def _act_dense_gradients(layer, prev, z, w, g, needs):
+    """Gradients of ``dense(act(z))`` as the differentiable composition of the activation's and the layer's own."""
+    from .activation import _GateBackwardFn
+
+    h = prev.act(z)  # differentiable in z
+    gz = _GateBackwardFn.apply(z, _DenseSlot.apply(_X, layer, w, g), prev.act) if needs[0] else None
+    return gz, _DenseSlot.apply(_WT, layer, h, g) if needs[1] else None
+
+
+def _layer_gradients(layer, prev, saved, g, needs):
+    """Differentiable gradients of a layer (``prev``: None) or of a layer behind the activation of another."""
+    x, w = saved
+    g = g.contiguous()
+    if prev is not None:
+        return _act_dense_gradients(layer, prev, x, w, g.clone() if g.data_ptr() % 16 else g, needs)
+    return _DenseSlot.apply(_X, layer, w, g) if needs[0] else None, _DenseSlot.apply(_WT, layer, x, g) if needs[1] else None
+
+
+_lib.connect({"layer_gradients": _layer_gradients})
 
 
 class _ActDenseFn(torch.autograd.Function):
@@ -93,15 +125,7 @@ class _ActDenseFn(torch.autograd.Function):
         if g.data_ptr() % 16:
             g = g.clone()
         if torch.is_grad_enabled():
-            from .activation import _GateBackwardFn
-
-            h = ctx.prev.act(z)  # differentiable in z
-            gz = gw = None
-            if ctx.needs_input_grad[0]:
-                gz = _GateBackwardFn.apply(z, _DenseSlot.apply(_X, ctx.layer, w, g), ctx.prev.act)
-            if ctx.needs_input_grad[1]:
-                gw = _DenseSlot.apply(_WT, ctx.layer, h, g)
-            return gz, gw, None, None
+            return (*_act_dense_gradients(ctx.layer, ctx.prev, z, w, g, ctx.needs_input_grad), None, None)
         gz = gw = None
         if ctx.needs_input_grad[0]:
             gz = bwd.forward(g, [(w.t() * ctx.scale).contiguous()], z)
@@ -213,16 +237,11 @@ class _FusedPlan:
         self.handle = h
         self.key = L.e3x_fc_plan_key(h).decode()
         self.workspace_bytes = L.e3x_fc_workspace_bytes(h)
+        # (owns the handle from here on)
+        self.native = _lib.native().FcPlan(h.value, hs[0], hs[-1], self.workspace_bytes)
 
     def __reduce__(self):  # copies and pickles rebuild the plan from its arguments
         return (_FusedPlan, self._args)
-
-    def __del__(self):
-        if getattr(self, "handle", None) is not None:
-            try:
-                _lib.lib().e3x_fc_plan_destroy(self.handle)
-            except Exception:
-                pass
 
     has_backward_w = False
 
@@ -295,6 +314,9 @@ class FullyConnectedNet(torch.nn.Sequential):
                 x2 = x.reshape(-1, self.hs[0]).contiguous()
                 if x2.data_ptr() % 16:
                     x2 = x2.clone()
+                out = _lib.native().fc_forward(plan.native, x2, [l.weight for l in layers])
+                if out is not None:
+                    return out.reshape(lead + (self.hs[-1],))
                 ws = [l.weight.detach().contiguous() for l in layers]
                 if all(w.is_cuda and w.dtype == torch.float32 for w in ws):
                     return plan.forward(x2, ws).reshape(lead + (self.hs[-1],))
@@ -320,7 +342,7 @@ class FullyConnectedNet(torch.nn.Sequential):
             x2 = x2.clone()
         z = _DenseFn.apply(x2, layers[0].weight, layers[0])
         for prev, layer in zip(layers, layers[1:]):
-            z = _ActDenseFn.apply(z, layer.weight, layer, prev)
+            z = _act_dense(z, layer.weight, layer, prev)
         last = layers[-1]
         if last.act is not None:
             z = last.act(z)

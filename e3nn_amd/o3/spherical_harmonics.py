@@ -99,8 +99,24 @@ class _ShBackwardFn(torch.autograd.Function):
         return gx.reshape(batch + (3,)), gg.reshape(g_shape), None, None, None
 
 
+@functools.lru_cache(maxsize=64)
+def _config(ls, normalize, normalization):
+    """The harmonics as the host path takes them."""
+    return _lib.native().Harmonics(ls, normalize, _NORMALIZATION[normalization])
+
+
+def _harmonics_gradient(x, g, ls, normalize, normalization):
+    return _sh_backward(x, g, ls, normalize, next(name for name, code in _NORMALIZATION.items() if code == normalization))
+
+
+_lib.connect({"harmonics_gradient": _harmonics_gradient})
+
+
 def _sh_forward(x, ls, normalize, normalization):
     ls = tuple(ls)
+    out = _lib.native().harmonics(_config(ls, bool(normalize), normalization), x)
+    if out is not None:
+        return out
     if _lib.unrecorded(x):
         return _forward(x, ls, normalize, normalization)
     return _SphericalHarmonicsFn.apply(x, ls, normalize, normalization)

@@ -59,7 +59,7 @@ def _num_elements(mode, m1, m2):
 
 
 class _Plan:
-    """Owner of one ``e3x_plan`` handle: a fused kernel specialised to one instruction set."""
+    """One ``e3x_plan`` handle: a fused kernel specialised to one instruction set."""
 
     _in_parts = False  # whether the scratch of a forward call depends on the batch
     _packs = True  # whether it holds repacked weights, whose kernels read rows with 16-byte loads
@@ -87,16 +87,12 @@ class _Plan:
         self.arithmetic = L.e3x_tp_plan_arithmetic(handle, 0).decode()  # which instruction forms the products
         self._in_parts = L.e3x_tp_forward_workspace_bytes(handle) > L.e3x_tp_forward_workspace_bytes_for(handle, -1)
         self._packs = L.e3x_tp_forward_workspace_bytes_for(handle, -1) > 0
+        self.native = _lib.native().Plan(  # owns the handle from here on
+            handle.value, irreps_in1.dim, self.in2_dim, self.out_dim, self.weight_numel, self._in_parts, self._packs, self.family == "uvw_node",
+            self.shared_weights, dtype == torch.bfloat16,
+        )  # fmt: skip
         self._fused_grad_w = None  # whether the plan has the message-step backward kernel; asked on first use
         self._by_destination = None  # ... and, on the forward plan, the one grouped by destination
-
-    def __del__(self):
-        try:
-            if self.handle:
-                _lib.lib().e3x_tp_plan_destroy(self.handle)
-                self.handle = None
-        except Exception:
-            pass
 
     def forward(self, x1, x2, w):
         Z = x1.shape[0]
@@ -300,9 +296,11 @@ def _w3j_swap_sign(tp, t):
 def _permuted_weights(tp, w, perm):
     """Per-instruction ``[..., U, V, W]`` weight blocks of a ``uvw`` product with their last three axes permuted: one
     gather along the weight axis through an index list built once per product, permutation and device."""
-    if tp.weight_numel == 0:
-        return w
-    key = ("weight permutation", perm, w.device)  # kept with the plans: dropped by copies and pickles alike
+    return w if tp.weight_numel == 0 else w.index_select(-1, _weight_permutation(tp, w.device, perm))
+
+
+def _weight_permutation(tp, device, perm):
+    key = ("weight permutation", perm, device)  # kept with the plans: dropped by copies and pickles alike
     index = tp._plans.get(key)
     if index is None:
         blocks, offset = [], 0
@@ -311,8 +309,8 @@ def _permuted_weights(tp, w, perm):
                 n = prod(t.path_shape)
                 blocks.append(torch.arange(offset, offset + n).view(t.path_shape).permute(*perm).reshape(-1))
                 offset += n
-        index = tp._plans[key] = torch.cat(blocks).to(w.device)
-    return w.index_select(-1, index)
+        index = tp._plans[key] = torch.cat(blocks).to(device)
+    return index
 
 
 # ---------------------------------------------------------------------------------------------------- autograd
@@ -507,21 +505,43 @@ class _GatherScatterShFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        from .spherical_harmonics import _sh_backward, _sh_forward
+        from .spherical_harmonics import _NORMALIZATION, _sh_backward, _sh_forward
 
         node_x, edge_vec, w = ctx.saved_tensors
         need1, need_vec, needw = ctx.needs_input_grad[:3]
         tp, edges = ctx.tp, ctx.edges
-        ls = tuple(range(len(tp.irreps_in2)))
         if torch.is_grad_enabled():
-            attr = _sh_forward(edge_vec, ls, *ctx.sh).to(node_x.dtype)  # differentiable in edge_vec
-            g1, g2, gw = _slot_backward(_MessageSlot, _OUT, (node_x, attr, w), g.contiguous(), (need1, need_vec, needw), tp, edges)
-            gvec = _sh_backward(edge_vec, g2.to(edge_vec.dtype), ls, *ctx.sh) if need_vec else None
-            return g1, gvec, gw, None, None, None, None
+            return (*_message_sh_gradients(tp, edges, ctx.saved_tensors, g, (need1, need_vec, needw), ctx.sh[0], _NORMALIZATION[ctx.sh[1]]), None, None, None, None)
+        ls = tuple(range(len(tp.irreps_in2)))
         attr = _sh_forward(edge_vec, ls, *ctx.sh).to(node_x.dtype)
         g1, g2, gw = _message_gradients(tp, edges, node_x, attr, w, g, need1, need_vec, needw)
         gvec = _sh_backward(edge_vec, g2.to(edge_vec.dtype), ls, *ctx.sh) if need_vec else None
         return g1, gvec, gw, None, None, None, None
+
+
+# what the nodes of the host path ask of Python: plans and weight permutations on first use, gradients that it leaves to the
+# functions above, and the backward passes that can be differentiated
+def _message_sh_gradients(tp, edges, saved, g, needs, normalize, normalization):
+    from .spherical_harmonics import _NORMALIZATION, _sh_backward, _sh_forward
+
+    node_x, edge_vec, w = saved
+    sh = (normalize, next(name for name, code in _NORMALIZATION.items() if code == normalization))
+    ls = tuple(range(len(tp.irreps_in2)))
+    attr = _sh_forward(edge_vec, ls, *sh).to(node_x.dtype)  # differentiable in edge_vec
+    g1, g2, gw = _slot_backward(_MessageSlot, _OUT, (node_x, attr, w), g.contiguous(), needs, tp, edges)
+    return g1, _sh_backward(edge_vec, g2.to(edge_vec.dtype), ls, *sh) if needs[1] else None, gw
+
+
+_lib.connect({
+    "plan": lambda tp, bf16, which: (
+        tp._plan(torch.bfloat16 if bf16 else torch.float32) if which == 0 else tp._grad_plan(("x1", "x2")[which - 1], torch.bfloat16 if bf16 else torch.float32)
+    ).native,
+    "weight_permutation": lambda tp, device, which: _weight_permutation(tp, device, ((2, 1, 0), (0, 2, 1))[which - 1]),
+    "dense_gradients": lambda tp, saved, g, needs: _slot_backward(_TpSlot, _OUT, saved, g.contiguous(), needs, tp),
+    "message_gradients": _message_gradients,
+    "message_gradients_graph": lambda tp, edges, saved, g, needs: _slot_backward(_MessageSlot, _OUT, saved, g.contiguous(), needs, tp, edges),
+    "message_sh_gradients": _message_sh_gradients,
+})  # fmt: skip
 
 
 class _Constants(torch.nn.Module):
@@ -926,6 +946,22 @@ class TensorProduct(torch.nn.Module):
             w = w.expand(batch + (-1,)).unsqueeze(-2).expand(batch + (d1, self.weight_numel))
         return self.forward(eye, yb, w if self.weight_numel else None)
 
+    def _native_plans(self):
+        """What the host path keeps of a product: ``(dense, message)``, None where a call is not of its kind."""
+        dense = self.shared_weights and self.weight_numel and self._compile_left_right and self._live_mode() == "uvw"
+        message = not self.shared_weights and self.weight_numel and self._all_uvu()
+        native = _lib.native()
+        pair = self._plans["native"] = (native.Dense() if dense else None, native.Message() if message else None)
+        return pair
+
+    def _native_message(self, edges, node_x, attr, weight, harmonics):
+        if edges is None or not isinstance(weight, torch.Tensor):
+            return None
+        native = self._plans.get("native") or self._native_plans()
+        if native[1] is None:
+            return None
+        return _lib.native().message(native[1], self, edges, edges.native(), self._in1_dim, self._in2_dim, self.weight_numel, node_x, attr, weight, harmonics)
+
     def _check_device(self, *tensors):
         for t in tensors:
             if not t.is_cuda:
@@ -934,6 +970,15 @@ class TensorProduct(torch.nn.Module):
     def forward(self, x, y, weight: Optional[Union[torch.Tensor, List[torch.Tensor]]] = None):
         r"""Evaluate :math:`w x \otimes y`: ``x[..., irreps_in1.dim]``, ``y[..., irreps_in2.dim]``,
         ``weight[weight_numel]`` (shared) or ``weight[..., weight_numel]`` -> ``[..., irreps_out.dim]``."""
+        native = self._plans.get("native")
+        if native is None:
+            native = self._native_plans()
+        if native[0] is not None:
+            w = self._parameters.get("weight") if weight is None else weight
+            if isinstance(w, torch.Tensor):
+                out = _lib.native().dense(native[0], self, self._in1_dim, self._in2_dim, self.weight_numel, x, y, w)
+                if out is not None:
+                    return out
         torch._assert(x.shape[-1] == self._in1_dim, "Incorrect last dimension for x")
         torch._assert(y.shape[-1] == self._in2_dim, "Incorrect last dimension for y")
         torch._assert(self._compile_left_right, "`left_right` method is not compiled, set `compile_left_right` to True when creating the TensorProduct")
@@ -980,6 +1025,9 @@ class TensorProduct(torch.nn.Module):
         Pass a prebuilt ``DstSortedEdges`` as ``edges`` to amortise the index preprocessing
         over several calls on the same graph.
         """
+        out = self._native_message(edges, node_x, edge_attr, weight, None)
+        if out is not None:
+            return out
         if not self._all_uvu():
             raise NotImplementedError("forward_gather_scatter needs an all-uvu TensorProduct")
         torch._assert(node_x.ndim == 2 and node_x.shape[-1] == self._in1_dim, "Incorrect shape for node_x")
@@ -1009,6 +1057,11 @@ class TensorProduct(torch.nn.Module):
         if not self._all_uvu():
             raise NotImplementedError("forward_gather_scatter_sh needs an all-uvu TensorProduct")
         assert normalization in ["integral", "component", "norm"]
+        from .spherical_harmonics import _config
+
+        out = self._native_message(edges, node_x, edge_vec, weight, _config(tuple(range(len(self.irreps_in2))), bool(normalize), normalization))
+        if out is not None:
+            return out
         torch._assert(node_x.ndim == 2 and node_x.shape[-1] == self._in1_dim, "Incorrect shape for node_x")
         torch._assert(edge_vec.shape == (edges.num_edges, 3), "edge_vec must be [num_edges, 3]")
         self._check_device(node_x, edge_vec)
