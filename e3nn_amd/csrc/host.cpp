@@ -424,8 +424,9 @@ struct MessageOp : Op {
     Tensor g1, g2, gw;
     // every gradient from one pass over the weights (as _message_gradients); other cases are Python's
     bool done = false;
-    if (need[0] && need[2] && w.size(1) > 0 && x.scalar_type() == at::kFloat) {
-      PlanPtr p = m->plan(tp, false, false);
+    if (need[0] && need[2] && w.size(1) > 0) {
+      const bool bf16 = x.scalar_type() == at::kBFloat16;
+      PlanPtr p = m->plan(tp, bf16, false);
       const size_t ws_bytes = e3x_tp_message_backward_workspace_bytes(p->h, e->num_edges);
       const EdgesPtr t = transposed();
       if (ws_bytes && p->has(p->by_destination, e3x_tp_plan_prepare_message_backward, true)) {
@@ -443,8 +444,8 @@ struct MessageOp : Op {
         }
       }
       if (!done) {
-        PlanPtr q = m->plan(tp, false, true);
-        if (q->has(q->fused_grad_w, e3x_tp_plan_prepare_gather_scatter_grad_w, false)) {
+        PlanPtr q = m->plan(tp, bf16, true);
+        if (q->has(q->fused_grad_w, e3x_tp_plan_prepare_gather_scatter_grad_w, bf16)) {
           g1 = rows_like(g, t->num_nodes, q->out_dim), gw = rows_like(g, t->num_edges, q->weight_numel);
           if (want_attr) g2 = at::empty_like(attr);
           OnDevice on(x);

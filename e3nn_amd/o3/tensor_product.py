@@ -173,10 +173,12 @@ class _Plan:
         groups by; None when the plan does not fit that kernel."""
         L = _lib.lib()
         if self._fused_grad_w is None:
+            # in bf16 storage a code object that cannot be had leaves the kernels that do the same in two passes
+            without = (_lib.ERR_INVALID,) if table.dtype == torch.float32 else (_lib.ERR_INVALID, _lib.ERR_COMPILE)
             rc = L.e3x_tp_plan_prepare_gather_scatter_grad_w(self.handle)
-            if rc != _lib.ERR_INVALID:
+            if rc not in without:
                 _lib.check(rc)
-            self._fused_grad_w = rc != _lib.ERR_INVALID
+            self._fused_grad_w = rc not in without
         if not self._fused_grad_w:
             return None
         out = torch.empty(edges.num_nodes, self.out_dim, dtype=table.dtype, device=table.device)
@@ -425,7 +427,7 @@ def _message_gradients(tp, edges, node_x, edge_attr, w, g, need1, need2, needw):
     dt = g.dtype
     g1 = g2 = gw = None
     needw = needw and tp.weight_numel > 0
-    if need1 and needw and dt == torch.float32:
+    if need1 and needw:
         # every gradient from one pass over the weights: grouped by destination where the messages are much wider than
         # the node features, else with one gather of g per edge
         res = tp._plan(dt).message_backward(node_x, edge_attr, w, g, edges, need2 and edge_attr.shape[1] > 0)
@@ -845,11 +847,11 @@ class TensorProduct(torch.nn.Module):
         self._grad_plan("x1", dtype)
         if self._live_mode() == "uvu":
             _lib.check(_lib.lib().e3x_tp_plan_prepare_backward_w(self._plan(dtype).handle))
-            if dtype == torch.float32 and not self.shared_weights and self.weight_numel:
+            if not self.shared_weights and self.weight_numel:
                 self._plan(dtype).has_message_backward()
                 # the message-step backward kernel on the transposed plan, where the instruction set fits it
                 rc = _lib.lib().e3x_tp_plan_prepare_gather_scatter_grad_w(self._grad_plan("x1", dtype).handle)
-                if rc != _lib.ERR_INVALID:
+                if rc != _lib.ERR_INVALID and (rc != _lib.ERR_COMPILE or dtype == torch.float32):
                     _lib.check(rc)
             if dtype != torch.float32 and self.shared_weights and self.weight_numel:  # summed over the batch in fp32
                 _lib.check(_lib.lib().e3x_tp_plan_prepare_backward_w(self._plan(torch.float32).handle))

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from e3nn_amd._lib import E3xError
 from e3nn_amd.nn import DstSortedEdges
 from oracle.torch_cpu import tp_forward_torch, tp_gather_scatter_torch
 from tests import kernel_sets as ks
@@ -126,6 +127,47 @@ def test_message_gradients_grouped_by_destination(maker, degrees, idx, grouped):
             assert_close(gx2, r2.numpy(), atol=1e-5 * max(1.0, float(r2.abs().max())), what="d/dedge_attr")
         again = plan.message_backward(x, a, ww, g, edges, want_x2)
         assert torch.equal(again[0], gx) and torch.equal(again[1], gw)
+
+
+@pytest.mark.parametrize("maker,one_kernel", [(lambda: ks.cfg3(True), True), (lambda: ks.cfg3(False), True), (ks.narrow_message, True), (ks.odd_mul, False),
+                                              (lambda: ks.cfg4("A"), False), (ks.ragged_wide_message, False)])  # fmt: skip
+@pytest.mark.parametrize("degrees,grouped", [([0, 1, 63, 64, 65, 0, 130, 2], True), ([300, 0, 7], False)])
+def test_message_gradients_in_bf16_storage(maker, one_kernel, degrees, grouped):
+    # one kernel for every gradient, grouped by source or by destination: against float64 on the same (rounded) inputs, with
+    # one rounding to bf16 (8 significant bits: 2^-8 of the value at most) and 1e-5 of the largest entry for the sums in fp32
+    tp = maker()
+    spec = oracle_spec(tp)
+    bf, N, E, n_src = torch.bfloat16, len(degrees), sum(degrees), 9
+    dst = torch.repeat_interleave(torch.arange(N), torch.tensor(degrees))
+    src = torch.randint(1, n_src, (E,), generator=torch.Generator().manual_seed(3))
+    if not grouped:
+        dst = dst[torch.randperm(E, generator=torch.Generator().manual_seed(4))]
+    node_x, attr, w = seeded(n_src, tp.irreps_in1.dim, seed=1).to(bf), seeded(E, tp.irreps_in2.dim, seed=2).to(bf), seeded(E, tp.weight_numel, seed=3).to(bf)
+    cot = seeded(N, tp.irreps_out.dim, seed=4).to(bf)
+    ref, grads = _oracle_grads(lambda a, b, c: tp_gather_scatter_torch(spec, a, b, c, src, dst, N), (node_x, attr, w), cot)
+
+    def close(got, want, what):
+        assert got.dtype == bf
+        err = (got.double().cpu() - want).abs() - 2**-8 * want.abs()
+        assert float(err.max()) <= 1e-5 * max(1.0, float(want.abs().max())), what
+
+    edges = DstSortedEdges(src.to(DEV), dst.to(DEV), N, n_src)
+    for with_attr in (False, True):
+        a, b, c = (t.to(DEV).requires_grad_(r) for t, r in ((node_x, True), (attr, with_attr), (w, True)))
+        out = tp.forward_gather_scatter(a, b, c, edges=edges)
+        junk = torch.full((E, tp.weight_numel), float("nan"), device=DEV, dtype=bf)  # see test_uvu_plain_gradients
+        del junk
+        if with_attr and not one_kernel:  # (shares of several kernels would be rounded one by one)
+            with pytest.raises(E3xError, match="single-kernel plan"):
+                out.backward(cot.to(DEV))
+            continue
+        out.backward(cot.to(DEV))
+        if one_kernel:  # (the matrix-core forward kernel rounds its operands too, and has a test of its own)
+            close(out.detach(), ref, "out")
+        for got, want, what in zip((a.grad, b.grad, c.grad), grads, ("d/dnode_x", "d/dedge_attr", "d/dweight")):
+            if got is not None:
+                close(got, want, what)
+        assert not a.grad[0].any()  # a source without edges
 
 
 @pytest.mark.parametrize("maker,Z", [(ks.mfma_full_tiles, 1), (ks.mfma_full_tiles, 31), (ks.mfma_full_tiles, 33), (ks.mfma_full_tiles, 400), (ks.node_block, 65)])
