@@ -247,14 +247,19 @@ int build_uvu_source(e3x_plan& P, SubKernel& K, std::string* src, bool bwd_only 
   int upl = 4;
   auto fits = [&](int u) {
     for (size_t a = 0; a < P.in1.size(); ++a) if (used1[a] && P.in1[a].mul % u) return false;
-    if (P.dtype == E3X_BF16 && u == 4 && accregs > 24) return false;  // measured: 2 per lane is faster there
+    // bf16 storage: two per lane where a wavefront then covers a row, also where four would fit (32 channels, l <= 2, 1.1 M
+    // edges, four / two per lane: forward 213 / 205 us, with all gradients 658 / 617)
+    if (P.dtype == E3X_BF16 && u == 4 && (accregs > 24 || (!bwd_only && max_mul <= 128))) return false;
     return u * (accregs + x1regs + wregs) + (int)P.in2_dim <= 200;
   };
   while (upl > 1 && !fits(upl)) upl /= 2;
   // narrow sets: a group of lanes is at least 8 wide, so fewer indices per lane keep its lanes busy (measured on
   // 500 000 edges, l <= 2: multiplicity 8 with 4 / 2 / 1 per lane 0.203 / 0.109 / 0.096 ms in fp32 and 0.485 / 0.138 /
-  // 0.085 ms in bf16 storage; multiplicity 16: 0.230 / 0.126 / 0.123 ms and 0.520 / 0.098 / 0.099 ms)
-  while (upl > 1 && max_mul / upl < 8) upl /= 2;
+  // 0.085 ms in bf16 storage; multiplicity 16: 0.230 / 0.126 / 0.123 ms and 0.520 / 0.098 / 0.099 ms); in fp32 a group of four
+  // lanes with four each reads whole 16-byte pieces (16 channels, 1.38 M edges: 256 -> 241 us; in bf16 143 -> 157)
+  const bool message = !bwd_only && (!tpl || tpl == e3x::kTplUvu);
+  const int min_lanes = message && P.dtype == E3X_F32 && upl == 4 && max_mul >= 16 ? 4 : 8;
+  while (upl > 1 && max_mul / upl < min_lanes) upl /= 2;
   upl = env_int("E3X_UVU_UPL", upl);
   // the backward kernel also holds the output gradient of its indices: one index per lane keeps it at several waves
   // per SIMD (measured on the 32-channel l <= 2 set: 1.39 ms against 1.85 ms with four)
@@ -270,7 +275,7 @@ int build_uvu_source(e3x_plan& P, SubKernel& K, std::string* src, bool bwd_only 
     if (used1[a] && P.in1[a].mul % upl) return fail(E3X_ERR_INVALID, "uvu kernel: multiplicity not divisible by UPL");
   const int lane_units = (max_mul + upl - 1) / upl;
   K.upl = upl;
-  K.lanes = lane_units > 32 ? 64 : pow2_at_least(lane_units, 8);
+  K.lanes = lane_units > 32 ? 64 : pow2_at_least(lane_units, min_lanes);
   K.chunks = (lane_units + K.lanes - 1) / K.lanes;
 
   std::ostringstream s;
@@ -364,10 +369,10 @@ int build_uvu_source(e3x_plan& P, SubKernel& K, std::string* src, bool bwd_only 
   // owns the whole output row.  Measured on the 32-channel l <= 2 set: the shuffle butterfly and the 128-byte stores
   // it replaces were 15 % of the kernel.
   {
-    bool ok = !bwd_only && !tpl && P.dtype == E3X_F32 && upl == 4 && K.lanes < 64 && K.chunks == 1 && P.out_dim % 4 == 0;
+    bool ok = !bwd_only && !tpl && upl >= 2 && K.lanes < 64 && K.chunks == 1 && P.out_dim % 4 == 0;
     for (size_t c = 0; c < P.out.size(); ++c) {
       if (P.out[c].mul == 0) continue;
-      if (!usedo[c] || P.offo[c] % 4 || P.out[c].mul % 4 || P.out[c].mul > K.lanes * upl) ok = false;
+      if (!usedo[c] || P.offo[c] % upl || P.out[c].mul % upl || P.out[c].mul > K.lanes * upl) ok = false;
     }
     const long long lds = (long long)K.waves_per_block * (64 / K.lanes) * P.out_dim * 4;
     if (ok && lds <= 49152 && env_int("E3X_UVU_LDS_REDUCE", 1)) s << "#define E3X_UVU_LDS_REDUCE 1\n";

@@ -23,7 +23,7 @@ GOLDEN_GPU_CASES = [
 BACKWARD_CASES = _ks.BACKWARD_CASES + ["uvu_merged_cfg3_like_mul4", "uvu_builderA_cfg4_like_mul2", "uvu_shared_v2", "fctp_small_cfg5_like",
                                        "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular", "zero_path_first", "zero_path_last",
                                        "dense_one_path", "node_ragged", "node_long_row", "few_channels", "few_channels_ragged",
-                                       "few_outputs", "few_outputs_per_sample"]  # fmt: skip
+                                       "few_outputs", "few_outputs_per_sample", "message_ragged_groups", "message_four_lanes"]  # fmt: skip
 BACKWARD_BF16_CASES = _ks.BACKWARD_BF16_CASES + ["uvu_shared_v2", "cfg3_builder", "cfg4_A", "odd_mul", "narrow_message", "ragged_wide_message"]
 
 
@@ -130,6 +130,16 @@ def few_outputs(per_sample=False):
     return o3.FullyConnectedTensorProduct("12x0e+7x1o", "20x0e+70x1o", "1x0e+2x1o+1x2e", **kw)
 
 
+def message_ragged_groups():
+    # 5 of the 8 lanes of a group have indices; rows summed over the groups through LDS
+    return _ks.message_tensor_product("20x0e+20x1o+20x2e", SH2, irreps_out="20x0e+20x1o+20x2e")
+
+
+def message_four_lanes():
+    # groups of four lanes whose rows are too wide to be summed through LDS
+    return _ks.message_tensor_product("16x0e+16x1o+16x2e", SH2, keep="0e+1o+2e")
+
+
 def golden_tensor_products():
     meta = golden_meta()
     return [(n, golden_tp(n, meta), (torch.float32,)) for n in GOLDEN_GPU_CASES]
@@ -143,6 +153,8 @@ def edge_case_tensor_products():
         ("node_long_row", node_long_row(), (torch.float32,)), ("few_channels", few_channels(), (torch.float32,)),
         ("few_channels_ragged", few_channels_ragged(), (torch.float32,)), ("few_outputs", few_outputs(), (torch.float32, torch.bfloat16)),
         ("few_outer_indices", few_outer_indices(), (torch.float32,)), ("few_outputs_per_sample", few_outputs(True), (torch.float32,)),
+        ("message_ragged_groups", message_ragged_groups(), (torch.float32, torch.bfloat16)),
+        ("message_four_lanes", message_four_lanes(), (torch.float32, torch.bfloat16)),
     ]  # fmt: skip
 
 

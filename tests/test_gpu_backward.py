@@ -49,7 +49,9 @@ def test_uvu_plain_gradients(maker, Z):
                                            (lambda: ks.cfg4("A"), 25, 300, torch.int32),
                                            # multiplicities that leave lane groups partly filled (80, 24, 5): every
                                            # weight-gradient column must still be written (the buffer is not zero-filled)
-                                           (ks.odd_mul, 40, 600, torch.int32), (ks.narrow_message, 60, 900, torch.int64)])  # fmt: skip
+                                           (ks.odd_mul, 40, 600, torch.int32), (ks.narrow_message, 60, 900, torch.int64),
+                                           # groups of four lanes, and of eight with some of them idle
+                                           (ks.message_ragged_groups, 30, 700, torch.int64), (ks.message_four_lanes, 30, 700, torch.int32)])  # fmt: skip
 def test_fused_message_gradients(maker, N, E, idx):
     tp = maker()
     spec = oracle_spec(tp)
@@ -130,6 +132,7 @@ def test_message_gradients_grouped_by_destination(maker, degrees, idx, grouped):
 
 
 @pytest.mark.parametrize("maker,one_kernel", [(lambda: ks.cfg3(True), True), (lambda: ks.cfg3(False), True), (ks.narrow_message, True), (ks.odd_mul, False),
+                                              (ks.message_ragged_groups, True), (ks.message_four_lanes, True),
                                               (lambda: ks.cfg4("A"), False), (ks.ragged_wide_message, False)])  # fmt: skip
 @pytest.mark.parametrize("degrees,grouped", [([0, 1, 63, 64, 65, 0, 130, 2], True), ([300, 0, 7], False)])
 def test_message_gradients_in_bf16_storage(maker, one_kernel, degrees, grouped):
