@@ -255,13 +255,13 @@ struct Plan : torch::CustomClassHolder {
   }
 
   // (as _Plan.backward_w_uvw, shared weights)
-  Tensor weight_gradient(Tensor x1, Tensor x2, Tensor g) const {
+  Tensor weight_gradient(Tensor x1, Tensor x2, Tensor g, bool bf16_values = false) const {
     Tensor gw = at::empty({weight_numel}, x1.options().requires_grad(false));
     if (!aligned(x1)) x1 = x1.clone();
     if (!aligned(x2)) x2 = x2.clone();
     if (!aligned(g)) g = g.clone();
     OnDevice on(x1);
-    check(e3x_tp_backward_w_uvw(h, in(x1), in(x2), in(g), ptr(gw), x1.size(0), stream_of(x1)));
+    check((bf16_values ? e3x_tp_backward_w_uvw_bf16_values : e3x_tp_backward_w_uvw)(h, in(x1), in(x2), in(g), ptr(gw), x1.size(0), stream_of(x1)));
     return gw;
   }
   // whether the plan has a kernel that is built on first use
@@ -319,7 +319,7 @@ struct Dense : torch::CustomClassHolder {
   Tensor grad_w(const PyRef& tp, const Tensor& x1, const Tensor& x2, const Tensor& g) {
     PlanPtr p = plan(tp, false, OUT);
     if (g.scalar_type() == at::kFloat) return p->weight_gradient(x1, x2, g);
-    return p->weight_gradient(x1.to(at::kFloat), x2.to(at::kFloat), g.to(at::kFloat)).to(g.scalar_type());
+    return p->weight_gradient(x1.to(at::kFloat), x2.to(at::kFloat), g.to(at::kFloat), g.scalar_type() == at::kBFloat16).to(g.scalar_type());
   }
 };
 using DensePtr = c10::intrusive_ptr<Dense>;

@@ -102,6 +102,10 @@ struct e3x_plan {
   // ... of products whose multiplicities are all multiples of 64: the kernel of uvw_dw_wide.inc (then `dw` is not built)
   std::unique_ptr<SubKernel> dw_wide;
   std::vector<std::pair<int, long long>> dw_wide_paths;  // per path: passes per outer index, tiles of a batch slice
+  // ... of operands that hold bf16 values (either kernel, as dw_wide / dw): built on first use, or found that it cannot be had
+  std::unique_ptr<SubKernel> dw_rounded;
+  bool dw_rounded_wide = false, dw_rounded_none = false;
+  long long dw_rounded_tiles = 0;
   // ... of node-wise layers (uvw_node): the kernel of uvw_node_dw.inc
   std::unique_ptr<SubKernel> dw_node;
   std::vector<std::pair<int, long long>> dw_node_paths;  // per path: components, tiles of a batch slice
@@ -897,7 +901,10 @@ bool mfma_dw_fits(const e3x_plan& P) {
 
 // Tables of the matrix-core weight-gradient kernel: per path the M operand is the input with the smaller l.
 
-int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
+// rounded: for operands that hold bf16 values, of which the one that goes to the matrix core as it is has no lower pieces:
+// three products in place of six, so split operands whatever the padding (64x0e+32x1o times 32x0e+32x1o+32x2e in bf16 storage,
+// forward and gradients of 31 154 rows 2278 -> 1852 us).
+int build_uvw_mfma_dw_source(e3x_plan& P, bool rounded, std::string* src) {
   bool split_operands = false;
   int obmax = 1, nrmax = 1;
   std::ostringstream s, nzs, ps;
@@ -923,10 +930,10 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
       const bool paired = pairing && c.mul == 32 && O % 2 == 0 && !synth_a;
       if (!paired && ((k_is_x2 ? b.mul : a.mul) % 64 || c.mul % 64)) full = false;
     }
-    const int split = env_int("E3X_DW_SPLIT", full ? 1 : 0);
+    const int split = env_int("E3X_DW_SPLIT", full || rounded ? 1 : 0);
     s << "#define E3X_DW_SPLIT " << split << "\n";
     split_operands = split != 0;
-    P.arithmetic_dw = split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
+    if (!rounded) P.arithmetic_dw = split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
   }
   if (std::getenv("E3X_DW_OCC")) s << "#define E3X_DW_OCC " << env_int("E3X_DW_OCC", 3) << "\n";
   int n_nz = 0, n_path = 0, dkmax = 1, drmax = 1;
@@ -966,6 +973,7 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
     tiles = std::max(tiles, (long long)((K + 63) / 64) * ((W + 63) / 64) * (O / ob));
     ++n_path;
   }
+  s << "constexpr bool BF16_VALUES = " << (rounded ? "true" : "false") << ";\n";
   s << "constexpr int WT = 64, OBMAX = " << obmax << ", NRMAX = " << nrmax << ", DKMAX = " << dkmax << ", DRMAX = " << drmax << ";\n";
   s << "struct Nz { int s, r, k; float c; };\nconstexpr int N_NZ = " << n_nz << ";\nconstexpr Nz nz[N_NZ] = {\n"
     << nzs.str() << "};\n";
@@ -973,8 +981,12 @@ int build_uvw_mfma_dw_source(e3x_plan& P, std::string* src) {
        "int nz_beg, nz_end; };\n";
   s << "constexpr int N_DPATH = " << n_path << ";\nconstexpr DPath dpaths[N_DPATH] = {\n" << ps.str() << "};\n";
   s << "}  // namespace cfg\n";
-  P.dw_tiles = tiles;
-  P.dw_paths = n_path;
+  if (rounded) {
+    P.dw_rounded_tiles = tiles;
+  } else {
+    P.dw_tiles = tiles;
+  }
+  if (P.dw_paths != n_path) P.dw_paths = n_path;
   *src = s.str() + e3x::kTplCommon + e3x::kTplPieces + e3x::kTplUvwMfmaDw;
   return E3X_OK;
 }
@@ -1000,10 +1012,10 @@ long long dw_wide_unit_jobs(const e3x_plan& P) {
 // ... so few that the batch is cut beyond what fills the chip: its slices alternate in sign
 bool dw_wide_few_tiles(const e3x_plan& P) { return 2048 / dw_wide_unit_jobs(P) > 1; }
 
-int build_uvw_dw_wide_source(e3x_plan& P, std::string* src) {
+int build_uvw_dw_wide_source(e3x_plan& P, bool rounded, std::string* src) {
   std::ostringstream s, nzs, ps;
   emit_header(s, P);
-  P.dw_wide_paths.clear();
+  std::vector<std::pair<int, long long>> path_tiles;
   int n_nz = 0;
   for (const auto& p : P.paths) {
     const e3x_irrep* ir[3] = {&P.in1[p.in1], &P.in2[p.in2], &P.out[p.out]};
@@ -1033,8 +1045,10 @@ int build_uvw_dw_wide_source(e3x_plan& P, std::string* src) {
     ps << "  {" << m << ", " << off[m] << ", " << d[m] << ", " << ir[m]->mul << ", " << n << ", " << off[n] << ", " << d[n] << ", "
        << ir[n]->mul << ", " << r << ", " << off[r] << ", " << d[r] << ", " << ir[r]->mul << ", " << (n == 2 ? "true" : "false") << ", "
        << p.woff << ", " << stride[m] << ", " << stride[n] << ", " << stride[r] << ", " << tiles << ", " << nz_beg << ", " << n_nz << "},\n";
-    P.dw_wide_paths.push_back({d[n], tiles});
+    path_tiles.push_back({d[n], tiles});
   }
+  if (P.dw_wide_paths.empty()) P.dw_wide_paths = path_tiles;  // (the same for both variants, and read without the lock by launches)
+  s << "constexpr bool BF16_VALUES = " << (rounded ? "true" : "false") << ";\n";
   s << "constexpr int DIMS[3] = {IN1_DIM, IN2_DIM, OUT_DIM};\nconstexpr bool ALTERNATE = " << (dw_wide_few_tiles(P) ? "true" : "false") << ";\n";
   s << "struct Nz { int s, r, k; float c; };\nconstexpr int N_NZ = " << n_nz << ";\nconstexpr Nz nz[N_NZ] = {\n" << nzs.str() << "};\n";
   s << "struct WPath { int m_src, m_off, dM, M, n_src, n_off, dN, N, r_src, r_off, dR, O; bool n_is_w; "
@@ -1090,7 +1104,7 @@ int prepare_mfma_dw(e3x_plan* P) {
   if (dw_wide_fits(*P)) {
     std::unique_ptr<SubKernel> K(new SubKernel);
     std::string src;
-    int rc = build_uvw_dw_wide_source(*P, &src);
+    int rc = build_uvw_dw_wide_source(*P, false, &src);
     if (!rc) rc = e3x::get_code_object("uvw_dw_wide", src, &K->key, &K->hsaco);
     if (!rc) {
       P->arithmetic_dw = "bf16 matrix instruction, six products of three-way split operands";
@@ -1102,16 +1116,37 @@ int prepare_mfma_dw(e3x_plan* P) {
   std::unique_ptr<SubKernel> K(new SubKernel);
   std::string src;
   int rc;
-  if ((rc = build_uvw_mfma_dw_source(*P, &src))) return rc;
+  if ((rc = build_uvw_mfma_dw_source(*P, false, &src))) return rc;
   if ((rc = e3x::get_code_object("uvw_mfma_dw", src, &K->key, &K->hsaco))) return rc;
   P->dw = std::move(K);
   return E3X_OK;
 }
 
-int load_dw_function(e3x_plan* P, int dev) {
+// ... and the one for operands that hold bf16 values.  Where it cannot be had (a cache made without it and E3X_NO_JIT) the
+// other one does the same.
+int prepare_mfma_dw_rounded(e3x_plan* P) {
   std::lock_guard<std::mutex> lock(P->mu);
-  SubKernel* K = P->dw_wide ? P->dw_wide.get() : P->dw.get();
-  const std::string name = P->dw_wide ? "e3x_uvw_dw_wide" : "e3x_uvw_mfma_dw";
+  if (P->dw_rounded) return E3X_OK;
+  if (P->dw_rounded_none || env_int("E3X_DW_SPLIT", 1) == 0) return E3X_ERR_COMPILE;
+  std::unique_ptr<SubKernel> K(new SubKernel);
+  std::string src;
+  const bool wide = dw_wide_fits(*P);
+  int rc = wide ? build_uvw_dw_wide_source(*P, true, &src) : build_uvw_mfma_dw_source(*P, true, &src);
+  if (!rc) rc = e3x::get_code_object(wide ? "uvw_dw_wide" : "uvw_mfma_dw", src, &K->key, &K->hsaco);
+  if (rc) {
+    P->dw_rounded_none = rc == E3X_ERR_COMPILE;
+    return rc;
+  }
+  P->dw_rounded_wide = wide;
+  P->dw_rounded = std::move(K);
+  return E3X_OK;
+}
+
+int load_dw_function(e3x_plan* P, bool rounded, int dev) {
+  std::lock_guard<std::mutex> lock(P->mu);
+  const bool wide = rounded ? P->dw_rounded_wide : P->dw_wide != nullptr;
+  SubKernel* K = rounded ? P->dw_rounded.get() : wide ? P->dw_wide.get() : P->dw.get();
+  const std::string name = wide ? "e3x_uvw_dw_wide" : "e3x_uvw_mfma_dw";
   if (K->module[dev]) return E3X_OK;
   hipModule_t mod = nullptr;
   hipError_t err = hipModuleLoad(&mod, K->hsaco.c_str());
@@ -2252,7 +2287,7 @@ extern "C" int e3x_tp_plan_prepare_backward_w(e3x_plan* P) {
 // 64x0e x 64x0e -> 64x0e, 12 000 / 50 000 / 400 000 rows: 89 / 201 / 1387 us, error against 64 bits 2.7e-7 / 3.8e-7 / 7.6e-7 of the
 // 2-norm; 24 slices at most 69 / 239 / 1826 us and 3.5e-7 / 9.0e-7 / 4.2e-6; uvw_mfma_dw.inc 94 / 270 / 1523 us and 3.1e-7 /
 // 4.2e-7 / 1.5e-6.
-static int launch_dw_wide(e3x_plan* P, int dev, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, hipStream_t st) {
+static int launch_dw_wide(e3x_plan* P, hipFunction_t fn, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, hipStream_t st) {
   auto rows_of = [](long long unit, int d) { return (unit / d + 15) / 16 * 16; };  // as in the kernel
   int unit_rows = 0, accumulate = 0;
   long long jobs = 0;
@@ -2282,7 +2317,7 @@ static int launch_dw_wide(e3x_plan* P, int dev, const void* x1, const void* x2, 
   if (accumulate && (rc = e3x::fill_zero_bytes(grad_w, (size_t)P->weight_numel * 4, st))) return rc;
   long long n_rows = Z;
   void* args[] = {(void*)&x1, (void*)&x2, (void*)&grad_out, (void*)&grad_w, (void*)&n_rows, (void*)&unit_rows, (void*)&accumulate};
-  hipError_t err = hipModuleLaunchKernel(P->dw_wide->fn_dw[dev], (unsigned)jobs, 1, 1, 256, 1, 1, 0, st, args, nullptr);
+  hipError_t err = hipModuleLaunchKernel(fn, (unsigned)jobs, 1, 1, 256, 1, 1, 0, st, args, nullptr);
   if (err != hipSuccess) return fail(E3X_ERR_HIP, std::string("e3x_tp_backward_w_uvw: launch failed: ") + hipGetErrorString(err));
   return E3X_OK;
 }
@@ -2334,8 +2369,9 @@ static int launch_node_dw(e3x_plan* P, int dev, const void* x1, const void* x2, 
   return E3X_OK;
 }
 
-extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2, const void* grad_out, void* grad_w,
-                                     int64_t Z, void* stream) {
+// rounded: every value of x1, x2 and grad_out is a bf16 value
+static int backward_w_uvw(e3x_plan* P, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, bool rounded,
+                          void* stream) {
   if (!P) return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: null plan");
   if (P->family != "uvw_small" && P->family != "uvw_mfma" && P->family != "uvw_node")
     return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: the plan must be all-uvw");
@@ -2362,11 +2398,17 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
   if (mfma) {
     if (((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)grad_out) & 15)
       return fail(E3X_ERR_INVALID, "e3x_tp_backward_w_uvw: x1, x2 and grad_out must be 16-byte aligned");
-    if ((rc = prepare_mfma_dw(P))) return rc;
-    if ((rc = load_dw_function(P, dev))) return rc;
-    if (P->dw_wide) return launch_dw_wide(P, dev, x1, x2, grad_out, grad_w, Z, st);
+    if (rounded) {
+      if ((rc = prepare_mfma_dw_rounded(P)) && rc != E3X_ERR_COMPILE) return rc;
+      rounded = rc == E3X_OK;
+    }
+    if (!rounded && (rc = prepare_mfma_dw(P))) return rc;
+    if ((rc = load_dw_function(P, rounded, dev))) return rc;
+    if (rounded ? P->dw_rounded_wide : P->dw_wide != nullptr)
+      return launch_dw_wide(P, (rounded ? P->dw_rounded : P->dw_wide)->fn_dw[dev], x1, x2, grad_out, grad_w, Z, st);
+    const long long tiles = rounded ? P->dw_rounded_tiles : P->dw_tiles;
     // batch slices: enough workgroups for a few waves of the chip, at least 256 rows each
-    const long long wgs = P->dw_tiles * P->dw_paths;
+    const long long wgs = tiles * P->dw_paths;
     long long slices = (2048 + wgs - 1) / wgs;
     slices = std::min(slices, (long long)((Z + 255) / 256));
     slices = std::max(1LL, std::min(slices, 1024LL));
@@ -2377,7 +2419,7 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
     if (accumulate && (rc = e3x::fill_zero_bytes(grad_w, (size_t)P->weight_numel * 4, st))) return rc;
     void* args[] = {(void*)&x1, (void*)&x2, (void*)&grad_out, (void*)&grad_w, (void*)&n_rows, (void*)&rows_per_slice,
                     (void*)&accumulate};
-    hipError_t err = hipModuleLaunchKernel(P->dw->fn_dw[dev], (unsigned)P->dw_tiles, (unsigned)P->dw_paths,
+    hipError_t err = hipModuleLaunchKernel((rounded ? P->dw_rounded : P->dw)->fn_dw[dev], (unsigned)tiles, (unsigned)P->dw_paths,
                                            (unsigned)slices, 256, 1, 1, 0, st, args, nullptr);
     if (err != hipSuccess)
       return fail(E3X_ERR_HIP, std::string("e3x_tp_backward_w_uvw: launch failed: ") + hipGetErrorString(err));
@@ -2421,4 +2463,22 @@ extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2
   if (err != hipSuccess)
     return fail(E3X_ERR_HIP, std::string("e3x_tp_backward_w_uvw: launch failed: ") + hipGetErrorString(err));
   return E3X_OK;
+}
+
+extern "C" int e3x_tp_backward_w_uvw(e3x_plan* P, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z, void* stream) {
+  return backward_w_uvw(P, x1, x2, grad_out, grad_w, Z, false, stream);
+}
+
+extern "C" int e3x_tp_backward_w_uvw_bf16_values(e3x_plan* P, const void* x1, const void* x2, const void* grad_out, void* grad_w, int64_t Z,
+                                                 void* stream) {
+  return backward_w_uvw(P, x1, x2, grad_out, grad_w, Z, true, stream);
+}
+
+extern "C" int e3x_tp_plan_prepare_backward_w_bf16_values(e3x_plan* P) {
+  if (!P) return fail(E3X_ERR_INVALID, "e3x_tp_plan_prepare_backward_w_bf16_values: null plan");
+  if (P->family == "uvw_mfma" && !mfma_dw_on_valu(P) && P->dtype == E3X_F32) {
+    const int rc = prepare_mfma_dw_rounded(P);
+    if (rc != E3X_ERR_COMPILE) return rc;
+  }
+  return e3x_tp_plan_prepare_backward_w(P);
 }

@@ -256,14 +256,15 @@ class _Plan:
         """Instruction of the matrix-core ``uvw`` weight gradient; "" before that kernel has been built."""
         return _lib.lib().e3x_tp_plan_arithmetic(self.handle, 1).decode()
 
-    def backward_w_uvw(self, x1, x2, grad_out, shared_weights):
+    def backward_w_uvw(self, x1, x2, grad_out, shared_weights, bf16_values=False):
+        """``bf16_values``: the (fp32) rows are widened bf16 ones."""
         shape = (self.weight_numel,) if shared_weights else (x1.shape[0], self.weight_numel)
         gw = torch.empty(shape, dtype=x1.dtype, device=x1.device)
         # the matrix-core kernel reads rows with 16-byte loads
         x1, x2, grad_out = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (x1, x2, grad_out))
         with _lib.on_device(x1.device):
             _lib.check(
-                _lib.lib().e3x_tp_backward_w_uvw(
+                (_lib.lib().e3x_tp_backward_w_uvw_bf16_values if bf16_values else _lib.lib().e3x_tp_backward_w_uvw)(
                     self.handle, _lib.ptr(x1), _lib.ptr(x2), _lib.ptr(grad_out), _lib.ptr(gw), x1.shape[0],
                     _lib.stream_ptr(x1.device),
                 )
@@ -354,7 +355,7 @@ def _tp_gradients(tp, x1, x2, w, g, need1, need2, needw):
         if needw:
             if dt != torch.float32:
                 # the weight-gradient kernels read fp32 rows: widened copies of the operands, result in storage type
-                gw = tp._plan(torch.float32).backward_w_uvw(x1.float(), x2.float(), g.float(), tp.shared_weights).to(dt)
+                gw = tp._plan(torch.float32).backward_w_uvw(x1.float(), x2.float(), g.float(), tp.shared_weights, dt == torch.bfloat16).to(dt)
             else:
                 gw = tp._plan(dt).backward_w_uvw(x1, x2, g, tp.shared_weights)
         if need1:
@@ -858,7 +859,8 @@ class TensorProduct(torch.nn.Module):
         if self._live_mode() == "uvw":
             self._grad_plan("x2", dtype)
             if self.weight_numel:  # the weight gradient always runs on the fp32 plan
-                _lib.check(_lib.lib().e3x_tp_plan_prepare_backward_w(self._plan(torch.float32).handle))
+                prepare = _lib.lib().e3x_tp_plan_prepare_backward_w_bf16_values if dtype == torch.bfloat16 else _lib.lib().e3x_tp_plan_prepare_backward_w
+                _lib.check(prepare(self._plan(torch.float32).handle))
         return self
 
     def __getstate__(self):

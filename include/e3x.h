@@ -360,6 +360,12 @@ int e3x_tp_message_backward(e3x_plan* plan, const void* node_x, const void* edge
 int e3x_tp_plan_prepare_backward_w(e3x_plan* plan);
 int e3x_tp_backward_w_uvw(e3x_plan* plan, const void* x1, const void* x2, const void* grad_out, void* grad_w,
                           int64_t Z, void* stream);
+/* The same where every value of x1, x2 and grad_out (fp32 storage) is a bf16 value, as with widened rows of bf16 storage: the
+ * matrix-core kernels then leave out the products that meet pieces which are zero.  A code object of its own, built on first use
+ * or ahead by e3x_tp_plan_prepare_backward_w_bf16_values; where it cannot be had the call above does the work. */
+int e3x_tp_plan_prepare_backward_w_bf16_values(e3x_plan* plan);
+int e3x_tp_backward_w_uvw_bf16_values(e3x_plan* plan, const void* x1, const void* x2, const void* grad_out, void* grad_w,
+                                      int64_t Z, void* stream);
 
 /* out[n, sum(2l+1 for l in ls)] = spherical harmonics of xyz[n, 3].  Replaces
  * SphericalHarmonics.forward (e3nn/o3/_spherical_harmonics.py:93-112) and the polynomial

@@ -24,7 +24,8 @@ BACKWARD_CASES = _ks.BACKWARD_CASES + ["uvu_merged_cfg3_like_mul4", "uvu_builder
                                        "fctp_per_sample_weights", "modes_uuu_uvuv_uuw_uvv", "modes_triangular", "zero_path_first", "zero_path_last",
                                        "dense_one_path", "node_ragged", "node_long_row", "few_channels", "few_channels_ragged",
                                        "few_outputs", "few_outputs_per_sample", "message_ragged_groups", "message_four_lanes"]  # fmt: skip
-BACKWARD_BF16_CASES = _ks.BACKWARD_BF16_CASES + ["uvu_shared_v2", "cfg3_builder", "cfg4_A", "odd_mul", "narrow_message", "ragged_wide_message"]
+BACKWARD_BF16_CASES = _ks.BACKWARD_BF16_CASES + ["uvu_shared_v2", "cfg3_builder", "cfg4_A", "odd_mul", "narrow_message", "ragged_wide_message",
+                                                 "mfma_full_tiles", "mfma_wide_blocks", "few_outer_indices", "unaligned_offsets", "cfg5"]  # fmt: skip
 
 
 def golden_meta():

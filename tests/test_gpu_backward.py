@@ -216,6 +216,24 @@ def test_uvw_weight_gradient_of_wide_blocks(Z):
         offset += n
 
 
+@pytest.mark.parametrize("maker", [ks.mfma_small, ks.mfma_full_tiles, ks.mfma_wide_blocks, ks.few_outer_indices, ks.unaligned_offsets])
+@pytest.mark.parametrize("Z", [1, 17, 33, 400])
+def test_uvw_weight_gradient_of_bf16_values(maker, Z):
+    # three products in place of six, of the same pieces: the bound of fp32 rows holds, path by path
+    tp = maker()
+    spec = oracle_spec(tp)
+    x1, x2, g = (seeded(Z, d, seed=i).bfloat16().float() for i, d in enumerate((tp.irreps_in1.dim, tp.irreps_in2.dim, tp.irreps_out.dim)))
+    w = torch.zeros(tp.weight_numel, dtype=torch.float64, requires_grad=True)
+    (ref,) = torch.autograd.grad(tp_forward_torch(spec, x1.double(), x2.double(), w), (w,), g.double())
+    got = tp._plan(torch.float32).backward_w_uvw(x1.to(DEV), x2.to(DEV), g.to(DEV), True, True).double().cpu()
+    offset = 0
+    for t in tp.instructions:
+        n = t.path_shape[0] * t.path_shape[1] * t.path_shape[2]
+        a, b = got[offset : offset + n], ref[offset : offset + n]
+        assert float((a - b).norm() / b.norm()) < 1e-6, t
+        offset += n
+
+
 @pytest.mark.parametrize("Z", [129, 50_003, 400_003])
 def test_uvw_weight_gradient_of_few_wide_tiles(Z):
     # 16 tiles for 512 workgroups: how many rows go into one sum decides the error
