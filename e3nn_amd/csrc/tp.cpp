@@ -651,18 +651,24 @@ int build_uvw_mfma_source(e3x_plan& P, std::string* src, bool half = false) {
   if (P.dtype != E3X_F32 || half) wt = 64;
   std::ostringstream s, nzs, ps, ts, scalar_width, parts;
   emit_header(s, P);
-  // split-operand matrix steps (see the template) in fp32 storage; weight chunks of 16 K rows then keep the LDS at
-  // 72 KB with 128 output channels (two workgroups per CU)
-  // Default where every block is a multiple of 64 wide (measured on 128-wide blocks, 65536 rows: 55.9 -> 50.0 ms);
-  // narrower blocks leave tiles half empty and keep the fp32 instruction, which needs no splitting.
-  bool full = true;
-  for (const auto& p : P.paths)
+  // split-operand matrix steps (see the template) in fp32 storage: where every block is a multiple of 64 wide (128-wide blocks,
+  // 65 536 rows: 55.9 -> 50.0 ms), in weight chunks of 16 K rows, which keep the LDS at 72 KB with 128 output channels (two
+  // workgroups per CU); and for narrower blocks up to l = 2, half empty tiles or not, in chunks of 32 rows (16: 674 and 106 us
+  // where 32 take 623 and 97).  Fp32 instruction / split, forward, input gradients, in us: 64x0e+32x1o times
+  // 32x0e+32x1o+32x2e onto 64x0e+64x1o+64x1e+64x2e, 30 000 rows 789, 898, 923 / 623, 688, 588, 3000 rows 133, 195, 159 / 97, 187,
+  // 150, 200 rows 29, 60, 37 / 27, 62, 38; 32x0e+32x1o+32x2e squared, 30 000 rows 634 / 492; error against 64 bits 1.6e-7, 3.0e-7,
+  // 1.9e-7 / 1.4e-7, 2.6e-7, 1.7e-7 of the 2-norm.  On either kind of set an infinity (and a number that rounds to one in bf16, from
+  // 3.39e38 on) makes NaN of the sums that it enters, where the fp32 instruction may leave an infinity, and of no others.
+  bool full = true, up_to_l2 = true;
+  for (const auto& p : P.paths) {
     if (P.in1[p.in1].mul % 64 || P.in2[p.in2].mul % 64 || P.out[p.out].mul % 64) full = false;
-  const int split = P.dtype == E3X_F32 ? env_int("E3X_UVW_SPLIT", full ? 1 : 0) : 0;
+    if (P.out[p.out].l > 2) up_to_l2 = false;
+  }
+  const int split = P.dtype == E3X_F32 ? env_int("E3X_UVW_SPLIT", full || up_to_l2 ? 1 : 0) : 0;
   if (split && !half) s << "#define E3X_UVW_SPLIT 1\n";
   if (!half)
     P.arithmetic = P.dtype != E3X_F32 ? "bf16 matrix instruction" : split ? "bf16 matrix instruction, six products of three-way split operands" : "fp32 matrix instruction";
-  if (P.dtype == E3X_F32 && !half) s << "#define E3X_UVW_KC " << env_int("E3X_UVW_KC", split ? 16 : 32) << "\n";
+  if (P.dtype == E3X_F32 && !half) s << "#define E3X_UVW_KC " << env_int("E3X_UVW_KC", split && full ? 16 : 32) << "\n";
   if (env_int("E3X_UVW_KS", 0)) s << "#define E3X_UVW_KS " << env_int("E3X_UVW_KS", 0) << "\n";
   // two waves per SIMD (256 registers) for 128-channel tiles and for l = 3 outputs, whose seven accumulator tiles do not
   // fit the 168 registers of three (64x1o+64x2e squared -> 32x3o: 3122 registers' worth of spills there, none here)

@@ -6,6 +6,7 @@ import torch
 
 from e3nn_amd import o3
 from oracle import tensor_product as otp
+from oracle.torch_cpu import tp_forward_torch
 from tests import kernel_sets as ks
 from tests.helpers import assert_close, oracle_spec, seeded
 
@@ -917,3 +918,23 @@ def test_provider_right_binding():
     assert mats.shape == (6, tp.irreps_in1.dim, tp.irreps_out.dim) and torch.equal(mats, tp.right(x2))
     ref = otp.tp_forward(oracle_spec(tp), x1.cpu().numpy(), x2.cpu().numpy(), tp.weight.detach().cpu().numpy())
     assert_close(torch.einsum("zi,zik->zk", x1, mats), ref, what="x @ right(y) through the provider")
+
+
+@pytest.mark.parametrize("Z", [1, 63, 65, 30_000])
+@pytest.mark.parametrize("scale", [1.0, 1e-25, 1e20])
+def test_uvw_narrow_blocks_on_split_operands(Z, scale):
+    # blocks of 32 and half-empty tiles, in parts and whole; products and input gradients keep 24 bits whatever their size
+    tp = ks.mfma_small()
+    spec = oracle_spec(tp)
+    rows = torch.unique(torch.tensor([0, Z // 2, Z - 1]))
+    x1, x2, w = seeded(Z, tp.irreps_in1.dim, seed=1) * scale, seeded(Z, tp.irreps_in2.dim, seed=2), seeded(tp.weight_numel, seed=3)
+    plan = tp._plan(torch.float32)
+    assert "split operands" in plan.arithmetic
+    got = plan.forward(x1.to(DEV), x2.to(DEV), w.to(DEV))
+    ref = tp_forward_torch(spec, x1[rows].double(), x2[rows].double(), w.double())
+    # sums of at most 64 x 32 x 25 products in fp32
+    assert float((got[rows.to(DEV)].double().cpu() - ref).norm() / ref.norm()) < 1e-6
+    if scale == 1.0:  # an infinity spoils its row, in the outputs that its irrep reaches, and nothing else
+        x1[0, 0] = float("inf")
+        bad = plan.forward(x1.to(DEV), x2.to(DEV), w.to(DEV))
+        assert torch.equal(bad[1:], got[1:]) and not torch.isfinite(bad[0, :64]).any()
