@@ -319,8 +319,9 @@ int e3x_tp_backward_w_x2(e3x_plan* plan, const void* x1, const void* x2, const v
  * wavefront are combined by a shuffle butterfly, there sometimes through LDS in another order).  grad_x2[E, in2_dim]
  * (may be NULL: not computed) is the gradient of edge_attr, summed over the multiplicity indices inside the kernel.
  * The reference obtains all of this by autograd through points_convolution.py:105-106 and the einsums of
- * e3nn/o3/_tensor_product/_codegen.py:166-187.  fp32, per-edge weights, multiplicities that one lane group of a
- * wavefront covers (instruction sets that run as several kernels over disjoint output irreps launch as many here)
+ * e3nn/o3/_tensor_product/_codegen.py:166-187.  Per-edge weights, multiplicities that one lane group of a
+ * wavefront covers (instruction sets that run as several kernels over disjoint output irreps launch as many here; in bf16
+ * storage a set has to run as one)
  * (e3x_tp_plan_prepare_gather_scatter_grad_w builds the code objects and returns E3X_ERR_INVALID, without a message,
  * for plans that do not fit); grad_w[E, weight_numel] 16-byte aligned. */
 int e3x_tp_plan_prepare_gather_scatter_grad_w(e3x_plan* plan);
@@ -339,8 +340,9 @@ int e3x_tp_gather_scatter_grad_w(e3x_plan* plan, const void* table, const void* 
  * edges: no atomics, run-to-run identical.  For messages several times as wide as the node features it moves a
  * fraction of the bytes of e3x_tp_gather_scatter_grad_w, which gathers a row of grad_out per edge.
  * e3x_tp_plan_prepare_message_backward builds the code object (no GPU needed) and returns E3X_ERR_INVALID, without a
- * message, for plans it is not meant for (fp32, per-edge weights, more than 32 channels, messages more than three times
- * as wide as the scratch row); the workspace size reads 0 then, and where it would exceed 16 GiB. */
+ * message, for plans it is not meant for (per-edge weights, more than 32 channels, messages more than three times
+ * as wide as the scratch row); the workspace size reads 0 then, and where it would exceed 16 GiB.  In bf16 storage sums and
+ * workspace are fp32, and grad_x2 is refused for sets that run as several kernels, as by e3x_tp_backward_w_x2. */
 int e3x_tp_plan_prepare_message_backward(e3x_plan* plan);
 size_t e3x_tp_message_backward_workspace_bytes(const e3x_plan* plan, int64_t E);
 int e3x_tp_message_backward(e3x_plan* plan, const void* node_x, const void* edge_attr, const void* w, const void* grad_out,
