@@ -260,8 +260,9 @@ int build_uvu_source(e3x_plan& P, SubKernel& K, std::string* src, bool bwd_only 
   // narrow sets: a group of lanes is at least 8 wide, so fewer indices per lane keep its lanes busy (measured on
   // 500 000 edges, l <= 2: multiplicity 8 with 4 / 2 / 1 per lane 0.203 / 0.109 / 0.096 ms in fp32 and 0.485 / 0.138 /
   // 0.085 ms in bf16 storage; multiplicity 16: 0.230 / 0.126 / 0.123 ms and 0.520 / 0.098 / 0.099 ms); in fp32 a group of four
-  // lanes with four each reads whole 16-byte pieces (16 channels, 1.38 M edges: 256 -> 241 us; in bf16 143 -> 157)
-  const bool message = !bwd_only && (!tpl || tpl == e3x::kTplUvu);
+  // lanes with four each reads whole 16-byte pieces (16 channels, 1.38 M edges: 256 -> 241 us; in bf16 143 -> 157), but not in
+  // the code object that also holds the product without a graph (400 000 rows 152 -> 166)
+  const bool message = !bwd_only && extra_cfg && (!tpl || tpl == e3x::kTplUvu);
   const int min_lanes = message && P.dtype == E3X_F32 && upl == 4 && max_mul >= 16 ? 4 : 8;
   while (upl > 1 && max_mul / upl < min_lanes) upl /= 2;
   upl = env_int("E3X_UVU_UPL", upl);
